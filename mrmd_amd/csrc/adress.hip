@@ -437,11 +437,8 @@ __global__ __launch_bounds__(BLOCK) void k_igTiled(IGArgs g, IGTiled tl, Pre p, 
         if (threadIdx.x == 0) partials[blk] = 0.0;
         return;
     }
-    if (threadIdx.x == 0)
-    {
-        ti = tl.tiles[blk];
-        queued = 0;
-    }
+    loadTile(ti, tl.tiles, blk);
+    if (threadIdx.x == 0) queued = 0;
     __syncthreads();
     // the first row's loads overlap the staging
     int s = -1, c = 0;

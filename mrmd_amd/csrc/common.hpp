@@ -358,15 +358,51 @@ inline void validatePred2(const mrmd_pred2* p)
 
 // ---------------------------------------------------------------------------------------
 // wave / block reductions (wave64 shuffles, then LDS across the 4 waves of a block)
+// Sums and maxima over the 64 lanes by DPP moves (register moves between lanes, no LDS
+// traffic and no address arithmetic: 3 instructions a step for a double instead of 7 with
+// shuffles): rows of 16 lanes by shifts of 1, 2, 4, 8, then lane 15 of each row into the next
+// row and lane 31 into the upper half, which leaves the result in lane 63.  Every lane of the
+// wave takes part; lanes without a source take `none`, the operation's neutral value.
+template <int CTRL, int ROWS>
+__device__ inline int dppMove(int v, int none)
+{
+    return __builtin_amdgcn_update_dpp(none, v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS>
+__device__ inline double dppMove(double v, double none)
+{
+    return __hiloint2double(dppMove<CTRL, ROWS>(__double2hiint(v), __double2hiint(none)),
+                            dppMove<CTRL, ROWS>(__double2loint(v), __double2loint(none)));
+}
+__device__ inline int lastLane(int v) { return __builtin_amdgcn_readlane(v, WAVE - 1); }
+__device__ inline double lastLane(double v)
+{
+    return __hiloint2double(lastLane(__double2hiint(v)), lastLane(__double2loint(v)));
+}
+template <class T, class Op>
+__device__ inline T waveReduce(T v, T none, Op op)
+{
+    v = op(v, dppMove<0x111, 0xf>(v, none));  // row_shr:1
+    v = op(v, dppMove<0x112, 0xf>(v, none));  // row_shr:2
+    v = op(v, dppMove<0x114, 0xf>(v, none));  // row_shr:4
+    v = op(v, dppMove<0x118, 0xf>(v, none));  // row_shr:8
+    v = op(v, dppMove<0x142, 0xa>(v, none));  // row_bcast:15 into rows 1 and 3
+    v = op(v, dppMove<0x143, 0xc>(v, none));  // row_bcast:31 into rows 2 and 3
+    return lastLane(v);
+}
 __device__ inline double waveSum(double v)
 {
-    for (int off = WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
-    return v;
+    return waveReduce(v, 0.0, [](double a, double b) { return a + b; });
 }
+// (of non-negative values)
 __device__ inline double waveMax(double v)
 {
-    for (int off = WAVE / 2; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, WAVE));
-    return v;
+    return waveReduce(v, 0.0, [](double a, double b) { return fmax(a, b); });
+}
+// (of non-negative values)
+__device__ inline int waveMaxInt(int v)
+{
+    return waveReduce(v, 0, [](int a, int b) { return max(a, b); });
 }
 // result valid in thread 0; lds holds blockDim.x / WAVE doubles (blockDim.x a multiple of WAVE, at most BLOCK)
 __device__ inline double blockSum(double v, double* lds)

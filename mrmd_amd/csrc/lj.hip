@@ -15,6 +15,7 @@
 #include <mutex>
 
 #include "nlist.hpp"
+#include "pairs.hpp"
 #include "physics.hpp"
 
 using namespace mrmd_hip;
@@ -106,137 +107,46 @@ struct TiledList
     int64_t gstageRecs; ///< records per tile slice of gstage
 };
 
-// 1/d^2 outside the cutoff made negligible with one select: the high word cleared leaves a
-// value below 2^-1022 whose square underflows to zero, so every term of the pair (f2^3, its
-// products and the force) comes out zero as from a zeroed reciprocal, with the same signs
-__device__ inline double maskReciprocal(double f2, bool in)
-{
-    const long long b = __double_as_longlong(f2);
-    return __hiloint2double(in ? int(b >> 32) : 0, int(b));
-}
-
-// Branch-free pair terms of one chunk of eight entries, written stage by stage over the
-// eight pairs so that the eight dependency chains (LDS read, distance, reciprocal, force)
-// are independent and interleave.  Padding entries (the sentinel record) and pairs beyond
-// rc get a zero factor.  CAP: the table has a capping distance, so the capped branch
-// (LennardJones.hpp:68-75) is evaluated too (single-type tables: only for the chunks where
-// a lane of the wave needs it).  Products and sums may contract to FMAs here
-// (the neighbour decision of the list is unaffected: it is made, unfused, at build time);
-// the forces then differ from the unfused CPU arithmetic by a few ulps per term.
-template <bool PRED, bool ONE, bool CAP>
-__device__ inline void ljChunk(const LJArgs& a, const Pre* tab, const Pre& p1, int ti0, const double4& pi,
-                               const void* st, const uint4 cur, double& fx, double& fy, double& fz, double& e,
-                               double& w, int& n)
+// Branch-free pair terms of four entries of a multi-type table (its records in LDS), stage by
+// stage so that the four dependency chains interleave; CAP: the table has a capping distance
+// (the capped branch per pair, LennardJones.hpp:68-75)
+template <bool PRED, bool CAP>
+__device__ inline void ljQuadTypes(const LJArgs& a, const Pre* tab, int ti0, const double4& pi, const Quad& q,
+                                   PairSums& s)
 {
 #pragma clang fp contract(fast)
-    const uint32_t wd[4] = {cur.x, cur.y, cur.z, cur.w};
-    double dx[CHUNK], dy[CHUNK], dz[CHUNK], d2[CHUNK], ty[CHUNK];
+    double dx[4], dy[4], dz[4], d2[4], frac2[4];
+    bool in[4];
+    quadDistances(pi, q, dx, dy, dz, d2);
 #pragma unroll
-    for (int u = 0; u < CHUNK; ++u)
+    for (int u = 0; u < 4; ++u)
     {
-        // single-type tables stage {x, y, z} only
-        const double4 pj = Staged<ONE>::get(st, int((wd[u >> 1] >> ((u & 1) * 16)) & 0x7fffu));
-        dx[u] = pi.x - pj.x;
-        dy[u] = pi.y - pj.y;
-        dz[u] = pi.z - pj.z;
-        ty[u] = pj.w;
-        if (PRED && !evalPred2(a.pred, pi.x, pi.y, pi.z, pj.x, pj.y, pj.z)) ty[u] = -1.0;
+        in[u] = d2[u] <= a.rcSqr;
+        if (PRED) in[u] = in[u] && evalPred2(a.pred, pi.x, pi.y, pi.z, q.x[u], q.y[u], q.z[u]);
     }
 #pragma unroll
-    for (int u = 0; u < CHUNK; ++u) d2[u] = dx[u] * dx[u] + dy[u] * dy[u] + dz[u] * dz[u];
-    double frac2[CHUNK];
+    for (int u = 0; u < 4; ++u) frac2[u] = recipNewton(d2[u]);
 #pragma unroll
-    for (int u = 0; u < CHUNK; ++u) frac2[u] = recipNewton(d2[u]);
-    auto accumulate = [&](int u, double ff, double en) {
-        // padding entries point at the sentinel record beyond every cutoff, so the cutoff test
-        // alone decides; the terms are finite for every entry and a 0 / 1 factor keeps them
-        bool in = d2[u] <= a.rcSqr;
-        if (PRED) in = in && ty[u] >= 0.0;
-        const double m = in ? 1.0 : 0.0;
+    for (int u = 0; u < 4; ++u)
+    {
+        const Pre& p = tab[ti0 + max(int(q.w[u]), 0)];
+        const double frac6 = frac2[u] * frac2[u] * frac2[u];
+        double ff = frac6 * (p.ff1 * frac6 - p.ff2) * frac2[u];
+        double en = frac6 * (p.ef1 * frac6 - p.ef2) - p.shift;
+        if (CAP && d2[u] < p.capDistSqr)
+        {
+            const double dist = sqrt(d2[u]);
+            ff = p.capCoeff / dist;
+            en = p.eCap - (dist - p.capDist) * p.capCoeff - p.shift;
+        }
+        // the terms are finite for every entry and a 0 / 1 factor keeps them
+        const double m = in[u] ? 1.0 : 0.0;
         ff *= m;
-        en *= m;
-        fx += dx[u] * ff;
-        fy += dy[u] * ff;
-        fz += dz[u] * ff;
-        e += en;
-        w += ff * d2[u];
-    };
-    if constexpr (ONE && !CAP)
-    {
-        // single-type table without capping: the reciprocal is masked (0 outside rc), and
-        // instead of each pair's energy and virial the lane keeps e = sum f6, w = sum g with
-        // g = f6 (ff1 f6 - ff2) = ff d^2, and n = pairs inside rc; the kernel turns them into
-        // energy ef1 sum f6^2 - ef2 sum f6 - shift n, sum f6^2 = (sum g + ff2 sum f6) / ff1
-#pragma unroll
-        for (int u = 0; u < CHUNK; ++u)
-        {
-            bool in = d2[u] <= a.rcSqr;
-            if (PRED) in = in && ty[u] >= 0.0;
-            const double f2 = maskReciprocal(frac2[u], in);
-            const double f6 = f2 * f2 * f2;
-            const double g = f6 * (p1.ff1 * f6 - p1.ff2);
-            const double ff = g * f2;
-            fx += dx[u] * ff;
-            fy += dy[u] * ff;
-            fz += dz[u] * ff;
-            e += f6;
-            w += g;
-            unsigned carry;  // the count takes the comparison as a carry (one add)
-            n = int(__builtin_addc(unsigned(n), 0u, unsigned(in), &carry));
-        }
-        return;
-    }
-    if constexpr (!CAP || !ONE)
-    {
-        // multi-type tables keep the capped branch per pair (the split form below would hold
-        // two table records per pair and cost occupancy)
-#pragma unroll
-        for (int u = 0; u < CHUNK; ++u)
-        {
-            const Pre& p = ONE ? p1 : tab[ti0 + max(int(ty[u]), 0)];
-            const double frac6 = frac2[u] * frac2[u] * frac2[u];
-            double ff = frac6 * (p.ff1 * frac6 - p.ff2) * frac2[u];
-            double en = frac6 * (p.ef1 * frac6 - p.ef2) - p.shift;
-            if (CAP && d2[u] < p.capDistSqr)
-            {
-                const double dist = sqrt(d2[u]);
-                ff = p.capCoeff / dist;
-                en = p.eCap - (dist - p.capDist) * p.capCoeff - p.shift;
-            }
-            accumulate(u, ff, en);
-        }
-    }
-    else
-    {
-        double ffv[CHUNK], env[CHUNK];
-        bool capped = false;
-#pragma unroll
-        for (int u = 0; u < CHUNK; ++u)
-        {
-            const Pre& p = ONE ? p1 : tab[ti0 + max(int(ty[u]), 0)];
-            const double frac6 = frac2[u] * frac2[u] * frac2[u];
-            ffv[u] = frac6 * (p.ff1 * frac6 - p.ff2) * frac2[u];
-            env[u] = frac6 * (p.ef1 * frac6 - p.ef2) - p.shift;
-            capped = capped || d2[u] < p.capDistSqr;
-        }
-        // pairs inside the capping distance are rare: the capped form runs, by selects over
-        // the chunk, only where some lane of the wave has one
-        if (__any(capped))
-        {
-            // keeps the block a branch: the compiler would otherwise evaluate it every chunk
-            asm volatile("" ::: "memory");
-#pragma unroll
-            for (int u = 0; u < CHUNK; ++u)
-            {
-                const Pre& p = ONE ? p1 : tab[ti0 + max(int(ty[u]), 0)];
-                const double dist = sqrt(d2[u]);
-                const bool c = d2[u] < p.capDistSqr;
-                ffv[u] = c ? p.capCoeff / dist : ffv[u];
-                env[u] = c ? p.eCap - (dist - p.capDist) * p.capCoeff - p.shift : env[u];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < CHUNK; ++u) accumulate(u, ffv[u], env[u]);
+        s.fx += dx[u] * ff;
+        s.fy += dy[u] * ff;
+        s.fz += dz[u] * ff;
+        s.e += en * m;
+        s.w += ff * d2[u];
     }
 }
 
@@ -245,17 +155,17 @@ __device__ inline void ljChunk(const LJArgs& a, const Pre* tab, const Pre& p1, i
 // GS: the neighbourhood is staged in the tile's slice of the list's global staging buffer
 // (dense inputs whose tiles exceed the LDS) instead of LDS
 template <bool PRED, bool ONE, bool CAP, bool ASSIGN = false, bool GS = false>
-__global__ __launch_bounds__(BLOCK) void k_ljTiled(LJArgs a, TiledList tl, Pre p1, double* partials)
+__global__ __launch_bounds__(BLOCK, PRED || (CAP && !ONE) ? 2 : 4) void k_ljTiled(LJArgs a, TiledList tl, Pre p1, double* partials)
 {
     extern __shared__ double4 stLds[];
     __shared__ Pre tab[ONE ? 1 : MAX_TYPES2];
     __shared__ TileInfo ti;
     __shared__ double red[BLOCK / WAVE];
     const unsigned blk = xcdBlock();
-    double4* const st = GS ? tl.gstage + int64_t(blk) * tl.gstageRecs : stLds;
+    const Stage<ONE> st(GS ? tl.gstage + int64_t(blk) * tl.gstageRecs : stLds, sentinelSlot(tl.maxStaged) + 1);
     if (!ONE)
         for (int t = threadIdx.x; t < a.nt2; t += blockDim.x) tab[t] = a.table[t];
-    if (threadIdx.x == 0) ti = tl.tiles[blk];
+    loadTile(ti, tl.tiles, blk);
     __syncthreads();
     // the first row's global loads (count, index, position, first index chunk) are issued
     // before the staging so that their latency overlaps it
@@ -272,14 +182,25 @@ __global__ __launch_bounds__(BLOCK) void k_ljTiled(LJArgs a, TiledList tl, Pre p
         pi = tl.sortedPos[s];
         cur = reinterpret_cast<const uint4*>(tl.nbr)[s];
     }
-    stageTile<ONE>(ti, tl.sortedPos, st);
-    putSentinel<ONE>(st, tl.maxStaged, tl.sentinel, 0.0);
+    stageTile(ti, tl.sortedPos, st);
+    putSentinel(st, tl.maxStaged, tl.sentinel, 0.0);
     __syncthreads();
-    double e = 0.0, w = 0.0;
-    int n = 0;
-    for (int t = threadIdx.x; t < ti.nrows; t += blockDim.x)
+    PairSums sum;
+    auto pairs = [&](const Quad& q, const double4& pi, int ti0) {
+        if constexpr (ONE)
+            ljQuadOne<CAP>(p1, a.rcSqr, pi, q, sum, [&](int u) {
+                return !PRED || evalPred2(a.pred, pi.x, pi.y, pi.z, q.x[u], q.y[u], q.z[u]);
+            });
+        else
+            ljQuadTypes<PRED, CAP>(a, tab, ti0, pi, q, sum);
+    };
+    // (a wave's lanes take their rows together: the pair count needs every lane at the end of a
+    // round)
+    for (int t0 = int(threadIdx.x) & ~(WAVE - 1); t0 < ti.nrows; t0 += blockDim.x)
     {
-        if (t != int(threadIdx.x))
+        const int t = t0 + int(threadIdx.x) % WAVE;
+        const bool live = t < ti.nrows;
+        if (live && t != int(threadIdx.x))
         {
             int self;
             s = tileRow(ti, t, self);
@@ -288,37 +209,29 @@ __global__ __launch_bounds__(BLOCK) void k_ljTiled(LJArgs a, TiledList tl, Pre p
             pi = tl.sortedPos[s];
             cur = reinterpret_cast<const uint4*>(tl.nbr)[s];
         }
-        if ((!ASSIGN && c == 0) || i >= a.rows) continue;
-        const int ti0 = ONE ? 0 : int(pi.w) * a.typeStride;
-        double fx = 0.0, fy = 0.0, fz = 0.0;
-        const uint4* chunk = reinterpret_cast<const uint4*>(tl.nbr) + s;
-        const int nch = (c + CHUNK - 1) / CHUNK;
-        for (int ch = 0; ch < nch; ++ch)
+        if (live && i < a.rows && (ASSIGN || c > 0))
         {
-            uint4 nxt = cur;
-            if (ch + 1 < nch) nxt = chunk[int64_t(ch + 1) * tl.strideS];
-            ljChunk<PRED, ONE, CAP>(a, tab, p1, ti0, pi, st, cur, fx, fy, fz, e, w, n);
-            cur = nxt;
+            const int ti0 = ONE ? 0 : int(pi.w) * a.typeStride;
+            sum.startRow();
+            walkRow<ONE && !CAP && !PRED>(st, reinterpret_cast<const uint4*>(tl.nbr) + s, tl.strideS, c, cur,
+                                          [&](const Quad& q) { pairs(q, pi, ti0); });
+            if (ASSIGN)
+            {
+                a.force[i] = 0.0 + sum.fx;
+                a.force[a.cap + i] = 0.0 + sum.fy;
+                a.force[2 * a.cap + i] = 0.0 + sum.fz;
+            }
+            else
+            {
+                a.force[i] += sum.fx;
+                a.force[a.cap + i] += sum.fy;
+                a.force[2 * a.cap + i] += sum.fz;
+            }
         }
-        if (ASSIGN)
-        {
-            a.force[i] = 0.0 + fx;
-            a.force[a.cap + i] = 0.0 + fy;
-            a.force[2 * a.cap + i] = 0.0 + fz;
-        }
-        else
-        {
-            a.force[i] += fx;
-            a.force[a.cap + i] += fy;
-            a.force[2 * a.cap + i] += fz;
-        }
+        if constexpr (ONE) sum.endRound();
     }
-    if constexpr (ONE && !CAP)
-    {
-        // e = sum f6, w = sum g over this lane's pairs (see ljChunk)
-        const double s12 = p1.ff1 != 0.0 ? (w + p1.ff2 * e) / p1.ff1 : 0.0;
-        e = p1.ef1 * s12 - p1.ef2 * e - p1.shift * double(n);
-    }
+    double e = sum.e, w = sum.w;
+    if constexpr (ONE) sum.finish<CAP>(p1, e, w);
     // every pair is visited from both ends: E = 1/2 sum, W = -1/2 sum(ff d2) / 2
     e = blockSum(0.5 * e, red);
     w = blockSum(-0.25 * w, red);
@@ -749,7 +662,7 @@ bool ljApplyImpl(mrmd_lj* lj, mrmd_atoms* at, mrmd_verlet_list* vl, const mrmd_p
             const Pre p1 = lj->table[0];
             const bool one = lj->table.size() == 1;
             const size_t lds = size_t(sentinelSlot(vl->maxStaged) + 1) *
-                               (one ? Staged<true>::bytes : Staged<false>::bytes);
+                               (one ? Stage<true>::bytes : Stage<false>::bytes);
             const dim3 g(grid), b(vl->block);
             bool cap = false;
             for (const auto& p : lj->table) cap = cap || p.capDistSqr > 0.0;
@@ -891,7 +804,7 @@ int mrmd_lj_apply_noalloc(mrmd_lj* lj, mrmd_atoms* at, mrmd_verlet_list* vl, dou
         const bool one = lj->table.size() == 1;
         bool cap = false;
         for (const auto& q : lj->table) cap = cap || q.capDistSqr > 0.0;
-        const size_t lds = size_t(sentinelSlot(vl->maxStaged) + 1) * (one ? Staged<true>::bytes : Staged<false>::bytes);
+        const size_t lds = size_t(sentinelSlot(vl->maxStaged) + 1) * (one ? Stage<true>::bytes : Stage<false>::bytes);
         const dim3 g(unsigned(vl->ntiles)), b(vl->block);
         auto launch2 = [&](auto kernel, auto kernelGS) {
             if (vl->globalStage)

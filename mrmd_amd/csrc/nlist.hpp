@@ -106,11 +106,19 @@ struct TileInfo
     int32_t selfRange[MAX_SELF], selfBegin[MAX_SELF], selfPrefix[MAX_SELF + 1];
 };
 
+// the tile's description into LDS, one word per lane
+__device__ inline void loadTile(TileInfo& ti, const TileInfo* tiles, int64_t t)
+{
+    constexpr int words = sizeof(TileInfo) / sizeof(int32_t);
+    const int32_t* src = reinterpret_cast<const int32_t*>(tiles + t);
+    for (int k = threadIdx.x; k < words; k += blockDim.x) reinterpret_cast<int32_t*>(&ti)[k] = src[k];
+}
+
 // sorted slot of the t-th row of a tile (its columns' rows one column after the other)
 __device__ inline int tileRow(const TileInfo& ti, int t, int& self)
 {
     int r = 0;
-    while (r + 1 < ti.nself && ti.selfPrefix[r + 1] <= t) ++r;
+    for (int q = 1; q < ti.nself; ++q) r += t >= ti.selfPrefix[q] ? 1 : 0;
     self = r;
     return ti.selfBegin[r] + (t - ti.selfPrefix[r]);
 }
@@ -157,6 +165,38 @@ struct Staged<false>
     __device__ static double4 get(const void* st, int q) { return static_cast<const double4*>(st)[q]; }
 };
 
+// The staged records of the force kernels: {x, y} pairs, then {z} (XYZ, 24 bytes a record, where
+// the kernel needs positions only) or {z, w} pairs (32 bytes, w = type or slab weight), each
+// array of `cap` records.  A neighbour is one 16-byte and one 8-byte read (or two 16-byte
+// ones): random gathers of 64 lanes take 19.7 LDS cycles per neighbour in this form, against
+// 32.0 for {x, y, z} records of 24 bytes, whose x and y come as one two-address read
+// (measured with 16 waves per CU; records a few places apart 14.6 against 22.6), and the LDS
+// pipe is what bounds the uncapped force kernel (with every lane reading one address it
+// runs in half the time).
+template <bool XYZ>
+struct Stage
+{
+    static constexpr int bytes = XYZ ? 24 : 32;
+    double2* xy;
+    double* z;
+    __device__ Stage(void* base, int64_t cap) : xy(static_cast<double2*>(base)), z(reinterpret_cast<double*>(xy + cap)) {}
+    __device__ void put(int q, const double4& v) const
+    {
+        xy[q] = make_double2(v.x, v.y);
+        if (XYZ)
+            z[q] = v.z;
+        else
+            reinterpret_cast<double2*>(z)[q] = make_double2(v.z, v.w);
+    }
+    __device__ double4 get(int q) const
+    {
+        const double2 a = xy[q];
+        if (XYZ) return make_double4(a.x, a.y, z[q], 0.0);
+        const double2 b = reinterpret_cast<const double2*>(z)[q];
+        return make_double4(a.x, a.y, b.x, b.y);
+    }
+};
+
 // Rows are padded to whole chunks with a sentinel entry: the LDS slot just past the largest
 // staged neighbourhood of the list, which every tiled force kernel fills with a record at
 // (c, c, c), c = the largest upper grid bound + SENTINEL_GAP + 4 r_n (the list's
@@ -168,6 +208,11 @@ template <bool XYZ>
 __device__ inline void putSentinel(void* st, int32_t maxStaged, double coord, double w)
 {
     if (threadIdx.x == 0) Staged<XYZ>::put(st, sentinelSlot(maxStaged), make_double4(coord, coord, coord, w));
+}
+template <bool XYZ>
+__device__ inline void putSentinel(const Stage<XYZ>& st, int32_t maxStaged, double coord, double w)
+{
+    if (threadIdx.x == 0) st.put(sentinelSlot(maxStaged), make_double4(coord, coord, coord, w));
 }
 
 // Sort the records of one cell by (z, record index) in a group of 32 lanes (half a wave):
@@ -297,31 +342,51 @@ __device__ inline void sortCellByZ(int32_t* recs, int n, const double4* __restri
     }
 }
 
-// copy the tile's neighbourhood (contiguous runs of sorted slots) into LDS; the copy is
-// unrolled so that four independent loads per lane are in flight
+// copy the tile's neighbourhood (contiguous runs of sorted slots) into LDS: each wave takes
+// every fourth run, four runs at a time, so that run starts and lengths are wave-uniform
+// (scalar) and a lane has four independent loads in flight; looking up the run of each record
+// instead took a tenth of the force kernel's vector instructions
+template <class Put>
+__device__ inline void stageRecords(const TileInfo& ti, const double4* __restrict__ sortedPos, Put put)
+{
+    constexpr int U = 4;
+    const int lane = int(threadIdx.x) % WAVE, waves = int(blockDim.x) / WAVE;
+    for (int r0 = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE); r0 < ti.nr; r0 += U * waves)
+    {
+        int begin[U], base[U], len[U], most = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+        {
+            const int r = r0 + u * waves;
+            const bool in = r < ti.nr;
+            const int rr = in ? r : 0;
+            begin[u] = __builtin_amdgcn_readfirstlane(ti.begin[rr]);
+            base[u] = __builtin_amdgcn_readfirstlane(ti.base[rr]);
+            const int end = __builtin_amdgcn_readfirstlane(rr + 1 < ti.nr ? ti.base[rr + 1] : ti.staged);
+            len[u] = in ? end - base[u] : 0;
+            most = max(most, len[u]);
+        }
+        for (int k = lane; k < most; k += WAVE)
+        {
+            double4 v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (k < len[u]) v[u] = sortedPos[begin[u] + k];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (k < len[u]) put(base[u] + k, v[u]);
+        }
+    }
+}
 template <bool XYZ>
 __device__ inline void stageTile(const TileInfo& ti, const double4* __restrict__ sortedPos, void* st)
 {
-    int r = 0;
-    const int step = blockDim.x;
-    auto source = [&](int q) -> int {
-        if (q >= ti.staged) return -1;
-        while (r + 1 < ti.nr && ti.base[r + 1] <= q) ++r;
-        return ti.begin[r] + (q - ti.base[r]);
-    };
-    for (int q0 = threadIdx.x; q0 < ti.staged; q0 += 4 * step)
-    {
-        const int i0 = source(q0), i1 = source(q0 + step), i2 = source(q0 + 2 * step), i3 = source(q0 + 3 * step);
-        double4 v0, v1, v2, v3;
-        v0 = sortedPos[i0];
-        if (i1 >= 0) v1 = sortedPos[i1];
-        if (i2 >= 0) v2 = sortedPos[i2];
-        if (i3 >= 0) v3 = sortedPos[i3];
-        Staged<XYZ>::put(st, q0, v0);
-        if (i1 >= 0) Staged<XYZ>::put(st, q0 + step, v1);
-        if (i2 >= 0) Staged<XYZ>::put(st, q0 + 2 * step, v2);
-        if (i3 >= 0) Staged<XYZ>::put(st, q0 + 3 * step, v3);
-    }
+    stageRecords(ti, sortedPos, [&](int q, const double4& v) { Staged<XYZ>::put(st, q, v); });
+}
+template <bool XYZ>
+__device__ inline void stageTile(const TileInfo& ti, const double4* __restrict__ sortedPos, const Stage<XYZ>& st)
+{
+    stageRecords(ti, sortedPos, [&](int q, const double4& v) { st.put(q, v); });
 }
 }  // namespace mrmd_hip
 

@@ -52,13 +52,6 @@ __device__ inline int64_t tileOfCell(const TileGeom& tg, int cell)
 }
 
 // one thread per tile: row ranges, neighbourhood column ranges and their LDS bases
-// the maximum of v over the 64 lanes of the wave (every lane active)
-__device__ inline int waveMaxInt(int v)
-{
-    for (int off = WAVE / 2; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, WAVE));
-    return v;
-}
-
 __device__ void tileSetup(const TileGeom& tg, int64_t t, const int32_t* offsets, const int32_t* counts,
                           TileInfo* tiles, int& stagedOut);
 
@@ -257,7 +250,7 @@ __global__ __launch_bounds__(BLOCK) void k_verletTiled(const double4* __restrict
     const int cz = tg.K + 2 * R + 1;
     int* cstart = GS ? reinterpret_cast<int*>(stRaw)
                      : reinterpret_cast<int*>(reinterpret_cast<double*>(stRaw) + 3 * (int64_t(stagedCap) + STAGE_PAD));
-    if (threadIdx.x == 0) ti = tiles[t];
+    loadTile(ti, tiles, t);
     __syncthreads();
     if (ti.nrows == 0) return;
     int i0, j0, k0, k1;
