@@ -261,7 +261,7 @@ __device__ inline int stagedSlot(const TileInfo& ti, int q)
 // pair terms of one chunk of eight entries (single-type table).  Returns the mask of
 // entries that pair the row with a flagged non-row partner.
 template <bool CAP>
-__device__ inline uint32_t igChunk(const IGArgs& g, const Pre& p, const double4& pi, const double4* st,
+__device__ inline uint32_t igChunk(const IGArgs& g, const Pre& p, const double4& pi, const Stage<false>& st,
                                    const uint4 cur, double& fx, double& fy, double& fz, double& ew, double& v)
 {
 #pragma clang fp contract(fast)
@@ -272,7 +272,7 @@ __device__ inline uint32_t igChunk(const IGArgs& g, const Pre& p, const double4&
     for (int u = 0; u < CHUNK; ++u)
     {
         const uint32_t e = (wd[u >> 1] >> ((u & 1) * 16)) & 0xffffu;
-        const double4 pj = st[e & 0x7fffu];
+        const double4 pj = st.at(e & 0x7fffu);
         dx[u] = pi.x - pj.x;
         dy[u] = pi.y - pj.y;
         dz[u] = pi.z - pj.z;
@@ -347,11 +347,11 @@ __device__ inline uint32_t igChunk(const IGArgs& g, const Pre& p, const double4&
 // molecule and its compensation sample (LJ_IdealGas.cpp:120-190), by atomics
 template <bool CAP>
 __device__ inline void igRemotePair(const IGArgs& g, const IGTiled& tl, const TileInfo& ti, const Pre& p,
-                                    const double4& pi, const double4* st, int q)
+                                    const double4& pi, const Stage<false>& st, uint32_t q)
 {
     const MolView& M = g.m;
     const AtomsView& A = g.a;
-    const double4 pj = st[q];
+    const double4 pj = st.at(q);
     const double lam = fabs(pj.w);
     const double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
     const double d2 = dx * dx + dy * dy + dz * dz;
@@ -370,7 +370,7 @@ __device__ inline void igRemotePair(const IGArgs& g, const IGTiled& tl, const Ti
         en = frac6 * (p.ef1 * frac6 - p.ef2) - p.shift;
     }
     const double ffw = ff * (0.5 * (pi.w + lam));
-    const int32_t k = tl.sorted[stagedSlot(ti, q)];
+    const int32_t k = tl.sorted[stagedSlot(ti, int(q >> 3))];
     const int64_t b = M.offset[k];
     atomicAddD(&A.force[b], -(dx * ffw));
     atomicAddD(&A.force[A.cap + b], -(dy * ffw));
@@ -395,7 +395,7 @@ __device__ inline void igRemotePair(const IGArgs& g, const IGTiled& tl, const Ti
 // its entries (used once the workgroup's queue of such pairs is full)
 template <bool CAP>
 __device__ void igRemoteRow(const IGArgs& g, const IGTiled& tl, const TileInfo& ti, const Pre& p,
-                            const double4& pi, const double4* st, int s, int c, int ch0)
+                            const double4& pi, const Stage<false>& st, int s, int c, int ch0)
 {
     const uint4* chunk = reinterpret_cast<const uint4*>(tl.nbr) + s;
     for (int ch = ch0; ch * CHUNK < c; ++ch)
@@ -405,8 +405,8 @@ __device__ void igRemoteRow(const IGArgs& g, const IGTiled& tl, const TileInfo& 
         for (int u = 0; u < CHUNK && ch * CHUNK + u < c; ++u)
         {
             const uint32_t e = (wd[u >> 1] >> ((u & 1) * 16)) & 0xffffu;
-            const int q = int(e & 0x7fffu);
-            const double4 pj = st[q];
+            const uint32_t q = e & 0x7fffu;
+            const double4 pj = st.at(q);
             if (!(e & 0x8000u) || !signbit(pj.w)) continue;
             const double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
             const double d2 = dx * dx + dy * dy + dz * dz;
@@ -422,10 +422,10 @@ constexpr uint32_t IG_SKIP = 0xffffffffu;  // a queue slot reserved by a reserva
 template <bool CAP>
 __global__ __launch_bounds__(BLOCK) void k_igTiled(IGArgs g, IGTiled tl, Pre p, double* partials)
 {
-    extern __shared__ double4 st[];
+    extern __shared__ double4 stLds[];
     __shared__ TileInfo ti;
     __shared__ double red[BLOCK / WAVE];
-    __shared__ uint32_t queue[IG_QUEUE];  // LDS slot of the row << 16 | LDS slot of the partner
+    __shared__ uint32_t queue[IG_QUEUE];  // LDS slot x 8 of the row << 16 | LDS slot x 8 of the partner
     __shared__ int queued;
     // consecutive tiles go to different XCDs: the pair work sits in the tiles of the
     // atomistic and hybrid slab, one contiguous range of tile indices, which an
@@ -454,13 +454,14 @@ __global__ __launch_bounds__(BLOCK) void k_igTiled(IGArgs g, IGTiled tl, Pre p, 
         pi = tl.igPos[s];
         cur = reinterpret_cast<const uint4*>(tl.nbr)[s];
     }
-    stageTile<false>(ti, tl.igPos, st);
-    putSentinel<false>(st, tl.maxStaged, tl.sentinel, 0.0);
+    const Stage<false> st(stLds, sentinelSlot(tl.maxStaged) + 1);
+    stageTile(ti, tl.igPos, st);
+    putSentinel(st, tl.maxStaged, tl.sentinel, 0.0);
     __syncthreads();
     // a neighbourhood of coarse-grained molecules only (lambda_mod = 0 everywhere) has no
     // pair work (LJ_IdealGas.cpp:95), no drift and no compensation term
     int busy = 0;
-    for (int q = threadIdx.x; q < ti.staged; q += blockDim.x) busy |= st[q].w != 0.0;
+    for (int q = threadIdx.x; q < ti.staged; q += blockDim.x) busy |= st.at(8 * q).w != 0.0;
     if (!__syncthreads_or(busy))
     {
         if (threadIdx.x == 0) partials[blk] = 0.0;
@@ -484,7 +485,7 @@ __global__ __launch_bounds__(BLOCK) void k_igTiled(IGArgs g, IGTiled tl, Pre p, 
             tileRow(ti, t, self);
         if (c == 0 || i >= tl.rowsEnd) continue;
         // the row's own record sits in its column's staged range
-        const uint32_t ownSlot = uint32_t(ldsSlot(ti, ti.selfRange[self], s));
+        const uint32_t ownSlot = 8 * uint32_t(ldsSlot(ti, ti.selfRange[self], s));
         double fx = 0.0, fy = 0.0, fz = 0.0, v = 0.0;
         const uint4* chunk = reinterpret_cast<const uint4*>(tl.nbr) + s;
         const int nch = (c + CHUNK - 1) / CHUNK;
@@ -542,7 +543,7 @@ __global__ __launch_bounds__(BLOCK) void k_igTiled(IGArgs g, IGTiled tl, Pre p, 
     {
         const uint32_t item = queue[k];
         if (item == IG_SKIP) continue;
-        igRemotePair<CAP>(g, tl, ti, p, st[item >> 16], st, int(item & 0x7fffu));
+        igRemotePair<CAP>(g, tl, ti, p, st.at(item >> 16), st, item & 0x7fffu);
     }
     eTile = blockSum(eTile, red);
     if (threadIdx.x == 0) partials[blk] = eTile;
@@ -918,7 +919,7 @@ int mrmd_ljig_run(mrmd_lj_idealgas* s, mrmd_molecules* m, mrmd_verlet_list* vl, 
         const IGTiled tl{vl->nbr16.p, vl->cnt16.p, vl->strideS, vl->tiles.p, vl->bin.sorted.p, s->igPos.p, rows,
                          s->queueCap, vl->maxStaged, vl->sentinel, vl->banded ? vl->tileSkip.p : nullptr};
         const Pre p = s->table[0];
-        const size_t lds = size_t(sentinelSlot(vl->maxStaged) + 1) * sizeof(double4);
+        const size_t lds = Stage<false>::bytes(sentinelSlot(vl->maxStaged) + 1);
         if (p.capDistSqr > 0.0)
             hipLaunchKernelGGL(k_igTiled<true>, dim3(grid), dim3(vl->block), lds, ctx->stream, g, tl, p, part);
         else

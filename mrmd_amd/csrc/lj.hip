@@ -213,7 +213,7 @@ __global__ __launch_bounds__(BLOCK, PRED || (CAP && !ONE) ? 2 : 4) void k_ljTile
         {
             const int ti0 = ONE ? 0 : int(pi.w) * a.typeStride;
             sum.startRow();
-            walkRow<ONE && !CAP && !PRED>(st, reinterpret_cast<const uint4*>(tl.nbr) + s, tl.strideS, c, cur,
+            walkRow<ONE && !CAP && !PRED, GS>(st, reinterpret_cast<const uint4*>(tl.nbr) + s, tl.strideS, c, cur,
                                           [&](const Quad& q) { pairs(q, pi, ti0); });
             if (ASSIGN)
             {
@@ -661,8 +661,8 @@ bool ljApplyImpl(mrmd_lj* lj, mrmd_atoms* at, mrmd_verlet_list* vl, const mrmd_p
                                vl->globalStage ? vl->gstage.p : nullptr, vl->gstageRecs};
             const Pre p1 = lj->table[0];
             const bool one = lj->table.size() == 1;
-            const size_t lds = size_t(sentinelSlot(vl->maxStaged) + 1) *
-                               (one ? Stage<true>::bytes : Stage<false>::bytes);
+            const int64_t recs = sentinelSlot(vl->maxStaged) + 1;
+            const size_t lds = one ? Stage<true>::bytes(recs) : Stage<false>::bytes(recs);
             const dim3 g(grid), b(vl->block);
             bool cap = false;
             for (const auto& p : lj->table) cap = cap || p.capDistSqr > 0.0;
@@ -804,7 +804,8 @@ int mrmd_lj_apply_noalloc(mrmd_lj* lj, mrmd_atoms* at, mrmd_verlet_list* vl, dou
         const bool one = lj->table.size() == 1;
         bool cap = false;
         for (const auto& q : lj->table) cap = cap || q.capDistSqr > 0.0;
-        const size_t lds = size_t(sentinelSlot(vl->maxStaged) + 1) * (one ? Stage<true>::bytes : Stage<false>::bytes);
+        const int64_t recs = sentinelSlot(vl->maxStaged) + 1;
+            const size_t lds = one ? Stage<true>::bytes(recs) : Stage<false>::bytes(recs);
         const dim3 g(unsigned(vl->ntiles)), b(vl->block);
         auto launch2 = [&](auto kernel, auto kernelGS) {
             if (vl->globalStage)

@@ -126,48 +126,21 @@ __device__ inline int tileRow(const TileInfo& ti, int t, int& self)
 // LDS slot of sorted slot s that lies in staged range r of the tile
 __device__ inline int ldsSlot(const TileInfo& ti, int r, int s) { return ti.base[r] + (s - ti.begin[r]); }
 
-// Neighbour entries are 16-bit LDS slots stored in chunks of 8 per row: entry k of sorted
+// Neighbour entries are 16-bit words stored in chunks of 8 per row: entry k of sorted
 // slot s sits at ((k / 8) * strideS + s) * 8 + k % 8, so one 16-byte load per lane brings
 // 8 entries and a wave's load is 1 KB contiguous.
 constexpr int CHUNK = 8;
+// An entry's low 15 bits: the LDS slot times 8 (slots stay below 4096, and the force kernels
+// use the product as a byte offset), or the slot itself where tiles stage in global memory
+// (slots up to 32766); bit 15 is the half-list flag.
+__host__ __device__ constexpr int entryShift(bool globalStage) { return globalStage ? 0 : 3; }
 __host__ __device__ inline int64_t entryIndex(int64_t k, int64_t s, int64_t strideS)
 {
     return ((k >> 3) * strideS + s) * CHUNK + (k & 7);
 }
 
-// A staged LDS record: {x, y, z} (24 bytes) where the kernel needs positions only, the full
-// {x, y, z, type} record (32 bytes) where it needs the type.  The smaller record fits more
-// workgroups into a CU's LDS.
-template <bool XYZ>
-struct Staged;
-template <>
-struct Staged<true>
-{
-    static constexpr int bytes = 24;
-    __device__ static void put(void* st, int q, const double4& v)
-    {
-        double* p = static_cast<double*>(st) + 3 * q;
-        p[0] = v.x;
-        p[1] = v.y;
-        p[2] = v.z;
-    }
-    __device__ static double4 get(const void* st, int q)
-    {
-        const double* p = static_cast<const double*>(st) + 3 * q;
-        return make_double4(p[0], p[1], p[2], 0.0);
-    }
-};
-template <>
-struct Staged<false>
-{
-    static constexpr int bytes = 32;
-    __device__ static void put(void* st, int q, const double4& v) { static_cast<double4*>(st)[q] = v; }
-    __device__ static double4 get(const void* st, int q) { return static_cast<const double4*>(st)[q]; }
-};
-
-// The staged records of the force kernels: {x, y} pairs, then {z} (XYZ, 24 bytes a record, where
-// the kernel needs positions only) or {z, w} pairs (32 bytes, w = type or slab weight), each
-// array of `cap` records.  A neighbour is one 16-byte and one 8-byte read (or two 16-byte
+// The staged records of the force kernels: {z} (XYZ, 24 bytes a record, where the kernel needs
+// positions only) or {z, w} pairs (32 bytes, w = type or slab weight), then {x, y} pairs.  A neighbour is one 16-byte and one 8-byte read (or two 16-byte
 // ones): random gathers of 64 lanes take 19.7 LDS cycles per neighbour in this form, against
 // 32.0 for {x, y, z} records of 24 bytes, whose x and y come as one two-address read
 // (measured with 16 waves per CU; records a few places apart 14.6 against 22.6), and the LDS
@@ -176,10 +149,16 @@ struct Staged<false>
 template <bool XYZ>
 struct Stage
 {
-    static constexpr int bytes = XYZ ? 24 : 32;
+    static constexpr int recBytes = XYZ ? 24 : 32;
+    double* z;    ///< first, so that an entry is its byte offset
     double2* xy;
-    double* z;
-    __device__ Stage(void* base, int64_t cap) : xy(static_cast<double2*>(base)), z(reinterpret_cast<double*>(xy + cap)) {}
+    /// LDS bytes of n records (an even number of them: the pairs are 16-byte aligned)
+    static size_t bytes(int64_t n) { return size_t((n + 1) / 2 * 2) * recBytes; }
+    __device__ Stage(void* base, int64_t n)
+        : z(static_cast<double*>(base)),
+          xy(reinterpret_cast<double2*>(static_cast<char*>(base) + (n + 1) / 2 * 2 * (XYZ ? 8 : 16)))
+    {
+    }
     __device__ void put(int q, const double4& v) const
     {
         xy[q] = make_double2(v.x, v.y);
@@ -188,12 +167,14 @@ struct Stage
         else
             reinterpret_cast<double2*>(z)[q] = make_double2(v.z, v.w);
     }
-    __device__ double4 get(int q) const
+    /// the record of the slot off / 8 (the form of the list entries)
+    __device__ double4 at(uint32_t off) const
     {
-        const double2 a = xy[q];
-        if (XYZ) return make_double4(a.x, a.y, z[q], 0.0);
-        const double2 b = reinterpret_cast<const double2*>(z)[q];
-        return make_double4(a.x, a.y, b.x, b.y);
+        const double2 a = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(xy) + 2 * off);
+        const char* const b = reinterpret_cast<const char*>(z) + (XYZ ? off : 2 * off);
+        if (XYZ) return make_double4(a.x, a.y, *reinterpret_cast<const double*>(b), 0.0);
+        const double2 zw = *reinterpret_cast<const double2*>(b);
+        return make_double4(a.x, a.y, zw.x, zw.y);
     }
 };
 
@@ -204,11 +185,6 @@ struct Stage
 // axis, so a padding pair lies beyond any cutoff and needs no test of its own.
 constexpr double SENTINEL_GAP = 1.0e3;
 __host__ __device__ inline int sentinelSlot(int32_t maxStaged) { return maxStaged > 1 ? maxStaged : 1; }
-template <bool XYZ>
-__device__ inline void putSentinel(void* st, int32_t maxStaged, double coord, double w)
-{
-    if (threadIdx.x == 0) Staged<XYZ>::put(st, sentinelSlot(maxStaged), make_double4(coord, coord, coord, w));
-}
 template <bool XYZ>
 __device__ inline void putSentinel(const Stage<XYZ>& st, int32_t maxStaged, double coord, double w)
 {
@@ -379,11 +355,6 @@ __device__ inline void stageRecords(const TileInfo& ti, const double4* __restric
     }
 }
 template <bool XYZ>
-__device__ inline void stageTile(const TileInfo& ti, const double4* __restrict__ sortedPos, void* st)
-{
-    stageRecords(ti, sortedPos, [&](int q, const double4& v) { Staged<XYZ>::put(st, q, v); });
-}
-template <bool XYZ>
 __device__ inline void stageTile(const TileInfo& ti, const double4* __restrict__ sortedPos, const Stage<XYZ>& st)
 {
     stageRecords(ti, sortedPos, [&](int q, const double4& v) { st.put(q, v); });
@@ -421,8 +392,8 @@ struct mrmd_verlet_list
     int32_t maxStaged = 0;
     int64_t strideS = 0;        ///< ELL stride over sorted slots (>= nrows, multiple of 64)
     mrmd_hip::DBuf<mrmd_hip::TileInfo> tiles;
-    /// entries per sorted slot s: nbr16[entryIndex(k, s, strideS)] = LDS slot (15 bits) |
-    /// half flag (bit 15)
+    /// entries per sorted slot s: nbr16[entryIndex(k, s, strideS)] = LDS slot << entryShift (15
+    /// bits) | half flag (bit 15)
     mrmd_hip::DBuf<uint16_t> nbr16;
     mrmd_hip::DBuf<int32_t> cnt16;  ///< count per sorted slot (0 for non-row records)
     /// The AdResS time loop builds only the rows that can interact before the next rebuild:

@@ -20,7 +20,7 @@ struct Quad
 {
     double x[4], y[4], z[4], w[4];
 };
-template <bool XYZ>
+template <bool GS, bool XYZ>
 __device__ inline Quad loadQuad(const Stage<XYZ>& st, uint32_t lo, uint32_t hi)
 {
     Quad q;
@@ -28,7 +28,7 @@ __device__ inline Quad loadQuad(const Stage<XYZ>& st, uint32_t lo, uint32_t hi)
 #pragma unroll
     for (int u = 0; u < 4; ++u)
     {
-        const double4 v = st.get(int(e[u]));
+        const double4 v = st.at(e[u] << (3 - entryShift(GS)));
         q.x[u] = v.x;
         q.y[u] = v.y;
         q.z[u] = v.z;
@@ -42,7 +42,7 @@ __device__ inline Quad loadQuad(const Stage<XYZ>& st, uint32_t lo, uint32_t hi)
 // chunk are laid out in a row (for bodies that leave registers for it), not in a loop.  (Two
 // fours in flight from LDS, the next loaded while one is computed, measured no faster: 419
 // against 415 us at 4M atoms.)
-template <bool BOTH, bool XYZ, class Body>
+template <bool BOTH, bool GS, bool XYZ, class Body>
 __device__ inline void walkRow(const Stage<XYZ>& st, const uint4* __restrict__ chunk, int64_t stride, int c, uint4 cur,
                                Body body)
 {
@@ -57,13 +57,13 @@ __device__ inline void walkRow(const Stage<XYZ>& st, const uint4* __restrict__ c
         if (ch + 2 < nch) nxt = chunk[int64_t(ch + 2) * stride];
         if constexpr (BOTH)
         {
-            body(loadQuad(st, now.x, now.y));
-            body(loadQuad(st, now.z, now.w));
+            body(loadQuad<GS>(st, now.x, now.y));
+            body(loadQuad<GS>(st, now.z, now.w));
         }
         else
         {
 #pragma unroll 1
-            for (int h = 0; h < 2; ++h) body(loadQuad(st, h ? now.z : now.x, h ? now.w : now.y));
+            for (int h = 0; h < 2; ++h) body(loadQuad<GS>(st, h ? now.z : now.x, h ? now.w : now.y));
         }
     }
 }

@@ -216,41 +216,67 @@ constexpr int MAX_SPAN = 64;  // cells of a tile's column range along z (K + 2R)
 // records of LDS past the staged neighbourhood that a candidate pass may read (its group of
 // four runs up to three records beyond the column run; their bits are cleared)
 constexpr int STAGE_PAD = 4;
+constexpr size_t LDS_LIMIT = 64000;  // dynamic LDS of a list build workgroup (64 KB less its static part)
 
-// One lane per row.  Every row scans its stencil columns in Cabana's i, j, k order with the
-// min-distance prune (the surviving cells of a column as one slot range, cut by binary
-// search to the z window of the row, the records being z-sorted), 32 candidates per pass in
-// groups of four (independent LDS reads and distances, hit bits shifted in by a funnel shift),
-// then the hits appended in slot order.
+// The list build.  S = 2R + 1 lanes share a row, one per j offset of the stencil, and walk the
+// S i offsets together, so a row's columns come in Cabana's i, j, k order: in each step a lane
+// takes one column, the S lanes' counts are summed in order, and every lane appends its
+// hits behind those of the lanes before it.
+//
+// What bounds it is vector instruction issue (one lane per row in FP64 took 180 instructions a
+// row: 10 per candidate, some 250 candidates, and 20 per entry in a loop that a wave ran 2.4
+// times as often as its mean lane).  Candidates are therefore tested on 16-bit coordinates,
+// relative to the tile's neighbourhood, 8 bytes a record: two packed subtractions and two
+// 16-bit dot products give the squared distance less the threshold in 4 instructions, with
+// one more for the hit bit and two for the bit of a pair too close to call.  A coordinate is
+// rounded by at most half a unit, so a distance is off by at most sqrt(3) units; pairs
+// within 1.75 units of r_n (about 1 in 1,500 candidates) are decided by the FP64 test on the
+// records in memory, the unfused expression of the reference, and so is the half-list bit
+// of partners whose x differs by less than two units: the list is the exact one.  A record
+// outside its tile's range (positions beyond the grid) makes every pair of the tile go that
+// way.  The window search runs on the 16-bit z, widened by two units.  Entries are collected
+// per row in LDS and stored as whole 16-byte chunks of neighbouring rows.
 // WIDE: list offsets in 64-bit arithmetic (lists of 2^31 entries or more); 32-bit otherwise
-// XCD: tiles in the chip's XCD-contiguous order (neighbouring tiles, which share most of
-// their staged records, on one XCD and its L2); otherwise plain block order
-template <int R, bool WIDE, bool XCD, bool GS>
+// GS (dense inputs): the 16-bit records in the tile's slice of global memory, entries stored
+// one by one
+typedef short Short2 __attribute__((ext_vector_type(2)));
+__device__ inline Short2 asShort2(uint32_t v)
+{
+    return __builtin_bit_cast(Short2, v);
+}
+constexpr double QUANT_RANGE = 32000.0;
+constexpr double QUANT_DOUBT = 1.75;
+
+template <int R, bool WIDE, bool GS>
 __global__ __launch_bounds__(BLOCK) void k_verletTiled(const double4* __restrict__ sortedPos,
                                                        const int32_t* __restrict__ sorted,
-                                                       const int32_t* __restrict__ cellOf,
                                                        const int32_t* __restrict__ offsets,
                                                        const TileInfo* __restrict__ tiles, TileGeom tg, GridD g,
-                                                       int64_t rowLo, int64_t rowHi, double rsq, uint16_t* nbr,
-                                                       int64_t strideS, int cap, int32_t* cnt, int32_t* maxCnt,
-                                                       int stagedCap, double4* gstage, int64_t gstageRecs,
-                                                       double bandLo, double bandHi, int8_t* tileSkip)
+                                                       int64_t rowLo, int64_t rowHi, double rsq, double rn,
+                                                       uint16_t* nbr, int64_t strideS, int cap, int32_t* cnt,
+                                                       int32_t* maxCnt, int stagedCap, double4* gstage,
+                                                       int64_t gstageRecs, double bandLo, double bandHi,
+                                                       int8_t* tileSkip)
 {
     constexpr int S = 2 * R + 1;
+    constexpr int RW = WAVE / S;  // rows of a wave
+    constexpr int SH = entryShift(GS);
     extern __shared__ double4 stRaw[];
     __shared__ TileInfo ti;
-    const int64_t t = XCD ? int64_t(xcdBlock()) : int64_t(blockIdx.x);
-    // the staged {x, y, z} records: in LDS, or (GS, dense inputs) in this tile's slice of
-    // global memory, with the per-cell start table alone in LDS
-    double* const st = GS ? reinterpret_cast<double*>(gstage + t * gstageRecs) : reinterpret_cast<double*>(stRaw);
-    // after the staged records and their pad: the LDS slot of the first record of cell
-    // kl + z of range r, cstart[r * cz + z] with cz = K + 2R + 1; entry z = nk closes the
-    // range (ranges outside the grid are empty).  Sized to the tile height, so that short
-    // tiles leave LDS for more workgroups.
+    __shared__ int wild;
+    const int64_t t = blockIdx.x;
+    const int lane = int(threadIdx.x) % WAVE, waves = int(blockDim.x) / WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    // LDS: the waves' row buffers (RW rows of cap entries), the 16-bit records, then the LDS slot
+    // of the first record of cell kl + z of range r, cstart[r * cz + z] with cz = K + 2R + 1;
+    // entry z = nk closes the range (ranges outside the grid are empty)
+    uint16_t* const rowBuf = reinterpret_cast<uint16_t*>(stRaw) + (GS ? 0 : wave * RW * cap);
+    uint2* const ldsRec = reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(stRaw) + (GS ? 0 : waves * RW * cap));
+    uint2* const rec = GS ? reinterpret_cast<uint2*>(gstage + t * gstageRecs) : ldsRec;
+    int* const cstart = reinterpret_cast<int*>(ldsRec + (GS ? 0 : stagedCap + STAGE_PAD));
     const int cz = tg.K + 2 * R + 1;
-    int* cstart = GS ? reinterpret_cast<int*>(stRaw)
-                     : reinterpret_cast<int*>(reinterpret_cast<double*>(stRaw) + 3 * (int64_t(stagedCap) + STAGE_PAD));
     loadTile(ti, tiles, t);
+    if (threadIdx.x == 0) wild = 0;
     __syncthreads();
     if (ti.nrows == 0) return;
     int i0, j0, k0, k1;
@@ -276,16 +302,28 @@ __global__ __launch_bounds__(BLOCK) void k_verletTiled(const double4* __restrict
     }
     const int span = tg.cols + 2 * R;
     const int kl = max(k0 - R, 0), nk = min(k1 + R, tg.n2) - kl;
-    // the first row's dependent loads (slot -> record -> cell) are issued before the staging
-    int s = -1, self = 0, cell = 0;
-    int32_t p = -1;
-    if (int(threadIdx.x) < ti.nrows)
-    {
-        s = tileRow(ti, threadIdx.x, self);
-        p = sorted[s];
-        cell = cellOf[p];
-    }
-    stageTile<true>(ti, sortedPos, st);
+    // units of the 16-bit coordinates: the neighbourhood's longest edge is QUANT_RANGE of them, so
+    // the differences of a row and a candidate (at most R + 1 of 2R + 1 cells) keep the dot
+    // products inside 32 bits
+    const double scale =
+        QUANT_RANGE / fmax(fmax(double(span) * g.dx[0], double(span) * g.dx[1]), double(tg.K + 2 * R) * g.dx[2]);
+    const double ox = g.min[0] + double(i0 - R) * g.dx[0], oy = g.min[1] + double(j0 - R) * g.dx[1],
+                 oz = g.min[2] + double(k0 - R) * g.dx[2];
+    const double rnq = rn * scale;
+    const int sure = int(floor((rnq - QUANT_DOUBT) * (rnq - QUANT_DOUBT)));  // d^2 <= sure: a neighbour
+    const uint32_t doubt = uint32_t(int(ceil((rnq + QUANT_DOUBT) * (rnq + QUANT_DOUBT))) - sure);
+    bool outside = false;
+    stageRecords(ti, sortedPos, [&](int q, const double4& v) {
+        const double u[3] = {(v.x - ox) * scale, (v.y - oy) * scale, (v.z - oz) * scale};
+        int c[3];
+        for (int d = 0; d < 3; ++d)
+        {
+            outside = outside || !(u[d] > -2.0 && u[d] < QUANT_RANGE + 2.0);
+            c[d] = int(rint(fmin(fmax(u[d], -512.0), QUANT_RANGE + 512.0)));
+        }
+        rec[q] = make_uint2((uint32_t(c[0]) << 16) | (uint32_t(c[1]) & 0xffffu), uint32_t(c[2]) & 0xffffu);
+    });
+    if (outside) wild = 1;
     for (int x = threadIdx.x; x < ti.nr * (nk + 1); x += blockDim.x)
     {
         const int r = x / (nk + 1), z = x % (nk + 1);
@@ -301,217 +339,249 @@ __global__ __launch_bounds__(BLOCK) void k_verletTiled(const double4* __restrict
         cstart[r * cz + z] = v;
     }
     __syncthreads();
+    const bool exactAll = wild != 0;
     using Off = std::conditional_t<WIDE, int64_t, uint32_t>;
+    const int sub = lane % S, group = lane / S, first = group * S;
     int localMax = 0;
-    for (int row = threadIdx.x; row < ti.nrows; row += blockDim.x)
+    for (int row0 = wave * RW; row0 < ti.nrows; row0 += waves * RW)
     {
-        if (row != int(threadIdx.x))
-        {
-            s = tileRow(ti, row, self);
-            p = sorted[s];
-            cell = cellOf[p];
-        }
-        if (p < rowLo || p >= rowHi)
-        {
-            cnt[s] = 0;
-            continue;
-        }
-        const int qSelf = ldsSlot(ti, ti.selfRange[self], s);
-        const double xpx = st[3 * qSelf], xpy = st[3 * qSelf + 1], xpz = st[3 * qSelf + 2];
-        const int ck = cell % tg.n2, i = (cell / tg.n2) / tg.n1, j = (cell / tg.n2) % tg.n1;
+        const int row = row0 + group;
+        const bool live = group < RW && row < ti.nrows;
+        int self = 0;
+        const int s = tileRow(ti, live ? row : 0, self);
+        const int32_t p = sorted[s];
+        const double4 xp = sortedPos[s];
+        const bool isRow = live && p >= rowLo && p < rowHi;
+        const int selfRange = ti.selfRange[self];
+        const int qSelf = ldsSlot(ti, selfRange, s);
+        const uint2 own = rec[qSelf];
+        const Short2 ownXY = asShort2(own.x), ownZ = asShort2(own.y);
+        const int zq = int(int16_t(own.y));
+        const int i = i0 - R + selfRange / span, jj = j0 - R + selfRange % span + sub - R;
+        const int ck = g.locate1(xp.z, 2);
         // per-axis terms of Cabana's minDistanceToPoint (r per axis of the cell box, summed
         // as r2 = ((0 + rx^2) + ry^2) + rz^2, so lateral part + rz^2 rounds exactly as the
         // full sum) and of the z window (the lateral distances shrunk by 1e-9 of a cell,
         // far more than a record binned across a face by rounding can stray)
-        double rx2[S], ry2[S], wx2[S], wy2[S], rz2[S];
-#pragma unroll
-        for (int a = 0; a < S; ++a)
-        {
-            const double cx = g.min[0] + (double(i - R + a) + 0.5) * g.dx[0];
-            const double cy = g.min[1] + (double(j - R + a) + 0.5) * g.dx[1];
-            const double czc = g.min[2] + (double(ck - R + a) + 0.5) * g.dx[2];
-            double r = fabs(xpx - cx) - 0.5 * g.dx[0];
+        auto boxDistSqr = [&](double x, int cell, int d, double shrink) {
+            const double c = g.min[d] + (double(cell) + 0.5) * g.dx[d];
+            double r = fabs(x - c) - 0.5 * g.dx[d] - shrink;
             r = r > 0.0 ? r : 0.0;
-            rx2[a] = r * r;
-            r = fabs(xpy - cy) - 0.5 * g.dx[1];
-            r = r > 0.0 ? r : 0.0;
-            ry2[a] = r * r;
-            r = fabs(xpz - czc) - 0.5 * g.dx[2];
-            r = r > 0.0 ? r : 0.0;
-            rz2[a] = r * r;
-            double e = fabs(xpx - cx) - 0.5 * g.dx[0] - 1e-9 * g.dx[0];
-            e = e > 0.0 ? e : 0.0;
-            wx2[a] = e * e;
-            e = fabs(xpy - cy) - 0.5 * g.dx[1] - 1e-9 * g.dx[1];
-            e = e > 0.0 ? e : 0.0;
-            wy2[a] = e * e;
-        }
-        // entries are collected eight at a time in four registers (each append shifts the
-        // eight 16-bit places down by one and puts the entry in the top place, so the first
-        // entry ends in the lowest) and stored as one 16-byte chunk: chunk k of slot s is
-        // chunk k * strideS + s of the list
-        uint4* const chunkBase = reinterpret_cast<uint4*>(nbr) + s;
-        uint32_t b0 = 0, b1 = 0, b2 = 0, b3 = 0;
-        int c = 0;
-        auto append = [&](uint16_t v) {
-            b0 = __builtin_amdgcn_alignbit(b1, b0, 16u);
-            b1 = __builtin_amdgcn_alignbit(b2, b1, 16u);
-            b2 = __builtin_amdgcn_alignbit(b3, b2, 16u);
-            b3 = __builtin_amdgcn_alignbit(uint32_t(v), b3, 16u);
-            if ((c & 7) == 7) chunkBase[Off(c >> 3) * Off(strideS)] = make_uint4(b0, b1, b2, b3);
-            ++c;
+            return r * r;
         };
+        const double ry2 = boxDistSqr(xp.y, jj, 1, 0.0), wy2 = boxDistSqr(xp.y, jj, 1, 1e-9 * g.dx[1]);
+        double rz2[S];
 #pragma unroll
-        for (int da = -R; da <= R; ++da)
-        {
+        for (int dc = 0; dc < S; ++dc) rz2[dc] = boxDistSqr(xp.z, ck - R + dc, 2, 0.0);
+        int n = 0;  // entries of the row so far (the same in its S lanes)
+        auto step = [&](auto daC) {
+            constexpr int da = decltype(daC)::value;
             const int ii = i + da;
-#pragma unroll
-            for (int db = -R; db <= R; ++db)
+            int lo = 0, hi = 0, range = 0;
+            if (isRow && ii >= 0 && ii < tg.n0 && jj >= 0 && jj < tg.n1)
             {
-                const int jj = j + db;
-                int lo = 0, hi = 0;
-                if (ii >= 0 && ii < tg.n0 && jj >= 0 && jj < tg.n1)
-                {
-                    const int* cs0 = cstart + ((ii - (i0 - R)) * span + (jj - (j0 - R))) * cz;
-                    // Cabana's prune per cell of the column: the distance is unimodal in k, so
-                    // the surviving cells are one run [kLo, kHi]
-                    const double lat = rx2[da + R] + ry2[db + R];
-                    int kLo = INT_MAX, kHi = -1;
+                range = (ii - (i0 - R)) * span + (jj - (j0 - R));
+                const int* cs0 = cstart + range * cz - kl;
+                // Cabana's prune per cell of the column: the distance is unimodal in k, so
+                // the surviving cells are one run [kLo, kHi]
+                const double lat = boxDistSqr(xp.x, ii, 0, 0.0) + ry2;
+                int kLo = INT_MAX, kHi = -1;
 #pragma unroll
-                    for (int dc = 0; dc < S; ++dc)
+                for (int dc = 0; dc < S; ++dc)
+                {
+                    const int kk = ck - R + dc;
+                    if (kk >= 0 && kk < tg.n2 && lat + rz2[dc] <= rsq)
                     {
-                        const int kk = ck - R + dc;
-                        if (kk >= 0 && kk < tg.n2 && lat + rz2[dc] <= rsq)
-                        {
-                            kLo = min(kLo, kk);
-                            kHi = kk;
-                        }
+                        kLo = min(kLo, kk);
+                        kHi = kk;
                     }
-                    if (kLo <= kHi)
+                }
+                if (kLo <= kHi)
+                {
+                    // records inside a column run are z-sorted: the candidates that can pass are
+                    // those whose |dz| stays within sqrt(rsq less the squared lateral distance
+                    // from the row to the column), widened by 1e-12 rsq, the float root's
+                    // rounding and two units; the window's lower edge lies in cell kLo and its
+                    // upper edge in cell kHi, so each binary search runs over one cell
+                    const double zsq = rsq - (boxDistSqr(xp.x, ii, 0, 1e-9 * g.dx[0]) + wy2) + 1e-12 * rsq;
+                    const int reach = zsq >= 0.0 ? int(sqrtf(float(zsq)) * float(scale) * 1.00001f) + 2 : -1;
+                    if (reach >= 0)
                     {
-                        // records inside a column run are z-sorted: the candidates that can pass
-                        // are those whose (dz)^2, as the test computes it, stays within rsq less
-                        // the squared lateral distance from the row to the column (widened by
-                        // 1e-12 rsq, more than the rounding of the test's sums), so the cut
-                        // changes no decision; the window's lower edge lies in cell kLo and its
-                        // upper edge in cell kHi, so each binary search runs over one cell
-                        const double zsq = rsq - (wx2[da + R] + wy2[db + R]) + 1e-12 * rsq;
-                        int a = cs0[kLo - kl], b = cs0[kLo + 1 - kl];
+                        int a = cs0[kLo], b = cs0[kLo + 1];
                         while (a < b)
                         {
                             const int m = (a + b) >> 1;
-                            const double dz = xpz - st[3 * m + 2];
-                            if (dz > 0.0 && dz * dz > zsq) a = m + 1;
+                            if (int(int16_t(rec[m].y)) < zq - reach) a = m + 1;
                             else b = m;
                         }
                         lo = a;
-                        a = max(lo, cs0[kHi - kl]);
-                        b = cs0[kHi + 1 - kl];
+                        a = max(lo, cs0[kHi]);
+                        b = cs0[kHi + 1];
                         while (a < b)
                         {
                             const int m = (a + b) >> 1;
-                            const double dz = xpz - st[3 * m + 2];
-                            if (dz < 0.0 && dz * dz > zsq) b = m;
+                            if (int(int16_t(rec[m].y)) > zq + reach) b = m;
                             else a = m + 1;
                         }
                         hi = a;
                     }
                 }
-                for (int qb = lo; qb < hi; qb += 32)
-                {
-                    // branch-free pass over up to 32 candidates in groups of four; each
-                    // group's reads may run up to three records past the run (inside the LDS
-                    // pad), their bits are cleared below.  hits (and, for the columns of the
-                    // row's own x index, the sign bits of dx and the dx == 0 ties) take one bit
-                    // per candidate, shifted in from the right (first candidate highest)
-                    // A bit is shifted in by one funnel shift of the sign word of a double:
-                    // rsq - d^2 is negative exactly when d^2 > rsq (a rounded difference keeps
-                    // the sign of the exact one and is +0 only for equal operands), and dx
-                    // is negative exactly when its sign bit is set (xp - xn is never -0)
-                    uint32_t miss = 0, neg = 0, tie = 0;
-                    const int nq = min(32, hi - qb);
-                    const double* q = st + 3 * qb;
-                    int m = 0;
-                    for (; m < nq; m += 4)
-                    {
-#pragma unroll
-                        for (int u = 0; u < 4; ++u)
-                        {
-                            const double dx = xpx - q[3 * (m + u)];
-                            const double dy = xpy - q[3 * (m + u) + 1];
-                            const double dz = xpz - q[3 * (m + u) + 2];
-                            const double r2 = dx * dx + dy * dy + dz * dz;
-                            miss = __builtin_amdgcn_alignbit(miss, uint32_t(__double2hiint(rsq - r2)), 31u);
-                            if (da == 0)
-                            {
-                                unsigned carry;
-                                neg = __builtin_amdgcn_alignbit(neg, uint32_t(__double2hiint(dx)), 31u);
-                                tie = __builtin_addc(tie, tie, unsigned(dx == 0.0), &carry);
-                            }
-                        }
-                    }
-                    // align: candidate u at bit 31 - u; drop the candidates past the run and
-                    // the row itself
-                    const int sh = 32 - m;  // m is 4..32
-                    uint32_t hits = ~miss << sh;
-                    hits &= ~((1u << (32 - nq)) - 1u);
-                    if (qSelf >= qb && qSelf < qb + nq) hits &= ~(0x80000000u >> (qSelf - qb));
-                    if (da == 0)
-                    {
-                        neg <<= sh;
-                        tie <<= sh;
-                    }
-                    // append the hits in slot order with their half-list bit, Cabana's
-                    // lexicographic discriminator (xn > xp || (xn == xp && (yn > yp || (yn ==
-                    // yp && zn > zp)))): columns of a larger x index hold larger x (binning is
-                    // monotone in x), smaller index smaller x; in the row's own x index the
-                    // sign of dx decides, and a tie dx == 0 compares y and z
-                    auto appendHits = [&](auto checked) {
-                        while (hits)
-                        {
-                            const int u = __builtin_clz(hits);
-                            hits ^= 0x80000000u >> u;
-                            uint32_t half = da > 0 ? 1u : 0u;
-                            if (da == 0)
-                            {
-                                half = (neg << u) >> 31;
-                                if ((tie << u) & 0x80000000u)
-                                {
-                                    const double ny = q[3 * u + 1], nz = q[3 * u + 2];
-                                    half = uint32_t((ny > xpy) | ((ny == xpy) & (nz > xpz)));
-                                }
-                            }
-                            const uint16_t v = uint16_t((qb + u) | (half << 15));
-                            if (!decltype(checked)::value || c < cap)
-                                append(v);
-                            else
-                                ++c;
-                        }
-                    };
-                    // a row that overflows the capacity counts its further hits without storing
-                    if (c + __builtin_popcount(hits) <= cap)
-                        appendHits(std::false_type{});
-                    else
-                        appendHits(std::true_type{});
-                }
             }
-        }
+            // hits (and, for the row's own x index, the half bits) of up to 32 candidates from
+            // qb: candidate u at bit 31 - u
+            auto test = [&](int qb, uint32_t& half) -> uint32_t {
+                half = 0;
+                const int nq = min(32, hi - qb);
+                if (nq <= 0) return 0u;
+                uint32_t hits = 0, unsure = 0, neg = 0;
+                const uint2* q = rec + qb;
+                int m = 0;
+                // groups of four, whose reads may run up to three records past the run (inside the
+                // LDS pad; their bits are cleared below)
+                for (; m < nq; m += 4)
+                {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                    {
+                        const uint2 w = q[m + u];
+                        const Short2 dxy = ownXY - asShort2(w.x), dz = ownZ - asShort2(w.y);
+                        const int over = __builtin_amdgcn_sdot2(
+                            dz, dz, __builtin_amdgcn_sdot2(dxy, dxy, -sure - 1, false), false);
+                        hits = __builtin_amdgcn_alignbit(hits, uint32_t(over), 31u);
+                        bool ask = uint32_t(over) < doubt;
+                        if constexpr (da == 0)
+                        {
+                            // the sign of dx (x is the upper half), near ties apart
+                            const uint32_t d = __builtin_bit_cast(uint32_t, dxy);
+                            neg = __builtin_amdgcn_alignbit(neg, d, 31u);
+                            ask = ask || d + 0x20000u < 0x50000u;
+                        }
+                        unsigned carry;
+                        unsure = __builtin_addc(unsure, unsure, unsigned(ask), &carry);
+                    }
+                }
+                // align; drop the candidates past the run and the row itself
+                const int sh = 32 - m;  // m is 4..32
+                uint32_t valid = ~((1u << (32 - nq)) - 1u);
+                if (nq == 32) valid = ~0u;
+                if (qSelf >= qb && qSelf < qb + nq) valid &= ~(0x80000000u >> (qSelf - qb));
+                hits = (hits << sh) & valid;
+                unsure = exactAll ? valid : (unsure << sh) & valid;
+                half = neg << sh;
+                while (unsure)
+                {
+                    // the reference's test and Cabana's lexicographic discriminator in FP64
+                    const int u = __builtin_clz(unsure);
+                    const uint32_t bit = 0x80000000u >> u;
+                    unsure ^= bit;
+                    const double4 xn = sortedPos[ti.begin[range] + (qb + u - ti.base[range])];
+                    const double dx = xp.x - xn.x, dy = xp.y - xn.y, dz = xp.z - xn.z;
+                    const bool in = dx * dx + dy * dy + dz * dz <= rsq;
+                    hits = in ? hits | bit : hits & ~bit;
+                    if constexpr (da == 0)
+                    {
+                        const bool h = xn.x > xp.x ||
+                                       (xn.x == xp.x && (xn.y > xp.y || (xn.y == xp.y && xn.z > xp.z)));
+                        half = h ? half | bit : half & ~bit;
+                    }
+                }
+                return hits;
+            };
+            // columns of a larger x index hold larger x (binning is monotone in x), smaller index
+            // smaller x: their half bit is the same for all
+            uint32_t half0, half1, halfT;
+            const uint32_t hits0 = test(lo, half0), hits1 = test(lo + 32, half1);
+            int mine = __builtin_popcount(hits0) + __builtin_popcount(hits1);
+            const bool longRun = __any(hi - lo > 64);  // (dense inputs: the rest is tested twice)
+            if (longRun)
+                for (int qb = lo + 64; qb < hi; qb += 32) mine += __builtin_popcount(test(qb, halfT));
+            // places: behind the row's entries so far and those of the lanes before this one
+            int at = n, total = 0;
+#pragma unroll
+            for (int k = 0; k < S; ++k)
+            {
+                const int c = __shfl(mine, first + k, WAVE);
+                at += k < sub ? c : 0;
+                total += c;
+            }
+            auto put = [&](int k, uint32_t v) {
+                if constexpr (GS)
+                    nbr[(Off(k >> 3) * Off(strideS) + Off(s)) * CHUNK + (k & 7)] = uint16_t(v);
+                else
+                    rowBuf[group * cap + k] = uint16_t(v);
+            };
+            auto append = [&](auto checked, int qb, uint32_t hits, uint32_t half) {
+                while (hits)
+                {
+                    const int u = __builtin_clz(hits);
+                    hits ^= 0x80000000u >> u;
+                    uint32_t v = uint32_t(qb + u) << SH;
+                    if (da > 0) v |= 0x8000u;
+                    if (da == 0) v |= ((half << u) >> 16) & 0x8000u;
+                    if (!decltype(checked)::value || at < cap) put(at, v);
+                    ++at;
+                }
+            };
+            // a row that overflows the capacity counts its further hits without storing
+            auto appendAll = [&](auto checked) {
+                append(checked, lo, hits0, half0);
+                append(checked, lo + 32, hits1, half1);
+                if (longRun)
+                    for (int qb = lo + 64; qb < hi; qb += 32)
+                    {
+                        const uint32_t h = test(qb, halfT);
+                        append(checked, qb, h, halfT);
+                    }
+            };
+            n += total;
+            if (__any(n > cap))
+                appendAll(std::true_type{});
+            else
+                appendAll(std::false_type{});
+        };
+        [&]<int... A>(std::integer_sequence<int, A...>) {
+            (step(std::integral_constant<int, A - R>{}), ...);
+        }(std::make_integer_sequence<int, S>{});
         // pad the last chunk with the sentinel slot (a record beyond every cutoff), so the
         // force kernels' chunk loop needs no bounds test
-        const int width = c;
-        while ((c & 7) != 0 && c < cap) append(uint16_t(sentinelSlot(stagedCap)));
-        cnt[s] = min(width, cap);  // the true width goes to maxCnt; reads stay inside the list
-        localMax = max(localMax, width);
+        const uint32_t pad = uint32_t(sentinelSlot(stagedCap)) << SH;
+        const int kept = min(n, cap), nch = (kept + CHUNK - 1) / CHUNK;
+        if (isRow)
+            for (int k = kept + sub; k < nch * CHUNK; k += S)
+            {
+                if constexpr (GS)
+                    nbr[(Off(k >> 3) * Off(strideS) + Off(s)) * CHUNK + (k & 7)] = uint16_t(pad);
+                else
+                    rowBuf[group * cap + k] = uint16_t(pad);
+            }
+        if (live && sub == 0) cnt[s] = isRow ? kept : 0;  // the true width goes to maxCnt
+        localMax = max(localMax, isRow ? n : 0);
+        if constexpr (!GS)
+        {
+            // the wave's rows go out chunk by chunk, neighbouring rows (mostly neighbouring slots)
+            // from neighbouring lanes
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            const int chunks = RW * waveMaxInt(isRow ? nch : 0);
+            for (int x = lane; x - lane < chunks; x += WAVE)
+            {
+                const int r = x % RW, ch = x / RW;
+                const int sr = __shfl(s, r * S, WAVE), nr = __shfl(isRow ? nch : 0, r * S, WAVE);
+                if (ch < nr)
+                    reinterpret_cast<uint4*>(nbr)[Off(ch) * Off(strideS) + Off(sr)] =
+                        reinterpret_cast<const uint4*>(rowBuf + r * cap)[ch];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        }
     }
     // one atomic per wave (every lane of the workgroup reaches this point)
     localMax = waveMaxInt(localMax);
-    if (threadIdx.x % WAVE == 0 && localMax > 0) atomicMax(maxCnt, localMax);
+    if (lane == 0 && localMax > 0) atomicMax(maxCnt, localMax);
 }
 
 // tiled rows (per sorted slot, LDS slots) -> global rows (per record begin+r, record indices)
 __global__ void k_toGlobal(const uint16_t* nbr16, const int32_t* cnt16, int64_t strideS, const TileInfo* tiles,
                            TileGeom tg, const int32_t* sorted, const int32_t* cellOf, int64_t nslots, int64_t rowLo,
-                           int64_t rowHi, uint32_t* nbr, int32_t* cnt, int64_t stride)
+                           int64_t rowHi, uint32_t* nbr, int32_t* cnt, int64_t stride, int shift)
 {
     const int64_t s = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (s >= nslots) return;
@@ -523,7 +593,7 @@ __global__ void k_toGlobal(const uint16_t* nbr16, const int32_t* cnt16, int64_t 
     for (int k = 0; k < c; ++k)
     {
         const uint16_t e = nbr16[entryIndex(k, s, strideS)];
-        const int q = e & 0x7fff;
+        const int q = (e & 0x7fff) >> shift;
         int rr = 0;
         while (rr + 1 < ti.nr && ti.base[rr + 1] <= q) ++rr;
         const int32_t jrec = sorted[ti.begin[rr] + (q - ti.base[rr])];
@@ -766,10 +836,7 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
     if (numAtoms && nall > 0)
         hipLaunchKernelGGL(k_countNotOne, dim3(gridFor(nall)), dim3(BLOCK), 0, ctx->stream, numAtoms, nall, dmulti);
     bool mono = false;
-    // staged records, then the per-cell start table of (a + 2R)^2 ranges x (K + 2R + 1)
     const int stagedCap = std::max(vl->maxStaged, 1);
-    const size_t lds = (vl->globalStage ? 0 : size_t(stagedCap + STAGE_PAD) * Staged<true>::bytes) +
-                       size_t((vl->tileCols + 2 * R) * (vl->tileCols + 2 * R) * (vl->tileK + 2 * R + 1)) * sizeof(int);
     for (int attempt = 0; attempt < 2; ++attempt)
     {
         vl->nbr16.ensure(ctx, int64_t(vl->capFull) * vl->strideS);
@@ -777,12 +844,22 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
         if (vl->ntiles > 0 && end > begin)
         {
             KTimer tk(ctx, "verlet_tiled");
+            // LDS: the row buffers (fewer waves where long rows would not fit), the 16-bit records
+            // and the per-cell start table of (a + 2R)^2 ranges x (K + 2R + 1)
+            const int W = vl->tileCols + 2 * R, rowsPerWave = WAVE / (2 * R + 1);
+            const size_t fixed = (vl->globalStage ? 0 : size_t(stagedCap + STAGE_PAD) * sizeof(uint2)) +
+                                 size_t(W * W * (vl->tileK + 2 * R + 1)) * sizeof(int);
+            const size_t perWave = vl->globalStage ? 0 : size_t(rowsPerWave) * vl->capFull * sizeof(uint16_t);
+            int waves = vl->block / WAVE;
+            while (waves > 1 && fixed + waves * perWave > LDS_LIMIT) --waves;
+            const size_t lds = fixed + waves * perWave;
+            if (lds > LDS_LIMIT)
+                fail(MRMD_ERR_UNSUP, "rows of %d neighbours do not fit the list build's LDS", vl->capFull);
             auto launch = [&](auto kernel) {
-                hipLaunchKernelGGL(kernel, dim3(unsigned(vl->ntiles)), dim3(vl->block), lds, ctx->stream,
-                                   vl->bin.sortedPos.p, vl->bin.sorted.p, vl->bin.cellOf.p, vl->bin.offsets.p,
-                                   vl->tiles.p, geom(vl), g, begin, end, rn * rn, vl->nbr16.p, vl->strideS,
-                                   vl->capFull, vl->cnt16.p, dmax, stagedCap, vl->gstage.p, vl->gstageRecs,
-                                   vl->bandLo, vl->bandHi, vl->tileSkip.p);
+                hipLaunchKernelGGL(kernel, dim3(unsigned(vl->ntiles)), dim3(waves * WAVE), lds, ctx->stream,
+                                   vl->bin.sortedPos.p, vl->bin.sorted.p, vl->bin.offsets.p, vl->tiles.p, geom(vl), g,
+                                   begin, end, rn * rn, rn, vl->nbr16.p, vl->strideS, vl->capFull, vl->cnt16.p, dmax,
+                                   stagedCap, vl->gstage.p, vl->gstageRecs, vl->bandLo, vl->bandHi, vl->tileSkip.p);
             };
             const bool wide = vl->forceWide || int64_t(vl->capFull) * vl->strideS >= (int64_t(1) << 31);
             // plain block order: measured faster here than the XCD-contiguous order (1.54 against
@@ -790,14 +867,14 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
             if (vl->globalStage)
             {
                 if (R == 1)
-                    wide ? launch(k_verletTiled<1, true, false, true>) : launch(k_verletTiled<1, false, false, true>);
+                    wide ? launch(k_verletTiled<1, true, true>) : launch(k_verletTiled<1, false, true>);
                 else
-                    wide ? launch(k_verletTiled<2, true, false, true>) : launch(k_verletTiled<2, false, false, true>);
+                    wide ? launch(k_verletTiled<2, true, true>) : launch(k_verletTiled<2, false, true>);
             }
             else if (R == 1)
-                wide ? launch(k_verletTiled<1, true, false, false>) : launch(k_verletTiled<1, false, false, false>);
+                wide ? launch(k_verletTiled<1, true, false>) : launch(k_verletTiled<1, false, false>);
             else
-                wide ? launch(k_verletTiled<2, true, false, false>) : launch(k_verletTiled<2, false, false, false>);
+                wide ? launch(k_verletTiled<2, true, false>) : launch(k_verletTiled<2, false, false>);
         }
         checkLaunch();
         int32_t hp[2];
@@ -866,7 +943,8 @@ void mrmd_verlet_list::ensureGlobal()
     {
         hipLaunchKernelGGL(k_zeroI32v, dim3(gridFor(rows)), dim3(BLOCK), 0, ctx->stream, cnt.p, rows);
         hipLaunchKernelGGL(k_toGlobal, dim3(gridFor(nrows)), dim3(BLOCK), 0, ctx->stream, nbr16.p, cnt16.p, strideS,
-                           tiles.p, geom(this), bin.sorted.p, bin.cellOf.p, nrows, begin, end, nbr.p, cnt.p, stride);
+                           tiles.p, geom(this), bin.sorted.p, bin.cellOf.p, nrows, begin, end, nbr.p, cnt.p, stride,
+                           entryShift(globalStage));
     }
     checkLaunch();
     globalValid = true;
