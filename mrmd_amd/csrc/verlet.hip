@@ -227,8 +227,8 @@ constexpr size_t LDS_LIMIT = 64000;  // dynamic LDS of a list build workgroup (6
 // row: 10 per candidate, some 250 candidates, and 20 per entry in a loop that a wave ran 2.4
 // times as often as its mean lane).  Candidates are therefore tested on 16-bit coordinates,
 // relative to the tile's neighbourhood, 8 bytes a record: two packed subtractions and two
-// 16-bit dot products give the squared distance less the threshold in 4 instructions, with
-// one more for the hit bit and two for the bit of a pair too close to call.  A coordinate is
+// 16-bit dot products give the squared distance less a threshold in 4 instructions, one more
+// shifts its sign into the hit bits and two the sign against a wider threshold.  A coordinate is
 // rounded by at most half a unit, so a distance is off by at most sqrt(3) units; pairs
 // within 1.75 units of r_n (about 1 in 1,500 candidates) are decided by the FP64 test on the
 // records in memory, the unfused expression of the reference, and so is the half-list bit
@@ -244,11 +244,14 @@ __device__ inline Short2 asShort2(uint32_t v)
 {
     return __builtin_bit_cast(Short2, v);
 }
+// a.x^2 + a.y^2 + c
+__device__ inline int dotSelf(Short2 a, int c) { return __builtin_amdgcn_sdot2(a, a, c, false); }
 constexpr double QUANT_RANGE = 32000.0;
 constexpr double QUANT_DOUBT = 1.75;
 
+// (5 waves per SIMD: 96 registers; with 98 it measured 1.14 instead of 1.08 ms at 4M atoms)
 template <int R, bool WIDE, bool GS>
-__global__ __launch_bounds__(BLOCK) void k_verletTiled(const double4* __restrict__ sortedPos,
+__global__ __launch_bounds__(BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTiled(const double4* __restrict__ sortedPos,
                                                        const int32_t* __restrict__ sorted,
                                                        const int32_t* __restrict__ offsets,
                                                        const TileInfo* __restrict__ tiles, TileGeom tg, GridD g,
@@ -311,7 +314,7 @@ __global__ __launch_bounds__(BLOCK) void k_verletTiled(const double4* __restrict
                  oz = g.min[2] + double(k0 - R) * g.dx[2];
     const double rnq = rn * scale;
     const int sure = int(floor((rnq - QUANT_DOUBT) * (rnq - QUANT_DOUBT)));  // d^2 <= sure: a neighbour
-    const uint32_t doubt = uint32_t(int(ceil((rnq + QUANT_DOUBT) * (rnq + QUANT_DOUBT))) - sure);
+    const int doubt = int(ceil((rnq + QUANT_DOUBT) * (rnq + QUANT_DOUBT))) - sure;  // d^2 < sure + doubt: perhaps
     bool outside = false;
     stageRecords(ti, sortedPos, [&](int q, const double4& v) {
         const double u[3] = {(v.x - ox) * scale, (v.y - oy) * scale, (v.z - oz) * scale};
@@ -427,57 +430,60 @@ __global__ __launch_bounds__(BLOCK) void k_verletTiled(const double4* __restrict
                     }
                 }
             }
-            // hits (and, for the row's own x index, the half bits) of up to 32 candidates from
-            // qb: candidate u at bit 31 - u
+            // the hits among up to 32 candidates from qb, candidate u at bit 31 - u, and, for the
+            // columns of the row's own x index, their half bits
             auto test = [&](int qb, uint32_t& half) -> uint32_t {
                 half = 0;
                 const int nq = min(32, hi - qb);
                 if (nq <= 0) return 0u;
-                uint32_t hits = 0, unsure = 0, neg = 0;
+                uint32_t near = 0, maybe = 0, tie = 0;
                 const uint2* q = rec + qb;
                 int m = 0;
                 // groups of four, whose reads may run up to three records past the run (inside the
-                // LDS pad; their bits are cleared below)
+                // LDS pad; their bits are cleared below); the bits are shifted in from the
+                // sign of the squared distance less either threshold
                 for (; m < nq; m += 4)
                 {
 #pragma unroll
                     for (int u = 0; u < 4; ++u)
                     {
                         const uint2 w = q[m + u];
-                        const Short2 dxy = ownXY - asShort2(w.x), dz = ownZ - asShort2(w.y);
-                        const int over = __builtin_amdgcn_sdot2(
-                            dz, dz, __builtin_amdgcn_sdot2(dxy, dxy, -sure - 1, false), false);
-                        hits = __builtin_amdgcn_alignbit(hits, uint32_t(over), 31u);
-                        bool ask = uint32_t(over) < doubt;
+                        const Short2 dxy = ownXY - asShort2(w.x);
+                        const int over = dotSelf(ownZ - asShort2(w.y), dotSelf(dxy, -sure - 1));
+                        near = __builtin_amdgcn_alignbit(near, uint32_t(over), 31u);
+                        maybe = __builtin_amdgcn_alignbit(maybe, uint32_t(over - doubt), 31u);
                         if constexpr (da == 0)
                         {
-                            // the sign of dx (x is the upper half), near ties apart
+                            // the sign of dx (the upper half), and whether it is within two units
                             const uint32_t d = __builtin_bit_cast(uint32_t, dxy);
-                            neg = __builtin_amdgcn_alignbit(neg, d, 31u);
-                            ask = ask || d + 0x20000u < 0x50000u;
+                            half = __builtin_amdgcn_alignbit(half, d, 31u);
+                            unsigned carry;
+                            tie = __builtin_addc(tie, tie, unsigned(d + 0x20000u < 0x50000u), &carry);
                         }
-                        unsigned carry;
-                        unsure = __builtin_addc(unsure, unsure, unsigned(ask), &carry);
                     }
                 }
                 // align; drop the candidates past the run and the row itself
                 const int sh = 32 - m;  // m is 4..32
                 uint32_t valid = ~((1u << (32 - nq)) - 1u);
-                if (nq == 32) valid = ~0u;
                 if (qSelf >= qb && qSelf < qb + nq) valid &= ~(0x80000000u >> (qSelf - qb));
-                hits = (hits << sh) & valid;
-                unsure = exactAll ? valid : (unsure << sh) & valid;
-                half = neg << sh;
+                uint32_t hits = (near << sh) & valid;
+                uint32_t unsure = ((maybe & (~near | tie)) << sh) & valid;
+                if constexpr (da == 0) half <<= sh;
+                if (exactAll)
+                {
+                    hits = 0;
+                    unsure = valid;
+                }
                 while (unsure)
                 {
-                    // the reference's test and Cabana's lexicographic discriminator in FP64
+                    // in FP64: the reference's test, and the half bit, Cabana's lexicographic
+                    // discriminator
                     const int u = __builtin_clz(unsure);
                     const uint32_t bit = 0x80000000u >> u;
                     unsure ^= bit;
                     const double4 xn = sortedPos[ti.begin[range] + (qb + u - ti.base[range])];
                     const double dx = xp.x - xn.x, dy = xp.y - xn.y, dz = xp.z - xn.z;
-                    const bool in = dx * dx + dy * dy + dz * dz <= rsq;
-                    hits = in ? hits | bit : hits & ~bit;
+                    hits = dx * dx + dy * dy + dz * dz <= rsq ? hits | bit : hits & ~bit;
                     if constexpr (da == 0)
                     {
                         const bool h = xn.x > xp.x ||
@@ -487,8 +493,6 @@ __global__ __launch_bounds__(BLOCK) void k_verletTiled(const double4* __restrict
                 }
                 return hits;
             };
-            // columns of a larger x index hold larger x (binning is monotone in x), smaller index
-            // smaller x: their half bit is the same for all
             uint32_t half0, half1, halfT;
             const uint32_t hits0 = test(lo, half0), hits1 = test(lo + 32, half1);
             int mine = __builtin_popcount(hits0) + __builtin_popcount(hits1);
@@ -504,12 +508,9 @@ __global__ __launch_bounds__(BLOCK) void k_verletTiled(const double4* __restrict
                 at += k < sub ? c : 0;
                 total += c;
             }
-            auto put = [&](int k, uint32_t v) {
-                if constexpr (GS)
-                    nbr[(Off(k >> 3) * Off(strideS) + Off(s)) * CHUNK + (k & 7)] = uint16_t(v);
-                else
-                    rowBuf[group * cap + k] = uint16_t(v);
-            };
+            uint16_t* out = rowBuf + group * cap + at;
+            // the half bit: columns of a larger x index hold larger x (binning is monotone in x),
+            // smaller index smaller x; in the row's own x index the sign of dx decides
             auto append = [&](auto checked, int qb, uint32_t hits, uint32_t half) {
                 while (hits)
                 {
@@ -518,8 +519,15 @@ __global__ __launch_bounds__(BLOCK) void k_verletTiled(const double4* __restrict
                     uint32_t v = uint32_t(qb + u) << SH;
                     if (da > 0) v |= 0x8000u;
                     if (da == 0) v |= ((half << u) >> 16) & 0x8000u;
-                    if (!decltype(checked)::value || at < cap) put(at, v);
-                    ++at;
+                    if (!decltype(checked)::value || at < cap)
+                    {
+                        if constexpr (GS)
+                            nbr[(Off(at >> 3) * Off(strideS) + Off(s)) * CHUNK + (at & 7)] = uint16_t(v);
+                        else
+                            *out = uint16_t(v);
+                    }
+                    if (GS || decltype(checked)::value) ++at;
+                    ++out;
                 }
             };
             // a row that overflows the capacity counts its further hits without storing
