@@ -13,6 +13,7 @@
 #include <cmath>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 
 #include "nlist.hpp"
 #include "pairs.hpp"
@@ -103,6 +104,7 @@ struct TiledList
     const double4* sortedPos;
     int32_t maxStaged;  ///< the sentinel record sits at sentinelSlot(maxStaged)
     double sentinel;    ///< at (sentinel, sentinel, sentinel)
+    int split;          ///< log2 of the lanes that share a row (SPLIT kernels)
     double4* gstage;    ///< the list's per-tile global staging (dense inputs), or null: LDS
     int64_t gstageRecs; ///< records per tile slice of gstage
 };
@@ -154,7 +156,8 @@ __device__ inline void ljQuadTypes(const LJArgs& a, const Pre* tab, int ti0, con
 // nothing there; 0.0 + F is what zeroing and adding leave, -0.0 included)
 // GS: the neighbourhood is staged in the tile's slice of the list's global staging buffer
 // (dense inputs whose tiles exceed the LDS) instead of LDS
-template <bool PRED, bool ONE, bool CAP, bool ASSIGN = false, bool GS = false>
+// SPLIT: 2^tl.split lanes share a row (small systems, see rowSplit)
+template <bool PRED, bool ONE, bool CAP, bool ASSIGN, bool GS, bool SPLIT>
 __global__ __launch_bounds__(BLOCK, PRED || (CAP && !ONE) ? 2 : 4) void k_ljTiled(LJArgs a, TiledList tl, Pre p1, double* partials)
 {
     extern __shared__ double4 stLds[];
@@ -169,19 +172,21 @@ __global__ __launch_bounds__(BLOCK, PRED || (CAP && !ONE) ? 2 : 4) void k_ljTile
     __syncthreads();
     // the first row's global loads (count, index, position, first index chunk) are issued
     // before the staging so that their latency overlaps it
+    const int lg = SPLIT ? tl.split : 0;
     int s = -1, c = 0;
     int32_t i = 0;
     double4 pi = make_double4(0.0, 0.0, 0.0, 0.0);
     uint4 cur = {0, 0, 0, 0};
-    if (int(threadIdx.x) < ti.nrows)
-    {
+    auto openRow = [&](int row) {
         int self;
-        s = tileRow(ti, threadIdx.x, self);
+        s = tileRow(ti, row, self);
         c = tl.cnt[s];
         i = tl.sorted[s];
         pi = tl.sortedPos[s];
-        cur = reinterpret_cast<const uint4*>(tl.nbr)[s];
-    }
+        if (!SPLIT) cur = reinterpret_cast<const uint4*>(tl.nbr)[s];
+    };
+    const int items = ti.nrows << lg;
+    if (int(threadIdx.x) < items) openRow(int(threadIdx.x) >> lg);
     stageTile(ti, tl.sortedPos, st);
     putSentinel(st, tl.maxStaged, tl.sentinel, 0.0);
     __syncthreads();
@@ -196,36 +201,40 @@ __global__ __launch_bounds__(BLOCK, PRED || (CAP && !ONE) ? 2 : 4) void k_ljTile
     };
     // (a wave's lanes take their rows together: the pair count needs every lane at the end of a
     // round)
-    for (int t0 = int(threadIdx.x) & ~(WAVE - 1); t0 < ti.nrows; t0 += blockDim.x)
+    for (int t0 = int(threadIdx.x) & ~(WAVE - 1); t0 < items; t0 += blockDim.x)
     {
         const int t = t0 + int(threadIdx.x) % WAVE;
-        const bool live = t < ti.nrows;
-        if (live && t != int(threadIdx.x))
-        {
-            int self;
-            s = tileRow(ti, t, self);
-            c = tl.cnt[s];
-            i = tl.sorted[s];
-            pi = tl.sortedPos[s];
-            cur = reinterpret_cast<const uint4*>(tl.nbr)[s];
-        }
+        const bool live = t < items;
+        if (live && t != int(threadIdx.x)) openRow(t >> lg);
         if (live && i < a.rows && (ASSIGN || c > 0))
         {
             const int ti0 = ONE ? 0 : int(pi.w) * a.typeStride;
+            const uint4* chunk = reinterpret_cast<const uint4*>(tl.nbr) + s;
             sum.startRow();
-            walkRow<ONE && !CAP && !PRED, GS>(st, reinterpret_cast<const uint4*>(tl.nbr) + s, tl.strideS, c, cur,
-                                          [&](const Quad& q) { pairs(q, pi, ti0); });
-            if (ASSIGN)
+            if constexpr (SPLIT)
             {
-                a.force[i] = 0.0 + sum.fx;
-                a.force[a.cap + i] = 0.0 + sum.fy;
-                a.force[2 * a.cap + i] = 0.0 + sum.fz;
+                walkRowSplit<GS>(st, chunk, tl.strideS, c, t & ((1 << lg) - 1), lg,
+                                 [&](const Quad& q) { pairs(q, pi, ti0); });
+                sum.joinRow(lg);
             }
             else
+                walkRow<ONE && !CAP && !PRED, GS>(st, chunk, tl.strideS, c, cur,
+                                                  [&](const Quad& q) { pairs(q, pi, ti0); });
+            // (the row's first lane stores)
+            if (!SPLIT || (t & ((1 << lg) - 1)) == 0)
             {
-                a.force[i] += sum.fx;
-                a.force[a.cap + i] += sum.fy;
-                a.force[2 * a.cap + i] += sum.fz;
+                if (ASSIGN)
+                {
+                    a.force[i] = 0.0 + sum.fx;
+                    a.force[a.cap + i] = 0.0 + sum.fy;
+                    a.force[2 * a.cap + i] = 0.0 + sum.fz;
+                }
+                else
+                {
+                    a.force[i] += sum.fx;
+                    a.force[a.cap + i] += sum.fy;
+                    a.force[2 * a.cap + i] += sum.fz;
+                }
             }
         }
         if constexpr (ONE) sum.endRound();
@@ -627,6 +636,52 @@ extern "C" int mrmd_lj_apply(mrmd_lj* lj, mrmd_atoms* at, mrmd_verlet_list* vl, 
 
 namespace
 {
+// the full-row kernel over a list whose slot-order positions are current; assign: in the store
+// form where the table has one (returns whether it was)
+bool launchTiled(mrmd_lj* lj, mrmd_verlet_list* vl, const LJArgs& a, bool assign, double* partials)
+{
+    mrmd_ctx* ctx = lj->ctx;
+    KTimer t(ctx, "lj_force");
+    const TiledList tl{vl->nbr16.p, vl->cnt16.p, vl->strideS, vl->tiles.p, vl->bin.sorted.p,
+                       vl->bin.sortedPos.p, vl->maxStaged, vl->sentinel, rowSplit(vl->end - vl->begin),
+                       vl->globalStage ? vl->gstage.p : nullptr, vl->gstageRecs};
+    const Pre p1 = lj->table[0];
+    const bool one = lj->table.size() == 1;
+    const int64_t recs = sentinelSlot(vl->maxStaged) + 1;
+    const size_t lds = vl->globalStage ? 0 : one ? Stage<true>::bytes(recs) : Stage<false>::bytes(recs);
+    bool cap = false;
+    for (const auto& p : lj->table) cap = cap || p.capDistSqr > 0.0;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(unsigned(std::max<int64_t>(vl->ntiles, 1))), dim3(vl->block), lds, ctx->stream,
+                           a, tl, p1, partials);
+    };
+    auto pick = [&](auto pred, auto single, auto capped, auto store) {
+        constexpr bool P = decltype(pred)::value, O = decltype(single)::value, C = decltype(capped)::value,
+                       A = decltype(store)::value;
+        if (vl->globalStage)
+            tl.split ? launch(k_ljTiled<P, O, C, A, true, true>) : launch(k_ljTiled<P, O, C, A, true, false>);
+        else
+            tl.split ? launch(k_ljTiled<P, O, C, A, false, true>) : launch(k_ljTiled<P, O, C, A, false, false>);
+    };
+    constexpr std::true_type yes;
+    constexpr std::false_type no;
+    if (assign && !a.usePred && one && !cap)
+    {
+        pick(no, yes, no, yes);
+        return true;
+    }
+    if (a.usePred)
+        one ? (cap ? pick(yes, yes, yes, no) : pick(yes, yes, no, no))
+            : (cap ? pick(yes, no, yes, no) : pick(yes, no, no, no));
+    else
+        one ? (cap ? pick(no, yes, yes, no) : pick(no, yes, no, no))
+            : (cap ? pick(no, no, yes, no) : pick(no, no, no, no));
+    return false;
+}
+}  // namespace
+
+namespace
+{
 bool ljApplyImpl(mrmd_lj* lj, mrmd_atoms* at, mrmd_verlet_list* vl, const mrmd_pred2* pred, bool assign)
 {
     bool assigned = false;
@@ -655,40 +710,7 @@ bool ljApplyImpl(mrmd_lj* lj, mrmd_atoms* at, mrmd_verlet_list* vl, const mrmd_p
             REQUIRE(!vl->banded, "the list holds only the rows within reach of the slab's weighted region (built "
                                  "inside the AdResS time loop); rebuild it for LennardJones");
             if (!fresh) vl->refreshSorted(at->pos.p);
-            KTimer t(ctx, "lj_force");
-            const TiledList tl{vl->nbr16.p, vl->cnt16.p, vl->strideS, vl->tiles.p, vl->bin.sorted.p,
-                               vl->bin.sortedPos.p, vl->maxStaged, vl->sentinel,
-                               vl->globalStage ? vl->gstage.p : nullptr, vl->gstageRecs};
-            const Pre p1 = lj->table[0];
-            const bool one = lj->table.size() == 1;
-            const int64_t recs = sentinelSlot(vl->maxStaged) + 1;
-            const size_t lds = one ? Stage<true>::bytes(recs) : Stage<false>::bytes(recs);
-            const dim3 g(grid), b(vl->block);
-            bool cap = false;
-            for (const auto& p : lj->table) cap = cap || p.capDistSqr > 0.0;
-            auto launch2 = [&](auto kernel, auto kernelGS) {
-                if (vl->globalStage)
-                    hipLaunchKernelGGL(kernelGS, g, b, 0, ctx->stream, a, tl, p1, partials);
-                else
-                    hipLaunchKernelGGL(kernel, g, b, lds, ctx->stream, a, tl, p1, partials);
-            };
-            const int variant = (a.usePred ? 4 : 0) | (one ? 2 : 0) | (cap ? 1 : 0);
-            if (assign && variant == 2)
-            {
-                launch2(k_ljTiled<false, true, false, true, false>, k_ljTiled<false, true, false, true, true>);
-                assigned = true;
-            }
-            else switch (variant)
-            {
-                case 0: launch2(k_ljTiled<false, false, false, false, false>, k_ljTiled<false, false, false, false, true>); break;
-                case 1: launch2(k_ljTiled<false, false, true, false, false>, k_ljTiled<false, false, true, false, true>); break;
-                case 2: launch2(k_ljTiled<false, true, false, false, false>, k_ljTiled<false, true, false, false, true>); break;
-                case 3: launch2(k_ljTiled<false, true, true, false, false>, k_ljTiled<false, true, true, false, true>); break;
-                case 4: launch2(k_ljTiled<true, false, false, false, false>, k_ljTiled<true, false, false, false, true>); break;
-                case 5: launch2(k_ljTiled<true, false, true, false, false>, k_ljTiled<true, false, true, false, true>); break;
-                case 6: launch2(k_ljTiled<true, true, false, false, false>, k_ljTiled<true, true, false, false, true>); break;
-                default: launch2(k_ljTiled<true, true, true, false, false>, k_ljTiled<true, true, true, false, true>); break;
-            }
+            assigned = launchTiled(lj, vl, a, assign, partials);
         }
         else
         {
@@ -797,29 +819,7 @@ int mrmd_lj_apply_noalloc(mrmd_lj* lj, mrmd_atoms* at, mrmd_verlet_list* vl, dou
         if (!fresh) vl->refreshSorted(at->pos.p);
         LJArgs a{at->pos.p, at->force.p, at->cap, 0, rows, 0, lj->dtable.p, int(lj->table.size()),
                  int(lj->typeStride), lj->rcSqr, mrmd_pred2{}, 0};
-        const TiledList tl{vl->nbr16.p, vl->cnt16.p, vl->strideS, vl->tiles.p, vl->bin.sorted.p,
-                           vl->bin.sortedPos.p, vl->maxStaged, vl->sentinel,
-                               vl->globalStage ? vl->gstage.p : nullptr, vl->gstageRecs};
-        const Pre p1 = lj->table[0];
-        const bool one = lj->table.size() == 1;
-        bool cap = false;
-        for (const auto& q : lj->table) cap = cap || q.capDistSqr > 0.0;
-        const int64_t recs = sentinelSlot(vl->maxStaged) + 1;
-            const size_t lds = one ? Stage<true>::bytes(recs) : Stage<false>::bytes(recs);
-        const dim3 g(unsigned(vl->ntiles)), b(vl->block);
-        auto launch2 = [&](auto kernel, auto kernelGS) {
-            if (vl->globalStage)
-                hipLaunchKernelGGL(kernelGS, g, b, 0, ctx->stream, a, tl, p1, part);
-            else
-                hipLaunchKernelGGL(kernel, g, b, lds, ctx->stream, a, tl, p1, part);
-        };
-        switch ((one ? 2 : 0) | (cap ? 1 : 0))
-        {
-            case 0: launch2(k_ljTiled<false, false, false, false, false>, k_ljTiled<false, false, false, false, true>); break;
-            case 1: launch2(k_ljTiled<false, false, true, false, false>, k_ljTiled<false, false, true, false, true>); break;
-            case 2: launch2(k_ljTiled<false, true, false, false, false>, k_ljTiled<false, true, false, false, true>); break;
-            default: launch2(k_ljTiled<false, true, true, false, false>, k_ljTiled<false, true, true, false, true>); break;
-        }
+        launchTiled(lj, vl, a, false, part);
         hipLaunchKernelGGL(k_sumPartialsTo, dim3(1), dim3(BLOCK), 0, ctx->stream, part, vl->ntiles, ev_dev, lj->ev.p);
     }
     else

@@ -130,6 +130,19 @@ __device__ inline int ldsSlot(const TileInfo& ti, int r, int s) { return ti.base
 // slot s sits at ((k / 8) * strideS + s) * 8 + k % 8, so one 16-byte load per lane brings
 // 8 entries and a wave's load is 1 KB contiguous.
 constexpr int CHUNK = 8;
+// Lanes of the tiled force kernels that share a row (log2).  One lane walks the ~77 neighbours of
+// a row of a liquid in twenty dependent fours, 12 us however few rows there are; a system too
+// small to fill the chip's 256 CUs x 8 waves x 64 lanes with rows splits each over up to eight
+// lanes (4,000 atoms: force 14.1 -> 6.1 us; 32,000 atoms, two types: 19.2 -> 12.4 us).  It follows
+// from the row count alone, so that a row's sums, whose order it sets, do not depend on the
+// tiling.
+constexpr int MAX_SPLIT = 3;
+inline int rowSplit(int64_t rows)
+{
+    int lg = 0;
+    while (lg < MAX_SPLIT && rows << (lg + 1) <= 256 * 8 * WAVE) ++lg;
+    return lg;
+}
 // An entry's low 15 bits: the LDS slot times 8 (slots stay below 4096, and the force kernels
 // use the product as a byte offset), or the slot itself where tiles stage in global memory
 // (slots up to 32766); bit 15 is the half-list flag.
@@ -384,6 +397,8 @@ struct mrmd_verlet_list
     // ---- tiled form (built on the device; what the force kernels read) ----
     int tileK = 0;              ///< cells per tile along z (0 = choose from the density)
     int tileCols = 2;           ///< a: tiles span a x a cell columns
+    bool tilingGiven = false;   ///< set_tiling chose the shape
+    int64_t tiledRows = -1;     ///< rows for which the shape was chosen
     int block = 256;            ///< workgroup size of the tiled kernels
     int tilesPerCol = 0;
     int64_t ntiles = 0;

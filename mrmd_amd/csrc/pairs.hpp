@@ -68,6 +68,23 @@ __device__ inline void walkRow(const Stage<XYZ>& st, const uint4* __restrict__ c
     }
 }
 
+// The same for one of the 2^lg lanes that share the row: fours sub, sub + 2^lg, ...
+template <bool GS, bool XYZ, class Body>
+__device__ inline void walkRowSplit(const Stage<XYZ>& st, const uint4* __restrict__ chunk, int64_t stride, int c,
+                                    int sub, int lg, Body body)
+{
+    const int nq = (c + 3) / 4, step = 1 << lg;
+    auto four = [&](int q) { return reinterpret_cast<const uint2*>(chunk + int64_t(q >> 1) * stride)[q & 1]; };
+    uint2 nxt = {0, 0};
+    if (sub < nq) nxt = four(sub);
+    for (int q = sub; q < nq; q += step)
+    {
+        const uint2 now = nxt;
+        if (q + step < nq) nxt = four(q + step);
+        body(loadQuad<GS>(st, now.x, now.y));
+    }
+}
+
 __device__ inline void quadDistances(const double4& pi, const Quad& q, double dx[4], double dy[4], double dz[4],
                                      double d2[4])
 {
@@ -97,6 +114,16 @@ struct PairSums
     {
         fx = fy = fz = 0.0;
         pairs = 0;
+    }
+    /// the row's force, summed over its 2^lg lanes (all of them, in a fixed order)
+    __device__ void joinRow(int lg)
+    {
+        for (int off = 1; off < 1 << lg; off <<= 1)
+        {
+            fx += __shfl_xor(fx, off, WAVE);
+            fy += __shfl_xor(fy, off, WAVE);
+            fz += __shfl_xor(fz, off, WAVE);
+        }
     }
     /// every lane of the wave, after its row of this round (if any)
     __device__ void endRound()

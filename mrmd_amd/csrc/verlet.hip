@@ -246,12 +246,13 @@ __device__ inline Short2 asShort2(uint32_t v)
 }
 // a.x^2 + a.y^2 + c
 __device__ inline int dotSelf(Short2 a, int c) { return __builtin_amdgcn_sdot2(a, a, c, false); }
+constexpr int BUILD_BLOCK = 12 * WAVE;
 constexpr double QUANT_RANGE = 32000.0;
 constexpr double QUANT_DOUBT = 1.75;
 
 // (5 waves per SIMD: 96 registers; with 98 it measured 1.14 instead of 1.08 ms at 4M atoms)
 template <int R, bool WIDE, bool GS>
-__global__ __launch_bounds__(BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTiled(const double4* __restrict__ sortedPos,
+__global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTiled(const double4* __restrict__ sortedPos,
                                                        const int32_t* __restrict__ sorted,
                                                        const int32_t* __restrict__ offsets,
                                                        const TileInfo* __restrict__ tiles, TileGeom tg, GridD g,
@@ -795,15 +796,31 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
     // tile shape: a x a columns (a <= 3; 1 when the stencil reaches two cells), height K
     // chosen to stage ~1650 records; shrink until every tile fits in LDS
     const int R = vl->range;
+    const int64_t rows = end - begin;
+    const double regionCells =
+        double(std::max(vl->rowExtent[0], 1)) * std::max(vl->rowExtent[1], 1) * std::max(vl->rowExtent[2], 1);
+    const double perCell = std::max(double(std::max<int64_t>(rows, 1)) / regionCells, 1e-3);
+    // a shape nobody asked for follows the rows: where they are too few to fill the chip, tiles of
+    // as many rows as a workgroup of the force kernel holds with its lanes per row, one cell
+    // column wide from four lanes on, so that there are more of them
+    if (!vl->tilingGiven && vl->tiledRows != rows)
+    {
+        const int lg = rowSplit(rows);
+        vl->tileCols = lg >= 2 ? 1 : 2;
+        vl->tileK = 0;
+        if (lg > 0)
+        {
+            const int a = R == 1 ? vl->tileCols : 1;
+            vl->tileK = std::max(1, int(double(vl->block >> lg) / (a * a * perCell)));
+        }
+        vl->tiledRows = rows;
+    }
     int a = std::max(1, std::min(vl->tileCols, R == 1 ? 3 : 1));
     const int W = a + 2 * R;
     int K = vl->tileK > 0 ? std::min(vl->tileK, g.n[2]) : 0;
     if (K <= 0)
     {
-        const double regionCells = double(std::max(vl->rowExtent[0], 1)) * std::max(vl->rowExtent[1], 1) *
-                                   std::max(vl->rowExtent[2], 1);
-        const double perCell = double(std::max<int64_t>(end - begin, 1)) / regionCells;
-        K = int(1650.0 / (W * W * std::max(perCell, 1e-3))) - 2 * R;
+        K = int(1650.0 / (W * W * perCell)) - 2 * R;
         K = std::max(1, std::min(K, g.n[2]));
     }
     K = std::min(K, MAX_SPAN - 2 * R);
@@ -858,7 +875,10 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
             const size_t fixed = (vl->globalStage ? 0 : size_t(stagedCap + STAGE_PAD) * sizeof(uint2)) +
                                  size_t(W * W * (vl->tileK + 2 * R + 1)) * sizeof(int);
             const size_t perWave = vl->globalStage ? 0 : size_t(rowsPerWave) * vl->capFull * sizeof(uint16_t);
+            // four waves a workgroup fill the chip from 1,280 tiles on (five waves a SIMD); with
+            // fewer tiles their rows go to up to twelve waves
             int waves = vl->block / WAVE;
+            if (!vl->tilingGiven) waves = int(std::max<int64_t>(waves, std::min<int64_t>(12, 5120 / vl->ntiles)));
             while (waves > 1 && fixed + waves * perWave > LDS_LIMIT) --waves;
             const size_t lds = fixed + waves * perWave;
             if (lds > LDS_LIMIT)
@@ -998,6 +1018,7 @@ int mrmd_verlet_set_tiling(mrmd_verlet_list* vl, int tile_cells, int tile_column
     MRMD_API_BEGIN(vl ? vl->ctx : nullptr)
     REQUIRE(vl && tile_cells >= 0 && tile_columns >= 1 && tile_columns <= 3, "invalid tiling");
     REQUIRE(block == 64 || block == 128 || block == 192 || block == 256, "workgroup size must be 64, 128, 192 or 256");
+    vl->tilingGiven = true;
     vl->tileK = tile_cells;
     vl->tileCols = tile_columns;
     vl->block = block;
