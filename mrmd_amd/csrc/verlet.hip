@@ -64,7 +64,7 @@ __global__ __launch_bounds__(BLOCK) void k_tileSetup(TileGeom tg, int64_t ntiles
     int staged = 0;
     if (t < ntiles) tileSetup(tg, t, offsets, counts, tiles, staged);
     staged = waveMaxInt(staged);
-    if (threadIdx.x % WAVE == 0 && staged > 0) atomicMax(maxStaged, staged);
+    if (threadIdx.x % WAVE == 0 && staged > 0) raiseTo(maxStaged, staged);
 }
 
 __device__ void tileSetup(const TileGeom& tg, int64_t t, const int32_t* offsets, const int32_t* counts,
@@ -200,9 +200,9 @@ __global__ __launch_bounds__(BLOCK) void k_rowCellBox(const int32_t* cellOf, int
         if (d < 3 ? v != INT32_MAX : v >= 0)
         {
             if (d < 3)
-                atomicMin(&box[d], v);
+                lowerTo(&box[d], v);
             else
-                atomicMax(&box[d], v);
+                raiseTo(&box[d], v);
         }
     }
 }
@@ -584,7 +584,7 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
     }
     // one atomic per wave (every lane of the workgroup reaches this point)
     localMax = waveMaxInt(localMax);
-    if (lane == 0 && localMax > 0) atomicMax(maxCnt, localMax);
+    if (lane == 0 && localMax > 0) raiseTo(maxCnt, localMax);
 }
 
 // tiled rows (per sorted slot, LDS slots) -> global rows (per record begin+r, record indices)
