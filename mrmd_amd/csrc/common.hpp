@@ -275,6 +275,9 @@ inline uint32_t tagValue(const mrmd_ctx* ctx, int word)
 }
 // n (<= READBACK_INTS) int32 device values to the host through the pinned buffer
 void readbackI32(mrmd_ctx* ctx, const int32_t* dev, int n, int32_t* out);
+// its two halves, for a host that has kernels to launch in between (no other readback may)
+uint32_t postI32(mrmd_ctx* ctx, const int32_t* dev, int n);
+void takeI32(mrmd_ctx* ctx, uint32_t tag, int n, int32_t* out);
 
 __host__ __device__ inline uint64_t tagWord(uint32_t tag, uint32_t v) { return (uint64_t(tag) << 32) | v; }
 

@@ -47,11 +47,23 @@ __global__ void k_scanSums(TO* sums, int64_t m, TO* total)
     if (threadIdx.x == 0 && total) *total = carry;
 }
 
-template <class TO>
-__global__ void k_tileScan(const int32_t* in, int64_t n, const TO* sums, TO* out)
+// SUM: sums holds the tile sums as they are, and every workgroup adds those before it up by
+// itself (the last one writes the total); else they are already scanned
+template <class TO, bool SUM>
+__global__ __launch_bounds__(BLOCK) void k_tileScan(const int32_t* in, int64_t n, const TO* sums, TO* out, TO* total)
 {
     __shared__ TO lds[BLOCK / WAVE];
     const int64_t base = int64_t(blockIdx.x) * TILE + int64_t(threadIdx.x) * 4;
+    TO before = 0;
+    if (SUM)
+    {
+        TO part = 0;
+        for (unsigned k = threadIdx.x; k < blockIdx.x; k += BLOCK) part += sums[k];
+        blockExclusiveScan<TO>(part, lds, &before);
+        __syncthreads();
+    }
+    else
+        before = sums[blockIdx.x];
     TO v[4];
     TO s = 0;
     for (int k = 0; k < 4; ++k)
@@ -60,13 +72,14 @@ __global__ void k_tileScan(const int32_t* in, int64_t n, const TO* sums, TO* out
         s += v[k];
     }
     TO tot;
-    TO ex = blockExclusiveScan<TO>(s, lds, &tot) + sums[blockIdx.x];
+    TO ex = blockExclusiveScan<TO>(s, lds, &tot) + before;
     for (int k = 0; k < 4; ++k)
         if (base + k < n)
         {
             out[base + k] = ex;
             ex += v[k];
         }
+    if (SUM && total && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total = before + tot;
 }
 
 // one workgroup per array (array k at in + k * n): exclusive scan in runs of TILE with a
@@ -103,6 +116,9 @@ __global__ __launch_bounds__(BLOCK) void k_scanSmall(const int32_t* in, TO* out,
     if (threadIdx.x == 0 && total) total[blockIdx.x] = carry;
 }
 
+// up to here a workgroup sums the tile sums before it in one round of loads (four a lane), less
+// than the launch of a kernel that scans them costs
+constexpr int64_t SUM_TILES = 4 * BLOCK;
 template <class TO>
 void scanImpl(mrmd_ctx* ctx, const int32_t* in, TO* out, int64_t n, TO* totalDev)
 {
@@ -115,8 +131,15 @@ void scanImpl(mrmd_ctx* ctx, const int32_t* in, TO* out, int64_t n, TO* totalDev
     const int64_t tiles = std::max<int64_t>(1, (n + TILE - 1) / TILE);
     TO* sums = static_cast<TO*>(ctxScratch(ctx, 0, size_t(tiles) * sizeof(TO)));
     hipLaunchKernelGGL(k_tileSums<TO>, dim3(unsigned(tiles)), dim3(BLOCK), 0, ctx->stream, in, n, sums);
-    hipLaunchKernelGGL(k_scanSums<TO>, dim3(1), dim3(BLOCK), 0, ctx->stream, sums, tiles, totalDev);
-    hipLaunchKernelGGL(k_tileScan<TO>, dim3(unsigned(tiles)), dim3(BLOCK), 0, ctx->stream, in, n, sums, out);
+    if (tiles <= SUM_TILES)
+        hipLaunchKernelGGL((k_tileScan<TO, true>), dim3(unsigned(tiles)), dim3(BLOCK), 0, ctx->stream, in, n, sums, out,
+                           totalDev);
+    else
+    {
+        hipLaunchKernelGGL(k_scanSums<TO>, dim3(1), dim3(BLOCK), 0, ctx->stream, sums, tiles, totalDev);
+        hipLaunchKernelGGL((k_tileScan<TO, false>), dim3(unsigned(tiles)), dim3(BLOCK), 0, ctx->stream, in, n, sums,
+                           out, nullptr);
+    }
     checkLaunch();
 }
 }  // namespace
@@ -193,16 +216,25 @@ __global__ void k_postI32(const int32_t* src, int n, uint64_t* host, uint32_t ta
 
 namespace mrmd_hip
 {
-void readbackI32(mrmd_ctx* ctx, const int32_t* dev, int n, int32_t* out)
+uint32_t postI32(mrmd_ctx* ctx, const int32_t* dev, int n)
 {
-    if (n < 0 || n > READBACK_INTS) fail(MRMD_ERR_ARG, "readback of %d values (at most %d)", n, READBACK_INTS);
-    if (n == 0) return;
+    if (n < 1 || n > READBACK_INTS) fail(MRMD_ERR_ARG, "readback of %d values (at most %d)", n, READBACK_INTS);
     const uint32_t tag = nextTag(ctx);
     hipLaunchKernelGGL(k_postI32, dim3(1), dim3(64), 0, ctx->stream, dev, n,
                        reinterpret_cast<uint64_t*>(ctx->pinned) + READBACK_WORD, tag);
     checkLaunch();
+    return tag;
+}
+
+void takeI32(mrmd_ctx* ctx, uint32_t tag, int n, int32_t* out)
+{
     waitTags(ctx, READBACK_WORD, n, tag);
     for (int k = 0; k < n; ++k) out[k] = int32_t(tagValue(ctx, READBACK_WORD + k));
+}
+
+void readbackI32(mrmd_ctx* ctx, const int32_t* dev, int n, int32_t* out)
+{
+    if (n != 0) takeI32(ctx, postI32(ctx, dev, n), n, out);
 }
 }  // namespace mrmd_hip
 

@@ -33,13 +33,18 @@ namespace
 {
 // WRAP: each position is first mapped into the box (PeriodicMapping) and written back; its
 // current value is wb.from[wb.slotOf[i]] when wb.from is set
-template <bool WRAP>
-__global__ void k_binCount(const double4* pos, int64_t begin, int64_t n, GridD g, int32_t* cellOf, int32_t* counts,
-                           double4* wrapPos, WrapBox wb)
+// BOX: the cell box of the records [rowLo, rowHi) too, a wave and then a workgroup maximum (of the
+// negated minima), and one conditional atomic per word and workgroup.  (Over cells in a pass of
+// its own it cost two launches of 1.5 and 6 us, and a wait of the host with the chip idle.)
+template <bool WRAP, bool BOX>
+__global__ __launch_bounds__(BLOCK) void k_binCount(const double4* pos, int64_t begin, int64_t n, GridD g,
+                                                    int32_t* cellOf, int32_t* counts, double4* wrapPos, WrapBox wb,
+                                                    int64_t rowLo, int64_t rowHi, int32_t* box)
 {
     const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     const bool valid = k < n;
     int c = -1;
+    int32_t ext[6] = {-INT32_MAX, -INT32_MAX, -INT32_MAX, -INT32_MAX, -INT32_MAX, -INT32_MAX};
     if (valid)
     {
         double4 p = (WRAP && wb.from) ? wb.from[wb.slotOf[begin + k]] : pos[begin + k];
@@ -48,11 +53,41 @@ __global__ void k_binCount(const double4* pos, int64_t begin, int64_t n, GridD g
             wrapInto(p, wb.min, wb.max, wb.diam);
             wrapPos[begin + k] = p;
         }
-        c = g.cell(p.x, p.y, p.z);
+        const int at[3] = {g.locate1(p.x, 0), g.locate1(p.y, 1), g.locate1(p.z, 2)};
+        c = (at[0] * g.n[1] + at[1]) * g.n[2] + at[2];
         cellOf[k] = c;
+        if (BOX && begin + k >= rowLo && begin + k < rowHi)
+            for (int d = 0; d < 3; ++d)
+            {
+                ext[d] = -at[d];
+                ext[3 + d] = at[d];
+            }
     }
     const Run r = laneRun(c, valid);
     if (valid && r.head == int(threadIdx.x) % WAVE) atomicAdd(&counts[c], r.len);
+    if constexpr (BOX)
+    {
+        __shared__ int32_t red[6][BLOCK / WAVE];
+        for (int d = 0; d < 6; ++d)
+        {
+            const int v = waveMaxInt(ext[d]);
+            if (threadIdx.x % WAVE == 0) red[d][threadIdx.x / WAVE] = v;
+        }
+        __syncthreads();
+        if (threadIdx.x < 6)
+        {
+            const int d = int(threadIdx.x);
+            int v = red[d][0];
+            for (int w = 1; w < BLOCK / WAVE; ++w) v = max(v, red[d][w]);
+            if (v != -INT32_MAX)
+            {
+                if (d < 3)
+                    lowerTo(&box[d], -v);
+                else
+                    raiseTo(&box[d], v);
+            }
+        }
+    }
 }
 
 __global__ void k_binFill(const int32_t* cellOf, int64_t begin, int64_t n, const int32_t* offsets, int32_t* fill,
@@ -201,15 +236,21 @@ __global__ void k_gatherPos(const double4* pos, const int32_t* sorted, int64_t n
     if (k < n) out[k] = pos[sorted[k]];
 }
 
-__global__ void k_zeroI32(int32_t* p, int64_t n)
+// the cells' counts and fill cursors, and (if not null) the cell box of no record
+__global__ void k_binClear(int32_t* counts, int32_t* fill, int64_t n, int32_t* box)
 {
     const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (k < n) p[k] = 0;
+    if (k < n)
+    {
+        counts[k] = 0;
+        fill[k] = 0;
+    }
+    if (box && k < 6) box[k] = k < 3 ? INT32_MAX : -1;
 }
 }  // namespace
 
 void Binning::build(mrmd_ctx* ctx, const double4* pos, int64_t b, int64_t e, const GridD& g, bool withPos,
-                    bool zOrder, double4* wrapPos, const WrapBox* wrap, int32_t* slotOfOut)
+                    bool zOrder, double4* wrapPos, const WrapBox* wrap, int32_t* slotOfOut, RowBox* rowBox)
 {
     grid = g;
     begin = b;
@@ -221,17 +262,22 @@ void Binning::build(mrmd_ctx* ctx, const double4* pos, int64_t b, int64_t e, con
     counts.ensure(ctx, ncell + 1);
     offsets.ensure(ctx, ncell + 1);
     fill.ensure(ctx, ncell + 1);
-    hipLaunchKernelGGL(k_zeroI32, dim3(gridFor(ncell)), dim3(BLOCK), 0, ctx->stream, counts.p, int64_t(ncell));
-    hipLaunchKernelGGL(k_zeroI32, dim3(gridFor(ncell)), dim3(BLOCK), 0, ctx->stream, fill.p, int64_t(ncell));
+    hipLaunchKernelGGL(k_binClear, dim3(gridFor(std::max(ncell, 6))), dim3(BLOCK), 0, ctx->stream, counts.p, fill.p,
+                       int64_t(ncell), rowBox ? rowBox->box : nullptr);
     if (n > 0)
     {
-        if (wrap)
-            hipLaunchKernelGGL(k_binCount<true>, dim3(gridFor(n)), dim3(BLOCK), 0, ctx->stream, pos, b, n, g, cellOf.p,
-                               counts.p, wrapPos, *wrap);
+        const WrapBox wb = wrap ? *wrap : WrapBox{};
+        auto count = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(gridFor(n)), dim3(BLOCK), 0, ctx->stream, pos, b, n, g, cellOf.p, counts.p,
+                               wrapPos, wb, rowBox ? rowBox->lo : 0, rowBox ? rowBox->hi : 0,
+                               rowBox ? rowBox->box : nullptr);
+        };
+        if (rowBox)
+            wrap ? count(k_binCount<true, true>) : count(k_binCount<false, true>);
         else
-            hipLaunchKernelGGL(k_binCount<false>, dim3(gridFor(n)), dim3(BLOCK), 0, ctx->stream, pos, b, n, g,
-                               cellOf.p, counts.p, nullptr, WrapBox{});
+            wrap ? count(k_binCount<true, false>) : count(k_binCount<false, false>);
     }
+    if (rowBox) rowBox->tag = postI32(ctx, rowBox->box, 6);
     scanExclusiveI32(ctx, counts.p, offsets.p, ncell, nullptr);
     if (n > 0)
     {

@@ -51,6 +51,16 @@ GridD makeGrid(const double* gmin, const double* gmax, const double* delta);
 // order is ascending record index inside every cell (a stable counting sort), or with
 // zOrder ascending z (record index breaking ties), which makes every column of cells one
 // z-sorted run
+// the box of the cells that hold records [lo, hi): box (6 words on the device: minimum cell index
+// per axis, then maximum) is filled by the binning's count pass and posted to the host behind it,
+// under tag, so that the host's wait (takeI32) overlaps with the rest of the binning
+struct RowBox
+{
+    int64_t lo, hi;
+    int32_t* box;
+    uint32_t tag;
+};
+
 struct Binning
 {
     GridD grid{};
@@ -64,10 +74,10 @@ struct Binning
 
     /// wrap (if given): every position is first mapped into that box and written to
     /// wrapPos (the same array as pos for an in-place wrap); slotOfOut (z order with
-    /// positions, begin 0): the slot of each record, written by the z sort
+    /// positions, begin 0): the slot of each record, written by the z sort; rowBox: see RowBox
     void build(mrmd_ctx* ctx, const double4* pos, int64_t b, int64_t e, const GridD& g, bool withPos,
                bool zOrder = false, double4* wrapPos = nullptr, const WrapBox* wrap = nullptr,
-               int32_t* slotOfOut = nullptr);
+               int32_t* slotOfOut = nullptr, RowBox* rowBox = nullptr);
 };
 }  // namespace mrmd_hip
 

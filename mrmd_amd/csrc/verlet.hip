@@ -51,165 +51,80 @@ __device__ inline int64_t tileOfCell(const TileGeom& tg, int cell)
     return (int64_t((i - tg.o0) / tg.cols) * tg.nbj + (j - tg.o1) / tg.cols) * tg.tilesPerCol + (k - tg.o2) / tg.K;
 }
 
-// one thread per tile: row ranges, neighbourhood column ranges and their LDS bases
-__device__ void tileSetup(const TileGeom& tg, int64_t t, const int32_t* offsets, const int32_t* counts,
-                          TileInfo* tiles, int& stagedOut);
-
-// one lane per tile; the largest staged neighbourhood goes to *maxStaged with one atomic per
-// wave
-__global__ __launch_bounds__(BLOCK) void k_tileSetup(TileGeom tg, int64_t ntiles, const int32_t* offsets, const int32_t* counts,
-                            TileInfo* tiles, int32_t* maxStaged)
+// half a wave per tile, a lane per range: row ranges, neighbourhood column ranges and their LDS
+// bases; the largest staged neighbourhood goes to *maxStaged.  The ranges' places are prefix sums
+// over the lanes and the description goes out in neighbouring words.  (One lane per tile, 150
+// scattered loads and 100 scattered stores each, took 12 us at any size up to 20,000 tiles.)
+constexpr int SETUP_LANES = 32;
+static_assert(MAX_RANGES <= SETUP_LANES);
+__global__ __launch_bounds__(BLOCK) void k_tileSetup(TileGeom tg, int64_t ntiles, const int32_t* offsets,
+                                                     const int32_t* counts, TileInfo* tiles, int32_t* maxStaged)
 {
-    const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    int staged = 0;
-    if (t < ntiles) tileSetup(tg, t, offsets, counts, tiles, staged);
-    staged = waveMaxInt(staged);
-    if (threadIdx.x % WAVE == 0 && staged > 0) raiseTo(maxStaged, staged);
-}
-
-__device__ void tileSetup(const TileGeom& tg, int64_t t, const int32_t* offsets, const int32_t* counts,
-                          TileInfo* tiles, int& stagedOut)
-{
+    const int64_t t = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / SETUP_LANES;
+    if (t >= ntiles) return;  // (whole groups leave together)
+    const int q = int(threadIdx.x) % SETUP_LANES;
     int i0, j0, k0, k1;
     tileCoords(tg, t, i0, j0, k0, k1);
-    TileInfo& ti = tiles[t];
-    const int span = tg.cols + 2 * tg.R;
+    const int span = tg.cols + 2 * tg.R, nr = span * span;
     const int kl = max(k0 - tg.R, 0), kh = min(k1 + tg.R, tg.n2);
     const int iEnd = min(i0 + tg.cols, tg.o0 + tg.e0), jEnd = min(j0 + tg.cols, tg.o1 + tg.e1);
-    // every range's table entries are loaded first (independent loads in flight together),
-    // then the ranges are laid out
-    int first[MAX_RANGES], last[MAX_RANGES], lastCount[MAX_RANGES], selfFirst[MAX_RANGES], selfLast[MAX_RANGES],
-        selfCount[MAX_RANGES];
-#pragma unroll
-    for (int q = 0; q < MAX_RANGES; ++q)
+    const int ii = i0 - tg.R + q / span, jj = j0 - tg.R + q % span;
+    const bool in = q < nr && ii >= 0 && ii < tg.n0 && jj >= 0 && jj < tg.n1;
+    const bool self = in && ii >= i0 && ii < iEnd && jj >= j0 && jj < jEnd;
+    const int col = (ii * tg.n1 + jj) * tg.n2;
+    int begin = 0, len = 0, selfBegin = 0, rows = 0;
+    if (in)
     {
-        const int a = q / 5, b = q % 5;  // (a, b) of a span x span neighbourhood, span <= 5
-        const int ii = i0 - tg.R + a, jj = j0 - tg.R + b;
-        const bool in = a < span && b < span && ii >= 0 && ii < tg.n0 && jj >= 0 && jj < tg.n1;
-        const bool self = in && ii >= i0 && ii < iEnd && jj >= j0 && jj < jEnd;
-        const int col = (ii * tg.n1 + jj) * tg.n2;
-        first[q] = in ? offsets[col + kl] : 0;
-        last[q] = in ? offsets[col + kh - 1] : 0;
-        lastCount[q] = in ? counts[col + kh - 1] : 0;
-        selfFirst[q] = self ? offsets[col + k0] : 0;
-        selfLast[q] = self ? offsets[col + k1 - 1] : 0;
-        selfCount[q] = self ? counts[col + k1 - 1] : -1;
+        begin = offsets[col + kl];
+        len = offsets[col + kh - 1] + counts[col + kh - 1] - begin;
     }
-    int nr = 0, staged = 0, nself = 0, nrows = 0;
-#pragma unroll
-    for (int q = 0; q < MAX_RANGES; ++q)
+    if (self)
     {
-        const int a = q / 5, b = q % 5;
-        if (a >= span || b >= span) continue;
-        const int ii = i0 - tg.R + a, jj = j0 - tg.R + b;
-        ti.base[nr] = staged;
-        ti.begin[nr] = first[q];
-        if (ii >= 0 && ii < tg.n0 && jj >= 0 && jj < tg.n1)
+        selfBegin = offsets[col + k0];
+        rows = offsets[col + k1 - 1] + counts[col + k1 - 1] - selfBegin;
+    }
+    // inclusive sums over the group's lanes
+    int lenTo = len, rowsTo = rows, selfTo = self ? 1 : 0;
+    for (int off = 1; off < SETUP_LANES; off <<= 1)
+    {
+        const int a = __shfl_up(lenTo, off, SETUP_LANES), b = __shfl_up(rowsTo, off, SETUP_LANES),
+                  c = __shfl_up(selfTo, off, SETUP_LANES);
+        if (q >= off)
         {
-            staged += last[q] + lastCount[q] - first[q];
-            if (selfCount[q] >= 0)
-            {
-                ti.selfRange[nself] = nr;
-                ti.selfBegin[nself] = selfFirst[q];
-                ti.selfPrefix[nself] = nrows;
-                nrows += selfLast[q] + selfCount[q] - selfFirst[q];
-                ++nself;
-            }
-        }
-        ++nr;
-    }
-    ti.selfPrefix[nself] = nrows;
-    ti.nr = nr;
-    ti.staged = staged;
-    ti.nself = nself;
-    ti.nrows = nrows;
-    stagedOut = staged;
-}
-
-// bounding box of the cells of the list rows (records [rowLo, rowHi) of the binning):
-// box[0..2] minimum cell index per axis, box[3..5] maximum.  A grid-stride pass with a
-// wave and then a workgroup reduction, so that only a few hundred workgroups post atomics
-// to the six words.
-constexpr int BOX_BLOCKS = 512;
-// q = c / n and r = c % n for 0 <= c < 2^31, 1 <= n < 2^31 (rn = 1.0 / n): the quotient from
-// a double product, off by at most one, corrected by the remainder's range
-__device__ inline int divCell(int c, int n, double rn, int& r)
-{
-    int q = int(double(c) * rn);
-    r = c - q * n;
-    if (r < 0)
-    {
-        --q;
-        r += n;
-    }
-    else if (r >= n)
-    {
-        ++q;
-        r -= n;
-    }
-    return q;
-}
-__global__ __launch_bounds__(BLOCK) void k_rowCellBox(const int32_t* cellOf, int64_t rowLo, int64_t rowHi, int n1,
-                                                       int n2, int32_t* box)
-{
-    __shared__ int red[6][BLOCK / WAVE];
-    int lo[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, hi[3] = {-1, -1, -1};
-    const double r1 = 1.0 / double(n1), r2 = 1.0 / double(n2);
-    const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-    // eight independent loads per lane in flight, then their cells
-    constexpr int U = 8;
-    for (int64_t k0 = rowLo + int64_t(blockIdx.x) * blockDim.x + threadIdx.x; k0 < rowHi; k0 += U * stride)
-    {
-        int c[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) c[u] = k0 + u * stride < rowHi ? cellOf[k0 + u * stride] : -1;
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-        {
-            if (c[u] < 0) continue;
-            int kc, jc;
-            const int ij = divCell(c[u], n2, r2, kc);
-            const int ic = divCell(ij, n1, r1, jc);
-            const int v[3] = {ic, jc, kc};
-            for (int d = 0; d < 3; ++d)
-            {
-                lo[d] = min(lo[d], v[d]);
-                hi[d] = max(hi[d], v[d]);
-            }
+            lenTo += a;
+            rowsTo += b;
+            selfTo += c;
         }
     }
-    for (int d = 0; d < 3; ++d)
-        for (int off = WAVE / 2; off > 0; off >>= 1)
-        {
-            lo[d] = min(lo[d], __shfl_xor(lo[d], off, WAVE));
-            hi[d] = max(hi[d], __shfl_xor(hi[d], off, WAVE));
-        }
-    const int w = threadIdx.x / WAVE;
-    if (threadIdx.x % WAVE == 0)
-        for (int d = 0; d < 3; ++d)
-        {
-            red[d][w] = lo[d];
-            red[3 + d][w] = hi[d];
-        }
-    __syncthreads();
-    if (threadIdx.x < 6)
+    TileInfo& ti = tiles[t];
+    if (q < nr)
     {
-        const int d = threadIdx.x;
-        int v = red[d][0];
-        for (int q = 1; q < int(blockDim.x) / WAVE; ++q) v = d < 3 ? min(v, red[d][q]) : max(v, red[d][q]);
-        if (d < 3 ? v != INT32_MAX : v >= 0)
-        {
-            if (d < 3)
-                lowerTo(&box[d], v);
-            else
-                raiseTo(&box[d], v);
-        }
+        ti.base[q] = lenTo - len;
+        ti.begin[q] = begin;
+    }
+    if (self)
+    {
+        ti.selfRange[selfTo - 1] = q;
+        ti.selfBegin[selfTo - 1] = selfBegin;
+        ti.selfPrefix[selfTo - 1] = rowsTo - rows;
+    }
+    if (q == SETUP_LANES - 1)
+    {
+        ti.selfPrefix[selfTo] = rowsTo;
+        ti.nr = nr;
+        ti.staged = lenTo;
+        ti.nself = selfTo;
+        ti.nrows = rowsTo;
+        raiseTo(maxStaged, lenTo);
     }
 }
 
-__global__ void k_initBox(int32_t* box)
+// the counts of all slots and the words of the build's maxima
+__global__ void k_listClear(int32_t* cnt, int64_t n, int32_t* words, int nw)
 {
-    if (threadIdx.x < 6) box[threadIdx.x] = threadIdx.x < 3 ? INT32_MAX : -1;
+    const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (k < n) cnt[k] = 0;
+    if (k < nw) words[k] = 0;
 }
 
 constexpr int MAX_SPAN = 64;  // cells of a tile's column range along z (K + 2R)
@@ -706,27 +621,22 @@ TileGeom geom(const mrmd_verlet_list* vl)
                     vl->rowExtent[0], vl->rowExtent[1], vl->rowExtent[2]};
 }
 
-// cell box of the list rows, from the binning (one device reduction and a readback)
-void rowRegion(mrmd_verlet_list* vl)
+// the words of a build in the context's scratch: the largest staged neighbourhood, the widest row,
+// the records of more than one atom; from word 8 the cell box of the rows
+constexpr int BUILD_WORDS = 3, BOX_WORD = 8;
+int32_t* buildWords(mrmd_ctx* ctx) { return static_cast<int32_t*>(ctxScratch(ctx, 2, 64)); }
+
+// cell box of the list rows, posted by the binning
+void rowRegion(mrmd_verlet_list* vl, const RowBox& rowBox)
 {
-    mrmd_ctx* ctx = vl->ctx;
     const int64_t rows = vl->end - vl->begin;
+    int32_t h[6];
+    takeI32(vl->ctx, rowBox.tag, 6, h);
     for (int d = 0; d < 3; ++d)
     {
         vl->rowOrigin[d] = 0;
         vl->rowExtent[d] = 0;
-    }
-    if (rows <= 0) return;
-    int32_t* box = static_cast<int32_t*>(ctxScratch(ctx, 2, 64)) + 8;
-    hipLaunchKernelGGL(k_initBox, dim3(1), dim3(64), 0, ctx->stream, box);
-    hipLaunchKernelGGL(k_rowCellBox, dim3(std::min<unsigned>(gridFor(rows), BOX_BLOCKS)), dim3(BLOCK), 0, ctx->stream,
-                       vl->bin.cellOf.p, vl->begin,
-                       vl->end, vl->bin.grid.n[1], vl->bin.grid.n[2], box);
-    checkLaunch();
-    int32_t h[6];
-    readbackI32(ctx, box, 6, h);
-    for (int d = 0; d < 3; ++d)
-    {
+        if (rows <= 0) continue;
         // rows exist, so every axis holds at least one cell of them
         if (h[d] < 0 || h[3 + d] < h[d] || h[3 + d] >= vl->bin.grid.n[d])
             fail(MRMD_ERR_STATE, "cell box of the list rows out of the grid: axis %d cells [%d, %d] of %d (%lld rows)",
@@ -736,6 +646,7 @@ void rowRegion(mrmd_verlet_list* vl)
     }
 }
 
+// (words[0] is zero before the call)
 void setupTiles(mrmd_verlet_list* vl, int K)
 {
     mrmd_ctx* ctx = vl->ctx;
@@ -744,15 +655,10 @@ void setupTiles(mrmd_verlet_list* vl, int K)
     const int a = vl->tileCols;
     vl->ntiles = int64_t((vl->rowExtent[0] + a - 1) / a) * ((vl->rowExtent[1] + a - 1) / a) * vl->tilesPerCol;
     vl->tiles.ensure(ctx, std::max<int64_t>(vl->ntiles, 1));
-    int32_t* dmax = static_cast<int32_t*>(ctxScratch(ctx, 2, 64));
-    hipLaunchKernelGGL(k_zeroI32v, dim3(1), dim3(64), 0, ctx->stream, dmax, int64_t(1));
     if (vl->ntiles > 0)
-        hipLaunchKernelGGL(k_tileSetup, dim3(gridFor(vl->ntiles)), dim3(BLOCK), 0, ctx->stream, geom(vl), vl->ntiles,
-                           vl->bin.offsets.p, vl->bin.counts.p, vl->tiles.p, dmax);
+        hipLaunchKernelGGL(k_tileSetup, dim3(gridFor(vl->ntiles * SETUP_LANES)), dim3(BLOCK), 0, ctx->stream, geom(vl),
+                           vl->ntiles, vl->bin.offsets.p, vl->bin.counts.p, vl->tiles.p, buildWords(ctx));
     checkLaunch();
-    int32_t h[1];
-    readbackI32(ctx, dmax, 1, h);
-    vl->maxStaged = h[0];
 }
 
 // records whose atom count is not 1 (molecule lists only)
@@ -786,8 +692,16 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
     vl->sentinel = std::max({gmax[0], gmax[1], gmax[2]}) + SENTINEL_GAP + 4.0 * rn;
     // the binning's z sort also writes each record's slot (slotOf)
     vl->slotOf.ensure(ctx, std::max<int64_t>(nall, 1));
-    vl->bin.build(ctx, pos, 0, nall, g, true, true, nullptr, nullptr, vl->slotOf.p);
-    rowRegion(vl);
+    int32_t* const words = buildWords(ctx);
+    RowBox rowBox{begin, end, words + BOX_WORD, 0};
+    vl->bin.build(ctx, pos, 0, nall, g, true, true, nullptr, nullptr, vl->slotOf.p, &rowBox);
+    vl->strideS = std::max<int64_t>(64, (nall + 63) / 64 * 64);
+    vl->cnt16.ensure(ctx, vl->strideS);
+    hipLaunchKernelGGL(k_listClear, dim3(gridFor(std::max<int64_t>(nall, BUILD_WORDS))), dim3(BLOCK), 0, ctx->stream,
+                       vl->cnt16.p, nall, words, BUILD_WORDS);
+    if (numAtoms && nall > 0)
+        hipLaunchKernelGGL(k_countNotOne, dim3(gridFor(nall)), dim3(BLOCK), 0, ctx->stream, numAtoms, nall, words + 2);
+    rowRegion(vl, rowBox);
     vl->globalValid = false;
     vl->halfValid = false;
     vl->banded = vl->bandLo <= vl->bandHi;
@@ -825,10 +739,12 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
     }
     K = std::min(K, MAX_SPAN - 2 * R);
     vl->globalStage = false;
-    for (;;)
+    for (bool again = false;; again = true)
     {
         vl->tileCols = a;
+        if (again) hipLaunchKernelGGL(k_zeroI32v, dim3(1), dim3(64), 0, ctx->stream, words, int64_t(1));
         setupTiles(vl, K);
+        readbackI32(ctx, words, 1, &vl->maxStaged);
         if (vl->maxStaged <= vl->stageLimit) break;
         if (K > 1)
             K = std::max(1, K / 2);
@@ -850,22 +766,15 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
         vl->gstage.ensure(ctx, std::max<int64_t>(vl->ntiles, 1) * vl->gstageRecs);
     }
     if (vl->banded) vl->tileSkip.ensure(ctx, std::max<int64_t>(vl->ntiles, 1));
-    vl->strideS = std::max<int64_t>(64, (nall + 63) / 64 * 64);
-    vl->cnt16.ensure(ctx, vl->strideS);
-    hipLaunchKernelGGL(k_zeroI32v, dim3(gridFor(nall)), dim3(BLOCK), 0, ctx->stream, vl->cnt16.p, nall);
     if (vl->capFull <= 0) vl->capFull = int32_t(std::max<int64_t>(2 * maxNeigh + 16, 96));
     vl->capFull = (vl->capFull + CHUNK - 1) / CHUNK * CHUNK;
-    int32_t* dmax = static_cast<int32_t*>(ctxScratch(ctx, 2, 64)) + 1;
-    int32_t* dmulti = dmax + 1;
-    hipLaunchKernelGGL(k_zeroI32v, dim3(1), dim3(64), 0, ctx->stream, dmulti, int64_t(1));
-    if (numAtoms && nall > 0)
-        hipLaunchKernelGGL(k_countNotOne, dim3(gridFor(nall)), dim3(BLOCK), 0, ctx->stream, numAtoms, nall, dmulti);
+    int32_t* const dmax = words + 1;
     bool mono = false;
     const int stagedCap = std::max(vl->maxStaged, 1);
     for (int attempt = 0; attempt < 2; ++attempt)
     {
         vl->nbr16.ensure(ctx, int64_t(vl->capFull) * vl->strideS);
-        hipLaunchKernelGGL(k_zeroI32v, dim3(1), dim3(64), 0, ctx->stream, dmax, int64_t(1));
+        if (attempt > 0) hipLaunchKernelGGL(k_zeroI32v, dim3(1), dim3(64), 0, ctx->stream, dmax, int64_t(1));
         if (vl->ntiles > 0 && end > begin)
         {
             KTimer tk(ctx, "verlet_tiled");
