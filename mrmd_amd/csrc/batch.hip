@@ -74,11 +74,20 @@ struct TileG
 struct TileB
 {
     int32_t nr, staged, nself, nrows;
+    int32_t near;  ///< the tile's rows can have pairs before the replica's next rebuild
     int32_t begin[B_RANGES], base[B_RANGES];
     int8_t sx[B_RANGES], sy[B_RANGES], sz[B_RANGES];
     int32_t colBase[B_STEN * B_STEN];
     int32_t selfPiece[B_SELF], selfBegin[B_SELF], selfPrefix[B_SELF + 1];
 };
+
+// the tile's description into LDS, one word per lane
+__device__ inline void loadTileB(TileB& ti, const TileB* tiles, int64_t t)
+{
+    static_assert(sizeof(TileB) % 4 == 0);
+    const int32_t* src = reinterpret_cast<const int32_t*>(tiles + t);
+    for (int k = threadIdx.x; k < int(sizeof(TileB) / 4); k += blockDim.x) reinterpret_cast<int32_t*>(&ti)[k] = src[k];
+}
 
 // sorted slot of the t-th row of a tile, and its self column
 __device__ inline int bTileRow(const TileB& ti, int t, int& sc)
@@ -457,6 +466,19 @@ __global__ __launch_bounds__(BLOCK) void k_bTiles(BS b)
             if (pc == 1) mainPiece = np;
             ++np;
         }
+    // an AdResS tile whose staged columns all lie out of reach of the weighted region (the slab's
+    // atomistic and hybrid x band widened by the displacement that triggers a rebuild; weights
+    // come from the records' own x in [0, L)) has no pair before its next rebuild: the build
+    // leaves its rows empty and the force kernel writes zeros without staging anything
+    bool near = col;
+    if (R.adress && col)
+    {
+        const double reach = 0.5 * R.slab.atomistic_diameter + R.slab.hybrid_diameter + R.halfSkin;
+        const double xlo = ii == 0 ? -HUGE_VAL : double(ii) * R.dxc[0] - 1e-9 * R.dxc[0];
+        const double xhi = ii == nx - 1 ? HUGE_VAL : double(ii + 1) * R.dxc[0] + 1e-9 * R.dxc[0];
+        near = !(xhi < R.slab.center[0] - reach || xlo > R.slab.center[0] + reach);
+    }
+    near = __any(near);
     if (self)
     {
         const int rf = cellIndex(R, ii, jj, G.k0), rl = cellIndex(R, ii, jj, G.k1 - 1);
@@ -500,6 +522,7 @@ __global__ __launch_bounds__(BLOCK) void k_bTiles(BS b)
         ti.staged = stTot;
         ti.nself = nself;
         ti.nrows = nrows;
+        ti.near = near ? 1 : 0;
     }
 }
 
@@ -744,36 +767,18 @@ __global__ __launch_bounds__(BLOCK) void k_bBuild(BS b)
     const unsigned t = blockIdx.x;
     const TileG G = b.tg[t];
     if (!b.flag[G.rep]) return;
-    if (threadIdx.x == 0) ti = b.tiles[t];
+    loadTileB(ti, b.tiles, t);
     __syncthreads();
     if (ti.nrows == 0) return;
     const RepD R = b.reps[G.rep];
-    if (R.adress)
+    if (!ti.near)
     {
-        // an AdResS tile whose staged columns all lie out of reach of the weighted region
-        // (the slab's atomistic and hybrid x band widened by the displacement that triggers
-        // a rebuild; weights come from the records' own x in [0, L)) keeps no pair before its
-        // next rebuild: empty rows, and the force kernel finds every weight 0
-        const double reach = 0.5 * R.slab.atomistic_diameter + R.slab.hybrid_diameter + R.halfSkin;
-        const double lo = R.slab.center[0] - reach, hi = R.slab.center[0] + reach;
-        bool near = false;
-        for (int sa = 0; sa < G.ni + 2; ++sa)
+        for (int t = threadIdx.x; t < ti.nrows; t += blockDim.x)
         {
-            int ii = G.i0 - 1 + sa;
-            ii = ii < 0 ? ii + R.nc[0] : (ii >= R.nc[0] ? ii - R.nc[0] : ii);
-            const double xlo = ii == 0 ? -HUGE_VAL : double(ii) * R.dxc[0] - 1e-9 * R.dxc[0];
-            const double xhi = ii == R.nc[0] - 1 ? HUGE_VAL : double(ii + 1) * R.dxc[0] + 1e-9 * R.dxc[0];
-            near = near || !(xhi < lo || xlo > hi);
+            int sc;
+            b.cnt[bTileRow(ti, t, sc)] = 0;
         }
-        if (!near)
-        {
-            for (int t = threadIdx.x; t < ti.nrows; t += blockDim.x)
-            {
-                int sc;
-                b.cnt[bTileRow(ti, t, sc)] = 0;
-            }
-            return;
-        }
+        return;
     }
     const bool fits = ti.staged <= b.stageCap;
     if (fits) stageShifted<true>(ti, b.sortedPos, stb, R);
@@ -952,11 +957,11 @@ __global__ __launch_bounds__(BLOCK) void k_bForce(BS b)
     __shared__ double red[BLOCK / WAVE];
     const unsigned t = unsigned(b.tileBase) + xcdBlock();
     const TileG G = b.tg[t];
-    if (threadIdx.x == 0) ti = b.tiles[t];
+    loadTileB(ti, b.tiles, t);
     __syncthreads();
     const bool fits = ti.staged <= b.stageCap;
     const RepD R = b.reps[G.rep];
-    const bool weighted = fits ? stageShifted<!W>(ti, b.sortedPos, stf, R) : true;
+    const bool weighted = !W || (ti.near && (fits ? stageShifted<!W>(ti, b.sortedPos, stf, R) : true));
     // an AdResS tile whose neighbourhood is all coarse-grained (every weight 0) has no pair
     // (LJ_IdealGas.cpp:95), hence zero forces, drift and energy: the rows get the +0.0 that
     // the pair loop would leave, without it
@@ -973,6 +978,7 @@ __global__ __launch_bounds__(BLOCK) void k_bForce(BS b)
         if (threadIdx.x == 0) b.ePart[t] = 0.0;
         return;
     }
+    if (!W && fits) stageShifted<true>(ti, b.sortedPos, stf, R);
     if (!W) __syncthreads();
     double eTile;
     if (!fits)
@@ -1267,35 +1273,45 @@ void mrmd_batch::layoutTiles()
         for (auto& R : reps)
         {
             if (R.adress != adress) continue;
-            const double perCell = double(R.n) / double(R.nc[0] * R.nc[1] * R.nc[2]);
-            const double cols = double(B_STEN * B_STEN);
-            int K = int(std::lround(double(targetStaged) / (cols * std::max(perCell, 1e-3)))) - 2;
+            // two by two columns, or one where three cells of two by two's sixteen columns
+            // already hold more records than wanted (dense cells; with two by two everywhere the
+            // densest replica's tiles set the LDS of the whole launch, 48 and 64 KB, and beyond
+            // that ran from global memory: 1.25 ms for one tile)
+            const double perCell = std::max(double(R.n) / double(R.nc[0] * R.nc[1] * R.nc[2]), 1e-3);
+            const double want = (adress ? 0.86 : 1.0) * targetStaged;  // whole records and a wider margin
+            int a = B_COLS, K = 0;
+            double cols = 0.0;
+            for (;; --a)
+            {
+                cols = double((a + 2) * (a + 2));
+                K = int(want / (cols * perCell) + 0.25) - 2;
+                if (K >= 1 || a == 1) break;
+            }
             K = std::max(1, std::min({K, R.nc[2], B_SPAN - 2}));
             R.K = K;
             R.tilesPerCol = (R.nc[2] + K - 1) / K;
             R.t0 = int32_t(t0);
-            const int bi = (R.nc[0] + B_COLS - 1) / B_COLS, bj = (R.nc[1] + B_COLS - 1) / B_COLS;
+            const int bi = (R.nc[0] + a - 1) / a, bj = (R.nc[1] + a - 1) / a;
             R.ntiles = bi * bj * R.tilesPerCol;
             for (int ib = 0; ib < bi; ++ib)
                 for (int jb = 0; jb < bj; ++jb)
                     for (int kb = 0; kb < R.tilesPerCol; ++kb)
-                        tg.push_back(TileG{int32_t(&R - reps.data()), ib * B_COLS, jb * B_COLS,
-                                           std::min(B_COLS, R.nc[0] - ib * B_COLS),
-                                           std::min(B_COLS, R.nc[1] - jb * B_COLS), kb * K,
-                                           std::min((kb + 1) * K, R.nc[2])});
+                        tg.push_back(TileG{int32_t(&R - reps.data()), ib * a, jb * a, std::min(a, R.nc[0] - ib * a),
+                                           std::min(a, R.nc[1] - jb * a), kb * K, std::min((kb + 1) * K, R.nc[2])});
             t0 += R.ntiles;
             maxStage[adress] = std::max(maxStage[adress], cols * (K + 2) * perCell);
         }
     }
     ntiles = t0;
-    // LDS capacity: the expected largest neighbourhood with room for density fluctuations
-    // (a tile beyond it reads its records from global memory, exactly)
-    auto capFor = [&](double m) {
-        int v = int(std::min(double(STAGE_MAX), std::ceil(1.25 * m + 64.0)));
+    // LDS capacity: the expected largest neighbourhood with room for density fluctuations, wider
+    // for AdResS replicas, whose ideal gas is denser or thinner than its liquid (a tile beyond it
+    // reads its records from global memory, exactly)
+    auto capFor = [&](double m, double room) {
+        int v = int(std::min(double(STAGE_MAX), std::ceil(room * m + 24.0)));
         return stageCapLimit > 0 ? std::min(v, stageCapLimit) : v;
     };
-    stageCapPlain = capFor(maxStage[0]);
-    stageCapAdress = capFor(maxStage[1]);
+    stageCapPlain = capFor(maxStage[0], 1.1);
+    stageCapAdress = capFor(maxStage[1], 1.25);
     stageCapBuild = std::max(stageCapPlain, stageCapAdress);
     mrmd_ctx* c = ctx;
     dreps.reserve(c, int64_t(reps.size()));
