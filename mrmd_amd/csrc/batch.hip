@@ -29,6 +29,7 @@
 
 #include "detmath.hpp"
 #include "nlist.hpp"
+#include "pairs.hpp"
 #include "physics.hpp"
 
 using namespace mrmd_hip;
@@ -40,6 +41,8 @@ constexpr int B_STEN = B_COLS + 2; // staged columns per axis
 constexpr int B_RANGES = B_STEN * B_STEN * 3;  // staged columns, up to three image pieces each
 constexpr int B_SELF = B_COLS * B_COLS;
 constexpr int B_SPAN = 18;         // cells of a tile's column run (K + 2), so K <= 16
+constexpr int TARGET_STAGED = 1400;  // staged records wanted per tile
+constexpr int B_ROW_LANES = 256;   // lanes that the force kernel lays a tile's rows out for
 constexpr int B_PAD = 4;           // staged records past the neighbourhood a candidate group may read
 constexpr int COMP_BINS = 200;     // LJ_IdealGas compensation bins (LJ_IdealGas.hpp:54)
 constexpr double COMP_SCALE = 4294967296.0;
@@ -52,6 +55,7 @@ struct RepD
     int64_t a0, n;
     int32_t c0, nc[3];
     int32_t t0, ntiles, K, tilesPerCol;
+    int32_t split;  ///< log2 of the lanes that share a row in the force kernels
     double L[3], dxc[3], rdxc[3];
     double dt, zeta, temperature, mass, halfSkin;
     double damping, sigma;  ///< O-step factors of the replica's mass, computed on the host
@@ -125,7 +129,8 @@ struct BS
     uint16_t* nbr;
     int32_t* cnt;
     int64_t strideS;
-    int32_t capList, stageCap;  ///< list width; staged records that fit the launch's LDS
+    int32_t capList;      ///< list width
+    int32_t stageCap[2];  ///< staged records that fit the LDS of the plain and the AdResS forces
     double* dispStep;
     double* dispAcc;
     int32_t* flag;
@@ -569,50 +574,22 @@ __global__ void k_bGather(BS b)
     }
 }
 
-// copy a tile's neighbourhood into LDS, shifting each piece by its periodic image: {x, y, z}
-// records (XYZ) or whole double4 records (the AdResS forces read the slab weight in w)
-// Returns whether a record this lane staged has a weight w > 0 (whole records only).
-template <bool XYZ>
-__device__ inline bool stageShifted(const TileB& ti, const double4* __restrict__ sp, double* st, const RepD& R)
+// a tile's records, each piece shifted by its periodic image, to put(slot, record)
+template <class Put>
+__device__ inline void stageShifted(const TileB& ti, const double4* __restrict__ sp, const RepD& R, Put put)
 {
-    bool weighted = false;
-    int r = 0;
-    for (int q = threadIdx.x; q < ti.staged; q += blockDim.x)
-    {
-        while (r + 1 < ti.nr && ti.base[r + 1] <= q) ++r;
-        double4 v = sp[ti.begin[r] + (q - ti.base[r])];
+    stageRecords(ti, sp, [&](int q, double4 v, int r) {
         v.x += double(ti.sx[r]) * R.L[0];
         v.y += double(ti.sy[r]) * R.L[1];
         v.z += double(ti.sz[r]) * R.L[2];
-        if (XYZ)
-        {
-            st[3 * q] = v.x;
-            st[3 * q + 1] = v.y;
-            st[3 * q + 2] = v.z;
-        }
-        else
-        {
-            reinterpret_cast<double4*>(st)[q] = v;
-            weighted = weighted || v.w > 0.0;
-        }
-    }
-    return weighted;
+        put(q, v);
+    });
 }
 
-// A tile's records by staged slot: from LDS when its neighbourhood fits the stage area, else
-// straight from the slot-ordered records with the same periodic shift (the same arithmetic,
-// so the same bits) -- a slower path that keeps tiles of crowded cells (lattice starts,
-// density fluctuations) exact instead of dropping them.
-struct LdsFetch3
-{
-    const double* st;
-    __device__ double4 operator()(int q) const { return make_double4(st[3 * q], st[3 * q + 1], st[3 * q + 2], 1.0); }
-};
-struct LdsFetch4
-{
-    const double4* st;
-    __device__ double4 operator()(int q) const { return st[q]; }
-};
+// A tile's neighbourhood that does not fit the stage area: records by staged slot straight from
+// the slot-ordered ones with the same periodic shift (the same arithmetic, so the same bits) --
+// a slower path that keeps tiles of crowded cells (lattice starts, density fluctuations) exact
+// instead of dropping them.  The entries of its rows are plain slots (bFits).
 struct GlobalFetch
 {
     const TileB* ti;
@@ -629,6 +606,18 @@ struct GlobalFetch
         v.z += double(ti->sz[r]) * L2;
         return v;
     }
+    __device__ double4 at(uint32_t off) const { return (*this)(int(off >> 3)); }
+};
+// whether a tile stages in LDS, in every kernel that reads or writes its entries (which then
+// hold slots times eight, else slots: entryShift)
+__device__ inline bool bFits(const BS& b, const RepD& R, const TileB& ti)
+{
+    return ti.staged <= b.stageCap[R.adress ? 1 : 0];
+}
+struct LdsFetch3
+{
+    const double* st;
+    __device__ double4 operator()(int q) const { return make_double4(st[3 * q], st[3 * q + 1], st[3 * q + 2], 1.0); }
 };
 
 // Full rows of one tile of a flagged replica, one lane per row, as the single-system build
@@ -637,7 +626,7 @@ struct GlobalFetch
 // column), 32 candidates per pass in groups of four with the hit bits shifted in by a
 // funnel shift, then the hits appended in slot order.  Entries are staged slots; rows are
 // padded to whole chunks with the row's own slot (distance 0, which the forces skip).
-template <class Fetch>
+template <int SH, class Fetch>
 __device__ void bBuildRows(const BS& b, const TileB& ti, const TileG& G, const RepD& R, const int* cstart,
                            const Fetch& fetch)
 {
@@ -742,13 +731,13 @@ __device__ void bBuildRows(const BS& b, const TileB& ti, const TileG& G, const R
                     {
                         const int u = __builtin_clz(hits);
                         hits ^= 0x80000000u >> u;
-                        if (c < b.capList) rowBase[int64_t(c >> 3) * chunkStride + (c & 7)] = uint16_t(qb + u);
+                        if (c < b.capList) rowBase[int64_t(c >> 3) * chunkStride + (c & 7)] = uint16_t((qb + u) << SH);
                         ++c;
                     }
                 }
             }
         for (int k = c; k < ((c + CHUNK - 1) / CHUNK) * CHUNK && k < b.capList; ++k)
-            rowBase[int64_t(k >> 3) * chunkStride + (k & 7)] = uint16_t(qSelf);
+            rowBase[int64_t(k >> 3) * chunkStride + (k & 7)] = uint16_t(qSelf << SH);
         b.cnt[s] = min(c, b.capList);  // an overflow is reported through err; reads stay in the list
         localMax = max(localMax, c);
     }
@@ -780,8 +769,13 @@ __global__ __launch_bounds__(BLOCK) void k_bBuild(BS b)
         }
         return;
     }
-    const bool fits = ti.staged <= b.stageCap;
-    if (fits) stageShifted<true>(ti, b.sortedPos, stb, R);
+    const bool fits = bFits(b, R, ti);
+    if (fits)
+        stageShifted(ti, b.sortedPos, R, [&](int q, const double4& v) {
+            stb[3 * q] = v.x;
+            stb[3 * q + 1] = v.y;
+            stb[3 * q + 2] = v.z;
+        });
     // LDS slot of the first record of cell k0 - 1 + z of each staged column
     const int nzr = G.k1 - G.k0 + 2;
     const int spanJ = G.nj + 2, ncol = (G.ni + 2) * spanJ;
@@ -802,147 +796,161 @@ __global__ __launch_bounds__(BLOCK) void k_bBuild(BS b)
     }
     __syncthreads();
     if (fits)
-        bBuildRows(b, ti, G, R, cstart, LdsFetch3{stb});
+        bBuildRows<entryShift(false)>(b, ti, G, R, cstart, LdsFetch3{stb});
     else
-        bBuildRows(b, ti, G, R, cstart, GlobalFetch{&ti, b.sortedPos, R.L[0], R.L[1], R.L[2]});
+        bBuildRows<entryShift(true)>(b, ti, G, R, cstart, GlobalFetch{&ti, b.sortedPos, R.L[0], R.L[1], R.L[2]});
 }
 
 // ---------------------------------------------------------------------------------------
 // forces: weighted LJ (LJ_IdealGas.cpp:80-200 with one atom per molecule; weight 1 for
 // plain replicas, which reduces to LennardJones.hpp:168-197), drift and compensation terms
 
-// W: weighted (AdResS replicas: slab weights in w, the unweighted energy e0 for the drift);
-// plain replicas have weight 1 and need neither
-template <bool CAP, bool W, class Fetch>
-__device__ inline void chunkW(const BS& b, const double4& pi, const Fetch& fetch, const uint4 cur, double& fx,
-                              double& fy, double& fz, double& ew, double& e0)
+// sums of one row of an AdResS replica over the pairs inside rc: the weighted force and energy,
+// the unweighted energy (for the drift)
+struct WeightedSums
 {
-    const uint32_t wd[4] = {cur.x, cur.y, cur.z, cur.w};
-    double dx[CHUNK], dy[CHUNK], dz[CHUNK], d2[CHUNK], lj[CHUNK], frac2[CHUNK];
-#pragma unroll
-    for (int u = 0; u < CHUNK; ++u)
-    {
-        const double4 pj = fetch(int((wd[u >> 1] >> ((u & 1) * 16)) & 0x7fffu));
-        dx[u] = pi.x - pj.x;
-        dy[u] = pi.y - pj.y;
-        dz[u] = pi.z - pj.z;
-        lj[u] = pj.w;
-    }
-#pragma unroll
-    for (int u = 0; u < CHUNK; ++u) d2[u] = dx[u] * dx[u] + dy[u] * dy[u] + dz[u] * dz[u];
-#pragma unroll
-    for (int u = 0; u < CHUNK; ++u) frac2[u] = recipNewton(d2[u]);
-    const Pre& p = b.lj;
-    auto accumulate = [&](int u, double ff, double en) {
-        if constexpr (W)
-        {
-            // both partners coarse-grained: no interaction (LJ_IdealGas.cpp:95)
-            const bool in = d2[u] <= b.rcSqr && d2[u] > 0.0 && !(pi.w <= 0.0 && lj[u] <= 0.0);
-            const double w = 0.5 * (pi.w + lj[u]);
-            const double ffw = in ? ff * w : 0.0;
-            fx += dx[u] * ffw;
-            fy += dy[u] * ffw;
-            fz += dz[u] * ffw;
-            ew += in ? en * w : 0.0;
-            e0 += in ? en : 0.0;
-        }
-        else
-        {
-            // padding entries are the row itself (distance 0)
-            const bool in = d2[u] <= b.rcSqr && d2[u] > 0.0;
-            const double ffw = in ? ff : 0.0;
-            fx += dx[u] * ffw;
-            fy += dy[u] * ffw;
-            fz += dz[u] * ffw;
-            ew += in ? en : 0.0;
-        }
-    };
-    if constexpr (!CAP)
-    {
-#pragma unroll
-        for (int u = 0; u < CHUNK; ++u)
-        {
-            const double frac6 = frac2[u] * frac2[u] * frac2[u];
-            accumulate(u, frac6 * (p.ff1 * frac6 - p.ff2) * frac2[u], frac6 * (p.ef1 * frac6 - p.ef2) - p.shift);
-        }
-        return;
-    }
-    double ffv[CHUNK], env[CHUNK];
-    bool capped = false;
-#pragma unroll
-    for (int u = 0; u < CHUNK; ++u)
-    {
-        const double frac6 = frac2[u] * frac2[u] * frac2[u];
-        ffv[u] = frac6 * (p.ff1 * frac6 - p.ff2) * frac2[u];
-        env[u] = frac6 * (p.ef1 * frac6 - p.ef2) - p.shift;
-        capped = capped || (d2[u] < p.capDistSqr && d2[u] > 0.0);  // padding (the row itself) is not a pair
-    }
-    // the capped form (LennardJones.hpp:68-75) only for chunks where some lane of the wave
-    // needs it
-    if (__any(capped))
-    {
-        // keeps the block a branch: the compiler would otherwise evaluate it for every chunk
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int u = 0; u < CHUNK; ++u)
-        {
-            const double dist = sqrt(d2[u]);
-            const bool c = d2[u] < p.capDistSqr;
-            ffv[u] = c ? p.capCoeff / dist : ffv[u];
-            env[u] = c ? p.eCap - (dist - p.capDist) * p.capCoeff - p.shift : env[u];
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < CHUNK; ++u) accumulate(u, ffv[u], env[u]);
-}
+    double fx, fy, fz, ew, e0;
+};
 
-// the rows of one tile: weighted pair forces, drift and compensation terms; returns the
-// lane's energy sum
-template <bool CAP, bool W, class Fetch>
-__device__ double bForceRows(const BS& b, const TileB& ti, const RepD& R, const Fetch& fetch)
+// Four weighted pair terms (w = the slab weight), stage by stage like ljQuadOne: pairs that do not
+// count have their reciprocal, weight and shift masked, so every term of theirs is zero.
+// Both partners coarse-grained: no interaction (LJ_IdealGas.cpp:95).
+template <bool CAP>
+__device__ inline void ljQuadWeighted(const Pre& p, double rcSqr, const double4& pi, const Quad& q, WeightedSums& s)
 {
-    const int64_t step = *b.step;
-    const bool sampling = W && R.adress && step % SAMPLING_INTERVAL == 0;
-    double eTile = 0.0;
-    for (int t = threadIdx.x; t < ti.nrows; t += blockDim.x)
+#pragma clang fp contract(fast)
+    double dx[4], dy[4], dz[4], d2[4], frac2[4];
+    bool in[4], capped = false;
+    quadDistances(pi, q, dx, dy, dz, d2);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
     {
-        int sc;
-        const int s = bTileRow(ti, t, sc);
-        const int c = b.cnt[s];
-        const int32_t i = b.sorted[s];
-        const double4 pi = b.sortedPos[s];
-        double fx = 0.0, fy = 0.0, fz = 0.0, ew = 0.0, e0 = 0.0;
-        const uint4* chunk = reinterpret_cast<const uint4*>(b.nbr) + s;
-        const int nch = (c + CHUNK - 1) / CHUNK;
-        uint4 cur = chunk[0];  // the first chunk column exists for every slot (read even when c = 0)
-        for (int ch = 0; ch < nch; ++ch)
+        // (padding entries are the row itself, at distance 0)
+        in[u] = d2[u] <= rcSqr && d2[u] > 0.0 && !(pi.w <= 0.0 && q.w[u] <= 0.0);
+        if (CAP) capped = capped || (in[u] && d2[u] < p.capDistSqr);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) frac2[u] = recipNewton(d2[u]);
+    if (CAP && __any(capped))
+    {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
         {
-            uint4 nxt = cur;
-            if (ch + 1 < nch) nxt = chunk[int64_t(ch + 1) * b.strideS];
-            chunkW<CAP, W>(b, pi, fetch, cur, fx, fy, fz, ew, e0);
-            cur = nxt;
-        }
-        if (W && R.adress && pi.w > 0.0 && pi.w < 1.0)
-        {
-            // hybrid atom: drift -1/2 sum_j E_ij grad(lambda) and the mean compensation
-            // energy (LJ_IdealGas.cpp:150-170, 208-224)
-            const double g = b.slotGrad[s];
-            fx += -(0.5 * e0) * g;
-            const int64_t bin = getBin(b.slotLam[s], 0.0, double(COMP_BINS), COMP_BINS);
-            if (bin != -1)
+            const bool c = in[u] && d2[u] < p.capDistSqr;
+            if (__any(c))
             {
-                fx += b.meanComp[R.cmp0 + bin] * g;
-                if (sampling)
-                {
-                    atomicAdd(&b.comp[R.cmp0 + bin], (unsigned long long)(long long)llrint(0.5 * e0 * COMP_SCALE));
-                    atomicAdd(&b.compCount[R.cmp0 + bin], 1ull);
-                }
+                // keeps the block a branch: the compiler would otherwise evaluate it every time
+                asm volatile("" ::: "memory");
+                const double dist = sqrt(d2[u]);
+                const double w = 0.5 * (pi.w + q.w[u]);
+                const double ff = c ? p.capCoeff / dist * w : 0.0;
+                const double en = c ? p.eCap - (dist - p.capDist) * p.capCoeff - p.shift : 0.0;
+                s.fx += dx[u] * ff;
+                s.fy += dy[u] * ff;
+                s.fz += dz[u] * ff;
+                s.ew += en * w;
+                s.e0 += en;
+                in[u] = in[u] && !c;
             }
         }
-        b.force[i] = fx;
-        b.force[b.cap + i] = fy;
-        b.force[2 * b.cap + i] = fz;
-        eTile += ew;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+    {
+        const double f2 = maskReciprocal(frac2[u], in[u]);
+        const double w = 0.5 * (pi.w + q.w[u]);
+        const double f6 = f2 * f2 * f2;
+        const double ff = f6 * (p.ff1 * f6 - p.ff2) * f2 * w;
+        const double en = f6 * (p.ef1 * f6 - p.ef2) - (in[u] ? p.shift : 0.0);
+        s.fx += dx[u] * ff;
+        s.fy += dy[u] * ff;
+        s.fz += dz[u] * ff;
+        s.ew += en * w;
+        s.e0 += en;
+    }
+}
+
+// The rows of one tile: pair forces (W: weighted, with the drift and compensation terms); returns
+// the lane's energy sum.  2^split lanes share a row (rowLanes).
+template <bool CAP, bool W, bool GS, class St>
+__device__ double bForceRows(const BS& b, const TileB& ti, const RepD& R, const St& st)
+{
+    const int64_t step = *b.step;
+    const bool sampling = W && step % SAMPLING_INTERVAL == 0;
+    const int lg = R.split;
+    const int items = ti.nrows << lg, mask = (1 << lg) - 1;
+    double eTile = 0.0;
+    PairSums sum;
+    // (a wave's lanes take their rows together: the pair count needs every lane at the end of a
+    // round)
+    for (int t0 = int(threadIdx.x) & ~(WAVE - 1); t0 < items; t0 += blockDim.x)
+    {
+        const int t = t0 + int(threadIdx.x) % WAVE;
+        if (t < items)
+        {
+            int sc;
+            const int s = bTileRow(ti, t >> lg, sc);
+            const int c = b.cnt[s];
+            const int32_t i = b.sorted[s];
+            const double4 pi = b.sortedPos[s];
+            const uint4* chunk = reinterpret_cast<const uint4*>(b.nbr) + s;
+            double f[3];
+            if constexpr (W)
+            {
+                WeightedSums ws{0.0, 0.0, 0.0, 0.0, 0.0};
+                walkRowSplit<GS>(st, chunk, b.strideS, c, t & mask, lg,
+                                 [&](const Quad& q) { ljQuadWeighted<CAP>(b.lj, b.rcSqr, pi, q, ws); });
+                for (int off = 1; off <= mask; off <<= 1)
+                {
+                    ws.fx += __shfl_xor(ws.fx, off, WAVE);
+                    ws.fy += __shfl_xor(ws.fy, off, WAVE);
+                    ws.fz += __shfl_xor(ws.fz, off, WAVE);
+                    ws.e0 += __shfl_xor(ws.e0, off, WAVE);
+                }
+                eTile += ws.ew;
+                if ((t & mask) == 0 && pi.w > 0.0 && pi.w < 1.0)
+                {
+                    // hybrid atom: drift -1/2 sum_j E_ij grad(lambda) and the mean compensation
+                    // energy (LJ_IdealGas.cpp:150-170, 208-224)
+                    const double g = b.slotGrad[s];
+                    ws.fx += -(0.5 * ws.e0) * g;
+                    const int64_t bin = getBin(b.slotLam[s], 0.0, double(COMP_BINS), COMP_BINS);
+                    if (bin != -1)
+                    {
+                        ws.fx += b.meanComp[R.cmp0 + bin] * g;
+                        if (sampling)
+                        {
+                            atomicAdd(&b.comp[R.cmp0 + bin],
+                                      (unsigned long long)(long long)llrint(0.5 * ws.e0 * COMP_SCALE));
+                            atomicAdd(&b.compCount[R.cmp0 + bin], 1ull);
+                        }
+                    }
+                }
+                f[0] = ws.fx;
+                f[1] = ws.fy;
+                f[2] = ws.fz;
+            }
+            else
+            {
+                sum.startRow();
+                walkRowSplit<GS>(st, chunk, b.strideS, c, t & mask, lg, [&](const Quad& q) {
+                    // (padding entries are the row itself, at distance 0)
+                    ljQuadOne<CAP>(b.lj, b.rcSqr, pi, q, sum, [](int, double d2) { return d2 > 0.0; });
+                });
+                sum.joinRow(lg);
+                f[0] = sum.fx;
+                f[1] = sum.fy;
+                f[2] = sum.fz;
+            }
+            if ((t & mask) == 0)
+                for (int d = 0; d < 3; ++d) b.force[d * b.cap + i] = f[d];
+        }
+        if constexpr (!W) sum.endRound();
+    }
+    if constexpr (!W)
+    {
+        double virial;
+        sum.finish<CAP>(b.lj, eTile, virial);
     }
     return eTile;
 }
@@ -952,20 +960,26 @@ __device__ double bForceRows(const BS& b, const TileB& ti, const RepD& R, const 
 template <bool CAP, bool W>
 __global__ __launch_bounds__(BLOCK) void k_bForce(BS b)
 {
-    extern __shared__ double stf[];
+    extern __shared__ double4 stLds[];
     __shared__ TileB ti;
     __shared__ double red[BLOCK / WAVE];
     const unsigned t = unsigned(b.tileBase) + xcdBlock();
     const TileG G = b.tg[t];
     loadTileB(ti, b.tiles, t);
     __syncthreads();
-    const bool fits = ti.staged <= b.stageCap;
-    const RepD R = b.reps[G.rep];
-    const bool weighted = !W || (ti.near && (fits ? stageShifted<!W>(ti, b.sortedPos, stf, R) : true));
+    const RepD& R = b.reps[G.rep];
+    const bool fits = bFits(b, R, ti);
+    const Stage<!W> st(stLds, b.stageCap[W]);
+    bool weighted = !fits;
+    if (fits && ti.near)
+        stageShifted(ti, b.sortedPos, R, [&](int q, const double4& v) {
+            st.put(q, v);
+            weighted = weighted || v.w > 0.0;
+        });
     // an AdResS tile whose neighbourhood is all coarse-grained (every weight 0) has no pair
     // (LJ_IdealGas.cpp:95), hence zero forces, drift and energy: the rows get the +0.0 that
     // the pair loop would leave, without it
-    if (W && !__syncthreads_or(weighted))
+    if (W && !__syncthreads_or(weighted && ti.near))
     {
         for (int t = threadIdx.x; t < ti.nrows; t += blockDim.x)
         {
@@ -978,15 +992,10 @@ __global__ __launch_bounds__(BLOCK) void k_bForce(BS b)
         if (threadIdx.x == 0) b.ePart[t] = 0.0;
         return;
     }
-    if (!W && fits) stageShifted<true>(ti, b.sortedPos, stf, R);
     if (!W) __syncthreads();
-    double eTile;
-    if (!fits)
-        eTile = bForceRows<CAP, W>(b, ti, R, GlobalFetch{&ti, b.sortedPos, R.L[0], R.L[1], R.L[2]});
-    else if constexpr (W)
-        eTile = bForceRows<CAP, W>(b, ti, R, LdsFetch4{reinterpret_cast<const double4*>(stf)});
-    else
-        eTile = bForceRows<CAP, W>(b, ti, R, LdsFetch3{stf});
+    const double eTile = fits ? bForceRows<CAP, W, false>(b, ti, R, st)
+                              : bForceRows<CAP, W, true>(b, ti, R,
+                                                         GlobalFetch{&ti, b.sortedPos, R.L[0], R.L[1], R.L[2]});
     const double e = blockSum(0.5 * eTile, red);
     if (threadIdx.x == 0) b.ePart[t] = e;
 }
@@ -1168,7 +1177,7 @@ struct mrmd_batch
     double rc = 2.5, skin = 0.3;
     Pre lj{};
     bool cap_ = false;
-    int targetStaged = 1400, block = 256;
+    int targetStaged = TARGET_STAGED, block = 256;
     int stageCapPlain = 1600, stageCapAdress = 1600, stageCapBuild = 1600;  ///< staged records in LDS per launch
     int stageCapLimit = 0;  ///< 0: the stage area follows the expected neighbourhood size
     int64_t plainTiles = 0;  ///< tiles of the plain replicas come first, then the AdResS replicas' tiles
@@ -1238,7 +1247,8 @@ BS mrmd_batch::state()
     b.cnt = cnt.p;
     b.strideS = cap;
     b.capList = capList;
-    b.stageCap = stageCapBuild;
+    b.stageCap[0] = stageCapPlain;
+    b.stageCap[1] = stageCapAdress;
     b.tileBase = 0;
     b.dispStep = dispStep.p;
     b.dispAcc = dispAcc.p;
@@ -1259,6 +1269,29 @@ BS mrmd_batch::state()
     return b;
 }
 
+// Tiles of two by two columns, or of one where three cells of two by two's sixteen columns already
+// hold more records than wanted (dense cells; with two by two everywhere the densest replica's
+// tiles set the LDS of the whole launch, 48 and 64 KB, and beyond that ran from global memory:
+// 1.25 ms for one tile), and of as many cells along z as hold the wanted records (fewer for AdResS
+// replicas, whose records are staged whole and need a wider margin)
+struct TileShape
+{
+    int a, K;
+    double perCell;
+};
+TileShape tileShape(const RepD& R, int target)
+{
+    TileShape t{B_COLS, 0, std::max(double(R.n) / double(R.nc[0] * R.nc[1] * R.nc[2]), 1e-3)};
+    const double want = (R.adress ? 0.86 : 1.0) * target;
+    for (;; --t.a)
+    {
+        t.K = int(want / (double((t.a + 2) * (t.a + 2)) * t.perCell) + 0.25) - 2;
+        if (t.K >= 1 || t.a == 1) break;
+    }
+    t.K = std::max(1, std::min({t.K, R.nc[2], B_SPAN - 2}));
+    return t;
+}
+
 // per-replica tile height from the target staged size, tile geometry, LDS capacity; the
 // plain replicas' tiles first, then the AdResS replicas' (their force launches stage
 // different records)
@@ -1273,21 +1306,16 @@ void mrmd_batch::layoutTiles()
         for (auto& R : reps)
         {
             if (R.adress != adress) continue;
-            // two by two columns, or one where three cells of two by two's sixteen columns
-            // already hold more records than wanted (dense cells; with two by two everywhere the
-            // densest replica's tiles set the LDS of the whole launch, 48 and 64 KB, and beyond
-            // that ran from global memory: 1.25 ms for one tile)
-            const double perCell = std::max(double(R.n) / double(R.nc[0] * R.nc[1] * R.nc[2]), 1e-3);
-            const double want = (adress ? 0.86 : 1.0) * targetStaged;  // whole records and a wider margin
-            int a = B_COLS, K = 0;
-            double cols = 0.0;
-            for (;; --a)
-            {
-                cols = double((a + 2) * (a + 2));
-                K = int(want / (cols * perCell) + 0.25) - 2;
-                if (K >= 1 || a == 1) break;
-            }
-            K = std::max(1, std::min({K, R.nc[2], B_SPAN - 2}));
+            const TileShape shape = tileShape(R, targetStaged), usual = tileShape(R, TARGET_STAGED);
+            const int a = shape.a, K = shape.K;
+            // Most tiles have fewer rows than a workgroup has lanes, and a row alone in its lane
+            // takes as long as twenty dependent fours do, so 2^split lanes share it: as many as
+            // the rows of a tile of the usual shape leave.  (By the replica alone, not by the tiling
+            // asked for: the order of a row's sum, and so its bits, follows from it.)
+            const double rows = double(usual.a * usual.a * usual.K) * usual.perCell;
+            R.split = 0;
+            while (R.split < MAX_SPLIT && rows * (2 << R.split) <= B_ROW_LANES) ++R.split;
+            const double cols = double((a + 2) * (a + 2)), perCell = shape.perCell;
             R.K = K;
             R.tilesPerCol = (R.nc[2] + K - 1) / K;
             R.t0 = int32_t(t0);
@@ -1356,22 +1384,22 @@ void mrmd_batch::enqueueSteps(int64_t n)
         hipLaunchKernelGGL(k_bGather, dim3(ga), dim3(BLOCK), 0, c->stream, b);
         hipLaunchKernelGGL(k_bBuild, dim3(unsigned(ntiles)), dim3(block), size_t(stageCapBuild + B_PAD) * 24, c->stream,
                            b);
-        auto force = [&](auto kernel, int64_t t0, int64_t t1, int capRecs, size_t bytes) {
+        auto force = [&](auto kernel, int64_t t0, int64_t t1, size_t lds) {
             if (t1 <= t0) return;
             BS f = b;
             f.tileBase = int32_t(t0);
-            f.stageCap = capRecs;
-            hipLaunchKernelGGL(kernel, dim3(unsigned(t1 - t0)), dim3(block), size_t(capRecs) * bytes, c->stream, f);
+            hipLaunchKernelGGL(kernel, dim3(unsigned(t1 - t0)), dim3(block), lds, c->stream, f);
         };
+        const size_t ldsPlain = Stage<true>::bytes(stageCapPlain), ldsAdress = Stage<false>::bytes(stageCapAdress);
         if (cap_)
         {
-            force(k_bForce<true, false>, 0, plainTiles, stageCapPlain, 24);
-            force(k_bForce<true, true>, plainTiles, ntiles, stageCapAdress, sizeof(double4));
+            force(k_bForce<true, false>, 0, plainTiles, ldsPlain);
+            force(k_bForce<true, true>, plainTiles, ntiles, ldsAdress);
         }
         else
         {
-            force(k_bForce<false, false>, 0, plainTiles, stageCapPlain, 24);
-            force(k_bForce<false, true>, plainTiles, ntiles, stageCapAdress, sizeof(double4));
+            force(k_bForce<false, false>, 0, plainTiles, ldsPlain);
+            force(k_bForce<false, true>, plainTiles, ntiles, ldsAdress);
         }
         hipLaunchKernelGGL(k_bCompUpdate, dim3(nr), dim3(BLOCK), 0, c->stream, b);
         hipLaunchKernelGGL(k_bTFUpdate, dim3(nr), dim3(BLOCK), 0, c->stream, b);

@@ -193,7 +193,7 @@ __global__ __launch_bounds__(BLOCK, PRED || (CAP && !ONE) ? 2 : 4) void k_ljTile
     PairSums sum;
     auto pairs = [&](const Quad& q, const double4& pi, int ti0) {
         if constexpr (ONE)
-            ljQuadOne<CAP>(p1, a.rcSqr, pi, q, sum, [&](int u) {
+            ljQuadOne<CAP>(p1, a.rcSqr, pi, q, sum, [&](int u, double) {
                 return !PRED || evalPred2(a.pred, pi.x, pi.y, pi.z, q.x[u], q.y[u], q.z[u]);
             });
         else

@@ -344,9 +344,9 @@ __device__ inline void sortCellByZ(int32_t* recs, int n, const double4* __restri
 // copy the tile's neighbourhood (contiguous runs of sorted slots) into LDS: each wave takes
 // every fourth run, four runs at a time, so that run starts and lengths are wave-uniform
 // (scalar) and a lane has four independent loads in flight; looking up the run of each record
-// instead took a tenth of the force kernel's vector instructions
-template <class Put>
-__device__ inline void stageRecords(const TileInfo& ti, const double4* __restrict__ sortedPos, Put put)
+// instead took a tenth of the force kernel's vector instructions; put(slot, record, run)
+template <class Tile, class Put>
+__device__ inline void stageRecords(const Tile& ti, const double4* __restrict__ sortedPos, Put put)
 {
     constexpr int U = 4;
     const int lane = int(threadIdx.x) % WAVE, waves = int(blockDim.x) / WAVE;
@@ -373,14 +373,14 @@ __device__ inline void stageRecords(const TileInfo& ti, const double4* __restric
                 if (k < len[u]) v[u] = sortedPos[begin[u] + k];
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                if (k < len[u]) put(base[u] + k, v[u]);
+                if (k < len[u]) put(base[u] + k, v[u], r0 + u * waves);
         }
     }
 }
 template <bool XYZ>
 __device__ inline void stageTile(const TileInfo& ti, const double4* __restrict__ sortedPos, const Stage<XYZ>& st)
 {
-    stageRecords(ti, sortedPos, [&](int q, const double4& v) { st.put(q, v); });
+    stageRecords(ti, sortedPos, [&](int q, const double4& v, int) { st.put(q, v); });
 }
 }  // namespace mrmd_hip
 

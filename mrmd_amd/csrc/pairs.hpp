@@ -20,8 +20,8 @@ struct Quad
 {
     double x[4], y[4], z[4], w[4];
 };
-template <bool GS, bool XYZ>
-__device__ inline Quad loadQuad(const Stage<XYZ>& st, uint32_t lo, uint32_t hi)
+template <bool GS, class St>
+__device__ inline Quad loadQuad(const St& st, uint32_t lo, uint32_t hi)
 {
     Quad q;
     const uint32_t e[4] = {lo & 0x7fffu, (lo >> 16) & 0x7fffu, hi & 0x7fffu, (hi >> 16) & 0x7fffu};
@@ -42,8 +42,8 @@ __device__ inline Quad loadQuad(const Stage<XYZ>& st, uint32_t lo, uint32_t hi)
 // chunk are laid out in a row (for bodies that leave registers for it), not in a loop.  (Two
 // fours in flight from LDS, the next loaded while one is computed, measured no faster: 419
 // against 415 us at 4M atoms.)
-template <bool BOTH, bool GS, bool XYZ, class Body>
-__device__ inline void walkRow(const Stage<XYZ>& st, const uint4* __restrict__ chunk, int64_t stride, int c, uint4 cur,
+template <bool BOTH, bool GS, class St, class Body>
+__device__ inline void walkRow(const St& st, const uint4* __restrict__ chunk, int64_t stride, int c, uint4 cur,
                                Body body)
 {
     const int nch = (c + CHUNK - 1) / CHUNK;
@@ -69,8 +69,8 @@ __device__ inline void walkRow(const Stage<XYZ>& st, const uint4* __restrict__ c
 }
 
 // The same for one of the 2^lg lanes that share the row: fours sub, sub + 2^lg, ...
-template <bool GS, bool XYZ, class Body>
-__device__ inline void walkRowSplit(const Stage<XYZ>& st, const uint4* __restrict__ chunk, int64_t stride, int c,
+template <bool GS, class St, class Body>
+__device__ inline void walkRowSplit(const St& st, const uint4* __restrict__ chunk, int64_t stride, int c,
                                     int sub, int lg, Body body)
 {
     const int nq = (c + 3) / 4, step = 1 << lg;
@@ -154,8 +154,8 @@ struct PairSums
 // beyond rc have their reciprocal masked, so every term of theirs is zero.  CAP: the table has a
 // capping distance; the capped form (LennardJones.hpp:68-75) runs, one entry after the other
 // (its square root and quotient need many registers), only where some lane of the wave has a
-// capped pair, and such a pair is masked out of the other sums.  allowed(u): whether the pair of
-// entry u counts at all.  Products and sums may contract to FMAs here (the neighbour decision of
+// capped pair, and such a pair is masked out of the other sums.  allowed(u, d2): whether the pair
+// of entry u counts at all.  Products and sums may contract to FMAs here (the neighbour decision of
 // the list is unaffected: it is made, unfused, at build time); the forces then differ from the
 // unfused CPU arithmetic by a few ulps per term.
 template <bool CAP, class Allowed>
@@ -171,8 +171,8 @@ __device__ inline void ljQuadOne(const Pre& p, double rcSqr, const double4& pi, 
     {
         // padding entries point at the sentinel record beyond every cutoff, so the cutoff test
         // alone decides
-        in[u] = d2[u] <= rcSqr && allowed(u);
-        if (CAP) capped = capped || d2[u] < p.capDistSqr;
+        in[u] = d2[u] <= rcSqr && allowed(u, d2[u]);
+        if (CAP) capped = capped || (in[u] && d2[u] < p.capDistSqr);
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) frac2[u] = recipNewton(d2[u]);

@@ -232,7 +232,7 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
     const int sure = int(floor((rnq - QUANT_DOUBT) * (rnq - QUANT_DOUBT)));  // d^2 <= sure: a neighbour
     const int doubt = int(ceil((rnq + QUANT_DOUBT) * (rnq + QUANT_DOUBT))) - sure;  // d^2 < sure + doubt: perhaps
     bool outside = false;
-    stageRecords(ti, sortedPos, [&](int q, const double4& v) {
+    stageRecords(ti, sortedPos, [&](int q, const double4& v, int) {
         const double u[3] = {(v.x - ox) * scale, (v.y - oy) * scale, (v.z - oz) * scale};
         int c[3];
         for (int d = 0; d < 3; ++d)
