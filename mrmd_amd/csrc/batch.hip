@@ -43,6 +43,7 @@ constexpr int B_SELF = B_COLS * B_COLS;
 constexpr int B_SPAN = 18;         // cells of a tile's column run (K + 2), so K <= 16
 constexpr int TARGET_STAGED = 1400;  // staged records wanted per tile
 constexpr int B_ROW_LANES = 256;   // lanes that the force kernel lays a tile's rows out for
+constexpr size_t B_BUILD_LDS = 60000;  // dynamic LDS of a build workgroup (64 KB less its static part)
 constexpr int B_PAD = 4;           // staged records past the neighbourhood a candidate group may read
 constexpr int COMP_BINS = 200;     // LJ_IdealGas compensation bins (LJ_IdealGas.hpp:54)
 constexpr double COMP_SCALE = 4294967296.0;
@@ -145,7 +146,8 @@ struct BS
     int64_t* step;
     int32_t* err;
     Pre lj;
-    double rcSqr, rnSqr;
+    double rcSqr, rnSqr, rn;
+    int32_t buildCap;  ///< staged records that fit the build's LDS
     int32_t tileBase;  ///< first tile of the launch (the force launches take plain and AdResS tiles apart)
 };
 
@@ -614,142 +616,230 @@ __device__ inline bool bFits(const BS& b, const RepD& R, const TileB& ti)
 {
     return ti.staged <= b.stageCap[R.adress ? 1 : 0];
 }
-struct LdsFetch3
+// the 16-bit records of a tile, from LDS or made from its records on each read
+struct LdsRec
 {
-    const double* st;
-    __device__ double4 operator()(int q) const { return make_double4(st[3 * q], st[3 * q + 1], st[3 * q + 2], 1.0); }
+    const uint2* rec;
+    __device__ uint2 operator()(int q) const { return rec[q]; }
+};
+struct GlobalRec
+{
+    GlobalFetch fetch;
+    Grid16 grid16;
+    __device__ uint2 operator()(int q) const
+    {
+        bool outside = false;
+        return grid16(fetch(q), outside);
+    }
 };
 
-// Full rows of one tile of a flagged replica, one lane per row, as the single-system build
-// forms them: per stencil column the cells that Cabana's min-distance prune keeps (one run
-// in z), cut by binary search to the z window of the row (records are z-sorted in a staged
-// column), 32 candidates per pass in groups of four with the hit bits shifted in by a
-// funnel shift, then the hits appended in slot order.  Entries are staged slots; rows are
-// padded to whole chunks with the row's own slot (distance 0, which the forces skip).
-template <int SH, class Fetch>
+// Full rows of one tile of a flagged replica, as the single-system build forms them: three lanes
+// share a row, one per j offset of the stencil, and walk the three i offsets together, so a row's
+// columns come in i, j order; per column the cells that Cabana's min-distance prune keeps (one
+// run in z), cut by binary search to the z window of the row, 32 candidates per pass tested on
+// 16-bit coordinates, those within the rounding of r_n in FP64; hits appended in slot order.
+// Entries are staged slots; rows are padded to whole chunks with the row's own slot (distance 0,
+// which the forces skip).  BUF: rows are collected in LDS (rowBuf, the wave's) and stored as
+// 16-byte chunks, else entry by entry.  What bounds the single-system kernel bounds this one
+// (vector issue), and with few replicas the chain of one row: one lane per row in FP64 took
+// 198 us a step at 2.8 million atoms and 54 at 31,000.
+template <bool BUF, class Rec>
 __device__ void bBuildRows(const BS& b, const TileB& ti, const TileG& G, const RepD& R, const int* cstart,
-                           const Fetch& fetch)
+                           const Rec& rec, const Grid16& grid16, bool exactAll, uint16_t* rowBuf)
 {
-    const int spanJ = G.nj + 2;
-    const int64_t chunkStride = b.strideS * CHUNK;
+    constexpr int S = 3, RW = WAVE / S;
+    const int lane = int(threadIdx.x) % WAVE, waves = int(blockDim.x) / WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int spanJ = G.nj + 2, cap = b.capList;
+    const int sh = entryShift(!bFits(b, R, ti));
     const double rsq = b.rnSqr;
+    int sure, doubt;
+    grid16.thresholds(b.rn, sure, doubt);
+    const GlobalFetch exact{&ti, b.sortedPos, R.L[0], R.L[1], R.L[2]};
+    const int sub = lane % S, group = lane / S, first = group * S;
     int localMax = 0;
-    for (int t = threadIdx.x; t < ti.nrows; t += blockDim.x)
+    for (int row0 = wave * RW; row0 < ti.nrows; row0 += waves * RW)
     {
+        const int row = row0 + group;
+        const bool live = group < RW && row < ti.nrows;
         int sc;
-        const int s = bTileRow(ti, t, sc);
+        const int s = bTileRow(ti, live ? row : 0, sc);
         const int pr = ti.selfPiece[sc];
         const int qSelf = ti.base[pr] + (s - ti.begin[pr]);
-        const double4 xp = fetch(qSelf);
-        const int kz = (b.cellOf[b.sorted[s]] - R.c0) % R.nc[2];
+        const double4 xp = b.sortedPos[s];  // (a self column's records are unshifted)
+        const uint2 own = rec(qSelf);
+        const Short2 ownXY = asShort2(own.x), ownZ = asShort2(own.y);
+        const int zq = int(int16_t(own.y));
+        const int kz = locate(xp.z, R.rdxc[2], R.nc[2]);
         const int sa = sc / G.nj, sb = sc % G.nj;
         const int i = G.i0 + sa, j = G.j0 + sb;
-        // per-axis distances from the row to the stencil cells' boxes (unwrapped indices) and
-        // the lateral terms of the z window, shrunk by 1e-9 of a cell
-        double rx2[3], ry2[3], wx2[3], wy2[3], rz2[3];
+        // squared distances from the row to the stencil cells' boxes (unwrapped indices), and the
+        // lateral terms of the z window, shrunk by 1e-9 of a cell
+        auto boxDistSqr = [&](double x, int cell, int d, double shrink) {
+            const double c = (double(cell) + 0.5) * R.dxc[d];
+            double r = fabs(x - c) - 0.5 * R.dxc[d] - shrink;
+            r = r > 0.0 ? r : 0.0;
+            return r * r;
+        };
+        const double ry2 = boxDistSqr(xp.y, j - 1 + sub, 1, 0.0),
+                     wy2 = boxDistSqr(xp.y, j - 1 + sub, 1, 1e-9 * R.dxc[1]);
+        double rz2[3];
 #pragma unroll
-        for (int a = 0; a < 3; ++a)
-        {
-            const double cx = (double(i - 1 + a) + 0.5) * R.dxc[0];
-            const double cy = (double(j - 1 + a) + 0.5) * R.dxc[1];
-            const double cz = (double(kz - 1 + a) + 0.5) * R.dxc[2];
-            double r = fabs(xp.x - cx) - 0.5 * R.dxc[0];
-            r = r > 0.0 ? r : 0.0;
-            rx2[a] = r * r;
-            r = fabs(xp.y - cy) - 0.5 * R.dxc[1];
-            r = r > 0.0 ? r : 0.0;
-            ry2[a] = r * r;
-            r = fabs(xp.z - cz) - 0.5 * R.dxc[2];
-            r = r > 0.0 ? r : 0.0;
-            rz2[a] = r * r;
-            double e = fabs(xp.x - cx) - 0.5 * R.dxc[0] - 1e-9 * R.dxc[0];
-            e = e > 0.0 ? e : 0.0;
-            wx2[a] = e * e;
-            e = fabs(xp.y - cy) - 0.5 * R.dxc[1] - 1e-9 * R.dxc[1];
-            e = e > 0.0 ? e : 0.0;
-            wy2[a] = e * e;
-        }
-        uint16_t* const rowBase = b.nbr + int64_t(s) * CHUNK;
-        int c = 0;
-#pragma unroll
+        for (int dc = 0; dc < 3; ++dc) rz2[dc] = boxDistSqr(xp.z, kz - 1 + dc, 2, 0.0);
+        int n = 0;  // entries of the row so far (the same in its lanes)
+#pragma unroll 1
         for (int da = -1; da <= 1; ++da)
+        {
+            int lo = 0, hi = 0;
+            // z index of the staged column: cell k of the run is entry k - (k0 - 1)
+            const int* cs = cstart + ((sa + 1 + da) * spanJ + (sb + sub)) * (B_SPAN + 1) - (G.k0 - 1);
+            const double lat = boxDistSqr(xp.x, i + da, 0, 0.0) + ry2;
+            int kLo = INT_MAX, kHi = INT_MIN;
 #pragma unroll
-            for (int db = -1; db <= 1; ++db)
+            for (int dc = 0; dc < 3; ++dc)
+                if (lat + rz2[dc] <= rsq)
+                {
+                    kLo = min(kLo, kz - 1 + dc);
+                    kHi = kz - 1 + dc;
+                }
+            if (live && kLo <= kHi)
             {
-                // z index of the staged column: cell k of the run is entry k - (k0 - 1)
-                const int* cs = cstart + ((sa + 1 + da) * spanJ + (sb + 1 + db)) * (B_SPAN + 1) - (G.k0 - 1);
-                const double lat = rx2[da + 1] + ry2[db + 1];
-                int kLo = INT_MAX, kHi = INT_MIN;
-#pragma unroll
-                for (int dc = 0; dc < 3; ++dc)
-                    if (lat + rz2[dc] <= rsq)
-                    {
-                        kLo = min(kLo, kz - 1 + dc);
-                        kHi = kz - 1 + dc;
-                    }
-                if (kLo > kHi) continue;
-                const double zsq = rsq - (wx2[da + 1] + wy2[db + 1]) + 1e-12 * rsq;
-                int lo = cs[kLo], hi = cs[kLo + 1];
-                while (lo < hi)
+                const double zsq = rsq - (boxDistSqr(xp.x, i + da, 0, 1e-9 * R.dxc[0]) + wy2) + 1e-12 * rsq;
+                const int reach = zsq >= 0.0 ? int(sqrtf(float(zsq)) * float(grid16.scale) * 1.00001f) + 2 : -1;
+                if (reach >= 0)
                 {
-                    const int m = (lo + hi) >> 1;
-                    const double dz = xp.z - fetch(m).z;
-                    if (dz > 0.0 && dz * dz > zsq) lo = m + 1;
-                    else hi = m;
-                }
-                const int wlo = lo;
-                lo = max(wlo, cs[kHi]);
-                hi = cs[kHi + 1];
-                while (lo < hi)
-                {
-                    const int m = (lo + hi) >> 1;
-                    const double dz = xp.z - fetch(m).z;
-                    if (dz < 0.0 && dz * dz > zsq) hi = m;
-                    else lo = m + 1;
-                }
-                const int whi = lo;
-                for (int qb = wlo; qb < whi; qb += 32)
-                {
-                    uint32_t miss = 0;
-                    const int nq = min(32, whi - qb);
-                    int m = 0;
-                    for (; m < nq; m += 4)
+                    int x = cs[kLo], y = cs[kLo + 1];
+                    while (x < y)
                     {
-#pragma unroll
-                        for (int u = 0; u < 4; ++u)
-                        {
-                            const double4 xn = fetch(qb + m + u);
-                            const double dx = xp.x - xn.x, dy = xp.y - xn.y, dz = xp.z - xn.z;
-                            const double r2 = dx * dx + dy * dy + dz * dz;
-                            miss = __builtin_amdgcn_alignbit(miss, uint32_t(__double2hiint(rsq - r2)), 31u);
-                        }
+                        const int m = (x + y) >> 1;
+                        if (int(int16_t(rec(m).y)) < zq - reach) x = m + 1;
+                        else y = m;
                     }
-                    uint32_t hits = ~miss << (32 - m);
-                    hits &= ~((1u << (32 - nq)) - 1u);
-                    if (qSelf >= qb && qSelf < qb + nq) hits &= ~(0x80000000u >> (qSelf - qb));
-                    while (hits)
+                    lo = x;
+                    x = max(lo, cs[kHi]);
+                    y = cs[kHi + 1];
+                    while (x < y)
                     {
-                        const int u = __builtin_clz(hits);
-                        hits ^= 0x80000000u >> u;
-                        if (c < b.capList) rowBase[int64_t(c >> 3) * chunkStride + (c & 7)] = uint16_t((qb + u) << SH);
-                        ++c;
+                        const int m = (x + y) >> 1;
+                        if (int(int16_t(rec(m).y)) > zq + reach) y = m;
+                        else x = m + 1;
                     }
+                    hi = x;
                 }
             }
-        for (int k = c; k < ((c + CHUNK - 1) / CHUNK) * CHUNK && k < b.capList; ++k)
-            rowBase[int64_t(k >> 3) * chunkStride + (k & 7)] = uint16_t(qSelf << SH);
-        b.cnt[s] = min(c, b.capList);  // an overflow is reported through err; reads stay in the list
-        localMax = max(localMax, c);
+            // the hits among up to 32 candidates from qb, candidate u at bit 31 - u
+            auto test = [&](int qb) -> uint32_t {
+                const int nq = min(32, hi - qb);
+                if (nq <= 0) return 0u;
+                uint32_t near = 0, maybe = 0;
+                int m = 0;
+                for (; m < nq; m += 4)
+                {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                    {
+                        const uint2 w = rec(qb + m + u);
+                        const int over = dotSelf(ownZ - asShort2(w.y), dotSelf(ownXY - asShort2(w.x), -sure - 1));
+                        near = __builtin_amdgcn_alignbit(near, uint32_t(over), 31u);
+                        maybe = __builtin_amdgcn_alignbit(maybe, uint32_t(over - doubt), 31u);
+                    }
+                }
+                const int up = 32 - m;  // m is 4..32
+                uint32_t valid = ~((1u << (32 - nq)) - 1u);
+                if (qSelf >= qb && qSelf < qb + nq) valid &= ~(0x80000000u >> (qSelf - qb));
+                uint32_t hits = (near << up) & valid;
+                uint32_t unsure = ((maybe & ~near) << up) & valid;
+                if (exactAll)
+                {
+                    hits = 0;
+                    unsure = valid;
+                }
+                while (unsure)
+                {
+                    const int u = __builtin_clz(unsure);
+                    const uint32_t bit = 0x80000000u >> u;
+                    unsure ^= bit;
+                    const double4 xn = exact(qb + u);
+                    const double dx = xp.x - xn.x, dy = xp.y - xn.y, dz = xp.z - xn.z;
+                    hits = dx * dx + dy * dy + dz * dz <= rsq ? hits | bit : hits & ~bit;
+                }
+                return hits;
+            };
+            const uint32_t hits0 = test(lo), hits1 = test(lo + 32);
+            int mine = __builtin_popcount(hits0) + __builtin_popcount(hits1);
+            const bool longRun = __any(hi - lo > 64);  // (dense inputs: the rest is tested twice)
+            if (longRun)
+                for (int qb = lo + 64; qb < hi; qb += 32) mine += __builtin_popcount(test(qb));
+            // places: behind the row's entries so far and those of the lanes before this one
+            int at = n, total = 0;
+#pragma unroll
+            for (int k = 0; k < S; ++k)
+            {
+                const int c = __shfl(mine, first + k, WAVE);
+                at += k < sub ? c : 0;
+                total += c;
+            }
+            auto append = [&](int qb, uint32_t hits) {
+                while (hits)
+                {
+                    const int u = __builtin_clz(hits);
+                    hits ^= 0x80000000u >> u;
+                    const uint16_t v = uint16_t((qb + u) << sh);
+                    if (at < cap)
+                    {
+                        if constexpr (BUF)
+                            rowBuf[group * cap + at] = v;
+                        else
+                            b.nbr[(int64_t(at >> 3) * b.strideS + s) * CHUNK + (at & 7)] = v;
+                    }
+                    ++at;
+                }
+            };
+            append(lo, hits0);
+            append(lo + 32, hits1);
+            if (longRun)
+                for (int qb = lo + 64; qb < hi; qb += 32) append(qb, test(qb));
+            n += total;
+        }
+        const int kept = min(n, cap), nch = (kept + CHUNK - 1) / CHUNK;
+        if (live)
+            for (int k = kept + sub; k < nch * CHUNK; k += S)
+            {
+                if constexpr (BUF)
+                    rowBuf[group * cap + k] = uint16_t(qSelf << sh);
+                else
+                    b.nbr[(int64_t(k >> 3) * b.strideS + s) * CHUNK + (k & 7)] = uint16_t(qSelf << sh);
+            }
+        if (live && sub == 0) b.cnt[s] = kept;  // an overflow is reported through err; reads stay in the list
+        localMax = max(localMax, live ? n : 0);
+        if constexpr (BUF)
+        {
+            // the wave's rows go out chunk by chunk, neighbouring rows from neighbouring lanes
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            const int chunks = RW * waveMaxInt(live ? nch : 0);
+            for (int x = lane; x - lane < chunks; x += WAVE)
+            {
+                const int r = x % RW, ch = x / RW;
+                const int sr = __shfl(s, r * S, WAVE), nr = __shfl(live ? nch : 0, r * S, WAVE);
+                if (ch < nr)
+                    reinterpret_cast<uint4*>(b.nbr)[int64_t(ch) * b.strideS + sr] =
+                        reinterpret_cast<const uint4*>(rowBuf + r * cap)[ch];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        }
     }
     if (localMax > b.capList) atomicOr(b.err, 1);
 }
 
-// full-row list of every tile of a flagged replica
-__global__ __launch_bounds__(BLOCK) void k_bBuild(BS b)
+// full-row list of every tile of a flagged replica; BUF: the launch's LDS holds the
+// waves' row buffers behind the records
+template <bool BUF>
+__global__ __launch_bounds__(BLOCK, 4) void k_bBuild(BS b)
 {
-    extern __shared__ double stb[];
+    extern __shared__ double4 stLds[];
     __shared__ TileB ti;
     __shared__ int cstart[B_STEN * B_STEN * (B_SPAN + 1)];
+    __shared__ int wild;
     // plain block order: when only some replicas rebuild, their tiles are contiguous, and the
     // hardware's round-robin of consecutive workgroups over the XCDs spreads them over all
     // eight (grouping consecutive tiles on one XCD would put a whole replica on one)
@@ -757,9 +847,10 @@ __global__ __launch_bounds__(BLOCK) void k_bBuild(BS b)
     const TileG G = b.tg[t];
     if (!b.flag[G.rep]) return;
     loadTileB(ti, b.tiles, t);
+    if (threadIdx.x == 0) wild = 0;
     __syncthreads();
     if (ti.nrows == 0) return;
-    const RepD R = b.reps[G.rep];
+    const RepD& R = b.reps[G.rep];
     if (!ti.near)
     {
         for (int t = threadIdx.x; t < ti.nrows; t += blockDim.x)
@@ -769,36 +860,46 @@ __global__ __launch_bounds__(BLOCK) void k_bBuild(BS b)
         }
         return;
     }
-    const bool fits = bFits(b, R, ti);
-    if (fits)
-        stageShifted(ti, b.sortedPos, R, [&](int q, const double4& v) {
-            stb[3 * q] = v.x;
-            stb[3 * q + 1] = v.y;
-            stb[3 * q + 2] = v.z;
-        });
-    // LDS slot of the first record of cell k0 - 1 + z of each staged column
     const int nzr = G.k1 - G.k0 + 2;
     const int spanJ = G.nj + 2, ncol = (G.ni + 2) * spanJ;
-    for (int col = threadIdx.x; col < ncol; col += blockDim.x)
+    const Grid16 grid16{double(G.i0 - 1) * R.dxc[0], double(G.j0 - 1) * R.dxc[1], double(G.k0 - 1) * R.dxc[2],
+                        QUANT_RANGE / fmax(fmax(double(G.ni + 2) * R.dxc[0], double(spanJ) * R.dxc[1]),
+                                           double(nzr) * R.dxc[2])};
+    uint2* const rec = reinterpret_cast<uint2*>(stLds);
+    const bool staged = ti.staged <= b.buildCap;
+    bool outside = !staged;
+    if (staged)
+        stageShifted(ti, b.sortedPos, R, [&](int q, const double4& v) { rec[q] = grid16(v, outside); });
+    if (outside) wild = 1;
+    // LDS slot of the first record of cell k0 - 1 + z of each staged column, whose pieces are cell
+    // nz - 1 below the box, the run from max(k0 - 1, 0) inside it and cell 0 above it
+    for (int x = threadIdx.x; x < ncol * (nzr + 1); x += blockDim.x)
     {
+        const int col = x / (nzr + 1), z = x % (nzr + 1);
         int ii = G.i0 - 1 + col / spanJ, jj = G.j0 - 1 + col % spanJ;
         ii = ii < 0 ? ii + R.nc[0] : (ii >= R.nc[0] ? ii - R.nc[0] : ii);
         jj = jj < 0 ? jj + R.nc[1] : (jj >= R.nc[1] ? jj - R.nc[1] : jj);
-        int run = ti.colBase[col];
-        for (int z = 0; z < nzr; ++z)
+        const int kz = G.k0 - 1 + z, last = cellIndex(R, ii, jj, R.nc[2] - 1);
+        int v = ti.colBase[col];
+        if (z == nzr)
+            v = col + 1 < ncol ? ti.colBase[col + 1] : ti.staged;
+        else if (kz >= 0)
         {
-            int kz = G.k0 - 1 + z;
-            kz = kz < 0 ? kz + R.nc[2] : (kz >= R.nc[2] ? kz - R.nc[2] : kz);
-            cstart[col * (B_SPAN + 1) + z] = run;
-            run += b.counts[cellIndex(R, ii, jj, kz)];
+            if (G.k0 == 0) v += b.counts[last];
+            v += (kz < R.nc[2] ? b.offsets[cellIndex(R, ii, jj, kz)] : b.offsets[last] + b.counts[last]) -
+                 b.offsets[cellIndex(R, ii, jj, max(G.k0 - 1, 0))];
         }
-        cstart[col * (B_SPAN + 1) + nzr] = run;
+        cstart[col * (B_SPAN + 1) + z] = v;
     }
     __syncthreads();
-    if (fits)
-        bBuildRows<entryShift(false)>(b, ti, G, R, cstart, LdsFetch3{stb});
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    uint16_t* const rowBuf = reinterpret_cast<uint16_t*>(rec + (b.buildCap + B_PAD + 1) / 2 * 2) + wave * (WAVE / 3) * b.capList;
+    if (staged)
+        bBuildRows<BUF>(b, ti, G, R, cstart, LdsRec{rec}, grid16, wild != 0, rowBuf);
     else
-        bBuildRows<entryShift(true)>(b, ti, G, R, cstart, GlobalFetch{&ti, b.sortedPos, R.L[0], R.L[1], R.L[2]});
+        bBuildRows<false>(b, ti, G, R, cstart,
+                          GlobalRec{GlobalFetch{&ti, b.sortedPos, R.L[0], R.L[1], R.L[2]}, grid16}, grid16, true,
+                          nullptr);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1265,7 +1366,9 @@ BS mrmd_batch::state()
     b.err = err.p;
     b.lj = lj;
     b.rcSqr = rc * rc;
+    b.rn = rc + skin;
     b.rnSqr = (rc + skin) * (rc + skin);
+    b.buildCap = stageCapBuild;
     return b;
 }
 
@@ -1367,6 +1470,9 @@ void mrmd_batch::enqueueSteps(int64_t n)
     const unsigned ga = gridFor(natoms), gc = gridFor(ncells);
     const unsigned gs = unsigned((ncells * SORT_GROUP + BLOCK - 1) / BLOCK);
     const unsigned nr = unsigned(reps.size());
+    // the build's LDS: 16-bit records, then the waves' row buffers where all fit
+    const size_t buildRecs = size_t(stageCapBuild + B_PAD + 1) / 2 * 2 * sizeof(uint2);
+    const size_t buildLds = buildRecs + size_t(block / WAVE * (WAVE / 3)) * capList * sizeof(uint16_t);
     hipLaunchKernelGGL(k_bPre<false>, dim3(ga), dim3(BLOCK), 0, c->stream, b);
     for (int64_t k = 0; k < n; ++k)
     {
@@ -1382,8 +1488,10 @@ void mrmd_batch::enqueueSteps(int64_t n)
         hipLaunchKernelGGL(k_bTiles, dim3(unsigned((ntiles + BLOCK / WAVE - 1) / (BLOCK / WAVE))), dim3(BLOCK), 0,
                            c->stream, b);
         hipLaunchKernelGGL(k_bGather, dim3(ga), dim3(BLOCK), 0, c->stream, b);
-        hipLaunchKernelGGL(k_bBuild, dim3(unsigned(ntiles)), dim3(block), size_t(stageCapBuild + B_PAD) * 24, c->stream,
-                           b);
+        if (buildLds <= B_BUILD_LDS)
+            hipLaunchKernelGGL(k_bBuild<true>, dim3(unsigned(ntiles)), dim3(block), buildLds, c->stream, b);
+        else
+            hipLaunchKernelGGL(k_bBuild<false>, dim3(unsigned(ntiles)), dim3(block), buildRecs, c->stream, b);
         auto force = [&](auto kernel, int64_t t0, int64_t t1, size_t lds) {
             if (t1 <= t0) return;
             BS f = b;

@@ -341,6 +341,43 @@ __device__ inline void sortCellByZ(int32_t* recs, int n, const double4* __restri
     }
 }
 
+// 16-bit coordinates of the list builds' candidate tests: units of 1/scale from (ox, oy, oz), the
+// tile's neighbourhood QUANT_RANGE units long, {x << 16 | y, z} in 8 bytes.  A coordinate is rounded by
+// at most half a unit, so the distance of two records is off by at most sqrt(3) units: with
+// doubt = QUANT_DOUBT units more, d^2 <= sure is a neighbour, d^2 >= sure + doubt none.
+typedef short Short2 __attribute__((ext_vector_type(2)));
+__device__ inline Short2 asShort2(uint32_t v)
+{
+    return __builtin_bit_cast(Short2, v);
+}
+// a.x^2 + a.y^2 + c
+__device__ inline int dotSelf(Short2 a, int c) { return __builtin_amdgcn_sdot2(a, a, c, false); }
+constexpr double QUANT_RANGE = 32000.0;
+constexpr double QUANT_DOUBT = 1.75;
+struct Grid16
+{
+    double ox, oy, oz, scale;
+    /// outside: set for a record beyond the neighbourhood's range (or not a number), which no
+    /// 16-bit test may decide
+    __device__ uint2 operator()(const double4& v, bool& outside) const
+    {
+        const double u[3] = {(v.x - ox) * scale, (v.y - oy) * scale, (v.z - oz) * scale};
+        int c[3];
+        for (int d = 0; d < 3; ++d)
+        {
+            outside = outside || !(u[d] > -2.0 && u[d] < QUANT_RANGE + 2.0);
+            c[d] = int(rint(fmin(fmax(u[d], -512.0), QUANT_RANGE + 512.0)));
+        }
+        return make_uint2((uint32_t(c[0]) << 16) | (uint32_t(c[1]) & 0xffffu), uint32_t(c[2]) & 0xffffu);
+    }
+    __device__ void thresholds(double rn, int& sure, int& doubt) const
+    {
+        const double rnq = rn * scale;
+        sure = int(floor((rnq - QUANT_DOUBT) * (rnq - QUANT_DOUBT)));
+        doubt = int(ceil((rnq + QUANT_DOUBT) * (rnq + QUANT_DOUBT))) - sure;
+    }
+};
+
 // copy the tile's neighbourhood (contiguous runs of sorted slots) into LDS: each wave takes
 // every fourth run, four runs at a time, so that run starts and lengths are wave-uniform
 // (scalar) and a lane has four independent loads in flight; looking up the run of each record

@@ -154,16 +154,7 @@ constexpr size_t LDS_LIMIT = 64000;  // dynamic LDS of a list build workgroup (6
 // WIDE: list offsets in 64-bit arithmetic (lists of 2^31 entries or more); 32-bit otherwise
 // GS (dense inputs): the 16-bit records in the tile's slice of global memory, entries stored
 // one by one
-typedef short Short2 __attribute__((ext_vector_type(2)));
-__device__ inline Short2 asShort2(uint32_t v)
-{
-    return __builtin_bit_cast(Short2, v);
-}
-// a.x^2 + a.y^2 + c
-__device__ inline int dotSelf(Short2 a, int c) { return __builtin_amdgcn_sdot2(a, a, c, false); }
 constexpr int BUILD_BLOCK = 12 * WAVE;
-constexpr double QUANT_RANGE = 32000.0;
-constexpr double QUANT_DOUBT = 1.75;
 
 // (5 waves per SIMD: 96 registers; with 98 it measured 1.14 instead of 1.08 ms at 4M atoms)
 template <int R, bool WIDE, bool GS>
@@ -228,19 +219,12 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
         QUANT_RANGE / fmax(fmax(double(span) * g.dx[0], double(span) * g.dx[1]), double(tg.K + 2 * R) * g.dx[2]);
     const double ox = g.min[0] + double(i0 - R) * g.dx[0], oy = g.min[1] + double(j0 - R) * g.dx[1],
                  oz = g.min[2] + double(k0 - R) * g.dx[2];
-    const double rnq = rn * scale;
-    const int sure = int(floor((rnq - QUANT_DOUBT) * (rnq - QUANT_DOUBT)));  // d^2 <= sure: a neighbour
-    const int doubt = int(ceil((rnq + QUANT_DOUBT) * (rnq + QUANT_DOUBT))) - sure;  // d^2 < sure + doubt: perhaps
+    const Grid16 grid16{ox, oy, oz, scale};
+    int sure, doubt;
+    grid16.thresholds(rn, sure, doubt);
     bool outside = false;
     stageRecords(ti, sortedPos, [&](int q, const double4& v, int) {
-        const double u[3] = {(v.x - ox) * scale, (v.y - oy) * scale, (v.z - oz) * scale};
-        int c[3];
-        for (int d = 0; d < 3; ++d)
-        {
-            outside = outside || !(u[d] > -2.0 && u[d] < QUANT_RANGE + 2.0);
-            c[d] = int(rint(fmin(fmax(u[d], -512.0), QUANT_RANGE + 512.0)));
-        }
-        rec[q] = make_uint2((uint32_t(c[0]) << 16) | (uint32_t(c[1]) & 0xffffu), uint32_t(c[2]) & 0xffffu);
+        rec[q] = grid16(v, outside);
     });
     if (outside) wild = 1;
     for (int x = threadIdx.x; x < ti.nr * (nk + 1); x += blockDim.x)
