@@ -43,7 +43,7 @@ constexpr int B_SELF = B_COLS * B_COLS;
 constexpr int B_SPAN = 18;         // cells of a tile's column run (K + 2), so K <= 16
 constexpr int TARGET_STAGED = 1400;  // staged records wanted per tile
 constexpr int B_ROW_LANES = 256;   // lanes that the force kernel lays a tile's rows out for
-constexpr size_t B_BUILD_LDS = 60000;  // dynamic LDS of a build workgroup (64 KB less its static part)
+constexpr int B_BUILD_BLOCK = 8 * WAVE;
 constexpr int B_PAD = 4;           // staged records past the neighbourhood a candidate group may read
 constexpr int COMP_BINS = 200;     // LJ_IdealGas compensation bins (LJ_IdealGas.hpp:54)
 constexpr double COMP_SCALE = 4294967296.0;
@@ -639,13 +639,15 @@ struct GlobalRec
 // run in z), cut by binary search to the z window of the row, 32 candidates per pass tested on
 // 16-bit coordinates, those within the rounding of r_n in FP64; hits appended in slot order.
 // Entries are staged slots; rows are padded to whole chunks with the row's own slot (distance 0,
-// which the forces skip).  BUF: rows are collected in LDS (rowBuf, the wave's) and stored as
-// 16-byte chunks, else entry by entry.  What bounds the single-system kernel bounds this one
-// (vector issue), and with few replicas the chain of one row: one lane per row in FP64 took
-// 198 us a step at 2.8 million atoms and 54 at 31,000.
-template <bool BUF, class Rec>
+// which the forces skip).  Only the flagged replicas' tiles build, a few thousand at a time, so
+// the chain of one tile weighs more than the vector issue that bounds the single-system kernel:
+// eight waves to a tile, so that most tiles are one or two rounds of rows, and entries stored one
+// by one (rows collected in LDS as there leave room for half the waves).  At 2.8 million atoms in
+// 256 replicas one lane per row in FP64 took 198 us a step, this with rows collected by four waves
+// 169, with twelve waves 181, as it is 155; at 31,000 in 24 replicas 54, 49, 28 and 33.
+template <class Rec>
 __device__ void bBuildRows(const BS& b, const TileB& ti, const TileG& G, const RepD& R, const int* cstart,
-                           const Rec& rec, const Grid16& grid16, bool exactAll, uint16_t* rowBuf)
+                           const Rec& rec, const Grid16& grid16, bool exactAll)
 {
     constexpr int S = 3, RW = WAVE / S;
     const int lane = int(threadIdx.x) % WAVE, waves = int(blockDim.x) / WAVE;
@@ -785,13 +787,7 @@ __device__ void bBuildRows(const BS& b, const TileB& ti, const TileG& G, const R
                     const int u = __builtin_clz(hits);
                     hits ^= 0x80000000u >> u;
                     const uint16_t v = uint16_t((qb + u) << sh);
-                    if (at < cap)
-                    {
-                        if constexpr (BUF)
-                            rowBuf[group * cap + at] = v;
-                        else
-                            b.nbr[(int64_t(at >> 3) * b.strideS + s) * CHUNK + (at & 7)] = v;
-                    }
+                    if (at < cap) b.nbr[entryIndex(at, s, b.strideS)] = v;
                     ++at;
                 }
             };
@@ -804,37 +800,15 @@ __device__ void bBuildRows(const BS& b, const TileB& ti, const TileG& G, const R
         const int kept = min(n, cap), nch = (kept + CHUNK - 1) / CHUNK;
         if (live)
             for (int k = kept + sub; k < nch * CHUNK; k += S)
-            {
-                if constexpr (BUF)
-                    rowBuf[group * cap + k] = uint16_t(qSelf << sh);
-                else
-                    b.nbr[(int64_t(k >> 3) * b.strideS + s) * CHUNK + (k & 7)] = uint16_t(qSelf << sh);
-            }
+                b.nbr[entryIndex(k, s, b.strideS)] = uint16_t(qSelf << sh);
         if (live && sub == 0) b.cnt[s] = kept;  // an overflow is reported through err; reads stay in the list
         localMax = max(localMax, live ? n : 0);
-        if constexpr (BUF)
-        {
-            // the wave's rows go out chunk by chunk, neighbouring rows from neighbouring lanes
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            const int chunks = RW * waveMaxInt(live ? nch : 0);
-            for (int x = lane; x - lane < chunks; x += WAVE)
-            {
-                const int r = x % RW, ch = x / RW;
-                const int sr = __shfl(s, r * S, WAVE), nr = __shfl(live ? nch : 0, r * S, WAVE);
-                if (ch < nr)
-                    reinterpret_cast<uint4*>(b.nbr)[int64_t(ch) * b.strideS + sr] =
-                        reinterpret_cast<const uint4*>(rowBuf + r * cap)[ch];
-            }
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        }
     }
     if (localMax > b.capList) atomicOr(b.err, 1);
 }
 
-// full-row list of every tile of a flagged replica; BUF: the launch's LDS holds the
-// waves' row buffers behind the records
-template <bool BUF>
-__global__ __launch_bounds__(BLOCK, 4) void k_bBuild(BS b)
+// full-row list of every tile of a flagged replica
+__global__ __launch_bounds__(B_BUILD_BLOCK, 4) void k_bBuild(BS b)
 {
     extern __shared__ double4 stLds[];
     __shared__ TileB ti;
@@ -860,12 +834,12 @@ __global__ __launch_bounds__(BLOCK, 4) void k_bBuild(BS b)
         }
         return;
     }
+    uint2* const rec = reinterpret_cast<uint2*>(stLds);
     const int nzr = G.k1 - G.k0 + 2;
     const int spanJ = G.nj + 2, ncol = (G.ni + 2) * spanJ;
     const Grid16 grid16{double(G.i0 - 1) * R.dxc[0], double(G.j0 - 1) * R.dxc[1], double(G.k0 - 1) * R.dxc[2],
                         QUANT_RANGE / fmax(fmax(double(G.ni + 2) * R.dxc[0], double(spanJ) * R.dxc[1]),
                                            double(nzr) * R.dxc[2])};
-    uint2* const rec = reinterpret_cast<uint2*>(stLds);
     const bool staged = ti.staged <= b.buildCap;
     bool outside = !staged;
     if (staged)
@@ -892,14 +866,11 @@ __global__ __launch_bounds__(BLOCK, 4) void k_bBuild(BS b)
         cstart[col * (B_SPAN + 1) + z] = v;
     }
     __syncthreads();
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    uint16_t* const rowBuf = reinterpret_cast<uint16_t*>(rec + (b.buildCap + B_PAD + 1) / 2 * 2) + wave * (WAVE / 3) * b.capList;
     if (staged)
-        bBuildRows<BUF>(b, ti, G, R, cstart, LdsRec{rec}, grid16, wild != 0, rowBuf);
+        bBuildRows(b, ti, G, R, cstart, LdsRec{rec}, grid16, wild != 0);
     else
-        bBuildRows<false>(b, ti, G, R, cstart,
-                          GlobalRec{GlobalFetch{&ti, b.sortedPos, R.L[0], R.L[1], R.L[2]}, grid16}, grid16, true,
-                          nullptr);
+        bBuildRows(b, ti, G, R, cstart, GlobalRec{GlobalFetch{&ti, b.sortedPos, R.L[0], R.L[1], R.L[2]}, grid16},
+                   grid16, true);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1470,9 +1441,6 @@ void mrmd_batch::enqueueSteps(int64_t n)
     const unsigned ga = gridFor(natoms), gc = gridFor(ncells);
     const unsigned gs = unsigned((ncells * SORT_GROUP + BLOCK - 1) / BLOCK);
     const unsigned nr = unsigned(reps.size());
-    // the build's LDS: 16-bit records, then the waves' row buffers where all fit
-    const size_t buildRecs = size_t(stageCapBuild + B_PAD + 1) / 2 * 2 * sizeof(uint2);
-    const size_t buildLds = buildRecs + size_t(block / WAVE * (WAVE / 3)) * capList * sizeof(uint16_t);
     hipLaunchKernelGGL(k_bPre<false>, dim3(ga), dim3(BLOCK), 0, c->stream, b);
     for (int64_t k = 0; k < n; ++k)
     {
@@ -1488,10 +1456,8 @@ void mrmd_batch::enqueueSteps(int64_t n)
         hipLaunchKernelGGL(k_bTiles, dim3(unsigned((ntiles + BLOCK / WAVE - 1) / (BLOCK / WAVE))), dim3(BLOCK), 0,
                            c->stream, b);
         hipLaunchKernelGGL(k_bGather, dim3(ga), dim3(BLOCK), 0, c->stream, b);
-        if (buildLds <= B_BUILD_LDS)
-            hipLaunchKernelGGL(k_bBuild<true>, dim3(unsigned(ntiles)), dim3(block), buildLds, c->stream, b);
-        else
-            hipLaunchKernelGGL(k_bBuild<false>, dim3(unsigned(ntiles)), dim3(block), buildRecs, c->stream, b);
+        hipLaunchKernelGGL(k_bBuild, dim3(unsigned(ntiles)), dim3(B_BUILD_BLOCK),
+                           size_t(stageCapBuild + B_PAD) * sizeof(uint2), c->stream, b);
         auto force = [&](auto kernel, int64_t t0, int64_t t1, size_t lds) {
             if (t1 <= t0) return;
             BS f = b;
