@@ -119,10 +119,9 @@ struct BS
     int32_t* fill;
     int32_t* sorted;
     int32_t* id;       ///< the atom's index in the ensemble as given (atoms move to slot order)
-    int32_t* tmpA;     ///< permutation scratch (given indices, cells)
-    int32_t* tmpB;
+    int32_t* tmpA;     ///< permutation scratch (given indices)
     double* tmpVel;
-    double4* sortedPos;
+    double4* sortedPos;  ///< permutation scratch (positions)
     double* slotLam;
     double* slotGrad;
     const TileG* tg;
@@ -162,6 +161,21 @@ __device__ inline int locate(double x, double rdx, int n)
 
 // ---------------------------------------------------------------------------------------
 // integration
+
+// the record's slab weight into w (1 in a plain replica), and the weighting's value and gradient,
+// which are read for hybrid records only (0 < weight < 1); places are atoms' and slots' alike
+__device__ inline void slabWeight(const BS& b, const RepD& R, int64_t i, double4& p)
+{
+    p.w = 1.0;
+    if (!R.adress) return;
+    double lam, g;
+    slabEval(R.slab, p.x, lam, p.w, g);
+    if (p.w > 0.0 && p.w < 1.0)
+    {
+        b.slotLam[i] = lam;
+        b.slotGrad[i] = g;
+    }
+}
 
 // VelocityVerletLangevinThermostat::preForceIntegrate (VelocityVerletLangevinThermostat.hpp:63-136);
 // POST: the previous step's post-force integration (k_bPost) first, in the same pass: the
@@ -238,6 +252,7 @@ __global__ __launch_bounds__(BLOCK) void k_bPre(BS b)
         p.x += dtHalf * vx;
         p.y += dtHalf * vy;
         p.z += dtHalf * vz;
+        slabWeight(b, *R, i, p);
         b.pos[i] = p;
         b.vel[i] = vx;
         b.vel[cap + i] = vy;
@@ -279,80 +294,49 @@ __global__ __launch_bounds__(BLOCK) void k_bPre(BS b)
     }
 }
 
-// rebuild criterion per replica (examples/02_LennardJones_NVE/02_LennardJones_NVE.cpp:138-165)
-__global__ void k_bCheck(BS b)
+// rebuild criterion per replica (examples/02_LennardJones_NVE/02_LennardJones_NVE.cpp:138-165),
+// from the displacements that no kernel changes before k_bScan does
+__device__ inline bool mustRebuild(const BS& b, int r, double& acc)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= b.nrep) return;
-    const double d = sqrt(b.dispStep[r]);
-    b.dispStep[r] = 0.0;
-    const double acc = b.dispAcc[r] + d;
-    if (acc >= b.reps[r].halfSkin)
-    {
-        b.flag[r] = 1;
-        b.dispAcc[r] = 0.0;
-        b.rebuilds[r] += 1;
-    }
-    else
-    {
-        b.flag[r] = 0;
-        b.dispAcc[r] = acc;
-    }
+    acc = b.dispAcc[r] + sqrt(b.dispStep[r]);
+    return acc >= b.reps[r].halfSkin;
 }
 
-// PeriodicMapping::mapIntoDomain (PeriodicMapping.cpp:30-58) on the box [0, L)
-__global__ void k_bWrap(BS b)
-{
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= b.natoms) return;
-    const int r = b.atomRep[i];
-    if (!b.flag[r]) return;
-    const RepD& R = b.reps[r];
-    double4 p = b.pos[i];
-    double x[3] = {p.x, p.y, p.z};
-    for (int d = 0; d < 3; ++d)
-    {
-        if (R.L[d] <= x[d])
-        {
-            x[d] -= R.L[d];
-            x[d] = fmax(x[d], 0.0);
-        }
-        if (x[d] < 0.0)
-        {
-            x[d] += R.L[d];
-            if (R.L[d] <= x[d]) x[d] = 0.0;
-        }
-    }
-    p.x = x[0];
-    p.y = x[1];
-    p.z = x[2];
-    b.pos[i] = p;
-}
-
-// ---------------------------------------------------------------------------------------
-// binning of flagged replicas (stable counting sort per replica)
-
-__global__ void k_bZeroCells(BS b)
-{
-    const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (c >= b.ncells || !b.flag[b.cellRep[c]]) return;
-    b.counts[c] = 0;
-    b.fill[c] = 0;
-}
-
-// atoms sit in cell order after their replica's last rebuild, so a wave's atoms share cells
-// over long runs: one atomic per run (laneRun; valid lanes are a prefix of the wave)
-__global__ void k_bCount(BS b)
+// Replicas that rebuild: PeriodicMapping::mapIntoDomain (PeriodicMapping.cpp:30-58) on the box
+// [0, L), the cell of each atom and the cells' counts (zero before, k_bEnd).  Atoms sit in cell
+// order after their replica's last rebuild, so a wave's atoms share cells over long runs: one
+// atomic per run (laneRun; valid lanes are a prefix of the wave).  (The binning is a stable
+// counting sort per replica.)
+__global__ void k_bWrapCount(BS b)
 {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     int c = -1;
     if (i < b.natoms)
     {
         const int r = b.atomRep[i];
-        if (b.flag[r])
+        double acc;
+        if (mustRebuild(b, r, acc))
         {
             const RepD& R = b.reps[r];
-            const double4 p = b.pos[i];
+            double4 p = b.pos[i];
+            double x[3] = {p.x, p.y, p.z};
+            for (int d = 0; d < 3; ++d)
+            {
+                if (R.L[d] <= x[d])
+                {
+                    x[d] -= R.L[d];
+                    x[d] = fmax(x[d], 0.0);
+                }
+                if (x[d] < 0.0)
+                {
+                    x[d] += R.L[d];
+                    if (R.L[d] <= x[d]) x[d] = 0.0;
+                }
+            }
+            p.x = x[0];
+            p.y = x[1];
+            p.z = x[2];
+            b.pos[i] = p;
             c = cellIndex(R, locate(p.x, R.rdxc[0], R.nc[0]), locate(p.y, R.rdxc[1], R.nc[1]),
                           locate(p.z, R.rdxc[2], R.nc[2]));
             b.cellOf[i] = c;
@@ -362,12 +346,26 @@ __global__ void k_bCount(BS b)
     if (c >= 0 && run.head == int(threadIdx.x) % WAVE) atomicAdd(&b.counts[c], run.len);
 }
 
-// one workgroup (BLOCK threads) per replica: offsets = a0 + exclusive scan of its counts
+// One workgroup (BLOCK threads) per replica: the rebuild decision into flag, the displacements
+// taken up or cleared, and offsets = a0 + exclusive scan of the replica's counts; the step count
+// goes up here, where nothing reads it (bStep).
+__device__ inline int64_t bStep(const BS& b) { return *b.step - 1; }
 __global__ __launch_bounds__(BLOCK) void k_bScan(BS b)
 {
     __shared__ int32_t lds[BLOCK / WAVE];
     const int r = blockIdx.x;
-    if (!b.flag[r]) return;
+    double acc;
+    const bool rebuild = mustRebuild(b, r, acc);
+    __syncthreads();
+    if (threadIdx.x == 0)
+    {
+        if (r == 0) *b.step += 1;
+        b.dispStep[r] = 0.0;
+        b.flag[r] = rebuild ? 1 : 0;
+        b.dispAcc[r] = rebuild ? 0.0 : acc;
+        if (rebuild) b.rebuilds[r] += 1;
+    }
+    if (!rebuild) return;
     const RepD& R = b.reps[r];
     const int ncell = R.nc[0] * R.nc[1] * R.nc[2];
     int32_t carry = int32_t(R.a0);
@@ -395,42 +393,46 @@ __global__ void k_bFill(BS b)
     if (c >= 0) b.sorted[b.offsets[c] + start + (lane - run.head)] = int32_t(i);
 }
 
-// ascending z inside each cell of a flagged replica, the atom's given index breaking ties
-// (the fill order of the atomics is arbitrary, and atoms move): one group of 32 lanes per
-// cell (sortCellByZ)
-__global__ __launch_bounds__(BLOCK) void k_bSortCells(BS b)
+// Ascending z inside each cell of a flagged replica, the atom's given index breaking ties (the fill
+// order of the atomics is arbitrary, and atoms move): one group of 32 lanes per cell
+// (sortCellByZ).  Then the replica's atoms move to that slot order (position, velocity and
+// given index; forces are written by the step's force pass before they are read), so that
+// slots and atoms are the same places: the group gathers them into scratch here, and
+// k_bMoveTiles copies them back.  Results do not depend on where an atom sits: its noise stream
+// follows its given index, and cell-order ties break by it.
+__global__ __launch_bounds__(BLOCK) void k_bSortGather(BS b)
 {
     const int64_t c = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / SORT_GROUP;
     if (c >= b.ncells || !b.flag[b.cellRep[c]]) return;
-    sortCellByZ<true>(b.sorted + b.offsets[c], b.counts[c], b.pos, int(threadIdx.x % SORT_GROUP), b.id);
+    const int lane = int(threadIdx.x % SORT_GROUP);
+    const int base = b.offsets[c], n = b.counts[c];
+    int32_t* recs = b.sorted + base;
+    sortCellByZ<true>(recs, n, b.pos, lane, b.id);
+    // every lane reads back only the places it wrote itself; a crowded cell, sorted by lane 0
+    // alone in memory, is gathered by lane 0 alone
+    const bool serial = n > 4 * SORT_GROUP;
+    if (serial && lane != 0) return;
+    for (int e = serial ? 0 : lane; e < n; e += serial ? 1 : SORT_GROUP)
+    {
+        const int32_t i = recs[e];
+        const int64_t s = base + e;
+        b.sortedPos[s] = b.pos[i];
+        for (int d = 0; d < 3; ++d) b.tmpVel[d * b.cap + s] = b.vel[d * b.cap + i];
+        b.tmpA[s] = b.id[i];
+    }
 }
 
-// A flagged replica's atoms move to its new slot order (position, velocity, given index and
-// cell; forces are written by the step's force pass before they are read), so that the
-// per-step slot gather, the force stores and the next binning run in atom order.  Pass 1
-// gathers into scratch (the slot positions serve for the positions), pass 2 copies back and
-// makes the slot map the identity.  Results do not depend on where an atom sits: its noise
-// stream follows its given index, and cell-order ties break by it.
-__global__ void k_bPermute1(BS b)
+// a flagged replica's atoms back from scratch, with the weights of their wrapped positions
+__device__ inline void bMove(const BS& b, int64_t s)
 {
-    const int64_t s = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (s >= b.natoms || !b.flag[b.atomRep[s]]) return;
-    const int32_t i = b.sorted[s];
-    b.sortedPos[s] = b.pos[i];
-    for (int d = 0; d < 3; ++d) b.tmpVel[d * b.cap + s] = b.vel[d * b.cap + i];
-    b.tmpA[s] = b.id[i];
-    b.tmpB[s] = b.cellOf[i];
-}
-
-__global__ void k_bPermute2(BS b)
-{
-    const int64_t s = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (s >= b.natoms || !b.flag[b.atomRep[s]]) return;
-    b.pos[s] = b.sortedPos[s];
+    if (s >= b.natoms) return;
+    const int r = b.atomRep[s];
+    if (!b.flag[r]) return;
+    double4 p = b.sortedPos[s];
+    slabWeight(b, b.reps[r], s, p);
+    b.pos[s] = p;
     for (int d = 0; d < 3; ++d) b.vel[d * b.cap + s] = b.tmpVel[d * b.cap + s];
     b.id[s] = b.tmpA[s];
-    b.cellOf[s] = b.tmpB[s];
-    b.sorted[s] = int32_t(s);
 }
 
 // slot ranges, image shifts and LDS bases of every tile of a flagged replica: the staged
@@ -440,9 +442,8 @@ __global__ void k_bPermute2(BS b)
 // (ni + 2) x (nj + 2) columns (i-major, the serial order of the layout), its up to three
 // pieces and, for a self column, its rows; wave prefix sums place the pieces, the LDS bases
 // and the rows in that order
-__global__ __launch_bounds__(BLOCK) void k_bTiles(BS b)
+__device__ inline void bTiles(const BS& b, int64_t t)
 {
-    const int64_t t = int64_t(blockIdx.x) * (BLOCK / WAVE) + threadIdx.x / WAVE;
     if (t >= b.ntiles) return;
     const TileG G = b.tg[t];
     if (!b.flag[G.rep]) return;
@@ -533,44 +534,30 @@ __global__ __launch_bounds__(BLOCK) void k_bTiles(BS b)
     }
 }
 
-// ---------------------------------------------------------------------------------------
-// per-step slot data: current positions in sorted order with the slab weights, and the
-// density sample of the thermodynamic force (AxialDensityProfile.cpp:21-51)
-__global__ void k_bGather(BS b)
+// the tiles first (they take longer), then the atoms
+__global__ __launch_bounds__(BLOCK) void k_bMoveTiles(BS b, unsigned tileBlocks)
 {
-    const int64_t s = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    const bool valid = s < b.natoms;
-    int64_t key = -1;  // density bin of the atom's replica, -1 for none
-    if (valid)
-    {
-        const int32_t i = b.sorted[s];
-        const double4 p = b.pos[i];
-        const RepD& R = b.reps[b.atomRep[i]];
-        double lam = 1.0, mod = 1.0, g = 0.0;
-        if (R.adress)
-        {
-            slabEval(R.slab, p.x, lam, mod, g);
-            const int64_t bin = getBin(p.x, 0.0, R.invBinWidth, R.nbins);
-            if (bin != -1) key = R.h0 + bin;
-        }
-        b.sortedPos[s] = make_double4(p.x, p.y, p.z, mod);
-        // lambda and its gradient are read for hybrid records only (0 < lambda_mod < 1)
-        if (mod > 0.0 && mod < 1.0)
-        {
-            b.slotLam[s] = lam;
-            b.slotGrad[s] = g;
-        }
-    }
-    // a wave's atoms (a few cells of one column, so one x-cell) fall into a few x-bins: one
-    // atomic per distinct bin of the wave (counts are integers, so the sums are exact in any
-    // order)
-    const int lane = int(threadIdx.x) % WAVE;
-    const int k32 = int(key);
-    for (unsigned long long pending = __ballot(k32 >= 0); pending;)
+    if (blockIdx.x < tileBlocks)
+        bTiles(b, int64_t(blockIdx.x) * (BLOCK / WAVE) + threadIdx.x / WAVE);
+    else
+        bMove(b, int64_t(blockIdx.x - tileBlocks) * BLOCK + threadIdx.x);
+}
+
+// ---------------------------------------------------------------------------------------
+
+// the density sample of the thermodynamic force (AxialDensityProfile.cpp:21-51) for the active
+// lanes' atoms of replica R: a wave's atoms (a few cells of one column, so one x-cell) fall into a
+// few x-bins, one atomic per distinct bin (counts are integers, so the sums are exact in any
+// order)
+__device__ inline void sampleDensity(const BS& b, const RepD& R, double x)
+{
+    const int64_t bin = getBin(x, 0.0, R.invBinWidth, R.nbins);
+    const int lane = int(threadIdx.x) % WAVE, key = bin != -1 ? int(R.h0 + bin) : -1;
+    for (unsigned long long pending = __ballot(key >= 0); pending;)
     {
         const int src = __builtin_ctzll(pending);
-        const int k0 = __shfl(k32, src, WAVE);
-        const unsigned long long m = __ballot(k32 == k0);
+        const int k0 = __shfl(key, src, WAVE);
+        const unsigned long long m = __ballot(key == k0);
         if (lane == src) atomicAddD(&b.tfDensity[k0], double(__popcll(m)));
         pending &= ~m;
     }
@@ -657,7 +644,7 @@ __device__ void bBuildRows(const BS& b, const TileB& ti, const TileG& G, const R
     const double rsq = b.rnSqr;
     int sure, doubt;
     grid16.thresholds(b.rn, sure, doubt);
-    const GlobalFetch exact{&ti, b.sortedPos, R.L[0], R.L[1], R.L[2]};
+    const GlobalFetch exact{&ti, b.pos, R.L[0], R.L[1], R.L[2]};
     const int sub = lane % S, group = lane / S, first = group * S;
     int localMax = 0;
     for (int row0 = wave * RW; row0 < ti.nrows; row0 += waves * RW)
@@ -668,7 +655,7 @@ __device__ void bBuildRows(const BS& b, const TileB& ti, const TileG& G, const R
         const int s = bTileRow(ti, live ? row : 0, sc);
         const int pr = ti.selfPiece[sc];
         const int qSelf = ti.base[pr] + (s - ti.begin[pr]);
-        const double4 xp = b.sortedPos[s];  // (a self column's records are unshifted)
+        const double4 xp = b.pos[s];  // (a self column's records are unshifted)
         const uint2 own = rec(qSelf);
         const Short2 ownXY = asShort2(own.x), ownZ = asShort2(own.y);
         const int zq = int(int16_t(own.y));
@@ -843,7 +830,7 @@ __global__ __launch_bounds__(B_BUILD_BLOCK, 4) void k_bBuild(BS b)
     const bool staged = ti.staged <= b.buildCap;
     bool outside = !staged;
     if (staged)
-        stageShifted(ti, b.sortedPos, R, [&](int q, const double4& v) { rec[q] = grid16(v, outside); });
+        stageShifted(ti, b.pos, R, [&](int q, const double4& v) { rec[q] = grid16(v, outside); });
     if (outside) wild = 1;
     // LDS slot of the first record of cell k0 - 1 + z of each staged column, whose pieces are cell
     // nz - 1 below the box, the run from max(k0 - 1, 0) inside it and cell 0 above it
@@ -869,7 +856,7 @@ __global__ __launch_bounds__(B_BUILD_BLOCK, 4) void k_bBuild(BS b)
     if (staged)
         bBuildRows(b, ti, G, R, cstart, LdsRec{rec}, grid16, wild != 0);
     else
-        bBuildRows(b, ti, G, R, cstart, GlobalRec{GlobalFetch{&ti, b.sortedPos, R.L[0], R.L[1], R.L[2]}, grid16},
+        bBuildRows(b, ti, G, R, cstart, GlobalRec{GlobalFetch{&ti, b.pos, R.L[0], R.L[1], R.L[2]}, grid16},
                    grid16, true);
 }
 
@@ -947,8 +934,7 @@ __device__ inline void ljQuadWeighted(const Pre& p, double rcSqr, const double4&
 template <bool CAP, bool W, bool GS, class St>
 __device__ double bForceRows(const BS& b, const TileB& ti, const RepD& R, const St& st)
 {
-    const int64_t step = *b.step;
-    const bool sampling = W && step % SAMPLING_INTERVAL == 0;
+    const bool sampling = W && bStep(b) % SAMPLING_INTERVAL == 0;
     const int lg = R.split;
     const int items = ti.nrows << lg, mask = (1 << lg) - 1;
     double eTile = 0.0;
@@ -963,8 +949,7 @@ __device__ double bForceRows(const BS& b, const TileB& ti, const RepD& R, const 
             int sc;
             const int s = bTileRow(ti, t >> lg, sc);
             const int c = b.cnt[s];
-            const int32_t i = b.sorted[s];
-            const double4 pi = b.sortedPos[s];
+            const double4 pi = b.pos[s];
             const uint4* chunk = reinterpret_cast<const uint4*>(b.nbr) + s;
             double f[3];
             if constexpr (W)
@@ -1014,8 +999,9 @@ __device__ double bForceRows(const BS& b, const TileB& ti, const RepD& R, const 
                 f[1] = sum.fy;
                 f[2] = sum.fz;
             }
+            if (W && (t & mask) == 0) sampleDensity(b, R, pi.x);
             if ((t & mask) == 0)
-                for (int d = 0; d < 3; ++d) b.force[d * b.cap + i] = f[d];
+                for (int d = 0; d < 3; ++d) b.force[d * b.cap + s] = f[d];
         }
         if constexpr (!W) sum.endRound();
     }
@@ -1044,7 +1030,7 @@ __global__ __launch_bounds__(BLOCK) void k_bForce(BS b)
     const Stage<!W> st(stLds, b.stageCap[W]);
     bool weighted = !fits;
     if (fits && ti.near)
-        stageShifted(ti, b.sortedPos, R, [&](int q, const double4& v) {
+        stageShifted(ti, b.pos, R, [&](int q, const double4& v) {
             st.put(q, v);
             weighted = weighted || v.w > 0.0;
         });
@@ -1056,10 +1042,9 @@ __global__ __launch_bounds__(BLOCK) void k_bForce(BS b)
         for (int t = threadIdx.x; t < ti.nrows; t += blockDim.x)
         {
             int sc;
-            const int32_t i = b.sorted[bTileRow(ti, t, sc)];
-            b.force[i] = 0.0;
-            b.force[b.cap + i] = 0.0;
-            b.force[2 * b.cap + i] = 0.0;
+            const int s = bTileRow(ti, t, sc);
+            for (int d = 0; d < 3; ++d) b.force[d * b.cap + s] = 0.0;
+            sampleDensity(b, R, b.pos[s].x);
         }
         if (threadIdx.x == 0) b.ePart[t] = 0.0;
         return;
@@ -1067,18 +1052,17 @@ __global__ __launch_bounds__(BLOCK) void k_bForce(BS b)
     if (!W) __syncthreads();
     const double eTile = fits ? bForceRows<CAP, W, false>(b, ti, R, st)
                               : bForceRows<CAP, W, true>(b, ti, R,
-                                                         GlobalFetch{&ti, b.sortedPos, R.L[0], R.L[1], R.L[2]});
+                                                         GlobalFetch{&ti, b.pos, R.L[0], R.L[1], R.L[2]});
     const double e = blockSum(0.5 * eTile, red);
     if (threadIdx.x == 0) b.ePart[t] = e;
 }
 
 // LJ_IdealGas::updateMeanCompensationEnergy (LJ_IdealGas.cpp:21-50) at the reference's
 // update interval; one workgroup per replica
-__global__ void k_bCompUpdate(BS b)
+__device__ inline void bCompUpdate(const BS& b, int r)
 {
-    const int r = blockIdx.x;
     const RepD& R = b.reps[r];
-    if (!R.adress || *b.step % COMP_UPDATE_INTERVAL != 0) return;
+    if (!R.adress || bStep(b) % COMP_UPDATE_INTERVAL != 0) return;
     for (int k = threadIdx.x; k < COMP_BINS; k += blockDim.x)
     {
         const int64_t idx = R.cmp0 + k;
@@ -1093,16 +1077,15 @@ __global__ void k_bCompUpdate(BS b)
 
 // ThermodynamicForce::update_if (ThermodynamicForce.hpp:124-152) every tfEvery steps with
 // the hybrid region as predicate; one workgroup per replica
-__global__ __launch_bounds__(BLOCK) void k_bTFUpdate(BS b)
+__device__ inline void bTFUpdate(const BS& b, int r)
 {
     __shared__ double dens[MAX_BINS];
     __shared__ double smooth[MAX_BINS];
-    const int r = blockIdx.x;
     const RepD& R = b.reps[r];
     if (!R.adress) return;
     __syncthreads();
     const int64_t samples = b.tfSamples[r] + 1;
-    if (R.tfEvery <= 0 || (*b.step + 1) % R.tfEvery != 0)
+    if (R.tfEvery <= 0 || (bStep(b) + 1) % R.tfEvery != 0)
     {
         if (threadIdx.x == 0) b.tfSamples[r] = samples;
         return;
@@ -1146,6 +1129,22 @@ __global__ __launch_bounds__(BLOCK) void k_bTFUpdate(BS b)
     if (threadIdx.x == 0) b.tfSamples[r] = 0;
 }
 
+// the end of a step: one workgroup per replica for its updates, then the cells of the replicas that
+// rebuilt, whose counts and fill cursors the next rebuild finds at zero
+__global__ __launch_bounds__(BLOCK) void k_bEnd(BS b)
+{
+    if (int(blockIdx.x) < b.nrep)
+    {
+        bCompUpdate(b, int(blockIdx.x));
+        bTFUpdate(b, int(blockIdx.x));
+        return;
+    }
+    const int64_t c = int64_t(blockIdx.x - b.nrep) * blockDim.x + threadIdx.x;
+    if (c >= b.ncells || !b.flag[b.cellRep[c]]) return;
+    b.counts[c] = 0;
+    b.fill[c] = 0;
+}
+
 // VelocityVerletLangevinThermostat::postForceIntegrate with the thermodynamic force
 // (ThermodynamicForce::apply, ThermodynamicForce.hpp:98-122) added first
 __global__ void k_bPost(BS b)
@@ -1167,11 +1166,6 @@ __global__ void k_bPost(BS b)
     b.vel[i] += dtfm * fx;
     b.vel[b.cap + i] += dtfm * b.force[b.cap + i];
     b.vel[2 * b.cap + i] += dtfm * b.force[2 * b.cap + i];
-}
-
-__global__ void k_bStepEnd(BS b)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) *b.step += 1;
 }
 
 // per-replica ordered sums: potential energy from the tile partials, kinetic energy
@@ -1260,7 +1254,7 @@ struct mrmd_batch
     DBuf<double4> pos, sortedPos;
     DBuf<double> vel, force, slotLam, slotGrad;
     DBuf<int32_t> atomRep, cellRep, cellOf, counts, offsets, fill, sorted, cnt, flag, err;
-    DBuf<int32_t> id, tmpA, tmpB;
+    DBuf<int32_t> id, tmpA;
     DBuf<double> tmpVel;
     DBuf<TileG> dtg;
     DBuf<TileB> tiles;
@@ -1308,7 +1302,6 @@ BS mrmd_batch::state()
     b.sorted = sorted.p;
     b.id = id.p;
     b.tmpA = tmpA.p;
-    b.tmpB = tmpB.p;
     b.tmpVel = tmpVel.p;
     b.sortedPos = sortedPos.p;
     b.slotLam = slotLam.p;
@@ -1431,7 +1424,8 @@ void mrmd_batch::layoutTiles()
     dropGraph();
 }
 
-// n steps; a step's post-force integration and the next step's pre-force integration run
+// n steps of ten launches each (a launch with nothing to do takes 4.5 us in a graph, and a step of
+// 24 replicas was eighteen of them); a step's post-force integration and the next step's pre-force integration run
 // as one pass (k_bPre<true>), the first pre-force and the last post-force pass alone
 void mrmd_batch::enqueueSteps(int64_t n)
 {
@@ -1440,22 +1434,15 @@ void mrmd_batch::enqueueSteps(int64_t n)
     const BS b = state();
     const unsigned ga = gridFor(natoms), gc = gridFor(ncells);
     const unsigned gs = unsigned((ncells * SORT_GROUP + BLOCK - 1) / BLOCK);
-    const unsigned nr = unsigned(reps.size());
+    const unsigned nr = unsigned(reps.size()), tileBlocks = unsigned((ntiles + BLOCK / WAVE - 1) / (BLOCK / WAVE));
     hipLaunchKernelGGL(k_bPre<false>, dim3(ga), dim3(BLOCK), 0, c->stream, b);
     for (int64_t k = 0; k < n; ++k)
     {
-        hipLaunchKernelGGL(k_bCheck, dim3(gridFor(nr)), dim3(BLOCK), 0, c->stream, b);
-        hipLaunchKernelGGL(k_bWrap, dim3(ga), dim3(BLOCK), 0, c->stream, b);
-        hipLaunchKernelGGL(k_bZeroCells, dim3(gc), dim3(BLOCK), 0, c->stream, b);
-        hipLaunchKernelGGL(k_bCount, dim3(ga), dim3(BLOCK), 0, c->stream, b);
+        hipLaunchKernelGGL(k_bWrapCount, dim3(ga), dim3(BLOCK), 0, c->stream, b);
         hipLaunchKernelGGL(k_bScan, dim3(nr), dim3(BLOCK), 0, c->stream, b);
         hipLaunchKernelGGL(k_bFill, dim3(ga), dim3(BLOCK), 0, c->stream, b);
-        hipLaunchKernelGGL(k_bSortCells, dim3(gs), dim3(BLOCK), 0, c->stream, b);
-        hipLaunchKernelGGL(k_bPermute1, dim3(ga), dim3(BLOCK), 0, c->stream, b);
-        hipLaunchKernelGGL(k_bPermute2, dim3(ga), dim3(BLOCK), 0, c->stream, b);
-        hipLaunchKernelGGL(k_bTiles, dim3(unsigned((ntiles + BLOCK / WAVE - 1) / (BLOCK / WAVE))), dim3(BLOCK), 0,
-                           c->stream, b);
-        hipLaunchKernelGGL(k_bGather, dim3(ga), dim3(BLOCK), 0, c->stream, b);
+        hipLaunchKernelGGL(k_bSortGather, dim3(gs), dim3(BLOCK), 0, c->stream, b);
+        hipLaunchKernelGGL(k_bMoveTiles, dim3(tileBlocks + ga), dim3(BLOCK), 0, c->stream, b, tileBlocks);
         hipLaunchKernelGGL(k_bBuild, dim3(unsigned(ntiles)), dim3(B_BUILD_BLOCK),
                            size_t(stageCapBuild + B_PAD) * sizeof(uint2), c->stream, b);
         auto force = [&](auto kernel, int64_t t0, int64_t t1, size_t lds) {
@@ -1475,9 +1462,7 @@ void mrmd_batch::enqueueSteps(int64_t n)
             force(k_bForce<false, false>, 0, plainTiles, ldsPlain);
             force(k_bForce<false, true>, plainTiles, ntiles, ldsAdress);
         }
-        hipLaunchKernelGGL(k_bCompUpdate, dim3(nr), dim3(BLOCK), 0, c->stream, b);
-        hipLaunchKernelGGL(k_bTFUpdate, dim3(nr), dim3(BLOCK), 0, c->stream, b);
-        hipLaunchKernelGGL(k_bStepEnd, dim3(1), dim3(64), 0, c->stream, b);
+        hipLaunchKernelGGL(k_bEnd, dim3(nr + gc), dim3(BLOCK), 0, c->stream, b);
         if (k + 1 < n)
             hipLaunchKernelGGL(k_bPre<true>, dim3(ga), dim3(BLOCK), 0, c->stream, b);
         else
@@ -1639,7 +1624,6 @@ int mrmd_batch_create(mrmd_ctx* c, const mrmd_replica* reps, int64_t nrep, doubl
         b->sorted.reserve(x, cp);
         b->id.reserve(x, cp);
         b->tmpA.reserve(x, cp);
-        b->tmpB.reserve(x, cp);
         b->tmpVel.reserve(x, 3 * cp);
         b->cnt.reserve(x, cp);
         b->cellRep.reserve(x, b->ncells);
@@ -1677,6 +1661,8 @@ int mrmd_batch_create(mrmd_ctx* c, const mrmd_replica* reps, int64_t nrep, doubl
         HIPCHECK(hipMemsetAsync(b->rebuilds.p, 0, size_t(nr) * 8, x->stream));
         HIPCHECK(hipMemsetAsync(b->tfSamples.p, 0, size_t(nr) * 8, x->stream));
         HIPCHECK(hipMemsetAsync(b->flag.p, 0, size_t(nr) * 4, x->stream));
+        HIPCHECK(hipMemsetAsync(b->counts.p, 0, size_t(b->ncells) * 4, x->stream));
+        HIPCHECK(hipMemsetAsync(b->fill.p, 0, size_t(b->ncells) * 4, x->stream));
         HIPCHECK(hipMemsetAsync(b->err.p, 0, 4, x->stream));
         HIPCHECK(hipMemsetAsync(b->step.p, 0, 8, x->stream));
         HIPCHECK(hipMemsetAsync(b->tfDensity.p, 0, size_t(b->nbins) * 8, x->stream));
