@@ -212,10 +212,32 @@ __global__ void k_postI32(const int32_t* src, int n, uint64_t* host, uint32_t ta
     const int32_t v = __hip_atomic_load(src + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(host + k, tagWord(tag, uint32_t(v)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+// the same for the maxima of n words over the MAX_SLOTS copies (one wave)
+__global__ __launch_bounds__(WAVE) void k_postMax(const int32_t* slots, int word, int n, uint64_t* host, uint32_t tag)
+{
+    static_assert(MAX_SLOTS == WAVE);
+    const int32_t* mine = slots + int(threadIdx.x) * MAX_WORDS + word;
+    for (int k = 0; k < n; ++k)
+    {
+        const int v = waveMaxInt(__hip_atomic_load(mine + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        if (threadIdx.x == 0)
+            __hip_atomic_store(host + k, tagWord(tag, uint32_t(v)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
 }  // namespace
 
 namespace mrmd_hip
 {
+uint32_t postMax(mrmd_ctx* ctx, const int32_t* slots, int word, int n)
+{
+    if (n < 1 || n > READBACK_INTS) fail(MRMD_ERR_ARG, "readback of %d values (at most %d)", n, READBACK_INTS);
+    const uint32_t tag = nextTag(ctx);
+    hipLaunchKernelGGL(k_postMax, dim3(1), dim3(WAVE), 0, ctx->stream, slots, word, n,
+                       reinterpret_cast<uint64_t*>(ctx->pinned) + READBACK_WORD, tag);
+    checkLaunch();
+    return tag;
+}
+
 uint32_t postI32(mrmd_ctx* ctx, const int32_t* dev, int n)
 {
     if (n < 1 || n > READBACK_INTS) fail(MRMD_ERR_ARG, "readback of %d values (at most %d)", n, READBACK_INTS);

@@ -33,13 +33,13 @@ namespace
 {
 // WRAP: each position is first mapped into the box (PeriodicMapping) and written back; its
 // current value is wb.from[wb.slotOf[i]] when wb.from is set
-// BOX: the cell box of the records [rowLo, rowHi) too, a wave and then a workgroup maximum (of the
-// negated minima), and one conditional atomic per word and workgroup.  (Over cells in a pass of
-// its own it cost two launches of 1.5 and 6 us, and a wait of the host with the chip idle.)
+// BOX: the cell box of the records [rowLo, rowHi) too (RowBox), a wave and then a workgroup
+// maximum.  (Over cells in a pass of its own it cost two launches of 1.5 and 6 us, and a wait of the
+// host with the chip idle.)
 template <bool WRAP, bool BOX>
 __global__ __launch_bounds__(BLOCK) void k_binCount(const double4* pos, int64_t begin, int64_t n, GridD g,
                                                     int32_t* cellOf, int32_t* counts, double4* wrapPos, WrapBox wb,
-                                                    int64_t rowLo, int64_t rowHi, int32_t* box)
+                                                    int64_t rowLo, int64_t rowHi, int32_t* slots)
 {
     const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     const bool valid = k < n;
@@ -79,13 +79,7 @@ __global__ __launch_bounds__(BLOCK) void k_binCount(const double4* pos, int64_t 
             const int d = int(threadIdx.x);
             int v = red[d][0];
             for (int w = 1; w < BLOCK / WAVE; ++w) v = max(v, red[d][w]);
-            if (v != -INT32_MAX)
-            {
-                if (d < 3)
-                    lowerTo(&box[d], -v);
-                else
-                    raiseTo(&box[d], v);
-            }
+            raiseTo(slots, BOX_WORD + d, v);
         }
     }
 }
@@ -236,8 +230,9 @@ __global__ void k_gatherPos(const double4* pos, const int32_t* sorted, int64_t n
     if (k < n) out[k] = pos[sorted[k]];
 }
 
-// the cells' counts and fill cursors, and (if not null) the cell box of no record
-__global__ void k_binClear(int32_t* counts, int32_t* fill, int64_t n, int32_t* box)
+// the cells' counts and fill cursors, and (if not null) the words of the slots (the cell box that of
+// no record)
+__global__ void k_binClear(int32_t* counts, int32_t* fill, int64_t n, int32_t* slots)
 {
     const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (k < n)
@@ -245,7 +240,7 @@ __global__ void k_binClear(int32_t* counts, int32_t* fill, int64_t n, int32_t* b
         counts[k] = 0;
         fill[k] = 0;
     }
-    if (box && k < 6) box[k] = k < 3 ? INT32_MAX : -1;
+    if (slots && k < MAX_SLOTS * MAX_WORDS) slots[k] = k % MAX_WORDS < BOX_WORD ? 0 : -INT32_MAX;
 }
 }  // namespace
 
@@ -262,22 +257,22 @@ void Binning::build(mrmd_ctx* ctx, const double4* pos, int64_t b, int64_t e, con
     counts.ensure(ctx, ncell + 1);
     offsets.ensure(ctx, ncell + 1);
     fill.ensure(ctx, ncell + 1);
-    hipLaunchKernelGGL(k_binClear, dim3(gridFor(std::max(ncell, 6))), dim3(BLOCK), 0, ctx->stream, counts.p, fill.p,
-                       int64_t(ncell), rowBox ? rowBox->box : nullptr);
+    hipLaunchKernelGGL(k_binClear, dim3(gridFor(std::max(ncell, MAX_SLOTS * MAX_WORDS))), dim3(BLOCK), 0, ctx->stream, counts.p, fill.p,
+                       int64_t(ncell), rowBox ? rowBox->slots : nullptr);
     if (n > 0)
     {
         const WrapBox wb = wrap ? *wrap : WrapBox{};
         auto count = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(gridFor(n)), dim3(BLOCK), 0, ctx->stream, pos, b, n, g, cellOf.p, counts.p,
                                wrapPos, wb, rowBox ? rowBox->lo : 0, rowBox ? rowBox->hi : 0,
-                               rowBox ? rowBox->box : nullptr);
+                               rowBox ? rowBox->slots : nullptr);
         };
         if (rowBox)
             wrap ? count(k_binCount<true, true>) : count(k_binCount<false, true>);
         else
             wrap ? count(k_binCount<true, false>) : count(k_binCount<false, false>);
     }
-    if (rowBox) rowBox->tag = postI32(ctx, rowBox->box, 6);
+    if (rowBox) rowBox->tag = postMax(ctx, rowBox->slots, BOX_WORD, 6);
     scanExclusiveI32(ctx, counts.p, offsets.p, ncell, nullptr);
     if (n > 0)
     {

@@ -51,15 +51,17 @@ GridD makeGrid(const double* gmin, const double* gmax, const double* delta);
 // order is ascending record index inside every cell (a stable counting sort), or with
 // zOrder ascending z (record index breaking ties), which makes every column of cells one
 // z-sorted run
-// the box of the cells that hold records [lo, hi): box (6 words on the device: minimum cell index
-// per axis, then maximum) is filled by the binning's count pass and posted to the host behind it,
-// under tag, so that the host's wait (takeI32) overlaps with the rest of the binning
+// the box of the cells that hold records [lo, hi): per axis the negated minimum, then the maximum
+// of their cell indices, raised in words BOX_WORD and on of slots (see raiseTo) by the binning's
+// count pass and posted to the host behind it, under tag, so that the host's wait (takeI32)
+// overlaps with the rest of the binning.  The binning clears all words of the slots.
 struct RowBox
 {
     int64_t lo, hi;
-    int32_t* box;
+    int32_t* slots;
     uint32_t tag;
 };
+constexpr int BOX_WORD = 8;
 
 struct Binning
 {

@@ -51,14 +51,19 @@ __device__ inline int64_t tileOfCell(const TileGeom& tg, int cell)
     return (int64_t((i - tg.o0) / tg.cols) * tg.nbj + (j - tg.o1) / tg.cols) * tg.tilesPerCol + (k - tg.o2) / tg.K;
 }
 
+// the maxima of a build (words of the slots in the context's scratch, see raiseTo): the largest staged
+// neighbourhood, the widest row, whether there is a record of more than one atom; the rows' cell box
+// from BOX_WORD
+constexpr int STAGED_WORD = 0, WIDTH_WORD = 1, MULTI_WORD = 2;
+
 // half a wave per tile, a lane per range: row ranges, neighbourhood column ranges and their LDS
-// bases; the largest staged neighbourhood goes to *maxStaged.  The ranges' places are prefix sums
+// bases.  The ranges' places are prefix sums
 // over the lanes and the description goes out in neighbouring words.  (One lane per tile, 150
 // scattered loads and 100 scattered stores each, took 12 us at any size up to 20,000 tiles.)
 constexpr int SETUP_LANES = 32;
 static_assert(MAX_RANGES <= SETUP_LANES);
 __global__ __launch_bounds__(BLOCK) void k_tileSetup(TileGeom tg, int64_t ntiles, const int32_t* offsets,
-                                                     const int32_t* counts, TileInfo* tiles, int32_t* maxStaged)
+                                                     const int32_t* counts, TileInfo* tiles, int32_t* slots)
 {
     const int64_t t = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / SETUP_LANES;
     if (t >= ntiles) return;  // (whole groups leave together)
@@ -115,16 +120,14 @@ __global__ __launch_bounds__(BLOCK) void k_tileSetup(TileGeom tg, int64_t ntiles
         ti.staged = lenTo;
         ti.nself = selfTo;
         ti.nrows = rowsTo;
-        raiseTo(maxStaged, lenTo);
+        raiseTo(slots, STAGED_WORD, lenTo);
     }
 }
 
-// the counts of all slots and the words of the build's maxima
-__global__ void k_listClear(int32_t* cnt, int64_t n, int32_t* words, int nw)
+__global__ void k_listClear(int32_t* cnt, int64_t n)
 {
     const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (k < n) cnt[k] = 0;
-    if (k < nw) words[k] = 0;
 }
 
 constexpr int MAX_SPAN = 64;  // cells of a tile's column range along z (K + 2R)
@@ -164,7 +167,7 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
                                                        const TileInfo* __restrict__ tiles, TileGeom tg, GridD g,
                                                        int64_t rowLo, int64_t rowHi, double rsq, double rn,
                                                        uint16_t* nbr, int64_t strideS, int cap, int32_t* cnt,
-                                                       int32_t* maxCnt, int stagedCap, double4* gstage,
+                                                       int32_t* slots, int stagedCap, double4* gstage,
                                                        int64_t gstageRecs, double bandLo, double bandHi,
                                                        int8_t* tileSkip)
 {
@@ -462,7 +465,7 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
                 else
                     rowBuf[group * cap + k] = uint16_t(pad);
             }
-        if (live && sub == 0) cnt[s] = isRow ? kept : 0;  // the true width goes to maxCnt
+        if (live && sub == 0) cnt[s] = isRow ? kept : 0;  // the true width goes to WIDTH_WORD
         localMax = max(localMax, isRow ? n : 0);
         if constexpr (!GS)
         {
@@ -483,7 +486,7 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
     }
     // one atomic per wave (every lane of the workgroup reaches this point)
     localMax = waveMaxInt(localMax);
-    if (lane == 0 && localMax > 0) raiseTo(maxCnt, localMax);
+    if (lane == 0 && localMax > 0) raiseTo(slots, WIDTH_WORD, localMax);
 }
 
 // tiled rows (per sorted slot, LDS slots) -> global rows (per record begin+r, record indices)
@@ -605,10 +608,10 @@ TileGeom geom(const mrmd_verlet_list* vl)
                     vl->rowExtent[0], vl->rowExtent[1], vl->rowExtent[2]};
 }
 
-// the words of a build in the context's scratch: the largest staged neighbourhood, the widest row,
-// the records of more than one atom; from word 8 the cell box of the rows
-constexpr int BUILD_WORDS = 3, BOX_WORD = 8;
-int32_t* buildWords(mrmd_ctx* ctx) { return static_cast<int32_t*>(ctxScratch(ctx, 2, 64)); }
+int32_t* buildSlots(mrmd_ctx* ctx)
+{
+    return static_cast<int32_t*>(ctxScratch(ctx, 2, sizeof(int32_t) * MAX_SLOTS * MAX_WORDS));
+}
 
 // cell box of the list rows, posted by the binning
 void rowRegion(mrmd_verlet_list* vl, const RowBox& rowBox)
@@ -622,15 +625,15 @@ void rowRegion(mrmd_verlet_list* vl, const RowBox& rowBox)
         vl->rowExtent[d] = 0;
         if (rows <= 0) continue;
         // rows exist, so every axis holds at least one cell of them
-        if (h[d] < 0 || h[3 + d] < h[d] || h[3 + d] >= vl->bin.grid.n[d])
+        if (-h[d] < 0 || h[3 + d] < -h[d] || h[3 + d] >= vl->bin.grid.n[d])
             fail(MRMD_ERR_STATE, "cell box of the list rows out of the grid: axis %d cells [%d, %d] of %d (%lld rows)",
-                 d, h[d], h[3 + d], vl->bin.grid.n[d], (long long)rows);
-        vl->rowOrigin[d] = h[d];
-        vl->rowExtent[d] = h[3 + d] - h[d] + 1;
+                 d, -h[d], h[3 + d], vl->bin.grid.n[d], (long long)rows);
+        vl->rowOrigin[d] = -h[d];
+        vl->rowExtent[d] = h[3 + d] + h[d] + 1;
     }
 }
 
-// (words[0] is zero before the call)
+// (the slots' STAGED_WORD is zero before the call)
 void setupTiles(mrmd_verlet_list* vl, int K)
 {
     mrmd_ctx* ctx = vl->ctx;
@@ -641,16 +644,18 @@ void setupTiles(mrmd_verlet_list* vl, int K)
     vl->tiles.ensure(ctx, std::max<int64_t>(vl->ntiles, 1));
     if (vl->ntiles > 0)
         hipLaunchKernelGGL(k_tileSetup, dim3(gridFor(vl->ntiles * SETUP_LANES)), dim3(BLOCK), 0, ctx->stream, geom(vl),
-                           vl->ntiles, vl->bin.offsets.p, vl->bin.counts.p, vl->tiles.p, buildWords(ctx));
+                           vl->ntiles, vl->bin.offsets.p, vl->bin.counts.p, vl->tiles.p, buildSlots(ctx));
     checkLaunch();
 }
 
-// records whose atom count is not 1 (molecule lists only)
-__global__ void k_countNotOne(const int64_t* numAtoms, int64_t n, int32_t* out)
+// whether there are records whose atom count is not 1 (molecule lists only)
+__global__ void k_anyNotOne(const int64_t* numAtoms, int64_t n, int32_t* slots)
 {
     const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (k < n && numAtoms[k] != 1) atomicAdd(out, 1);
+    if (k < n && numAtoms[k] != 1) raiseTo(slots, MULTI_WORD, 1);
 }
+
+__global__ void k_clearWord(int32_t* slots, int word) { slots[int(threadIdx.x) * MAX_WORDS + word] = 0; }
 
 // numAtoms (molecule lists) is checked for records of one atom; returns whether all are
 bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t begin, int64_t end, double rn,
@@ -676,15 +681,15 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
     vl->sentinel = std::max({gmax[0], gmax[1], gmax[2]}) + SENTINEL_GAP + 4.0 * rn;
     // the binning's z sort also writes each record's slot (slotOf)
     vl->slotOf.ensure(ctx, std::max<int64_t>(nall, 1));
-    int32_t* const words = buildWords(ctx);
-    RowBox rowBox{begin, end, words + BOX_WORD, 0};
+    int32_t* const slots = buildSlots(ctx);
+    RowBox rowBox{begin, end, slots, 0};
     vl->bin.build(ctx, pos, 0, nall, g, true, true, nullptr, nullptr, vl->slotOf.p, &rowBox);
     vl->strideS = std::max<int64_t>(64, (nall + 63) / 64 * 64);
     vl->cnt16.ensure(ctx, vl->strideS);
-    hipLaunchKernelGGL(k_listClear, dim3(gridFor(std::max<int64_t>(nall, BUILD_WORDS))), dim3(BLOCK), 0, ctx->stream,
-                       vl->cnt16.p, nall, words, BUILD_WORDS);
+    if (nall > 0)
+        hipLaunchKernelGGL(k_listClear, dim3(gridFor(nall)), dim3(BLOCK), 0, ctx->stream, vl->cnt16.p, nall);
     if (numAtoms && nall > 0)
-        hipLaunchKernelGGL(k_countNotOne, dim3(gridFor(nall)), dim3(BLOCK), 0, ctx->stream, numAtoms, nall, words + 2);
+        hipLaunchKernelGGL(k_anyNotOne, dim3(gridFor(nall)), dim3(BLOCK), 0, ctx->stream, numAtoms, nall, slots);
     rowRegion(vl, rowBox);
     vl->globalValid = false;
     vl->halfValid = false;
@@ -726,9 +731,9 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
     for (bool again = false;; again = true)
     {
         vl->tileCols = a;
-        if (again) hipLaunchKernelGGL(k_zeroI32v, dim3(1), dim3(64), 0, ctx->stream, words, int64_t(1));
+        if (again) hipLaunchKernelGGL(k_clearWord, dim3(1), dim3(MAX_SLOTS), 0, ctx->stream, slots, STAGED_WORD);
         setupTiles(vl, K);
-        readbackI32(ctx, words, 1, &vl->maxStaged);
+        takeI32(ctx, postMax(ctx, slots, STAGED_WORD, 1), 1, &vl->maxStaged);
         if (vl->maxStaged <= vl->stageLimit) break;
         if (K > 1)
             K = std::max(1, K / 2);
@@ -752,13 +757,12 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
     if (vl->banded) vl->tileSkip.ensure(ctx, std::max<int64_t>(vl->ntiles, 1));
     if (vl->capFull <= 0) vl->capFull = int32_t(std::max<int64_t>(2 * maxNeigh + 16, 96));
     vl->capFull = (vl->capFull + CHUNK - 1) / CHUNK * CHUNK;
-    int32_t* const dmax = words + 1;
     bool mono = false;
     const int stagedCap = std::max(vl->maxStaged, 1);
     for (int attempt = 0; attempt < 2; ++attempt)
     {
         vl->nbr16.ensure(ctx, int64_t(vl->capFull) * vl->strideS);
-        if (attempt > 0) hipLaunchKernelGGL(k_zeroI32v, dim3(1), dim3(64), 0, ctx->stream, dmax, int64_t(1));
+        if (attempt > 0) hipLaunchKernelGGL(k_clearWord, dim3(1), dim3(MAX_SLOTS), 0, ctx->stream, slots, WIDTH_WORD);
         if (vl->ntiles > 0 && end > begin)
         {
             KTimer tk(ctx, "verlet_tiled");
@@ -779,7 +783,7 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
             auto launch = [&](auto kernel) {
                 hipLaunchKernelGGL(kernel, dim3(unsigned(vl->ntiles)), dim3(waves * WAVE), lds, ctx->stream,
                                    vl->bin.sortedPos.p, vl->bin.sorted.p, vl->bin.offsets.p, vl->tiles.p, geom(vl), g,
-                                   begin, end, rn * rn, rn, vl->nbr16.p, vl->strideS, vl->capFull, vl->cnt16.p, dmax,
+                                   begin, end, rn * rn, rn, vl->nbr16.p, vl->strideS, vl->capFull, vl->cnt16.p, slots,
                                    stagedCap, vl->gstage.p, vl->gstageRecs, vl->bandLo, vl->bandHi, vl->tileSkip.p);
             };
             const bool wide = vl->forceWide || int64_t(vl->capFull) * vl->strideS >= (int64_t(1) << 31);
@@ -799,7 +803,7 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
         }
         checkLaunch();
         int32_t hp[2];
-        readbackI32(ctx, dmax, 2, hp);
+        takeI32(ctx, postMax(ctx, slots, WIDTH_WORD, 2), 2, hp);
         const int32_t hmax = hp[0];
         mono = hp[1] == 0;
         vl->maxFull = hmax;
