@@ -154,11 +154,13 @@ struct HistD;
 // k) each local atom's molecule force (ContributeMoleculeForceToAtoms) and the thermodynamic
 // force of its x-bin (ThermodynamicForce::apply) are added to its force first.  With
 // sortedPos / slotOf each new position is stored at the atom's slot too; slotsOnly: the
-// positions are read from the slots and stored there alone (the positions array goes stale)
+// positions are read from the slots and stored there alone (the positions array goes stale).
+// With tag, the call does not wait for the displacement: takeDisp(a, *tag, maxDisp) does
 int fusedPostPre(mrmd_atoms* a, double dt, bool langevin, double zeta, double temperature, uint64_t seed,
                  uint64_t call, double* maxDisp, double4* sortedPos = nullptr, const int32_t* slotOf = nullptr,
                  const mrmd_molecules* adrMol = nullptr, const double* tfForce = nullptr,
-                 const HistD* tfHd = nullptr, bool slotsOnly = false);
+                 const HistD* tfHd = nullptr, bool slotsOnly = false, uint32_t* tag = nullptr);
+void takeDisp(mrmd_atoms* a, uint32_t tag, double* maxDisp);
 // whether mrmd_lj_apply without a predicate uses the full-row kernel (no ghost forces)
 bool ljFullRows(const mrmd_lj* lj);
 // device address of the allocation-free apply's scratch array on `device` (the current

@@ -380,9 +380,12 @@ uint64_t* dispHost(mrmd_atoms* a, const double* maxDisp, uint32_t* tag)
 }  // namespace
 
 // the fused post/pre step of time loops (k_postPre); synchronises for the displacement
+void mrmd_hip::takeDisp(mrmd_atoms* a, uint32_t tag, double* maxDisp) { finishDisp(a, maxDisp, tag); }
+
 int mrmd_hip::fusedPostPre(mrmd_atoms* a, double dt, bool langevin, double zeta, double temperature, uint64_t seed,
                            uint64_t call, double* maxDisp, double4* sortedPos, const int32_t* slotOf,
-                           const mrmd_molecules* adrMol, const double* tfForce, const HistD* tfHd, bool slotsOnly)
+                           const mrmd_molecules* adrMol, const double* tfForce, const HistD* tfHd, bool slotsOnly,
+                           uint32_t* tagOut)
 {
     MRMD_API_BEGIN(a ? a->ctx : nullptr)
     REQUIRE(a && maxDisp, "invalid arguments");
@@ -427,7 +430,10 @@ int mrmd_hip::fusedPostPre(mrmd_atoms* a, double dt, bool langevin, double zeta,
                            tag);
     }
     checkLaunch();
-    finishDisp(a, maxDisp, tag);
+    if (tagOut)
+        *tagOut = tag;
+    else
+        finishDisp(a, maxDisp, tag);
     MRMD_API_END
 }
 

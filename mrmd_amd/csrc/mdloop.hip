@@ -83,6 +83,16 @@ int mrmd_md_run(mrmd_atoms* a, mrmd_ghost_layer* gl, mrmd_verlet_list* vl, mrmd_
     // the ghost records' forces are zero: nothing between two rebuilds writes them on the
     // store-form path, so they are filled once after each ghost creation
     bool ghostForcesZero = false;
+    // The host decides about the rebuild from the largest displacement, and a chip that waits for
+    // that stands still for some 10 us a step.  Where the displacements so far say that the next
+    // step will not rebuild, its ghost update and forces are enqueued before the wait (ahead).  If
+    // it rebuilds all the same they are void: the ghosts are made and the forces stored again,
+    // and the ghost update wrote ghosts' slots only.  A wrong guess costs one force call, so the
+    // guess leaves a quarter of a step (a step's largest displacement changes by a few percent
+    // from one to the next).  With rebuilds, 4,000 atoms 37 -> 33.5 us a step, 256,000 atoms
+    // 109 -> 103.
+    bool ahead = false;
+    constexpr double DISP_MARGIN = 1.25;
     for (int64_t k = 0; k < nsteps; ++k)
     {
         if (s->langevin) ++s->call;
@@ -91,6 +101,7 @@ int mrmd_md_run(mrmd_atoms* a, mrmd_ghost_layer* gl, mrmd_verlet_list* vl, mrmd_
         if (s->max_disp >= s->skin * 0.5)
         {
             s->max_disp = 0.0;
+            ahead = false;
             // the positions, from the slots when they are kept there, back in the positions array
             const double4* from = slots.held ? vl->bin.sortedPos.p : nullptr;
             const int32_t* slotOf = slots.held ? vl->slotOf.p : nullptr;
@@ -119,6 +130,9 @@ int mrmd_md_run(mrmd_atoms* a, mrmd_ghost_layer* gl, mrmd_verlet_list* vl, mrmd_
             ++s->rebuilds;
             fresh = vl->nrows == a->nlocal + a->nghost;  // the build binned (and gathered) every record
         }
+        else if (ahead)
+        {
+        }
         else if (localsScattered && vl->nrows == a->nlocal + a->nghost)
         {
             MD_CALL(ghostUpdateSorted(gl, a, box, vl->bin.sortedPos.p, vl->ensureSlotOf(), slots.held));
@@ -129,8 +143,11 @@ int mrmd_md_run(mrmd_atoms* a, mrmd_ghost_layer* gl, mrmd_verlet_list* vl, mrmd_
             slots.release();
             MD_CALL(mrmd_halo_update(gl, a, box));
         }
-        vl->sortedFresh = fresh;
-        if (ljAssignable(lj) && vl->begin == 0 && vl->end == a->nlocal)
+        if (!ahead) vl->sortedFresh = fresh;
+        if (ahead)
+        {
+        }
+        else if (ljAssignable(lj) && vl->begin == 0 && vl->end == a->nlocal)
         {
             // the force kernel stores the rows' forces (0.0 + F, what zeroing and adding
             // leave) and writes no ghost record; only the ghost records need their zero,
@@ -158,11 +175,22 @@ int mrmd_md_run(mrmd_atoms* a, mrmd_ghost_layer* gl, mrmd_verlet_list* vl, mrmd_
             // own gather or the copies above), so the slots hold the current positions
             const bool slotsOnly = scatter && ljFullRows(lj);
             if (!slotsOnly) slots.release();
+            uint32_t tag = 0;
             MD_CALL(fusedPostPre(a, s->dt, s->langevin != 0, s->zeta, s->temperature, s->seed, s->call, &d,
                                  scatter ? vl->bin.sortedPos.p : nullptr, scatter ? vl->ensureSlotOf() : nullptr,
-                                 nullptr, nullptr, nullptr, slotsOnly));
+                                 nullptr, nullptr, nullptr, slotsOnly, &tag));
             localsScattered = scatter;
             if (slotsOnly) slots.held = true;
+            // (the conditions of the store form and of the ghost update at the slots, above)
+            ahead = slotsOnly && ghostForcesZero && ljAssignable(lj) && vl->begin == 0 && vl->end == a->nlocal &&
+                    s->max_disp + DISP_MARGIN * d < s->skin * 0.5;
+            if (ahead)
+            {
+                MD_CALL(ghostUpdateSorted(gl, a, box, vl->bin.sortedPos.p, vl->ensureSlotOf(), true));
+                vl->sortedFresh = true;
+                MD_CALL(ljApplyAssign(lj, a, vl));
+            }
+            takeDisp(a, tag, &d);
         }
         else
             MD_CALL(mrmd_vv_post(a, s->dt));
