@@ -235,6 +235,7 @@ struct IGTiled
     int queueCap;          ///< queued non-row partner pairs per workgroup (<= IG_QUEUE)
     int32_t maxStaged;     ///< the sentinel record sits at sentinelSlot(maxStaged)
     double sentinel;       ///< at (sentinel, sentinel, sentinel)
+    int32_t split;         ///< 2^split lanes share a row (the list's splitRows)
     const int8_t* skip;    ///< per tile: 1 = no record of its neighbourhood can be weighted (or null)
 };
 
@@ -391,14 +392,14 @@ __device__ inline void igRemotePair(const IGArgs& g, const IGTiled& tl, const Ti
     }
 }
 
-// the (row, flagged non-row) pairs of one row's chunks from ch0 on, by a second pass over
-// its entries (used once the workgroup's queue of such pairs is full)
+// the (row, flagged non-row) pairs of one row's chunks ch0, ch0 + step, ... by a second pass over
+// their entries (used once the workgroup's queue of such pairs is full)
 template <bool CAP>
 __device__ void igRemoteRow(const IGArgs& g, const IGTiled& tl, const TileInfo& ti, const Pre& p,
-                            const double4& pi, const Stage<false>& st, int s, int c, int ch0)
+                            const double4& pi, const Stage<false>& st, int s, int c, int ch0, int step)
 {
     const uint4* chunk = reinterpret_cast<const uint4*>(tl.nbr) + s;
-    for (int ch = ch0; ch * CHUNK < c; ++ch)
+    for (int ch = ch0; ch * CHUNK < c; ch += step)
     {
         const uint4 cur = chunk[int64_t(ch) * tl.strideS];
         const uint32_t wd[4] = {cur.x, cur.y, cur.z, cur.w};
@@ -440,20 +441,23 @@ __global__ __launch_bounds__(BLOCK) void k_igTiled(IGArgs g, IGTiled tl, Pre p, 
     loadTile(ti, tl.tiles, blk);
     if (threadIdx.x == 0) queued = 0;
     __syncthreads();
-    // the first row's loads overlap the staging
-    int s = -1, c = 0;
+    // the first row's loads overlap the staging; 2^lg lanes share a row, each with every 2^lg-th
+    // chunk (the rows that can have pairs are those of a slab, too few to fill the chip with a
+    // lane each: with 21,000 molecules, four and then eight lanes, 39 -> 28 us between events; with
+    // 160,000, one and then two, 69 -> 62)
+    const int lg = tl.split, mask = (1 << lg) - 1, items = ti.nrows << lg;
+    int s = -1, c = 0, self = 0;
     int32_t i = 0;
     double4 pi = make_double4(0.0, 0.0, 0.0, 0.0);
     uint4 cur = {0, 0, 0, 0};
-    if (int(threadIdx.x) < ti.nrows)
-    {
-        int self;
-        s = tileRow(ti, threadIdx.x, self);
+    auto openRow = [&](int t) {
+        s = tileRow(ti, t >> lg, self);
         c = tl.cnt[s];
         i = tl.sorted[s];
         pi = tl.igPos[s];
-        cur = reinterpret_cast<const uint4*>(tl.nbr)[s];
-    }
+        if ((t & mask) * CHUNK < c) cur = reinterpret_cast<const uint4*>(tl.nbr)[s + int64_t(t & mask) * tl.strideS];
+    };
+    if (int(threadIdx.x) < items) openRow(threadIdx.x);
     const Stage<false> st(stLds, sentinelSlot(tl.maxStaged) + 1);
     stageTile(ti, tl.igPos, st);
     putSentinel(st, tl.maxStaged, tl.sentinel, 0.0);
@@ -470,19 +474,9 @@ __global__ __launch_bounds__(BLOCK) void k_igTiled(IGArgs g, IGTiled tl, Pre p, 
     const MolView& M = g.m;
     const AtomsView& A = g.a;
     double eTile = 0.0;
-    for (int t = threadIdx.x; t < ti.nrows; t += blockDim.x)
+    for (int t = threadIdx.x; t < items; t += blockDim.x)
     {
-        int self = 0;
-        if (t != int(threadIdx.x))
-        {
-            s = tileRow(ti, t, self);
-            c = tl.cnt[s];
-            i = tl.sorted[s];
-            pi = tl.igPos[s];
-            cur = reinterpret_cast<const uint4*>(tl.nbr)[s];
-        }
-        else
-            tileRow(ti, t, self);
+        if (t != int(threadIdx.x)) openRow(t);
         if (c == 0 || i >= tl.rowsEnd) continue;
         // the row's own record sits in its column's staged range
         const uint32_t ownSlot = 8 * uint32_t(ldsSlot(ti, ti.selfRange[self], s));
@@ -490,10 +484,10 @@ __global__ __launch_bounds__(BLOCK) void k_igTiled(IGArgs g, IGTiled tl, Pre p, 
         const uint4* chunk = reinterpret_cast<const uint4*>(tl.nbr) + s;
         const int nch = (c + CHUNK - 1) / CHUNK;
         int overflow = -1;  // first chunk whose partner sides did not fit into the queue
-        for (int ch = 0; ch < nch; ++ch)
+        for (int ch = t & mask; ch < nch; ch += mask + 1)
         {
             uint4 nxt = cur;
-            if (ch + 1 < nch) nxt = chunk[int64_t(ch + 1) * tl.strideS];
+            if (ch + mask + 1 < nch) nxt = chunk[int64_t(ch + mask + 1) * tl.strideS];
             uint32_t remote = igChunk<CAP>(g, p, pi, st, cur, fx, fy, fz, eTile, v);
             if (remote && overflow < 0)
             {
@@ -519,7 +513,15 @@ __global__ __launch_bounds__(BLOCK) void k_igTiled(IGArgs g, IGTiled tl, Pre p, 
             cur = nxt;
         }
         // partner sides that did not fit are deposited by the row itself
-        if (overflow >= 0) igRemoteRow<CAP>(g, tl, ti, p, pi, st, s, c, overflow);
+        if (overflow >= 0) igRemoteRow<CAP>(g, tl, ti, p, pi, st, s, c, overflow, mask + 1);
+        for (int off = 1; off <= mask; off <<= 1)
+        {
+            fx += __shfl_xor(fx, off, WAVE);
+            fy += __shfl_xor(fy, off, WAVE);
+            fz += __shfl_xor(fz, off, WAVE);
+            v += __shfl_xor(v, off, WAVE);
+        }
+        if (t & mask) continue;
         const int64_t a = M.offset[i];
         A.force[a] += fx;
         A.force[A.cap + a] += fy;
@@ -917,22 +919,24 @@ int mrmd_ljig_run(mrmd_lj_idealgas* s, mrmd_molecules* m, mrmd_verlet_list* vl, 
                                vl->bin.sorted.p, vl->nrows, rows, s->igPos.p);
         }
         const IGTiled tl{vl->nbr16.p, vl->cnt16.p, vl->strideS, vl->tiles.p, vl->bin.sorted.p, s->igPos.p, rows,
-                         s->queueCap, vl->maxStaged, vl->sentinel, vl->banded ? vl->tileSkip.p : nullptr};
+                         s->queueCap, vl->maxStaged, vl->sentinel, rowSplit(vl->splitRows), vl->banded ? vl->tileSkip.p : nullptr};
         const Pre p = s->table[0];
         const size_t lds = Stage<false>::bytes(sentinelSlot(vl->maxStaged) + 1);
         if (p.capDistSqr > 0.0)
             hipLaunchKernelGGL(k_igTiled<true>, dim3(grid), dim3(vl->block), lds, ctx->stream, g, tl, p, part);
         else
             hipLaunchKernelGGL(k_igTiled<false>, dim3(grid), dim3(vl->block), lds, ctx->stream, g, tl, p, part);
-        hipLaunchKernelGGL(k_sumOrdered, dim3(1), dim3(BLOCK), 0, ctx->stream, part, int64_t(grid), part + grid,
-                           host);
+        if (host)
+            hipLaunchKernelGGL(k_sumOrdered, dim3(1), dim3(BLOCK), 0, ctx->stream, part, int64_t(grid), part + grid,
+                               host);
     }
     else if (rows > 0)
     {
         KTimer t(ctx, "lj_idealgas");
         hipLaunchKernelGGL(k_ljIdealGas, dim3(grid), dim3(BLOCK), 0, ctx->stream, g, part);
-        hipLaunchKernelGGL(k_sumOrdered, dim3(1), dim3(BLOCK), 0, ctx->stream, part, int64_t(grid), part + grid,
-                           host);
+        if (host)
+            hipLaunchKernelGGL(k_sumOrdered, dim3(1), dim3(BLOCK), 0, ctx->stream, part, int64_t(grid), part + grid,
+                               host);
     }
     else
         hipLaunchKernelGGL(k_zeroD, dim3(1), dim3(64), 0, ctx->stream, part + grid, int64_t(1));

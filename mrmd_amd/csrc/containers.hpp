@@ -177,7 +177,7 @@ void adressCollectGhosts(mrmd_atoms* a, mrmd_molecules* m, const mrmd_ghost_laye
 void adressContributeLocal(mrmd_atoms* a, mrmd_molecules* m);
 // the thermodynamic force's device table and histogram geometry
 void thermoForceTable(const mrmd_thermo_force* tf, const double** force, HistD* hd);
-// whether the table has the store form (single type, no capping): ljApplyAssign then
+// whether the table has the store form (a symmetric one): ljApplyAssign then
 // computes what zeroing the forces of the list rows and mrmd_lj_apply(pred = NULL) leave
 bool ljAssignable(const mrmd_lj* lj);
 int ljApplyAssign(mrmd_lj* lj, mrmd_atoms* atoms, mrmd_verlet_list* vl);

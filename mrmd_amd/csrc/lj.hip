@@ -613,8 +613,7 @@ bool ljApplyImpl(mrmd_lj* lj, mrmd_atoms* at, mrmd_verlet_list* vl, const mrmd_p
 
 bool mrmd_hip::ljAssignable(const mrmd_lj* lj)
 {
-    if (!lj || !lj->symmetric || lj->table.size() != 1) return false;
-    return !(lj->table[0].capDistSqr > 0.0);
+    return lj && lj->symmetric;
 }
 
 int mrmd_hip::ljApplyAssign(mrmd_lj* lj, mrmd_atoms* at, mrmd_verlet_list* vl)
@@ -665,9 +664,10 @@ bool launchTiled(mrmd_lj* lj, mrmd_verlet_list* vl, const LJArgs& a, bool assign
     };
     constexpr std::true_type yes;
     constexpr std::false_type no;
-    if (assign && !a.usePred && one && !cap)
+    if (assign && !a.usePred)
     {
-        pick(no, yes, no, yes);
+        one ? (cap ? pick(no, yes, yes, yes) : pick(no, yes, no, yes))
+            : (cap ? pick(no, no, yes, yes) : pick(no, no, no, yes));
         return true;
     }
     if (a.usePred)

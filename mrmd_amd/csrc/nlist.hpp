@@ -448,6 +448,8 @@ struct mrmd_verlet_list
     int tileCols = 2;           ///< a: tiles span a x a cell columns
     bool tilingGiven = false;   ///< set_tiling chose the shape
     int64_t tiledRows = -1;     ///< rows for which the shape was chosen
+    /// rows that can have entries: all, or in a banded list about the band's share of them
+    int64_t splitRows = 0;
     int block = 256;            ///< workgroup size of the tiled kernels
     int tilesPerCol = 0;
     int64_t ntiles = 0;

@@ -706,9 +706,17 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
     // a shape nobody asked for follows the rows: where they are too few to fill the chip, tiles of
     // as many rows as a workgroup of the force kernel holds with its lanes per row, one cell
     // column wide from four lanes on, so that there are more of them
-    if (!vl->tilingGiven && vl->tiledRows != rows)
+    vl->splitRows = rows;
+    if (vl->banded)
     {
-        const int lg = rowSplit(rows);
+        // (the neighbourhoods that reach into the band)
+        const double width = gmax[0] - gmin[0];
+        const double part = std::min(gmax[0], vl->bandHi + rn) - std::max(gmin[0], vl->bandLo - rn);
+        vl->splitRows = int64_t(double(rows) * std::min(1.0, std::max(0.0, part / width)));
+    }
+    if (!vl->tilingGiven && vl->tiledRows != vl->splitRows)
+    {
+        const int lg = rowSplit(vl->splitRows);
         vl->tileCols = lg >= 2 ? 1 : 2;
         vl->tileK = 0;
         if (lg > 0)
@@ -716,7 +724,7 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
             const int a = R == 1 ? vl->tileCols : 1;
             vl->tileK = std::max(1, int(double(vl->block >> lg) / (a * a * perCell)));
         }
-        vl->tiledRows = rows;
+        vl->tiledRows = vl->splitRows;
     }
     int a = std::max(1, std::min(vl->tileCols, R == 1 ? 3 : 1));
     const int W = a + 2 * R;
