@@ -41,7 +41,7 @@ constexpr int B_STEN = B_COLS + 2; // staged columns per axis
 constexpr int B_RANGES = B_STEN * B_STEN * 3;  // staged columns, up to three image pieces each
 constexpr int B_SELF = B_COLS * B_COLS;
 constexpr int B_SPAN = 18;         // cells of a tile's column run (K + 2), so K <= 16
-constexpr int TARGET_STAGED = 1400;  // staged records wanted per tile
+constexpr int TARGET_STAGED = 1300;  // staged records wanted per tile (1400: 1 to 4 % slower, 1100: up to 12 %)
 constexpr int B_ROW_LANES = 256;   // lanes that the force kernel lays a tile's rows out for
 constexpr int B_BUILD_BLOCK = 8 * WAVE;
 constexpr int B_PAD = 4;           // staged records past the neighbourhood a candidate group may read
@@ -1013,15 +1013,11 @@ __device__ double bForceRows(const BS& b, const TileB& ti, const RepD& R, const 
     return eTile;
 }
 
-// tiles [tileBase, tileBase + gridDim.x): the plain replicas' tiles (W = false, {x, y, z}
-// staged) or the AdResS replicas' (W = true, whole records staged)
+// one tile of a plain replica (W = false, {x, y, z} staged) or of an AdResS replica (W = true, whole
+// records staged)
 template <bool CAP, bool W>
-__global__ __launch_bounds__(BLOCK) void k_bForce(BS b)
+__device__ inline void bForceTile(const BS& b, unsigned t, double4* stLds, TileB& ti, double* red)
 {
-    extern __shared__ double4 stLds[];
-    __shared__ TileB ti;
-    __shared__ double red[BLOCK / WAVE];
-    const unsigned t = unsigned(b.tileBase) + xcdBlock();
     const TileG G = b.tg[t];
     loadTileB(ti, b.tiles, t);
     __syncthreads();
@@ -1055,6 +1051,29 @@ __global__ __launch_bounds__(BLOCK) void k_bForce(BS b)
                                                          GlobalFetch{&ti, b.pos, R.L[0], R.L[1], R.L[2]});
     const double e = blockSum(0.5 * eTile, red);
     if (threadIdx.x == 0) b.ePart[t] = e;
+}
+
+// tiles [tileBase, tileBase + gridDim.x), all plain or all AdResS
+template <bool CAP, bool W>
+__global__ __launch_bounds__(BLOCK) void k_bForce(BS b)
+{
+    extern __shared__ double4 stLds[];
+    __shared__ TileB ti;
+    __shared__ double red[BLOCK / WAVE];
+    bForceTile<CAP, W>(b, unsigned(b.tileBase) + xcdBlock(), stLds, ti, red);
+}
+
+// the tiles of all replicas in one launch (the plain ones are those below tileBase)
+template <bool CAP>
+__global__ __launch_bounds__(BLOCK) void k_bForceAll(BS b)
+{
+    extern __shared__ double4 stLds[];
+    __shared__ TileB ti;
+    __shared__ double red[BLOCK / WAVE];
+    if (int(blockIdx.x) < b.tileBase)
+        bForceTile<CAP, false>(b, blockIdx.x, stLds, ti, red);
+    else
+        bForceTile<CAP, true>(b, blockIdx.x, stLds, ti, red);
 }
 
 // LJ_IdealGas::updateMeanCompensationEnergy (LJ_IdealGas.cpp:21-50) at the reference's
@@ -1452,7 +1471,20 @@ void mrmd_batch::enqueueSteps(int64_t n)
             hipLaunchKernelGGL(kernel, dim3(unsigned(t1 - t0)), dim3(block), lds, c->stream, f);
         };
         const size_t ldsPlain = Stage<true>::bytes(stageCapPlain), ldsAdress = Stage<false>::bytes(stageCapAdress);
-        if (cap_)
+        // With no more tiles than the chip holds at once (two of the larger a CU) a launch takes as
+        // long as one tile does, and one for all takes 22 us where one each take 22 and 18
+        // (31,000 atoms); with more the plain tiles want their own registers and LDS
+        if (plainTiles > 0 && plainTiles < ntiles && ntiles <= 2 * 256)
+        {
+            BS f = b;
+            f.tileBase = int32_t(plainTiles);
+            const size_t lds = std::max(ldsPlain, ldsAdress);
+            if (cap_)
+                hipLaunchKernelGGL(k_bForceAll<true>, dim3(unsigned(ntiles)), dim3(block), lds, c->stream, f);
+            else
+                hipLaunchKernelGGL(k_bForceAll<false>, dim3(unsigned(ntiles)), dim3(block), lds, c->stream, f);
+        }
+        else if (cap_)
         {
             force(k_bForce<true, false>, 0, plainTiles, ldsPlain);
             force(k_bForce<true, true>, plainTiles, ntiles, ldsAdress);
