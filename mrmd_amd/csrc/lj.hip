@@ -305,17 +305,26 @@ __global__ __launch_bounds__(BLOCK) void k_ljHalf(LJArgs a, const int32_t* __res
     }
 }
 
-// ordered sum of per-workgroup partials (one workgroup)
-__global__ void k_sumPartials(const double* partials, int64_t n, int width, double* out)
+// ordered sums of per-workgroup partials, a workgroup for each of the `width` columns (one for all
+// took 13 us for the eight of a two-type table's gradients)
+__global__ __launch_bounds__(BLOCK) void k_sumPartials(const double* partials, int64_t n, int width, double* out)
 {
     __shared__ double red[BLOCK / WAVE];
-    for (int c = 0; c < width; ++c)
+    const int c = int(blockIdx.x);
+    // (eight loads in flight, added in order)
+    double s = 0.0;
+    int64_t k = threadIdx.x;
+    for (; k + 7 * blockDim.x < n; k += 8 * blockDim.x)
     {
-        double s = 0.0;
-        for (int64_t k = threadIdx.x; k < n; k += blockDim.x) s += partials[k * width + c];
-        s = blockSum(s, red);
-        if (threadIdx.x == 0) out[c] = s;
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = partials[(k + u * blockDim.x) * width + c];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s += v[u];
     }
+    for (; k < n; k += blockDim.x) s += partials[k * width + c];
+    s = blockSum(s, red);
+    if (threadIdx.x == 0) out[c] = s;
 }
 
 __global__ void k_ljEval(const Pre* table, const double* d2, const int64_t* idx, int64_t n, double* ff, double* e)
@@ -840,7 +849,7 @@ int mrmd_lj_energy_virial(mrmd_lj* lj, double* e, double* w)
     if (!lj->evValid)
     {
         if (lj->nPartials > 0)
-            hipLaunchKernelGGL(k_sumPartials, dim3(1), dim3(BLOCK), 0, lj->ctx->stream, lj->partials.p, lj->nPartials, 2,
+            hipLaunchKernelGGL(k_sumPartials, dim3(2), dim3(BLOCK), 0, lj->ctx->stream, lj->partials.p, lj->nPartials, 2,
                                lj->ev.p);
         checkLaunch();
         lj->nPartials = 0;
@@ -920,7 +929,7 @@ extern "C" int mrmd_lj_adjoint(mrmd_lj* lj, const mrmd_atoms* at, mrmd_verlet_li
             cap ? launch(k_ljAdjoint<true, true>) : launch(k_ljAdjoint<true, false>);
         else
             cap ? launch(k_ljAdjoint<false, true>) : launch(k_ljAdjoint<false, false>);
-        hipLaunchKernelGGL(k_sumPartials, dim3(1), dim3(BLOCK), 0, ctx->stream, pg, int64_t(adjGrid), 2 * nt2, pgSum);
+        hipLaunchKernelGGL(k_sumPartials, dim3(unsigned(2 * nt2)), dim3(BLOCK), 0, ctx->stream, pg, int64_t(adjGrid), 2 * nt2, pgSum);
     }
     checkLaunch();
     // outputs: dL/dx back to row-major, the parameter sums to the host (one synchronisation)

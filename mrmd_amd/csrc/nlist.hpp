@@ -145,9 +145,9 @@ constexpr int CHUNK = 8;
 // Lanes of the tiled force kernels that share a row (log2).  One lane walks the ~77 neighbours of
 // a row of a liquid in twenty dependent fours, 12 us however few rows there are; a system too
 // small to fill the chip's 256 CUs x 8 waves x 64 lanes with rows splits each over up to eight
-// lanes (4,000 atoms: force 14.1 -> 6.1 us; 32,000 atoms, two types: 19.2 -> 12.4 us).  It follows
-// from the row count alone, so that a row's sums, whose order it sets, do not depend on the
-// tiling.
+// lanes (force between events, 4,000 atoms: 15.9 -> 11.0 us; 32,000 atoms, two types: 21.4 -> 14.6
+// us; 62,000 atoms of a gas: 18.1 -> 16.4 us).  It follows from the row count alone, so that a row's
+// sums, whose order it sets, do not depend on the tiling.
 constexpr int MAX_SPLIT = 3;
 inline int rowSplit(int64_t rows)
 {
@@ -165,12 +165,11 @@ __host__ __device__ inline int64_t entryIndex(int64_t k, int64_t s, int64_t stri
 }
 
 // The staged records of the force kernels: {z} (XYZ, 24 bytes a record, where the kernel needs
-// positions only) or {z, w} pairs (32 bytes, w = type or slab weight), then {x, y} pairs.  A neighbour is one 16-byte and one 8-byte read (or two 16-byte
-// ones): random gathers of 64 lanes take 19.7 LDS cycles per neighbour in this form, against
-// 32.0 for {x, y, z} records of 24 bytes, whose x and y come as one two-address read
-// (measured with 16 waves per CU; records a few places apart 14.6 against 22.6), and the LDS
-// pipe is what bounds the uncapped force kernel (with every lane reading one address it
-// runs in half the time).
+// positions only) or {z, w} pairs (32 bytes, w = type or slab weight), then {x, y} pairs.  A
+// neighbour is one 16-byte and one 8-byte read (or two 16-byte ones): random gathers of 64 lanes
+// take 19.7 LDS cycles per neighbour in this form, against 32.0 for {x, y, z} records of 24 bytes,
+// whose x and y come as one two-address read (measured with 16 waves per CU; records a few places
+// apart 14.6 against 22.6).
 template <bool XYZ>
 struct Stage
 {
