@@ -159,7 +159,7 @@ constexpr size_t LDS_LIMIT = 64000;  // dynamic LDS of a list build workgroup (6
 // one by one
 constexpr int BUILD_BLOCK = 12 * WAVE;
 
-// (5 waves per SIMD: 96 registers; with 98 it measured 1.14 instead of 1.08 ms at 4M atoms)
+// (5 waves per SIMD: 96 registers; with 98 it measured 1.14 instead of 1.06 ms at 4M atoms)
 template <int R, bool WIDE, bool GS>
 __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTiled(const double4* __restrict__ sortedPos,
                                                        const int32_t* __restrict__ sorted,
@@ -717,12 +717,14 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
     if (!vl->tilingGiven && vl->tiledRows != vl->splitRows)
     {
         const int lg = rowSplit(vl->splitRows);
-        vl->tileCols = lg >= 2 ? 1 : 2;
+        // (in sparse cells even the tallest tile of one column has fewer rows than that: two columns)
+        const double cells = double(vl->block >> lg) / perCell;
+        vl->tileCols = lg >= 2 && cells <= double(std::min(g.n[2], MAX_SPAN - 2 * R)) ? 1 : 2;
         vl->tileK = 0;
         if (lg > 0)
         {
             const int a = R == 1 ? vl->tileCols : 1;
-            vl->tileK = std::max(1, int(double(vl->block >> lg) / (a * a * perCell)));
+            vl->tileK = std::max(1, int(std::min(cells / (a * a), double(MAX_SPAN))));
         }
         vl->tiledRows = vl->splitRows;
     }
