@@ -930,7 +930,7 @@ __device__ inline void ljQuadWeighted(const Pre& p, double rcSqr, const double4&
 }
 
 // The rows of one tile: pair forces (W: weighted, with the drift and compensation terms); returns
-// the lane's energy sum.  2^split lanes share a row (rowLanes).
+// the lane's energy sum.  2^split lanes share a row (layoutTiles).
 template <bool CAP, bool W, bool GS, class St>
 __device__ double bForceRows(const BS& b, const TileB& ti, const RepD& R, const St& st)
 {

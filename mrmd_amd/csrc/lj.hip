@@ -157,6 +157,10 @@ __device__ inline void ljQuadTypes(const LJArgs& a, const Pre* tab, int ti0, con
 // GS: the neighbourhood is staged in the tile's slice of the list's global staging buffer
 // (dense inputs whose tiles exceed the LDS) instead of LDS
 // SPLIT: 2^tl.split lanes share a row (small systems, see rowSplit)
+// Bound by vector instruction issue (some 80 % of the time at 4 million atoms, of which staging is
+// a tenth): ~27 cycles per list entry, the reciprocal being a quarter-rate instruction.  With
+// records read by two-address LDS reads, run starts looked up per staged record and shuffles in
+// the reductions 441 us at 4 million atoms, in this form 395 to 415.
 template <bool PRED, bool ONE, bool CAP, bool ASSIGN, bool GS, bool SPLIT>
 __global__ __launch_bounds__(BLOCK, PRED || (CAP && !ONE) ? 2 : 4) void k_ljTiled(LJArgs a, TiledList tl, Pre p1, double* partials)
 {

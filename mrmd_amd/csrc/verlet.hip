@@ -148,7 +148,7 @@ constexpr size_t LDS_LIMIT = 64000;  // dynamic LDS of a list build workgroup (6
 // 16-bit dot products give the squared distance less a threshold in 4 instructions, one more
 // shifts its sign into the hit bits and two the sign against a wider threshold.  A coordinate is
 // rounded by at most half a unit, so a distance is off by at most sqrt(3) units; pairs
-// within 1.75 units of r_n (about 1 in 1,500 candidates) are decided by the FP64 test on the
+// within 1.75 units of r_n (about 1 in 2,000 candidates) are decided by the FP64 test on the
 // records in memory, the unfused expression of the reference, and so is the half-list bit
 // of partners whose x differs by less than two units: the list is the exact one.  A record
 // outside its tile's range (positions beyond the grid) makes every pair of the tile go that
