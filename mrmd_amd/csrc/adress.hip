@@ -1360,6 +1360,8 @@ void mrmd_hip::adressPrepare(mrmd_atoms* a, mrmd_molecules* m, const mrmd_ghost_
     ig->igPosList = vl;
 }
 
+void mrmd_hip::adressForget(mrmd_lj_idealgas* ig) { ig->igPosFresh = false; }
+
 void mrmd_hip::adressCollectGhosts(mrmd_atoms* a, mrmd_molecules* m, const mrmd_ghost_layer* gl)
 {
     mrmd_ctx* ctx = a->ctx;

@@ -173,6 +173,7 @@ int64_t ghostCorrSize(const mrmd_ghost_layer* gl);
 bool adressIdentityLayout(const mrmd_molecules* m, const mrmd_atoms* a);
 void adressPrepare(mrmd_atoms* a, mrmd_molecules* m, const mrmd_ghost_layer* gl, const mrmd_box* box,
                    const mrmd_slab* slab, mrmd_lj_idealgas* ig, mrmd_verlet_list* vl);
+void adressForget(mrmd_lj_idealgas* ig);  // the slot records of an adressPrepare that a rebuild voids
 void adressCollectGhosts(mrmd_atoms* a, mrmd_molecules* m, const mrmd_ghost_layer* gl);
 void adressContributeLocal(mrmd_atoms* a, mrmd_molecules* m);
 // the thermodynamic force's device table and histogram geometry

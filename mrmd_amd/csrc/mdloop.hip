@@ -35,6 +35,9 @@ struct SlotPositions
         if (held) vl->positionsFromSlotsNoThrow(a->pos.p);
     }
 };
+
+// the part of the last step's largest displacement that the next step's is expected to stay below
+constexpr double DISP_MARGIN = 1.25;
 }  // namespace
 
 extern "C" {
@@ -92,7 +95,6 @@ int mrmd_md_run(mrmd_atoms* a, mrmd_ghost_layer* gl, mrmd_verlet_list* vl, mrmd_
     // from one to the next).  With rebuilds, 4,000 atoms 37 -> 33.5 us a step, 256,000 atoms
     // 109 -> 103.
     bool ahead = false;
-    constexpr double DISP_MARGIN = 1.25;
     for (int64_t k = 0; k < nsteps; ++k)
     {
         if (s->langevin) ++s->call;
@@ -243,6 +245,10 @@ int mrmd_adress_md_run(mrmd_atoms* a, mrmd_molecules* m, mrmd_ghost_layer* gl, m
     const double* tfForce = nullptr;
     HistD tfHd{};
     thermoForceTable(tf, &tfForce, &tfHd);
+    // as above: where the next step will hardly rebuild, its adressPrepare is enqueued before the
+    // wait for the displacement.  (LJ_IdealGas counts its runs, so it is not.)  A rebuild makes all
+    // that it wrote again: ghosts, molecules, zero forces, slot records.
+    bool ahead = false;
     for (int64_t k = 0; k < nsteps; ++k)
     {
         ++s->call;
@@ -251,6 +257,7 @@ int mrmd_adress_md_run(mrmd_atoms* a, mrmd_molecules* m, mrmd_ghost_layer* gl, m
         if (rebuild)
         {
             s->max_disp = 0.0;
+            if (ahead) adressForget(ig);
             MD_CALL(mrmd_molecules_update(m, a, nullptr));
             MD_CALL(mrmd_multires_wrap(m, a, box));
             MD_CALL(mrmd_multires_halo_create(gl, m, a, box));
@@ -277,7 +284,9 @@ int mrmd_adress_md_run(mrmd_atoms* a, mrmd_molecules* m, mrmd_ghost_layer* gl, m
                 MD_CALL(mrmd_verlet_build_molecules(vl, m, 0, m->nlocal, rn, 1.0, gridMin, gridMax, 0));
         }
         if (fused)
-            adressPrepare(a, m, rebuild ? nullptr : gl, box, slab, ig, vl);
+        {
+            if (rebuild || !ahead) adressPrepare(a, m, rebuild ? nullptr : gl, box, slab, ig, vl);
+        }
         else
         {
             if (!rebuild) MD_CALL(mrmd_halo_update(gl, a, box));
@@ -297,9 +306,16 @@ int mrmd_adress_md_run(mrmd_atoms* a, mrmd_molecules* m, mrmd_ghost_layer* gl, m
         ++s->steps;
         if (s->tf_every && s->steps % s->tf_every == 0)
             MD_CALL(mrmd_tf_update(tf, s->tf_sigma, s->tf_range, &s->tf_pred));
+        ahead = false;
         if (k + 1 < nsteps && fused)
+        {
+            uint32_t tag = 0;
             MD_CALL(fusedPostPre(a, s->dt, true, s->zeta, s->temperature, s->seed, s->call, &d, nullptr, nullptr, m,
-                                 tfForce, &tfHd));
+                                 tfForce, &tfHd, false, &tag));
+            ahead = s->max_disp + DISP_MARGIN * d < s->skin * 0.5;
+            if (ahead) adressPrepare(a, m, gl, box, slab, ig, vl);
+            takeDisp(a, tag, &d);
+        }
         else
         {
             if (fused) adressContributeLocal(a, m);
