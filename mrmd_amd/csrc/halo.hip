@@ -216,9 +216,9 @@ __device__ inline unsigned waveCodes(unsigned m)
 }
 
 // per tile of `rounds` x BLOCK atoms: atoms of each code, cnt[(b - 1) * tiles + tile]; a
-// wave counts only the codes present in it
+// wave counts only the codes present in it.  The real atoms' own entries of corr become -1.
 __global__ __launch_bounds__(BLOCK) void k_ghostCount3(const double4* pos, int64_t n, SubD s, int32_t* cnt,
-                                                       int64_t tiles, int rounds)
+                                                       int64_t tiles, int rounds, int32_t* corr)
 {
     __shared__ int sc[BLOCK / WAVE][GHOST_BLOCKS];
     const int64_t base = int64_t(blockIdx.x) * rounds * BLOCK;
@@ -227,6 +227,7 @@ __global__ __launch_bounds__(BLOCK) void k_ghostCount3(const double4* pos, int64
     for (int r = 0; r < rounds; ++r)
     {
         const int64_t e = base + r * BLOCK + threadIdx.x;
+        if (e < n) corr[e] = -1;
         const unsigned codes = e < n ? ghostCodes(ghostFlags(pos[e], s)) : 0u;
         if (__ballot(codes != 0) == 0) continue;
         for (unsigned present = waveCodes(codes); present; present &= present - 1)
@@ -246,8 +247,9 @@ __global__ __launch_bounds__(BLOCK) void k_ghostCount3(const double4* pos, int64
     }
 }
 
-// block bases in output order from the 26 totals (tot[b - 1]); bases[b] by code, *count = sum
-__global__ void k_ghostBases(const int32_t* tot, int32_t* bases, int32_t* count)
+// block bases in output order from the 26 totals (tot[b - 1]); bases[b] by code, the sum to the
+// host's tagged word
+__global__ void k_ghostBases(const int32_t* tot, int32_t* bases, uint64_t* host, uint32_t tag)
 {
     if (threadIdx.x != 0) return;
     int byOrder[GHOST_BLOCKS];
@@ -260,7 +262,7 @@ __global__ void k_ghostBases(const int32_t* tot, int32_t* bases, int32_t* count)
     }
     bases[0] = 0;
     for (int b = 1; b <= GHOST_BLOCKS; ++b) bases[b] = start[ghostBlockOrder(b)];
-    *count = acc;
+    __hip_atomic_store(host, tagWord(tag, uint32_t(acc)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // every real atom writes its ghosts: ghost index n + bases[b] + the tile's offset + its rank
@@ -806,10 +808,11 @@ __global__ __launch_bounds__(BLOCK) void k_molGhostScatter3(MolView m, AtomsView
 // =========================================================================================
 namespace
 {
-void resetCorr(mrmd_ghost_layer* gl, int64_t nlocal)
+// fill = false: the caller's next pass over the real atoms writes their -1
+void resetCorr(mrmd_ghost_layer* gl, int64_t nlocal, bool fill = true)
 {
     gl->corr.reserve(gl->ctx, growCap(nlocal), 0);
-    if (nlocal > 0)
+    if (fill && nlocal > 0)
         hipLaunchKernelGGL(k_fillI32, dim3(gridFor(nlocal)), dim3(BLOCK), 0, gl->ctx->stream, gl->corr.p, nlocal,
                            -1);
     gl->corrSize = nlocal;
@@ -864,15 +867,16 @@ void createAll(mrmd_ghost_layer* gl, mrmd_atoms* a, const mrmd_box* box)
     gl->blocks.ensure(ctx, 64);
     int32_t* tot = gl->blocks.p;
     int32_t* bases = tot + 32;
-    int32_t* count = bases + 27;
     hipLaunchKernelGGL(k_ghostCount3, dim3(unsigned(tiles)), dim3(BLOCK), 0, ctx->stream, a->pos.p, n, s,
-                       gl->tileCnt.p, tiles, rounds);
+                       gl->tileCnt.p, tiles, rounds, gl->corr.p);
     checkLaunch();
     scanExclusiveI32Multi(ctx, gl->tileCnt.p, gl->tileOff.p, tiles, GHOST_BLOCKS, tot);
-    hipLaunchKernelGGL(k_ghostBases, dim3(1), dim3(64), 0, ctx->stream, tot, bases, count);
+    const uint32_t tag = nextTag(ctx);
+    hipLaunchKernelGGL(k_ghostBases, dim3(1), dim3(64), 0, ctx->stream, tot, bases,
+                       reinterpret_cast<uint64_t*>(ctx->pinned) + READBACK_WORD, tag);
     checkLaunch();
     int32_t h[1];
-    readbackI32(ctx, count, 1, h);
+    takeI32(ctx, tag, 1, h);
     const int64_t newTotal = n + h[0];
     a->ensureCap(newTotal);
     a->size = newTotal;
@@ -1046,7 +1050,7 @@ int mrmd_halo_create(mrmd_ghost_layer* gl, mrmd_atoms* a, const mrmd_box* box, i
     REQUIRE(gl && a && a->ctx == gl->ctx, "invalid arguments");
     checkBox(box);
     KTimer t(gl->ctx, "halo_create");
-    resetCorr(gl, a->nlocal);
+    resetCorr(gl, a->nlocal, false);
     a->nghost = 0;
     createAll(gl, a, box);
     if (nghost) *nghost = a->nghost;
