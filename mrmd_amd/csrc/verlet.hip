@@ -135,6 +135,17 @@ constexpr int MAX_SPAN = 64;  // cells of a tile's column range along z (K + 2R)
 // four runs up to three records beyond the column run; their bits are cleared)
 constexpr int STAGE_PAD = 4;
 constexpr size_t LDS_LIMIT = 64000;  // dynamic LDS of a list build workgroup (64 KB less its static part)
+// entries of a row that the list build collects in LDS (the least list width, and the least number
+// of entries: bufCap); a row's further entries are stored one by one.  A liquid's rows of some 80 fit.
+// With buffers of the list's width, at 260,000 atoms a caller's hint of 0, 60, 150 or 300
+// neighbours made it 114, 121, 191 or 323 us, and wider rows did not fit at all; now 110 for any
+// hint, and rows of 240 take 303 instead of 385.
+constexpr int ROW_BUF = 96;
+// Up to here every workgroup has its LDS to itself (two a CU), and buffers of the list's width are
+// taken if four waves have room for them (4,000 atoms, rows of 140 and 240: 31 and 47 us, with 96
+// entries 37 and 62)
+constexpr int64_t WIDE_BUF_TILES = 2 * 256;
+static_assert(ROW_BUF % CHUNK == 0);
 
 // The list build.  S = 2R + 1 lanes share a row, one per j offset of the stencil, and walk the
 // S i offsets together, so a row's columns come in Cabana's i, j, k order: in each step a lane
@@ -152,8 +163,8 @@ constexpr size_t LDS_LIMIT = 64000;  // dynamic LDS of a list build workgroup (6
 // records in memory, the unfused expression of the reference, and so is the half-list bit
 // of partners whose x differs by less than two units: the list is the exact one.  A record
 // outside its tile's range (positions beyond the grid) makes every pair of the tile go that
-// way.  The window search runs on the 16-bit z, widened by two units.  Entries are collected
-// per row in LDS and stored as whole 16-byte chunks of neighbouring rows.
+// way.  The window search runs on the 16-bit z, widened by two units.  A row's first bufCap
+// entries are collected in LDS and stored as whole 16-byte chunks of neighbouring rows.
 // WIDE: list offsets in 64-bit arithmetic (lists of 2^31 entries or more); 32-bit otherwise
 // GS (dense inputs): the 16-bit records in the tile's slice of global memory, entries stored
 // one by one
@@ -166,7 +177,7 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
                                                        const int32_t* __restrict__ offsets,
                                                        const TileInfo* __restrict__ tiles, TileGeom tg, GridD g,
                                                        int64_t rowLo, int64_t rowHi, double rsq, double rn,
-                                                       uint16_t* nbr, int64_t strideS, int cap, int32_t* cnt,
+                                                       uint16_t* nbr, int64_t strideS, int cap, int bufCap, int32_t* cnt,
                                                        int32_t* slots, int stagedCap, double4* gstage,
                                                        int64_t gstageRecs, double bandLo, double bandHi,
                                                        int8_t* tileSkip)
@@ -180,11 +191,11 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
     const int64_t t = blockIdx.x;
     const int lane = int(threadIdx.x) % WAVE, waves = int(blockDim.x) / WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    // LDS: the waves' row buffers (RW rows of cap entries), the 16-bit records, then the LDS slot
+    // LDS: the waves' row buffers (RW rows of bufCap entries), the 16-bit records, then the LDS slot
     // of the first record of cell kl + z of range r, cstart[r * cz + z] with cz = K + 2R + 1;
     // entry z = nk closes the range (ranges outside the grid are empty)
-    uint16_t* const rowBuf = reinterpret_cast<uint16_t*>(stRaw) + (GS ? 0 : wave * RW * cap);
-    uint2* const ldsRec = reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(stRaw) + (GS ? 0 : waves * RW * cap));
+    uint16_t* const rowBuf = reinterpret_cast<uint16_t*>(stRaw) + (GS ? 0 : wave * RW * bufCap);
+    uint2* const ldsRec = reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(stRaw) + (GS ? 0 : waves * RW * bufCap));
     uint2* const rec = GS ? reinterpret_cast<uint2*>(gstage + t * gstageRecs) : ldsRec;
     int* const cstart = reinterpret_cast<int*>(ldsRec + (GS ? 0 : stagedCap + STAGE_PAD));
     const int cz = tg.K + 2 * R + 1;
@@ -411,7 +422,7 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
                 at += k < sub ? c : 0;
                 total += c;
             }
-            uint16_t* out = rowBuf + group * cap + at;
+            uint16_t* out = rowBuf + group * bufCap + at;
             // the half bit: columns of a larger x index hold larger x (binning is monotone in x),
             // smaller index smaller x; in the row's own x index the sign of dx decides
             auto append = [&](auto checked, int qb, uint32_t hits, uint32_t half) {
@@ -422,13 +433,10 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
                     uint32_t v = uint32_t(qb + u) << SH;
                     if (da > 0) v |= 0x8000u;
                     if (da == 0) v |= ((half << u) >> 16) & 0x8000u;
-                    if (!decltype(checked)::value || at < cap)
-                    {
-                        if constexpr (GS)
-                            nbr[(Off(at >> 3) * Off(strideS) + Off(s)) * CHUNK + (at & 7)] = uint16_t(v);
-                        else
-                            *out = uint16_t(v);
-                    }
+                    if (!GS && (!decltype(checked)::value || at < bufCap))
+                        *out = uint16_t(v);
+                    else if (!decltype(checked)::value || at < cap)
+                        nbr[(Off(at >> 3) * Off(strideS) + Off(s)) * CHUNK + (at & 7)] = uint16_t(v);
                     if (GS || decltype(checked)::value) ++at;
                     ++out;
                 }
@@ -445,7 +453,7 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
                     }
             };
             n += total;
-            if (__any(n > cap))
+            if (__any(n > (GS ? cap : bufCap)))
                 appendAll(std::true_type{});
             else
                 appendAll(std::false_type{});
@@ -460,10 +468,10 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
         if (isRow)
             for (int k = kept + sub; k < nch * CHUNK; k += S)
             {
-                if constexpr (GS)
-                    nbr[(Off(k >> 3) * Off(strideS) + Off(s)) * CHUNK + (k & 7)] = uint16_t(pad);
+                if (!GS && k < bufCap)
+                    rowBuf[group * bufCap + k] = uint16_t(pad);
                 else
-                    rowBuf[group * cap + k] = uint16_t(pad);
+                    nbr[(Off(k >> 3) * Off(strideS) + Off(s)) * CHUNK + (k & 7)] = uint16_t(pad);
             }
         if (live && sub == 0) cnt[s] = isRow ? kept : 0;  // the true width goes to WIDTH_WORD
         localMax = max(localMax, isRow ? n : 0);
@@ -472,14 +480,15 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
             // the wave's rows go out chunk by chunk, neighbouring rows (mostly neighbouring slots)
             // from neighbouring lanes
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            const int chunks = RW * waveMaxInt(isRow ? nch : 0);
+            const int bufCh = isRow ? min(nch, bufCap / CHUNK) : 0;
+            const int chunks = RW * waveMaxInt(bufCh);
             for (int x = lane; x - lane < chunks; x += WAVE)
             {
                 const int r = x % RW, ch = x / RW;
-                const int sr = __shfl(s, r * S, WAVE), nr = __shfl(isRow ? nch : 0, r * S, WAVE);
+                const int sr = __shfl(s, r * S, WAVE), nr = __shfl(bufCh, r * S, WAVE);
                 if (ch < nr)
                     reinterpret_cast<uint4*>(nbr)[Off(ch) * Off(strideS) + Off(sr)] =
-                        reinterpret_cast<const uint4*>(rowBuf + r * cap)[ch];
+                        reinterpret_cast<const uint4*>(rowBuf + r * bufCap)[ch];
             }
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         }
@@ -765,7 +774,7 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
         vl->gstage.ensure(ctx, std::max<int64_t>(vl->ntiles, 1) * vl->gstageRecs);
     }
     if (vl->banded) vl->tileSkip.ensure(ctx, std::max<int64_t>(vl->ntiles, 1));
-    if (vl->capFull <= 0) vl->capFull = int32_t(std::max<int64_t>(2 * maxNeigh + 16, 96));
+    if (vl->capFull <= 0) vl->capFull = int32_t(std::max<int64_t>(2 * maxNeigh + 16, ROW_BUF));
     vl->capFull = (vl->capFull + CHUNK - 1) / CHUNK * CHUNK;
     bool mono = false;
     const int stagedCap = std::max(vl->maxStaged, 1);
@@ -776,24 +785,27 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
         if (vl->ntiles > 0 && end > begin)
         {
             KTimer tk(ctx, "verlet_tiled");
-            // LDS: the row buffers (fewer waves where long rows would not fit), the 16-bit records
-            // and the per-cell start table of (a + 2R)^2 ranges x (K + 2R + 1)
+            // LDS: the row buffers, the 16-bit records and the per-cell start table of (a + 2R)^2 ranges
+            // x (K + 2R + 1); at most 23,000 bytes without the row buffers, so eight waves of the narrow
+            // ones fit
             const int W = vl->tileCols + 2 * R, rowsPerWave = WAVE / (2 * R + 1);
             const size_t fixed = (vl->globalStage ? 0 : size_t(stagedCap + STAGE_PAD) * sizeof(uint2)) +
                                  size_t(W * W * (vl->tileK + 2 * R + 1)) * sizeof(int);
-            const size_t perWave = vl->globalStage ? 0 : size_t(rowsPerWave) * vl->capFull * sizeof(uint16_t);
+            auto perWave = [&](int entries) {
+                return vl->globalStage ? 0 : size_t(rowsPerWave) * entries * sizeof(uint16_t);
+            };
+            const bool wideBuf = vl->ntiles <= WIDE_BUF_TILES && fixed + 4 * perWave(vl->capFull) <= LDS_LIMIT;
+            const int bufCap = wideBuf ? vl->capFull : ROW_BUF;
             // four waves a workgroup fill the chip from 1,280 tiles on (five waves a SIMD); with
             // fewer tiles their rows go to up to twelve waves
             int waves = vl->block / WAVE;
             if (!vl->tilingGiven) waves = int(std::max<int64_t>(waves, std::min<int64_t>(12, 5120 / vl->ntiles)));
-            while (waves > 1 && fixed + waves * perWave > LDS_LIMIT) --waves;
-            const size_t lds = fixed + waves * perWave;
-            if (lds > LDS_LIMIT)
-                fail(MRMD_ERR_UNSUP, "rows of %d neighbours do not fit the list build's LDS", vl->capFull);
+            while (waves > 1 && fixed + waves * perWave(bufCap) > LDS_LIMIT) --waves;
+            const size_t lds = fixed + waves * perWave(bufCap);
             auto launch = [&](auto kernel) {
                 hipLaunchKernelGGL(kernel, dim3(unsigned(vl->ntiles)), dim3(waves * WAVE), lds, ctx->stream,
                                    vl->bin.sortedPos.p, vl->bin.sorted.p, vl->bin.offsets.p, vl->tiles.p, geom(vl), g,
-                                   begin, end, rn * rn, rn, vl->nbr16.p, vl->strideS, vl->capFull, vl->cnt16.p, slots,
+                                   begin, end, rn * rn, rn, vl->nbr16.p, vl->strideS, vl->capFull, bufCap, vl->cnt16.p, slots,
                                    stagedCap, vl->gstage.p, vl->gstageRecs, vl->bandLo, vl->bandHi, vl->tileSkip.p);
             };
             const bool wide = vl->forceWide || int64_t(vl->capFull) * vl->strideS >= (int64_t(1) << 31);
