@@ -373,8 +373,9 @@ struct Grid16
     }
     __device__ void thresholds(double rn, int& sure, int& doubt) const
     {
-        const double rnq = rn * scale;
-        sure = int(floor((rnq - QUANT_DOUBT) * (rnq - QUANT_DOUBT)));
+        const double rnq = rn * scale, in = rnq - QUANT_DOUBT;
+        // (a radius of less than QUANT_DOUBT units has no sure neighbours)
+        sure = in >= 0.0 ? int(floor(in * in)) : -1;
         doubt = int(ceil((rnq + QUANT_DOUBT) * (rnq + QUANT_DOUBT))) - sure;
     }
 };

@@ -71,3 +71,22 @@ def test_clusters_within_the_radius(M, ctx, n, ratio):
     vl.build(a, 0, *kw)
     ov.build(c, 1000, 0, *kw)
     _same_lists(vl, ov, 1000, True)
+
+
+def test_radius_far_below_the_cells(M, ctx):
+    """a radius of less than a unit of the tiles' 16-bit coordinates (three cells of 10,000 radii an
+    axis): every pair within a few units is decided on the records themselves, also across a cell
+    face, where no column ties decide it"""
+    g = np.random.default_rng(14)
+    n, pos = 300, []
+    for d in (0.004, 0.0095, 0.0105, 0.013, 0.02, 0.04):
+        u = g.normal(size=(n, 3))
+        u[:, 0] = np.abs(u[:, 0]) + 1.0
+        u *= d / np.linalg.norm(u, axis=1, keepdims=True)
+        base = g.uniform(5.0, 295.0, (n, 3))
+        base[:, 0] = np.where(g.uniform(size=n) < 0.5, 100.0, 200.0) - u[:, 0] * g.uniform(0.1, 0.9, n)
+        pos += [base, base + u]
+    pos = np.concatenate(pos)
+    _, _, vl, ov = _lists(M, ctx, pos, 0.01, 1e4, 300.0)
+    assert ov.total() >= 2 * n
+    _same_lists(vl, ov, pos.shape[0], True)
