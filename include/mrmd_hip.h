@@ -531,7 +531,9 @@ int mrmd_batch_set_stage_cap(mrmd_batch* b, int limit);
 int mrmd_batch_upload(mrmd_batch* b, int field, const double* host);
 int mrmd_batch_download(mrmd_batch* b, int field, double* host);
 /* advance every replica by nsteps; graph_steps > 0 replays a captured graph of that many
- * steps (a remainder runs as plain launches), 0 launches every kernel directly */
+ * steps (a remainder runs as plain launches), 0 launches every kernel directly.  Fails where a
+ * neighbour row exceeded the list's width, or lay past the 32,768 records of a tile's
+ * neighbourhood that list entries tell apart (the steps are then not to be used) */
 int mrmd_batch_run(mrmd_batch* b, int64_t nsteps, int graph_steps);
 /* per-replica potential energy of the last force evaluation and current kinetic energy */
 int mrmd_batch_energies(mrmd_batch* b, double* potential, double* kinetic);

@@ -25,6 +25,7 @@
 #include <cfloat>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "detmath.hpp"
@@ -44,6 +45,9 @@ constexpr int B_SPAN = 18;         // cells of a tile's column run (K + 2), so K
 constexpr int TARGET_STAGED = 1300;  // staged records wanted per tile (1400: 1 to 4 % slower, 1100: up to 12 %)
 constexpr int B_ROW_LANES = 256;   // lanes that the force kernel lays a tile's rows out for
 constexpr int B_BUILD_BLOCK = 8 * WAVE;
+constexpr int B_MAX_SLOT = 0x7fff; // largest staged slot of a list entry (15 bits)
+// bits of BS::err, reported when the run ends
+constexpr int ERR_WIDTH = 1, ERR_SLOT = 2;
 constexpr int B_PAD = 4;           // staged records past the neighbourhood a candidate group may read
 constexpr int COMP_BINS = 200;     // LJ_IdealGas compensation bins (LJ_IdealGas.hpp:54)
 constexpr double COMP_SCALE = 4294967296.0;
@@ -647,6 +651,7 @@ __device__ void bBuildRows(const BS& b, const TileB& ti, const TileG& G, const R
     const GlobalFetch exact{&ti, b.pos, R.L[0], R.L[1], R.L[2]};
     const int sub = lane % S, group = lane / S, first = group * S;
     int localMax = 0;
+    bool beyond = false;  // a slot that no entry holds (staged records are far fewer in LDS)
     for (int row0 = wave * RW; row0 < ti.nrows; row0 += waves * RW)
     {
         const int row = row0 + group;
@@ -774,6 +779,7 @@ __device__ void bBuildRows(const BS& b, const TileB& ti, const TileG& G, const R
                     const int u = __builtin_clz(hits);
                     hits ^= 0x80000000u >> u;
                     const uint16_t v = uint16_t((qb + u) << sh);
+                    if constexpr (!std::is_same_v<Rec, LdsRec>) beyond = beyond || qb + u > B_MAX_SLOT;
                     if (at < cap) b.nbr[entryIndex(at, s, b.strideS)] = v;
                     ++at;
                 }
@@ -790,8 +796,10 @@ __device__ void bBuildRows(const BS& b, const TileB& ti, const TileG& G, const R
                 b.nbr[entryIndex(k, s, b.strideS)] = uint16_t(qSelf << sh);
         if (live && sub == 0) b.cnt[s] = kept;  // an overflow is reported through err; reads stay in the list
         localMax = max(localMax, live ? n : 0);
+        if constexpr (!std::is_same_v<Rec, LdsRec>) beyond = beyond || (live && n > 0 && qSelf > B_MAX_SLOT);
     }
-    if (localMax > b.capList) atomicOr(b.err, 1);
+    if (localMax > b.capList) atomicOr(b.err, ERR_WIDTH);
+    if (beyond) atomicOr(b.err, ERR_SLOT);
 }
 
 // full-row list of every tile of a flagged replica
@@ -1835,7 +1843,11 @@ int mrmd_batch_run(mrmd_batch* b, int64_t nsteps, int graphSteps)
     HIPCHECK(hipMemcpyAsync(&e, b->err.p, 4, hipMemcpyDeviceToHost, c->stream));
     sync(c);
     b->steps += nsteps;
-    if (e & 1) fail(MRMD_ERR_STATE, "a neighbour row exceeded the list width %d (density too high)", b->capList);
+    if (e & ERR_SLOT)
+        fail(MRMD_ERR_STATE, "neighbours beyond the first %d records of a tile's neighbourhood (cells too crowded)",
+             B_MAX_SLOT + 1);
+    if (e & ERR_WIDTH)
+        fail(MRMD_ERR_STATE, "a neighbour row exceeded the list width %d (density too high)", b->capList);
     MRMD_API_END
 }
 
