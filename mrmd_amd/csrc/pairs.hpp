@@ -138,7 +138,8 @@ struct PairSums
     {
 #pragma clang fp contract(fast)
         const double s12 = p.ff1 != 0.0 ? (w + p.ff2 * e) / p.ff1 : 0.0;
-        energy = p.ef1 * s12 - p.ef2 * e;
+        // (where sum f6 overflows so does sum f6^2, and the energy is the latter's infinity)
+        energy = p.ef1 * s12 - (isinf(e) ? 0.0 : p.ef2 * e);
         virial = w;
         if (CAP)
         {

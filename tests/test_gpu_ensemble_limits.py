@@ -1,4 +1,4 @@
-"""Ensembles at the limits of their lists."""
+"""Ensembles at the limits of their lists and sums."""
 import numpy as np
 import pytest
 
@@ -54,3 +54,12 @@ def test_neighbourhoods_beyond_the_entries_are_refused(M, ctx, side):
         f = d * (f6 * (48.0 * f6 - 24.0) / w)[:, None]
         # 5,000 terms in another order: sqrt(5000) roundings of 1.1e-16 of the summed magnitudes
         assert np.abs(F[k] - f.sum(axis=0)).max() <= 1e-14 * np.abs(f).sum(axis=0).max()
+
+
+@pytest.mark.parametrize("cap", [0.0, 1e-100])
+def test_energy_of_an_overflowing_pair_is_infinite(M, ctx, cap):
+    """two atoms 1e-60 apart: r^-12 and r^-6 overflow, and their difference is the first, not a NaN"""
+    pos = np.array([[0.0, 0.0, 0.0], [1e-60, 0.0, 0.0], [3.0, 3.0, 3.0]])
+    e = _cold(M, ctx, pos, [6.0] * 3, 2.5, cap=cap)
+    e.run(1, 0)
+    assert e.energies()[0][0] == np.inf
