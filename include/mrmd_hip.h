@@ -267,8 +267,9 @@ int mrmd_verlet_count_within(mrmd_verlet_list* vl, const mrmd_atoms* atoms, doub
                              int64_t* full_entries);
 /* Launch shape of the tiled list and the tiled force kernel (no reference counterpart; the
  * reference's Cabana list has no tiling): a tile is tile_cells cells along z (0 = chosen
- * from the density at the next build) in tile_columns x tile_columns cell columns (1-3;
+ * at each build, from the density) in tile_columns x tile_columns cell columns (1-3;
  * 1 when the cell ratio is below 1); block = workgroup size (64, 128, 192 or 256).
+ * tile_cells 0 with tile_columns 2 is the default: small systems then get narrower tiles.
  * Applies from the next build; results do not depend on it. */
 int mrmd_verlet_set_tiling(mrmd_verlet_list* vl, int tile_cells, int tile_columns, int block);
 /* No counterpart in the reference (a test knob): on != 0 builds the list with the 64-bit

@@ -409,7 +409,8 @@ class HalfVerletList:
 
     def set_tiling(self, tile_cells=0, block=256, tile_columns=1):
         """cells per tile along z (0 = from the density), tile width in cell columns and
-        workgroup size of the tiled list build and force kernel; applies from the next build"""
+        workgroup size of the tiled list build and force kernel; applies from the next build
+        ((0, 256, 2) is what a list has without this call)"""
         self.ctx.check(_L.mrmd_verlet_set_tiling(self.h, int(tile_cells), int(tile_columns), int(block)))
 
     def set_stage_limit(self, limit=0):

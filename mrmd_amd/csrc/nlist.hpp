@@ -444,8 +444,9 @@ struct mrmd_verlet_list
     mrmd_hip::DBuf<double4> gstage;
 
     // ---- tiled form (built on the device; what the force kernels read) ----
+    static constexpr int DEFAULT_COLS = 2;
     int tileK = 0;              ///< cells per tile along z (0 = choose from the density)
-    int tileCols = 2;           ///< a: tiles span a x a cell columns
+    int tileCols = DEFAULT_COLS;  ///< a: tiles span a x a cell columns
     bool tilingGiven = false;   ///< set_tiling chose the shape
     int64_t tiledRows = -1;     ///< rows for which the shape was chosen
     /// rows that can have entries: all, or in a banded list about the band's share of them

@@ -728,7 +728,7 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
         const int lg = rowSplit(vl->splitRows);
         // (in sparse cells even the tallest tile of one column has fewer rows than that: two columns)
         const double cells = double(vl->block >> lg) / perCell;
-        vl->tileCols = lg >= 2 && cells <= double(std::min(g.n[2], MAX_SPAN - 2 * R)) ? 1 : 2;
+        vl->tileCols = lg >= 2 && cells <= double(std::min(g.n[2], MAX_SPAN - 2 * R)) ? 1 : mrmd_verlet_list::DEFAULT_COLS;
         vl->tileK = 0;
         if (lg > 0)
         {
@@ -798,8 +798,7 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
             const int bufCap = wideBuf ? vl->capFull : ROW_BUF;
             // four waves a workgroup fill the chip from 1,280 tiles on (five waves a SIMD); with
             // fewer tiles their rows go to up to twelve waves
-            int waves = vl->block / WAVE;
-            if (!vl->tilingGiven) waves = int(std::max<int64_t>(waves, std::min<int64_t>(12, 5120 / vl->ntiles)));
+            int waves = int(std::max<int64_t>(vl->block / WAVE, std::min<int64_t>(12, 5120 / vl->ntiles)));
             while (waves > 1 && fixed + waves * perWave(bufCap) > LDS_LIMIT) --waves;
             const size_t lds = fixed + waves * perWave(bufCap);
             auto launch = [&](auto kernel) {
@@ -937,7 +936,8 @@ int mrmd_verlet_set_tiling(mrmd_verlet_list* vl, int tile_cells, int tile_column
     MRMD_API_BEGIN(vl ? vl->ctx : nullptr)
     REQUIRE(vl && tile_cells >= 0 && tile_columns >= 1 && tile_columns <= 3, "invalid tiling");
     REQUIRE(block == 64 || block == 128 || block == 192 || block == 256, "workgroup size must be 64, 128, 192 or 256");
-    vl->tilingGiven = true;
+    vl->tilingGiven = tile_cells > 0 || tile_columns != mrmd_verlet_list::DEFAULT_COLS;
+    vl->tiledRows = -1;
     vl->tileK = tile_cells;
     vl->tileCols = tile_columns;
     vl->block = block;

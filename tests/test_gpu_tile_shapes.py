@@ -1,0 +1,45 @@
+"""The tile shape that a list build chooses: what a fresh list would choose, whatever the list object
+has built before or was asked for, and the lists themselves are the same."""
+import numpy as np
+import pytest
+
+from test_gpu_split_rows import _jittered
+
+pytestmark = pytest.mark.gpu
+
+RN = 2.8
+
+
+@pytest.fixture(scope="module")
+def M():
+    import mrmd_amd
+    return mrmd_amd
+
+
+@pytest.fixture(scope="module")
+def ctx(M):
+    c = M.Context(0)
+    yield c
+    c.close()
+
+
+def _build(M, ctx, pos, L, vl=None, ratio=1.0):
+    a = M.Atoms.from_arrays(ctx, pos)
+    vl = vl or M.HalfVerletList(ctx)
+    vl.build(a, 0, pos.shape[0], RN, ratio, [0.0] * 3, [L] * 3)
+    return vl, vl.tiling()
+
+
+@pytest.mark.parametrize("n", [4000, 70000])
+def test_default_shape_can_be_asked_for(M, ctx, n):
+    """4,000 atoms: one column by one cell; 70,000: two by two columns of three cells"""
+    pos, L = _jittered(n, 0.8442, 3)
+    fresh, shape = _build(M, ctx, pos, L)
+    vl = M.HalfVerletList(ctx)
+    for cells, columns in ((2, 3), (0, 1), (0, 2)):
+        vl.set_tiling(cells, 256, columns)
+        _, other = _build(M, ctx, pos, L, vl)
+        if columns != 2:
+            assert other["tile_columns"] == columns
+    assert other == shape
+    np.testing.assert_array_equal(vl.half_counts(n)[0], fresh.half_counts(n)[0])
