@@ -445,10 +445,19 @@ struct mrmd_verlet_list
 
     // ---- tiled form (built on the device; what the force kernels read) ----
     static constexpr int DEFAULT_COLS = 2;
-    int tileK = 0;              ///< cells per tile along z (0 = choose from the density)
+    int givenCells = 0, givenCols = 0;  ///< the shape that set_tiling asked for (0 = choose)
+    int tileK = 0;              ///< cells per tile along z
     int tileCols = DEFAULT_COLS;  ///< a: tiles span a x a cell columns
-    bool tilingGiven = false;   ///< set_tiling chose the shape
-    int64_t tiledRows = -1;     ///< rows for which the shape was chosen
+    /// what the last build's shape was chosen for, before it shrank
+    struct TileChoice
+    {
+        int cols = 0, cells = 0, range = 0, n0 = 0, n1 = 0, n2 = 0, limit = 0;
+        bool operator==(const TileChoice& o) const
+        {
+            return cols == o.cols && cells == o.cells && range == o.range && n0 == o.n0 && n1 == o.n1 && n2 == o.n2 &&
+                   limit == o.limit;
+        }
+    } tileChoice;
     /// rows that can have entries: all, or in a banded list about the band's share of them
     int64_t splitRows = 0;
     int block = 256;            ///< workgroup size of the tiled kernels

@@ -712,9 +712,6 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
     const double regionCells =
         double(std::max(vl->rowExtent[0], 1)) * std::max(vl->rowExtent[1], 1) * std::max(vl->rowExtent[2], 1);
     const double perCell = std::max(double(std::max<int64_t>(rows, 1)) / regionCells, 1e-3);
-    // a shape nobody asked for follows the rows: where they are too few to fill the chip, tiles of
-    // as many rows as a workgroup of the force kernel holds with its lanes per row, one cell
-    // column wide from four lanes on, so that there are more of them
     vl->splitRows = rows;
     if (vl->banded)
     {
@@ -723,29 +720,38 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
         const double part = std::min(gmax[0], vl->bandHi + rn) - std::max(gmin[0], vl->bandLo - rn);
         vl->splitRows = int64_t(double(rows) * std::min(1.0, std::max(0.0, part / width)));
     }
-    if (!vl->tilingGiven && vl->tiledRows != vl->splitRows)
-    {
-        const int lg = rowSplit(vl->splitRows);
-        // (in sparse cells even the tallest tile of one column has fewer rows than that: two columns)
-        const double cells = double(vl->block >> lg) / perCell;
-        vl->tileCols = lg >= 2 && cells <= double(std::min(g.n[2], MAX_SPAN - 2 * R)) ? 1 : mrmd_verlet_list::DEFAULT_COLS;
-        vl->tileK = 0;
-        if (lg > 0)
-        {
-            const int a = R == 1 ? vl->tileCols : 1;
-            vl->tileK = std::max(1, int(std::min(cells / (a * a), double(MAX_SPAN))));
-        }
-        vl->tiledRows = vl->splitRows;
-    }
-    int a = std::max(1, std::min(vl->tileCols, R == 1 ? 3 : 1));
-    const int W = a + 2 * R;
-    int K = vl->tileK > 0 ? std::min(vl->tileK, g.n[2]) : 0;
+    // A shape nobody asked for follows the rows: where they are too few to fill the chip, tiles of
+    // as many rows as a workgroup of the force kernel holds with its lanes per row, one cell
+    // column wide from four lanes on, so that there are more of them.  It is chosen at every build:
+    // a list object may meet another system.
+    const int lg = rowSplit(vl->splitRows);
+    // (in sparse cells even the tallest tile of one column has fewer rows than that: two columns)
+    const double cells = double(vl->block >> lg) / perCell;
+    const bool narrow = lg >= 2 && cells <= double(std::min(g.n[2], MAX_SPAN - 2 * R));
+    const int wantCols = vl->givenCols > 0 ? vl->givenCols : narrow ? 1 : mrmd_verlet_list::DEFAULT_COLS;
+    int a = std::min(wantCols, R == 1 ? 3 : 1);
+    int K = vl->givenCells;
+    if (K <= 0 && vl->givenCols <= 0 && lg > 0) K = std::max(1, int(std::min(cells / (a * a), double(MAX_SPAN))));
     if (K <= 0)
     {
-        K = int(1650.0 / (W * W * perCell)) - 2 * R;
-        K = std::max(1, std::min(K, g.n[2]));
+        const int W = a + 2 * R;
+        K = std::max(1, int(1650.0 / (W * W * perCell) - 2 * R));
     }
-    K = std::min(K, MAX_SPAN - 2 * R);
+    K = std::min({K, g.n[2], MAX_SPAN - 2 * R});
+    // A shape that had to shrink is where the next build of the same system starts (a shape that does
+    // not fit costs a launch and a wait), unless the chosen shape would now fit at the density of
+    // its fullest neighbourhood, which larger neighbourhoods do not exceed
+    const mrmd_verlet_list::TileChoice choice{a, K, R, g.n[0], g.n[1], g.n[2], vl->stageLimit};
+    auto cellsAround = [&](int cols, int height) {
+        return double(std::min(cols + 2 * R, g.n[0])) * std::min(cols + 2 * R, g.n[1]) * std::min(height + 2 * R, g.n[2]);
+    };
+    if (choice == vl->tileChoice && vl->tileK > 0 &&
+        vl->maxStaged * cellsAround(a, K) > vl->stageLimit * cellsAround(vl->tileCols, vl->tileK))
+    {
+        a = vl->tileCols;
+        K = vl->tileK;
+    }
+    vl->tileChoice = choice;
     vl->globalStage = false;
     for (bool again = false;; again = true)
     {
@@ -936,10 +942,11 @@ int mrmd_verlet_set_tiling(mrmd_verlet_list* vl, int tile_cells, int tile_column
     MRMD_API_BEGIN(vl ? vl->ctx : nullptr)
     REQUIRE(vl && tile_cells >= 0 && tile_columns >= 1 && tile_columns <= 3, "invalid tiling");
     REQUIRE(block == 64 || block == 128 || block == 192 || block == 256, "workgroup size must be 64, 128, 192 or 256");
-    vl->tilingGiven = tile_cells > 0 || tile_columns != mrmd_verlet_list::DEFAULT_COLS;
-    vl->tiledRows = -1;
+    vl->givenCells = tile_cells;
+    vl->givenCols = tile_cells > 0 || tile_columns != mrmd_verlet_list::DEFAULT_COLS ? tile_columns : 0;
     vl->tileK = tile_cells;
     vl->tileCols = tile_columns;
+    vl->tileChoice = {};
     vl->block = block;
     MRMD_API_END
 }

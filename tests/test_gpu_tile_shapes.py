@@ -43,3 +43,25 @@ def test_default_shape_can_be_asked_for(M, ctx, n):
             assert other["tile_columns"] == columns
     assert other == shape
     np.testing.assert_array_equal(vl.half_counts(n)[0], fresh.half_counts(n)[0])
+
+
+def test_shape_follows_the_system(M, ctx):
+    """a list object that has built another density, a wider stencil and a crowd whose tiles had to
+    shrink; the shape after the crowd is back with the second ordinary build at the latest"""
+    n = 70000
+    pos, L = _jittered(n, 0.8442, 4)
+    _, shape = _build(M, ctx, pos, L)
+    vl = M.HalfVerletList(ctx)
+    thin, thin_L = _jittered(n, 0.1, 5)
+    for p, edge, ratio in ((thin, thin_L, 1.0), (pos, L, 0.5)):
+        _, other = _build(M, ctx, p, edge, vl, ratio)
+        assert other != shape
+        assert _build(M, ctx, pos, L, vl)[1] == shape
+    g = np.random.default_rng(6)
+    crowd = pos.copy()
+    crowd[g.permutation(n)[:1500]] = 0.5 * L + g.uniform(-0.7, 0.7, (1500, 3))
+    _, other = _build(M, ctx, crowd, L, vl)
+    assert (other["tile_columns"], other["tile_cells"]) < (shape["tile_columns"], shape["tile_cells"])
+    assert _build(M, ctx, crowd, L, vl)[1] == other
+    _build(M, ctx, pos, L, vl)
+    assert _build(M, ctx, pos, L, vl)[1] == shape
