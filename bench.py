@@ -368,14 +368,11 @@ def main():
     n = pos.shape[0]
     dt = 0.005
     s.run(args.warmup, dt)
-    tiling = None
     if not args.no_tune:
         from mrmd_amd.autotune import tune_lj_system
-        best, _ = tune_lj_system(s)
-        tiling = {"tile_columns": best[0], "tile_cells": best[1], "block": best[2]}
+        tune_lj_system(s)
         s.run(3, dt)
-    else:
-        tiling = {k: v for k, v in s.vl.tiling().items() if k != "max_staged"}
+    tiling = {k: v for k, v in s.vl.tiling().items() if k != "max_staged"}
     ctx.synchronize()
     # the timed steps carry HIP events around the force kernel only (the roofline's
     # measurement, on the library stream); the other kernels are timed in a separate pass

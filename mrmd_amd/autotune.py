@@ -10,7 +10,8 @@ time plus the build time spread over the expected steps between rebuilds.
 """
 import itertools
 
-DEFAULT_SHAPES = ((1, 6), (2, 2), (2, 3), (2, 4), (3, 1), (3, 2))  # (columns, cells)
+# (columns, cells); (2, 0) is the shape that the list chooses by itself
+DEFAULT_SHAPES = ((2, 0), (1, 6), (2, 2), (2, 3), (2, 4), (3, 1), (3, 2))
 DEFAULT_BLOCKS = (192, 256)
 
 
@@ -52,7 +53,8 @@ def tune_lj_system(system, shapes=DEFAULT_SHAPES, blocks=DEFAULT_BLOCKS, force_r
     return best, table
 
 
-ENSEMBLE_TARGETS = (1000, 1400, 1800)  # staged records per workgroup a replica's tile height aims at
+# staged records per workgroup a replica's tile height aims at (1300: an ensemble's own choice)
+ENSEMBLE_TARGETS = (1000, 1300, 1800)
 ENSEMBLE_BLOCKS = (128, 256)
 
 

@@ -65,3 +65,26 @@ def test_shape_follows_the_system(M, ctx):
     assert _build(M, ctx, crowd, L, vl)[1] == other
     _build(M, ctx, pos, L, vl)
     assert _build(M, ctx, pos, L, vl)[1] == shape
+
+
+def test_tuners_try_the_default_shapes(M, ctx):
+    """a system's or an ensemble's own choice is among the candidates, so tuning cannot lose it"""
+    from mrmd_amd.autotune import ENSEMBLE_BLOCKS, ENSEMBLE_TARGETS, tune_lj_system
+    from mrmd_amd.drivers import LJSystem
+    from mrmd_amd.ensemble import Ensemble, cubic_box, replica
+    pos, L = _jittered(4000, 0.8442, 7)
+    s = LJSystem(ctx, pos, np.zeros_like(pos), L)
+    s.rebuild()
+    own, tried = s.vl.tiling(), []
+    rebuild = s.rebuild
+
+    def recorded():
+        rebuild()
+        tried.append(s.vl.tiling())
+
+    s.rebuild = recorded
+    tune_lj_system(s, force_reps=1)
+    assert own in tried
+    e = Ensemble(ctx, [replica(600, cubic_box(600, 0.8), 1.0, 1)])
+    own = e.tiling()
+    assert own["target_staged"] in ENSEMBLE_TARGETS and own["block"] in ENSEMBLE_BLOCKS
