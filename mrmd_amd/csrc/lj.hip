@@ -160,9 +160,11 @@ __device__ inline void ljQuadTypes(const LJArgs& a, const Pre* tab, int ti0, con
 // Bound by vector instruction issue (some 80 % of the time at 4 million atoms, of which staging is
 // a tenth): ~27 cycles per list entry, the reciprocal being a quarter-rate instruction.  With
 // records read by two-address LDS reads, run starts looked up per staged record and shuffles in
-// the reductions 441 us at 4 million atoms, in this form 395 to 415.
+// the reductions 441 us at 4 million atoms, in this form 395 to 415.  (Two-type tables without
+// capping, at 260,000 atoms: 80 us with the fours of a chunk in a loop and 124 registers, 69 in a row
+// with 170 at hand; their 32-byte records leave LDS for three waves a SIMD.)
 template <bool PRED, bool ONE, bool CAP, bool ASSIGN, bool GS, bool SPLIT>
-__global__ __launch_bounds__(BLOCK, PRED || (CAP && !ONE) ? 2 : 4) void k_ljTiled(LJArgs a, TiledList tl, Pre p1, double* partials)
+__global__ __launch_bounds__(BLOCK, PRED || (CAP && !ONE) ? 2 : ONE ? 4 : 3) void k_ljTiled(LJArgs a, TiledList tl, Pre p1, double* partials)
 {
     extern __shared__ double4 stLds[];
     __shared__ Pre tab[ONE ? 1 : MAX_TYPES2];
@@ -222,7 +224,7 @@ __global__ __launch_bounds__(BLOCK, PRED || (CAP && !ONE) ? 2 : 4) void k_ljTile
                 sum.joinRow(lg);
             }
             else
-                walkRow<ONE && !CAP && !PRED, GS>(st, chunk, tl.strideS, c, cur,
+                walkRow<!CAP && !PRED, GS>(st, chunk, tl.strideS, c, cur,
                                                   [&](const Quad& q) { pairs(q, pi, ti0); });
             // (the row's first lane stores)
             if (!SPLIT || (t & ((1 << lg) - 1)) == 0)
