@@ -963,7 +963,7 @@ __device__ double bForceRows(const BS& b, const TileB& ti, const RepD& R, const 
             if constexpr (W)
             {
                 WeightedSums ws{0.0, 0.0, 0.0, 0.0, 0.0};
-                walkRowSplit<GS>(st, chunk, b.strideS, c, t & mask, lg,
+                walkRowSplit<false, GS>(st, chunk, b.strideS, c, t & mask, lg,
                                  [&](const Quad& q) { ljQuadWeighted<CAP>(b.lj, b.rcSqr, pi, q, ws); });
                 for (int off = 1; off <= mask; off <<= 1)
                 {
@@ -998,7 +998,7 @@ __device__ double bForceRows(const BS& b, const TileB& ti, const RepD& R, const 
             else
             {
                 sum.startRow();
-                walkRowSplit<GS>(st, chunk, b.strideS, c, t & mask, lg, [&](const Quad& q) {
+                walkRowSplit<false, GS>(st, chunk, b.strideS, c, t & mask, lg, [&](const Quad& q) {
                     // (padding entries are the row itself, at distance 0)
                     ljQuadOne<CAP>(b.lj, b.rcSqr, pi, q, sum, [](int, double d2) { return d2 > 0.0; });
                 });

@@ -147,8 +147,9 @@ __device__ inline void ljQuadTypes(const LJArgs& a, const Pre* tab, int ti0, con
         s.fx += dx[u] * ff;
         s.fy += dy[u] * ff;
         s.fz += dz[u] * ff;
-        s.e += en * m;
-        s.w += ff * d2[u];
+        // (spelt out, as in ljQuadOne)
+        s.e = __builtin_fma(en, m, s.e);
+        s.w = __builtin_fma(ff, d2[u], s.w);
     }
 }
 
@@ -161,17 +162,18 @@ __device__ inline void ljQuadTypes(const LJArgs& a, const Pre* tab, int ti0, con
 // a tenth): ~27 cycles per list entry, the reciprocal being a quarter-rate instruction.  With
 // records read by two-address LDS reads, run starts looked up per staged record and shuffles in
 // the reductions 441 us at 4 million atoms, in this form 395 to 415.  (Two-type tables without
-// capping, at 260,000 atoms: 80 us with the fours of a chunk in a loop and 124 registers, 69 in a row
-// with 170 at hand; their 32-byte records leave LDS for three waves a SIMD.)
+// capping, at 260,000 atoms: 80 us with the fours of a chunk in a loop and 124 registers, 70 in a row
+// and 86; their 32-byte records leave LDS for three waves a SIMD.)
 template <bool PRED, bool ONE, bool CAP, bool ASSIGN, bool GS, bool SPLIT>
-__global__ __launch_bounds__(BLOCK, PRED || (CAP && !ONE) ? 2 : ONE ? 4 : 3) void k_ljTiled(LJArgs a, TiledList tl, Pre p1, double* partials)
+__global__ __launch_bounds__(BLOCK, PRED || GS || (CAP && !ONE) ? 2 : ONE ? 4 : 3) void k_ljTiled(LJArgs a, TiledList tl, Pre p1, double* partials)
 {
     extern __shared__ double4 stLds[];
     __shared__ Pre tab[ONE ? 1 : MAX_TYPES2];
     __shared__ TileInfo ti;
     __shared__ double red[BLOCK / WAVE];
     const unsigned blk = xcdBlock();
-    const Stage<ONE> st(GS ? tl.gstage + int64_t(blk) * tl.gstageRecs : stLds, sentinelSlot(tl.maxStaged) + 1);
+    const std::conditional_t<GS && !SPLIT, GlobalStage<ONE>, Stage<ONE>> st(
+        GS ? tl.gstage + int64_t(blk) * tl.gstageRecs : stLds, sentinelSlot(tl.maxStaged) + 1);
     if (!ONE)
         for (int t = threadIdx.x; t < a.nt2; t += blockDim.x) tab[t] = a.table[t];
     loadTile(ti, tl.tiles, blk);
@@ -219,7 +221,7 @@ __global__ __launch_bounds__(BLOCK, PRED || (CAP && !ONE) ? 2 : ONE ? 4 : 3) voi
             sum.startRow();
             if constexpr (SPLIT)
             {
-                walkRowSplit<GS>(st, chunk, tl.strideS, c, t & ((1 << lg) - 1), lg,
+                walkRowSplit<GS, GS>(st, chunk, tl.strideS, c, t & ((1 << lg) - 1), lg,
                                  [&](const Quad& q) { pairs(q, pi, ti0); });
                 sum.joinRow(lg);
             }

@@ -39,9 +39,10 @@ __device__ inline Quad loadQuad(const St& st, uint32_t lo, uint32_t hi)
 
 // The entries of one row (c of them, chunks of eight at `chunk`, the first already in `cur`),
 // four at a time in order; an index chunk is requested a chunk ahead.  BOTH: the two fours of a
-// chunk are laid out in a row (for bodies that leave registers for it), not in a loop.  (Two
-// fours in flight from LDS, the next loaded while one is computed, measured no faster: 419
-// against 415 us at 4M atoms.)
+// chunk are laid out in a row (for bodies that leave registers for it), not in a loop.  From global
+// memory (GS) both fours and then the next index chunk are loaded before either is computed: few
+// tiles are in flight there, and a four's loads are a wait for memory.  (Two fours in flight from
+// LDS, the next loaded while one is computed, measured no faster: 419 against 415 us at 4M atoms.)
 template <bool BOTH, bool GS, class St, class Body>
 __device__ inline void walkRow(const St& st, const uint4* __restrict__ chunk, int64_t stride, int c, uint4 cur,
                                Body body)
@@ -54,6 +55,14 @@ __device__ inline void walkRow(const St& st, const uint4* __restrict__ chunk, in
     {
         const uint4 now = cur;
         cur = nxt;
+        if constexpr (GS)
+        {
+            const Quad a = loadQuad<GS>(st, now.x, now.y), b = loadQuad<GS>(st, now.z, now.w);
+            if (ch + 2 < nch) nxt = chunk[int64_t(ch + 2) * stride];
+            body(a);
+            body(b);
+            continue;
+        }
         if (ch + 2 < nch) nxt = chunk[int64_t(ch + 2) * stride];
         if constexpr (BOTH)
         {
@@ -68,8 +77,9 @@ __device__ inline void walkRow(const St& st, const uint4* __restrict__ chunk, in
     }
 }
 
-// The same for one of the 2^lg lanes that share the row: fours sub, sub + 2^lg, ...
-template <bool GS, class St, class Body>
+// The same for one of the 2^lg lanes that share the row: fours sub, sub + 2^lg, ...  PAIR: two of them
+// loaded before either is computed
+template <bool PAIR, bool GS, class St, class Body>
 __device__ inline void walkRowSplit(const St& st, const uint4* __restrict__ chunk, int64_t stride, int c,
                                     int sub, int lg, Body body)
 {
@@ -77,6 +87,23 @@ __device__ inline void walkRowSplit(const St& st, const uint4* __restrict__ chun
     auto four = [&](int q) { return reinterpret_cast<const uint2*>(chunk + int64_t(q >> 1) * stride)[q & 1]; };
     uint2 nxt = {0, 0};
     if (sub < nq) nxt = four(sub);
+    if constexpr (PAIR)
+    {
+        // (a lane without a second four loads some record for it; every four is computed inside the
+        // loop, so that the lane with the most of them takes part wherever another does: PairSums
+        // counts on it)
+        uint2 nxt2 = {0, 0};
+        if (sub + step < nq) nxt2 = four(sub + step);
+        for (int q = sub; q < nq; q += 2 * step)
+        {
+            const Quad a = loadQuad<GS>(st, nxt.x, nxt.y), b = loadQuad<GS>(st, nxt2.x, nxt2.y);
+            if (q + 2 * step < nq) nxt = four(q + 2 * step);
+            if (q + 3 * step < nq) nxt2 = four(q + 3 * step);
+            body(a);
+            if (q + step < nq) body(b);
+        }
+        return;
+    }
     for (int q = sub; q < nq; q += step)
     {
         const uint2 now = nxt;
@@ -206,14 +233,16 @@ __device__ inline void ljQuadOne(const Pre& p, double rcSqr, const double4& pi, 
     for (int u = 0; u < 4; ++u)
     {
         const double f2 = maskReciprocal(frac2[u], in[u]);
-        const double f6 = f2 * f2 * f2;
-        const double g = f6 * (p.ff1 * f6 - p.ff2);
+        const double f4 = f2 * f2, f6 = f4 * f2;
+        const double t = p.ff1 * f6 - p.ff2, g = f6 * t;
         const double ff = g * f2;
         s.fx += dx[u] * ff;
         s.fy += dy[u] * ff;
         s.fz += dz[u] * ff;
-        s.e += f6;
-        s.w += g;
+        // (spelt out: contracted or not according to the block that the compiler leaves them in,
+        // the kernels of one table would differ in the last bit of their energies)
+        s.e = __builtin_fma(f4, f2, s.e);
+        s.w = __builtin_fma(f6, t, s.w);
     }
 }
 }  // namespace mrmd_hip

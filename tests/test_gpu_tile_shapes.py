@@ -88,3 +88,29 @@ def test_tuners_try_the_default_shapes(M, ctx):
     e = Ensemble(ctx, [replica(600, cubic_box(600, 0.8), 1.0, 1)])
     own = e.tiling()
     assert own["target_staged"] in ENSEMBLE_TARGETS and own["block"] in ENSEMBLE_BLOCKS
+
+
+@pytest.mark.parametrize("n", [5000, 66000])
+@pytest.mark.parametrize("num_types", [1, 2])
+@pytest.mark.parametrize("cap", [0.0, 0.9])
+def test_global_staging_gives_the_same_bits(M, ctx, n, num_types, cap):
+    """rows of eight lanes and of one, every table, from a tile's slice of memory and from LDS"""
+    pos, L = _jittered(n, 0.8442, n)
+    pos[1] = pos[0] + [1e-3, 0.0, 0.0] if cap else pos[1]  # one pair far inside the capping distance
+    types = (np.arange(n) % num_types).astype(np.int64)
+    k = num_types * num_types
+    lj = M.LennardJones(ctx, [2.5] * k, [1.0, 0.93, 0.93, 0.86][:k], [1.0, 0.75, 0.75, 0.5][:k],
+                        capping_distance=[cap] * k, num_types=num_types, shifted=True, type_stride=num_types)
+    out = []
+    for limit in (0, 64):
+        a = M.Atoms.from_arrays(ctx, pos, type=types)
+        vl = M.HalfVerletList(ctx)
+        vl.set_tiling(1, 256, 1)
+        vl.set_stage_limit(limit)
+        vl.build(a, 0, n, RN, 1.0, [0.0] * 3, [L] * 3)
+        assert limit == 0 or vl.tiling()["max_staged"] > limit
+        a.set_force(0.0)
+        lj.apply(a, vl)
+        out.append((a.download(M.FORCE, n), lj.energy_virial()))
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    assert out[0][1] == out[1][1]
