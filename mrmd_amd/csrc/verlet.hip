@@ -141,11 +141,15 @@ constexpr size_t LDS_LIMIT = 64000;  // dynamic LDS of a list build workgroup (6
 // neighbours made it 114, 121, 191 or 323 us, and wider rows did not fit at all; now 110 for any
 // hint, and rows of 240 take 303 instead of 385.
 constexpr int ROW_BUF = 96;
+// Where the widest row met so far is a little wider the buffers hold it: rows of up to 109 and 129
+// entries, 129 and 154 us, with 96 entries 139 and 174; rows of up to 200 take 288 us with 96 and 313
+// with 128 or 144.
+constexpr int ROW_BUF_MOST = 144;
 // Up to here every workgroup has its LDS to itself (two a CU), and buffers of the list's width are
 // taken if four waves have room for them (4,000 atoms, rows of 140 and 240: 31 and 47 us, with 96
 // entries 37 and 62)
 constexpr int64_t WIDE_BUF_TILES = 2 * 256;
-static_assert(ROW_BUF % CHUNK == 0);
+static_assert(ROW_BUF % CHUNK == 0 && ROW_BUF_MOST % CHUNK == 0);
 
 // The list build.  S = 2R + 1 lanes share a row, one per j offset of the stencil, and walk the
 // S i offsets together, so a row's columns come in Cabana's i, j, k order: in each step a lane
@@ -792,8 +796,7 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
         {
             KTimer tk(ctx, "verlet_tiled");
             // LDS: the row buffers, the 16-bit records and the per-cell start table of (a + 2R)^2 ranges
-            // x (K + 2R + 1); at most 23,000 bytes without the row buffers, so eight waves of the narrow
-            // ones fit
+            // x (K + 2R + 1); at most 23,000 bytes without the row buffers, so that six waves fit
             const int W = vl->tileCols + 2 * R, rowsPerWave = WAVE / (2 * R + 1);
             const size_t fixed = (vl->globalStage ? 0 : size_t(stagedCap + STAGE_PAD) * sizeof(uint2)) +
                                  size_t(W * W * (vl->tileK + 2 * R + 1)) * sizeof(int);
@@ -801,7 +804,8 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
                 return vl->globalStage ? 0 : size_t(rowsPerWave) * entries * sizeof(uint16_t);
             };
             const bool wideBuf = vl->ntiles <= WIDE_BUF_TILES && fixed + 4 * perWave(vl->capFull) <= LDS_LIMIT;
-            const int bufCap = wideBuf ? vl->capFull : ROW_BUF;
+            const int widest = (vl->maxFull + CHUNK - 1) / CHUNK * CHUNK;  // (of the last build)
+            const int bufCap = wideBuf ? vl->capFull : widest > ROW_BUF && widest <= ROW_BUF_MOST ? widest : ROW_BUF;
             // four waves a workgroup fill the chip from 1,280 tiles on (five waves a SIMD); with
             // fewer tiles their rows go to up to twelve waves
             int waves = int(std::max<int64_t>(vl->block / WAVE, std::min<int64_t>(12, 5120 / vl->ntiles)));

@@ -50,10 +50,18 @@ def test_width_hints(M, ctx, ratio):
 @pytest.mark.parametrize("ratio", [1.0, 0.5])
 @pytest.mark.parametrize("density", [1.05, 1.6])
 def test_rows_about_and_beyond_the_row_buffers(M, ctx, density, ratio):
-    """rows of 40 to 110 and of 60 to 170 entries"""
-    pos, L = _jittered(3000, density, 12)
-    _, _, vl, ov = _lists(M, ctx, pos, RN, ratio, L)
-    _same_lists(vl, ov, 3000, True)
+    """rows of 40 to 110 and of 60 to 170 entries, in more tiles than take buffers of the list's width;
+    the second build knows the widest row"""
+    n = 30000
+    pos, L = _jittered(n, density, 12)
+    g, _, vl, ov = _lists(M, ctx, pos, RN, ratio, L)
+    _same_lists(vl, ov, n, False)
+    ref = ov.neighbors()
+    sets = [set(ref[i, :c].tolist()) for i, c in enumerate(ov.counts()[:2000])]
+    for _ in range(2):
+        rows = vl.half_rows(n)
+        assert all(rows[i] == s for i, s in enumerate(sets))
+        vl.build(g, 0, n, RN, ratio, [0.0] * 3, [L] * 3)
 
 
 @pytest.mark.parametrize("ratio", [1.0, 0.5])
