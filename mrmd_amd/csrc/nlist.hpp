@@ -473,14 +473,18 @@ struct mrmd_verlet_list
     int givenCells = 0, givenCols = 0;  ///< the shape that set_tiling asked for (0 = choose)
     int tileK = 0;              ///< cells per tile along z
     int tileCols = DEFAULT_COLS;  ///< a: tiles span a x a cell columns
-    /// what the last build's shape was chosen for, before it shrank
+    /// what the shape was chosen for, and the shape before it shrank
     struct TileChoice
     {
-        int cols = 0, cells = 0, range = 0, n0 = 0, n1 = 0, n2 = 0, limit = 0;
-        bool operator==(const TileChoice& o) const
+        int64_t rows = -1, splitRows = -1;
+        int n[3] = {0, 0, 0}, range = 0, limit = 0;
+        double regionCells = 0.0;
+        int cols = 0, cells = 0;
+        bool sameSystem(const TileChoice& o) const
         {
-            return cols == o.cols && cells == o.cells && range == o.range && n0 == o.n0 && n1 == o.n1 && n2 == o.n2 &&
-                   limit == o.limit;
+            return rows == o.rows && splitRows == o.splitRows && n[0] == o.n[0] && n[1] == o.n[1] && n[2] == o.n[2] &&
+                   range == o.range && limit == o.limit && regionCells <= 4.0 * o.regionCells &&
+                   o.regionCells <= 4.0 * regionCells;
         }
     } tileChoice;
     /// rows that can have entries: all, or in a banded list about the band's share of them

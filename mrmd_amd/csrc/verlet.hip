@@ -726,8 +726,7 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
     }
     // A shape nobody asked for follows the rows: where they are too few to fill the chip, tiles of
     // as many rows as a workgroup of the force kernel holds with its lanes per row, one cell
-    // column wide from four lanes on, so that there are more of them.  It is chosen at every build:
-    // a list object may meet another system.
+    // column wide from four lanes on, so that there are more of them.
     const int lg = rowSplit(vl->splitRows);
     // (in sparse cells even the tallest tile of one column has fewer rows than that: two columns)
     const double cells = double(vl->block >> lg) / perCell;
@@ -742,14 +741,23 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
         K = std::max(1, int(1650.0 / (W * W * perCell) - 2 * R));
     }
     K = std::min({K, g.n[2], MAX_SPAN - 2 * R});
-    // A shape that had to shrink is where the next build of the same system starts (a shape that does
-    // not fit costs a launch and a wait), unless the chosen shape would now fit at the density of
-    // its fullest neighbourhood, which larger neighbourhoods do not exceed
-    const mrmd_verlet_list::TileChoice choice{a, K, R, g.n[0], g.n[1], g.n[2], vl->stageLimit};
+    // The shape is kept for as long as the system is the same: its rows, its grid, and the cells that
+    // hold rows within a factor of four (atoms that just reach into further cells do not make it
+    // another one).  A shape that had to shrink is where its next build starts (a shape that does not
+    // fit costs a launch and a wait), unless the chosen one would now fit at the density of its
+    // fullest neighbourhood, which larger neighbourhoods do not exceed.
+    mrmd_verlet_list::TileChoice choice{rows, vl->splitRows, {g.n[0], g.n[1], g.n[2]}, R, vl->stageLimit, regionCells, a, K};
+    const bool sameSystem = choice.sameSystem(vl->tileChoice);
+    if (sameSystem)
+    {
+        choice = vl->tileChoice;
+        a = choice.cols;
+        K = choice.cells;
+    }
     auto cellsAround = [&](int cols, int height) {
         return double(std::min(cols + 2 * R, g.n[0])) * std::min(cols + 2 * R, g.n[1]) * std::min(height + 2 * R, g.n[2]);
     };
-    if (choice == vl->tileChoice && vl->tileK > 0 &&
+    if (sameSystem && vl->tileK > 0 &&
         vl->maxStaged * cellsAround(a, K) > vl->stageLimit * cellsAround(vl->tileCols, vl->tileK))
     {
         a = vl->tileCols;

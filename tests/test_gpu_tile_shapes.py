@@ -46,8 +46,8 @@ def test_default_shape_can_be_asked_for(M, ctx, n):
 
 
 def test_shape_follows_the_system(M, ctx):
-    """a list object that has built another density, a wider stencil and a crowd whose tiles had to
-    shrink; the shape after the crowd is back with the second ordinary build at the latest"""
+    """a list object that has built another density, a wider stencil, a corner of the grid and a crowd whose
+    tiles had to shrink; the shape after the crowd is back with the second ordinary build at the latest"""
     n = 70000
     pos, L = _jittered(n, 0.8442, 4)
     _, shape = _build(M, ctx, pos, L)
@@ -57,6 +57,10 @@ def test_shape_follows_the_system(M, ctx):
         _, other = _build(M, ctx, p, edge, vl, ratio)
         assert other != shape
         assert _build(M, ctx, pos, L, vl)[1] == shape
+    # as many atoms in a corner of the same grid
+    corner, _ = _jittered(n, 0.8442 * 27, 5)
+    assert _build(M, ctx, corner, L, vl)[1] != shape
+    assert _build(M, ctx, pos, L, vl)[1] == shape
     g = np.random.default_rng(6)
     crowd = pos.copy()
     crowd[g.permutation(n)[:1500]] = 0.5 * L + g.uniform(-0.7, 0.7, (1500, 3))
