@@ -403,10 +403,9 @@ __device__ inline double waveMax(double v)
 {
     return waveReduce(v, 0.0, [](double a, double b) { return fmax(a, b); });
 }
-// (of non-negative values)
 __device__ inline int waveMaxInt(int v)
 {
-    return waveReduce(v, 0, [](int a, int b) { return max(a, b); });
+    return waveReduce(v, INT32_MIN, [](int a, int b) { return max(a, b); });
 }
 // result valid in thread 0; lds holds blockDim.x / WAVE doubles (blockDim.x a multiple of WAVE, at most BLOCK)
 __device__ inline double blockSum(double v, double* lds)
