@@ -379,9 +379,11 @@ uint64_t* dispHost(mrmd_atoms* a, const double* maxDisp, uint32_t* tag)
 }
 }  // namespace
 
-// the fused post/pre step of time loops (k_postPre); synchronises for the displacement
+// the wait for the displacement of a fused step that did not wait for it
 void mrmd_hip::takeDisp(mrmd_atoms* a, uint32_t tag, double* maxDisp) { finishDisp(a, maxDisp, tag); }
 
+// the fused post/pre step of time loops (k_postPre); synchronises for the displacement, or gives its
+// tag for takeDisp
 int mrmd_hip::fusedPostPre(mrmd_atoms* a, double dt, bool langevin, double zeta, double temperature, uint64_t seed,
                            uint64_t call, double* maxDisp, double4* sortedPos, const int32_t* slotOf,
                            const mrmd_molecules* adrMol, const double* tfForce, const HistD* tfHd, bool slotsOnly,

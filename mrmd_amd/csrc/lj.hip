@@ -1,12 +1,12 @@
 // Lennard-Jones pair force (action::LennardJones), its precomputed table, and the adjoint.
 //
 // Force kernel design (gfx950, FP64): one lane per local atom over its full neighbour row
-// (both directions of every pair), so F_i is owned by one lane and no atomics are needed;
-// the pair work is done twice, which on a chip with 78.6 TFLOP/s FP64 costs less than the
-// L2 atomics of a half list.  One workgroup per Verlet-list tile stages the neighbourhood's
-// {x,y,z,type} records in LDS once; rows then read neighbours from LDS through 16-bit slot
-// entries.  Energy and virial are reduced with wave shuffles, per-workgroup partials and
-// one ordered final pass (deterministic).
+// (both directions of every pair), or up to eight lanes of a wave in systems too small to fill
+// the chip (rowSplit), so F_i is summed inside a wave and no atomics are needed; the pair work is
+// done twice, which on a chip with 78.6 TFLOP/s FP64 costs less than the L2 atomics of a half
+// list.  One workgroup per Verlet-list tile stages the neighbourhood's records in LDS once; rows
+// then read neighbours from LDS through 16-bit entries.  Energy and virial are summed over the
+// lanes by DPP moves, into per-workgroup partials and in one ordered final pass (deterministic).
 // The reference's half-list algorithm (atomic F_j, LennardJones.hpp:158-205) is kept for
 // asymmetric pair predicates and asymmetric parameter tables.
 #include <algorithm>
@@ -20,10 +20,6 @@
 #include "physics.hpp"
 
 using namespace mrmd_hip;
-
-namespace
-{
-}  // namespace
 
 struct mrmd_lj
 {
@@ -623,8 +619,8 @@ int mrmd_lj_eval(mrmd_lj* lj, const double* d2, const int64_t* idx, int64_t n, d
 namespace
 {
 // the body of mrmd_lj_apply; assign: store the rows' forces instead of adding them, honoured
-// only by the full-row kernel of a single-type table without capping and predicate
-// (returns whether it was)
+// by the full-row kernel without a predicate, which serves every symmetric table (returns whether
+// it was)
 bool ljApplyImpl(mrmd_lj* lj, mrmd_atoms* at, mrmd_verlet_list* vl, const mrmd_pred2* pred, bool assign);
 }  // namespace
 

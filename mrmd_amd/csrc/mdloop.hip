@@ -36,7 +36,7 @@ struct SlotPositions
     }
 };
 
-// the part of the last step's largest displacement that the next step's is expected to stay below
+// the next step's largest displacement is expected to stay below this many times the last one's
 constexpr double DISP_MARGIN = 1.25;
 }  // namespace
 

@@ -6,11 +6,12 @@
 // contiguous range of sorted slots per column, and every cell of its stencils lies in the
 // (a + 2R)^2 columns around it, each again a contiguous slot range.  One workgroup per tile
 // copies those ranges into LDS once and every row scans its stencil cells (Cabana's i, j, k
-// order and min-distance prune) from LDS.  An entry is the 15-bit LDS slot of the neighbour plus a flag bit for
-// the pairs Cabana's position-lexicographic half discriminator keeps, so the exact half
-// list is a sub-list and the force kernels stage the same tile and never gather from
-// global memory in their inner loop.  Global-index rows (for the API, the adjoint and the
-// half-list kernels) are converted from this form on demand.
+// order and min-distance prune) from LDS.  An entry's low 15 bits are the LDS slot of the
+// neighbour times eight (the slot itself where the tile stages in global memory, see entryShift),
+// the highest flags the pairs that Cabana's position-lexicographic half discriminator keeps, so
+// the exact half list is a sub-list and the force kernels stage the same tile and never gather
+// from global memory in their inner loop (dense tiles aside).  Global-index rows (for the API, the
+// adjoint and the half-list kernels) are converted from this form on demand.
 #include <algorithm>
 #include <climits>
 #include <cmath>
