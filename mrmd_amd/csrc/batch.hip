@@ -1929,6 +1929,27 @@ int mrmd_batch_state_load(mrmd_batch* b, const void* host, int64_t bytes)
     mrmd_ctx* c = b->ctx;
     const char* in = static_cast<const char*>(host);
     size_t off = sizeof hdr;
+    // the device writes by the given indices (k_bToGiven): each replica's have to be its own atoms, once
+    for (const StatePart& p : stateParts(b))
+    {
+        if (p.dev == b->id.p)
+        {
+            std::vector<int32_t> id(static_cast<size_t>(b->natoms));
+            std::memcpy(id.data(), in + off, p.bytes);
+            std::vector<bool> seen(static_cast<size_t>(b->natoms), false);
+            for (const RepD& R : b->reps)
+                for (int64_t i = R.a0; i < R.a0 + R.n; ++i)
+                {
+                    const int64_t k = id[size_t(i)];
+                    REQUIRE(k >= R.a0 && k < R.a0 + R.n && !seen[size_t(k)],
+                            "the state's atom indices are no order of the replicas' atoms (%lld at %lld)",
+                            (long long)k, (long long)i);
+                    seen[size_t(k)] = true;
+                }
+        }
+        off += p.bytes;
+    }
+    off = sizeof hdr;
     for (const StatePart& p : stateParts(b))
     {
         HIPCHECK(hipMemcpyAsync(p.dev, in + off, p.bytes, hipMemcpyHostToDevice, c->stream));

@@ -1,4 +1,4 @@
-"""Ensembles at the limits of their lists and sums."""
+"""Ensembles at the limits of their lists and sums, and saved states that are none."""
 import numpy as np
 import pytest
 
@@ -63,3 +63,30 @@ def test_energy_of_an_overflowing_pair_is_infinite(M, ctx, cap):
     e = _cold(M, ctx, pos, [6.0] * 3, 2.5, cap=cap)
     e.run(1, 0)
     assert e.energies()[0][0] == np.inf
+
+
+@pytest.mark.parametrize("bad", [-1, 300, 100, 1 << 30])
+def test_states_with_foreign_atom_indices_are_refused(M, ctx, bad):
+    """a negative index, one past the atoms, one of the other replica (or a second of its own) and one far
+    beyond; the refused load leaves the ensemble as it was"""
+    from mrmd_amd.ensemble import Ensemble, cubic_box, replica
+    reps = [replica(n, cubic_box(n, 0.3), 1.0, n) for n in (200, 100)]
+    g = rng(8)
+    e = Ensemble(ctx, reps)
+    e.set_lj(cap=0.7)
+    e.upload(M.POS, [g.uniform(0.0, 1.0, (r["num_atoms"], 3)) * np.asarray(r["box"]) for r in reps])
+    e.run(5, 0)
+    state, pos = e.state(), np.concatenate(e.positions())
+    header, n = 64, 300
+    index = header + n * 32 + 6 * n * 8  # after the positions, three velocities and three forces
+    order = state[index: index + 4 * n].view(np.int32)
+    assert sorted(order.tolist()) == list(range(n))
+    for place in (0, 250):
+        broken = state.copy()
+        broken[index + 4 * place: index + 4 * place + 4] = np.array([bad], np.int32).view(np.uint8)
+        if broken.tobytes() == state.tobytes():
+            continue
+        with pytest.raises(M.MrmdError, match="indices"):
+            e.load_state(broken)
+    np.testing.assert_array_equal(np.concatenate(e.positions()), pos)
+    e.load_state(state)
