@@ -470,14 +470,17 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
         // force kernels' chunk loop needs no bounds test
         const uint32_t pad = uint32_t(sentinelSlot(stagedCap)) << SH;
         const int kept = min(n, cap), nch = (kept + CHUNK - 1) / CHUNK;
-        if (isRow)
+        auto padRow = [&](auto checked) {
             for (int k = kept + sub; k < nch * CHUNK; k += S)
             {
-                if (!GS && k < bufCap)
+                if (!GS && (!decltype(checked)::value || k < bufCap))
                     rowBuf[group * bufCap + k] = uint16_t(pad);
                 else
                     nbr[(Off(k >> 3) * Off(strideS) + Off(s)) * CHUNK + (k & 7)] = uint16_t(pad);
             }
+        };
+        const bool beyond = !GS && __any(n > bufCap);
+        if (isRow) beyond ? padRow(std::true_type{}) : padRow(std::false_type{});
         if (live && sub == 0) cnt[s] = isRow ? kept : 0;  // the true width goes to WIDTH_WORD
         localMax = max(localMax, isRow ? n : 0);
         if constexpr (!GS)
@@ -485,7 +488,7 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
             // the wave's rows go out chunk by chunk, neighbouring rows (mostly neighbouring slots)
             // from neighbouring lanes
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            const int bufCh = isRow ? min(nch, bufCap / CHUNK) : 0;
+            const int bufCh = !isRow ? 0 : beyond ? min(nch, bufCap / CHUNK) : nch;
             const int chunks = RW * waveMaxInt(bufCh);
             for (int x = lane; x - lane < chunks; x += WAVE)
             {
