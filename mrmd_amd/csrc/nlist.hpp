@@ -407,8 +407,9 @@ struct Grid16
 
 // copy the tile's neighbourhood (contiguous runs of sorted slots) into LDS: each wave takes
 // every fourth run, four runs at a time, so that run starts and lengths are wave-uniform
-// (scalar) and a lane has four independent loads in flight; looking up the run of each record
-// instead took a tenth of the force kernel's vector instructions; put(slot, record, run)
+// (scalar; the four loads stand apart from the puts, but the compiler waits for each before it
+// issues the next); looking up the run of each record instead took a tenth of the force kernel's
+// vector instructions; put(slot, record, run)
 template <class Tile, class Put>
 __device__ inline void stageRecords(const Tile& ti, const double4* __restrict__ sortedPos, Put put)
 {

@@ -1,6 +1,6 @@
 """The native time loops where a step's work was enqueued ahead of the wait for the displacement and
 the step rebuilds all the same, which voids it: a cold start with one close pair, whose largest
-displacement grows by more than half from one step to the next, and a skin that the guess keeps
+displacement grows by more than a third from one step to the next, and a skin that the guess keeps
 within and the step exceeds.  Against the same actions called one by one."""
 import numpy as np
 import pytest
