@@ -173,16 +173,18 @@ static_assert(ROW_BUF % CHUNK == 0 && ROW_BUF_MOST % CHUNK == 0);
 // WIDE: list offsets in 64-bit arithmetic (lists of 2^31 entries or more); 32-bit otherwise
 // GS (dense inputs): the 16-bit records in the tile's slice of global memory, entries stored
 // one by one
+// BUF: the row buffers' entries where the compiler knows them (ROW_BUF, the usual case: 1 % faster)
+// or 0 (bufEntries)
 constexpr int BUILD_BLOCK = 12 * WAVE;
 
 // (5 waves per SIMD: 96 registers; with 98 it measured 1.14 instead of 1.06 ms at 4M atoms)
-template <int R, bool WIDE, bool GS>
+template <int R, bool WIDE, bool GS, int BUF>
 __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTiled(const double4* __restrict__ sortedPos,
                                                        const int32_t* __restrict__ sorted,
                                                        const int32_t* __restrict__ offsets,
                                                        const TileInfo* __restrict__ tiles, TileGeom tg, GridD g,
                                                        int64_t rowLo, int64_t rowHi, double rsq, double rn,
-                                                       uint16_t* nbr, int64_t strideS, int cap, int bufCap, int32_t* cnt,
+                                                       uint16_t* nbr, int64_t strideS, int cap, int bufEntries, int32_t* cnt,
                                                        int32_t* slots, int stagedCap, double4* gstage,
                                                        int64_t gstageRecs, double bandLo, double bandHi,
                                                        int8_t* tileSkip)
@@ -190,6 +192,7 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
     constexpr int S = 2 * R + 1;
     constexpr int RW = WAVE / S;  // rows of a wave
     constexpr int SH = entryShift(GS);
+    const int bufCap = BUF > 0 ? BUF : bufEntries;
     extern __shared__ double4 stRaw[];
     __shared__ TileInfo ti;
     __shared__ int wild;
@@ -835,14 +838,16 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
             if (vl->globalStage)
             {
                 if (R == 1)
-                    wide ? launch(k_verletTiled<1, true, true>) : launch(k_verletTiled<1, false, true>);
+                    wide ? launch(k_verletTiled<1, true, true, 0>) : launch(k_verletTiled<1, false, true, 0>);
                 else
-                    wide ? launch(k_verletTiled<2, true, true>) : launch(k_verletTiled<2, false, true>);
+                    wide ? launch(k_verletTiled<2, true, true, 0>) : launch(k_verletTiled<2, false, true, 0>);
             }
-            else if (R == 1)
-                wide ? launch(k_verletTiled<1, true, false>) : launch(k_verletTiled<1, false, false>);
+            else if (wide)
+                R == 1 ? launch(k_verletTiled<1, true, false, 0>) : launch(k_verletTiled<2, true, false, 0>);
+            else if (bufCap == ROW_BUF)
+                R == 1 ? launch(k_verletTiled<1, false, false, ROW_BUF>) : launch(k_verletTiled<2, false, false, ROW_BUF>);
             else
-                wide ? launch(k_verletTiled<2, true, false>) : launch(k_verletTiled<2, false, false>);
+                R == 1 ? launch(k_verletTiled<1, false, false, 0>) : launch(k_verletTiled<2, false, false, 0>);
         }
         checkLaunch();
         int32_t hp[2];
