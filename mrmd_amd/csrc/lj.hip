@@ -154,11 +154,11 @@ __device__ inline void ljQuadTypes(const LJArgs& a, const Pre* tab, int ti0, con
 // GS: the neighbourhood is staged in the tile's slice of the list's global staging buffer
 // (dense inputs whose tiles exceed the LDS) instead of LDS
 // SPLIT: 2^tl.split lanes share a row (small systems, see rowSplit)
-// Bound by vector instruction issue (the vector unit is busy 72 % of the time at 4 million atoms,
+// Bound by vector instruction issue (the vector unit is busy some 70 % of the time at 4 million atoms,
 // the LDS stage area leaves four workgroups a CU to hide the rest): ~27 cycles per list entry, the
 // reciprocal being a quarter-rate instruction.  With records read by two-address LDS reads, run
 // starts looked up per staged record and shuffles in the reductions 441 us at 4 million atoms, in
-// this form 399 to 419.  (Two-type tables without
+// this form 399 to 428.  (Two-type tables without
 // capping, at 260,000 atoms: 80 us with the fours of a chunk in a loop and 124 registers, 70 in a row
 // and 86; their 32-byte records leave LDS for three waves a SIMD.)
 template <bool PRED, bool ONE, bool CAP, bool ASSIGN, bool GS, bool SPLIT>

@@ -184,8 +184,8 @@ __global__ __launch_bounds__(BUILD_BLOCK, R == 1 && !GS ? 5 : 4) void k_verletTi
                                                        const int32_t* __restrict__ offsets,
                                                        const TileInfo* __restrict__ tiles, TileGeom tg, GridD g,
                                                        int64_t rowLo, int64_t rowHi, double rsq, double rn,
-                                                       uint16_t* nbr, int64_t strideS, int cap, int bufEntries, int32_t* cnt,
-                                                       int32_t* slots, int stagedCap, double4* gstage,
+                                                       uint16_t* nbr, int64_t strideS, int cap, int bufEntries,
+                                                       int32_t* cnt, int32_t* slots, int stagedCap, double4* gstage,
                                                        int64_t gstageRecs, double bandLo, double bandHi,
                                                        int8_t* tileSkip)
 {
@@ -753,7 +753,8 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
     // another one).  A shape that had to shrink is where its next build starts (a shape that does not
     // fit costs a launch and a wait), unless the chosen one would now fit at the density of its
     // fullest neighbourhood, which larger neighbourhoods do not exceed.
-    mrmd_verlet_list::TileChoice choice{rows, vl->splitRows, {g.n[0], g.n[1], g.n[2]}, R, vl->stageLimit, regionCells, a, K};
+    mrmd_verlet_list::TileChoice choice{rows, vl->splitRows, {g.n[0], g.n[1], g.n[2]}, R, vl->stageLimit,
+                                        regionCells, a, K};
     const bool sameSystem = choice.sameSystem(vl->tileChoice);
     if (sameSystem)
     {
@@ -762,7 +763,8 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
         K = choice.cells;
     }
     auto cellsAround = [&](int cols, int height) {
-        return double(std::min(cols + 2 * R, g.n[0])) * std::min(cols + 2 * R, g.n[1]) * std::min(height + 2 * R, g.n[2]);
+        return double(std::min(cols + 2 * R, g.n[0])) * std::min(cols + 2 * R, g.n[1]) *
+               std::min(height + 2 * R, g.n[2]);
     };
     if (sameSystem && vl->tileK > 0 &&
         vl->maxStaged * cellsAround(a, K) > vl->stageLimit * cellsAround(vl->tileCols, vl->tileK))
@@ -829,8 +831,8 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
             auto launch = [&](auto kernel) {
                 hipLaunchKernelGGL(kernel, dim3(unsigned(vl->ntiles)), dim3(waves * WAVE), lds, ctx->stream,
                                    vl->bin.sortedPos.p, vl->bin.sorted.p, vl->bin.offsets.p, vl->tiles.p, geom(vl), g,
-                                   begin, end, rn * rn, rn, vl->nbr16.p, vl->strideS, vl->capFull, bufCap, vl->cnt16.p, slots,
-                                   stagedCap, vl->gstage.p, vl->gstageRecs, vl->bandLo, vl->bandHi, vl->tileSkip.p);
+                                   begin, end, rn * rn, rn, vl->nbr16.p, vl->strideS, vl->capFull, bufCap,
+                                   vl->cnt16.p, slots, stagedCap, vl->gstage.p, vl->gstageRecs, vl->bandLo, vl->bandHi, vl->tileSkip.p);
             };
             const bool wide = vl->forceWide || int64_t(vl->capFull) * vl->strideS >= (int64_t(1) << 31);
             // plain block order: measured faster here than the XCD-contiguous order (1.54 against
@@ -845,7 +847,8 @@ bool verletBuild(mrmd_verlet_list* vl, const double4* pos, int64_t nall, int64_t
             else if (wide)
                 R == 1 ? launch(k_verletTiled<1, true, false, 0>) : launch(k_verletTiled<2, true, false, 0>);
             else if (bufCap == ROW_BUF)
-                R == 1 ? launch(k_verletTiled<1, false, false, ROW_BUF>) : launch(k_verletTiled<2, false, false, ROW_BUF>);
+                R == 1 ? launch(k_verletTiled<1, false, false, ROW_BUF>)
+                       : launch(k_verletTiled<2, false, false, ROW_BUF>);
             else
                 R == 1 ? launch(k_verletTiled<1, false, false, 0>) : launch(k_verletTiled<2, false, false, 0>);
         }
