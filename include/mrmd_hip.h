@@ -548,7 +548,8 @@ int mrmd_batch_tf_get(mrmd_batch* b, int64_t replica, int which, double* host, i
  * device), the step counter that keys the Langevin noise, rebuild
  * and density-sample counts, thermodynamic-force and density bins, compensation-energy
  * sums, counts and means.  state_bytes gives the blob's size; save writes it, load reads a
- * blob of the same replicas into an ensemble created with the same replica descriptions.
+ * blob of the same replicas into an ensemble created with the same replica descriptions, and
+ * refuses one whose given indices are not each replica's own atoms, each once.
  * Both end the current list epoch (every replica rebuilds at its next step), so the run
  * that continues after a save and the run restored from it stay bit-identical. */
 int mrmd_batch_state_bytes(const mrmd_batch* b, int64_t* bytes);
